@@ -99,8 +99,9 @@ ACLNN_API aclnnStatus opscvGridSampler2DNoAlloc(const aclTensor* input, const ac
  *   "resize_variant"        OPSCV_RESIZE_VARIANT=generic|register|band   0 automatic, 1 per-element kernels,
  *                                                            2 register-band kernel, 3 no flat LDS kernel
  *   "nearest_variant"       OPSCV_NEAREST_VARIANT=gather     0 automatic, 1 gather from memory
- *   "gs3d_grad_variant"     OPSCV_GS3D_GRAD_VARIANT=ordered|gather   0 automatic, 1 ordered kernel, 2 gather variant
- *                                                            wherever it can run (input gradient of the 3-D sampler)
+ *   "gs3d_grad_variant"     OPSCV_GS3D_GRAD_VARIANT=ordered|gather|sorted   0 automatic, 1 ordered kernel, 2 gather
+ *                                                            variant, 3 sorting variant, wherever it can run (input
+ *                                                            gradient of the 3-D sampler)
  * The last four pick among kernels with identical results (tests and benchmarks use them); the first three can
  * change result bits.  Returns ACLNN_ERR_PARAM_INVALID for an unknown name or a value out of range.
  */

@@ -156,6 +156,9 @@ struct GridSampler3DGradArgs {
     // optional scratch of gs3d_grad_list_words() 32-bit words, 16-byte aligned: cell slots and corner weights of the
     // variant that gathers every voxel's contributions (gs3d_grad_lists.hip); null: the ordered kernel does all items
     void* lists = nullptr;
+    // optional scratch of gs3d_grad_gather_words() 32-bit words, 16-byte aligned: the variant that sorts every voxel's
+    // contributions (gs_grad_gather.hip), which then does all items
+    void* gather = nullptr;
 };
 
 enum class ResizeMode : int {

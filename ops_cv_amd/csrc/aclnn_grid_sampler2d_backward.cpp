@@ -201,7 +201,10 @@ aclnnStatus aclnnGridSampler2DBackwardGetWorkspaceSize(const aclTensor* gradOutp
     }
     if (want_dx) {
         // scratch of the input gradient's list variant (0 words when the shape does not qualify)
-        const int64_t words = gs2d_grad_csr_words(a);
+        int64_t words = gs2d_grad_csr_words(a);
+        if (words == 0) {
+            words = gs2d_grad_gather_words(a);
+        }
         if (words > 0) {
             ex->scratch.in_workspace = true;
             ex->scratch.ws_offset = (ex->workspace_bytes + 255) / 256 * 256;

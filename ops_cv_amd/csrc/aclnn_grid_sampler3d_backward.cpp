@@ -214,9 +214,14 @@ aclnnStatus aclnnGridSampler3DBackwardGetWorkspaceSize(const aclTensor* gradOutp
     if (want_dx) {
         // scratch of the input-gradient kernels: the voxel span of every chunk of grid points, then (from the next
         // 256-byte boundary) the cell slots and corner weights of the gather variant
+        const int64_t gather_words = gs3d_grad_gather_words(a);
         const int64_t range_words = gs3d_grad_range_words(a);
         const int64_t list_words = gs3d_grad_list_words(a);
-        if (range_words > 0 || list_words > 0) {
+        if (gather_words > 0) {
+            ex->scratch.in_workspace = true;
+            ex->scratch.ws_offset = (ex->workspace_bytes + 255) / 256 * 256;
+            ex->workspace_bytes = ex->scratch.ws_offset + (uint64_t)gather_words * 4;
+        } else if (range_words > 0 || list_words > 0) {
             ex->scratch.in_workspace = true;
             ex->scratch.ws_offset = (ex->workspace_bytes + 255) / 256 * 256;
             ex->workspace_bytes = ex->scratch.ws_offset + (list_words > 0 ? gs3d_grad_lists_offset(range_words) +

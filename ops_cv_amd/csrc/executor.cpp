@@ -153,9 +153,10 @@ aclnnStatus execute_plan(void* workspace, const aclOpExecutor* ex, aclrtStream s
         a.dgrid = ex->want_out1 ? resolve(ex->out1, workspace) : nullptr;
         if (ex->scratch.in_workspace) {
             char* scratch = static_cast<char*>(resolve(ex->scratch, workspace));
+            a.gather = gs3d_grad_gather_words(a) > 0 ? scratch : nullptr;
             const int64_t range_words = gs3d_grad_range_words(a);
-            a.chunk_ranges = range_words > 0 ? scratch : nullptr;
-            a.lists = gs3d_grad_list_words(a) > 0 ? scratch + gs3d_grad_lists_offset(range_words) : nullptr;
+            a.chunk_ranges = (range_words > 0 && a.gather == nullptr) ? scratch : nullptr;
+            a.lists = (a.gather == nullptr && gs3d_grad_list_words(a) > 0) ? scratch + gs3d_grad_lists_offset(range_words) : nullptr;
         }
         if (a.gout == nullptr || a.x == nullptr || a.grid == nullptr || (ex->want_out0 && a.dx == nullptr) ||
             (ex->want_out1 && a.dgrid == nullptr)) {

@@ -99,16 +99,20 @@ const char* opscvExecutorVariant(const aclOpExecutor* executor)
         case OpKind::GridSampler2DGrad:
             // the grid gradient has a variant that stages the input planes through LDS
         {
-            // input gradient: elections or lists; grid gradient: one lane per point or the LDS-ring variant
-            const bool lists = executor->want_out0 && executor->scratch.in_workspace;
+            // input gradient: stored lists, or the contributions put in order call by call (elections, or for larger
+            // planes sorting); grid gradient: one lane per point or the LDS-ring variant
+            const bool lists = executor->want_out0 && gs2d_grad_csr_words(executor->gsg) > 0;
             const bool rings = executor->want_out1 && gs2d_grad_grid_uses_lds(executor->gsg);
             return lists ? (rings ? "gs2d_grad_lists_lds" : "gs2d_grad_lists")
                          : (rings ? "gs2d_grad_ordered_lds" : "gs2d_grad_ordered");
         }
         case OpKind::GridSampler3DGrad:
-            // input gradient: a gather over every voxel's contributions, or elections in their order
-            return (executor->want_out0 && gs3d_grad_list_words(executor->gsg3) > 0) ? "gs3d_grad_lists"
-                                                                                      : "gs3d_grad_ordered";
+            // input gradient: cell slots and a gather over every voxel's contributions, or these put in order (elections,
+            // or for larger grids and volumes sorting)
+            return (executor->want_out0 && gs3d_grad_gather_words(executor->gsg3) == 0 &&
+                    gs3d_grad_list_words(executor->gsg3) > 0)
+                       ? "gs3d_grad_lists"
+                       : "gs3d_grad_ordered";
         case OpKind::GridSampler3D:
             if (executor->gs3.channels_last) {
                 return executor->gs3.interp == 0 ? "gs3d_ndhwc_bilinear" : "gs3d_ndhwc_nearest";
@@ -159,7 +163,7 @@ int32_t opscvVariantRevision(const char* variant)
         {"nchw_band_lds", 1},  {"nchw_flat_lds", 1},    {"nchw_band", 1},       {"nchw_generic", 1},
         {"nhwc_", 1},          {"nearest_", 1},         {"copy", 1},            {"point_copy", 1},
         {"broadcast", 1},      {"first_pixel", 1},      {"resize_grad", 1},     {"gs2d_grad", 4},
-        {"gs3d_grad", 1},      {"gs3d_", 1},
+        {"gs2d_grad_ordered", 5}, {"gs3d_grad", 1}, {"gs3d_grad_ordered", 2},      {"gs3d_", 1},
     };
     if (variant == nullptr) {
         return 0;

@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "gs2d_grad_math.hpp"
+#include "gs_grad_gather.hpp"
 #include "kernels.hpp"
 
 namespace opscv {
@@ -366,6 +367,26 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __res
     ElemIO<T>::store(dgrid + 2 * idx + 1, as_fp32_value(tp.my * giy));
 }
 
+GradGatherArgs gather_args(const GridSamplerGradArgs& a)
+{
+    GradGatherArgs g;
+    g.elem = a.elem;
+    g.dim = 2;
+    g.interp = a.interp;
+    g.pad = a.pad;
+    g.align = a.align;
+    g.N = a.N;
+    g.C = a.C;
+    g.H = a.Hin;
+    g.W = a.Win;
+    g.points = a.Hout * a.Wout;
+    g.gout = a.gout;
+    g.grid = a.grid;
+    g.dx = a.dx;
+    g.scratch = a.scratch;
+    return g;
+}
+
 template <typename T, int INTERP>
 hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
 {
@@ -406,6 +427,13 @@ hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
                 return e;
             }
         }
+    }
+    if (a.dx != nullptr && !dx_done && a.scratch != nullptr && gs2d_grad_gather_words(a) > 0) {
+        const hipError_t e = run_grad_gather(gather_args(a), stream);
+        if (e != hipSuccess) {
+            return e;
+        }
+        dx_done = true;
     }
     if (a.dx != nullptr && !dx_done) {
         const int64_t bands = (plane_px + p.band_px - 1) / p.band_px;
@@ -467,6 +495,21 @@ hipError_t launch_typed(const GridSamplerGradArgs& a, hipStream_t stream)
 }
 
 }  // namespace
+
+int64_t gs2d_grad_gather_words(const GridSamplerGradArgs& a)
+{
+    if (gs2d_grad_csr_words(a) > 0) {
+        return 0;
+    }
+    // The elections take about 3 us per chunk of 256 grid points (bilinear; 1.2 us nearest, 6 us bicubic) and once more
+    // for every turn of bands over the chip, the sorting variant 20 us (bicubic 40) at the least.  Device time of a call
+    // with both gradients, elections / sorting, fp32 N1 C3: bilinear 4 chunks 17 / 20 us, 9 chunks 32 / 22, 64 chunks
+    // 126 / 23; nearest 9 chunks 13 / 19, 16 chunks 21 / 19; bicubic 1 chunk 24 / 36, 3 chunks 50 / 41, 9 chunks
+    // 135 / 45.  From 24 tap passes over a chunk on the sorting variant is taken.
+    const int64_t chunks = (a.Hout * a.Wout + kThreads - 1) / kThreads;
+    const int64_t taps = (a.interp == 0) ? 4 : ((a.interp == 1) ? 1 : 16);
+    return chunks * taps > 24 ? grad_gather_words(gather_args(a)) : 0;
+}
 
 hipError_t launch_grid_sampler2d_grad(const GridSamplerGradArgs& a, hipStream_t stream)
 {

@@ -23,7 +23,9 @@
 
 #include "gs2d_grad_math.hpp"
 #include "gs3d_grad_math.hpp"
+#include "gs_grad_gather.hpp"
 #include "kernels.hpp"
+#include "options.hpp"
 
 namespace opscv {
 
@@ -319,6 +321,28 @@ int64_t band_voxels(const GridSampler3DGradArgs& a)
     return vol < band ? vol : band;
 }
 
+GradGatherArgs gather_args(const GridSampler3DGradArgs& a)
+{
+    GradGatherArgs g;
+    g.elem = a.elem;
+    g.dim = 3;
+    g.interp = a.interp;
+    g.pad = a.pad;
+    g.align = a.align;
+    g.N = a.N;
+    g.C = a.C;
+    g.D = a.Din;
+    g.H = a.Hin;
+    g.W = a.Win;
+    g.points = a.Dout * a.Hout * a.Wout;
+    g.items_per_core = a.items_per_core;
+    g.gout = a.gout;
+    g.grid = a.grid;
+    g.dx = a.dx;
+    g.scratch = a.gather;
+    return g;
+}
+
 template <typename T, int INTERP>
 hipError_t launch_interp(const GridSampler3DGradArgs& a, hipStream_t stream)
 {
@@ -340,7 +364,12 @@ hipError_t launch_interp(const GridSampler3DGradArgs& a, hipStream_t stream)
         p.tags *= 2;
     }
     bool dgrid_done = false;  // the gather variant's first kernel computes the grid gradient on its way
-    if (a.dx != nullptr) {
+    if (a.dx != nullptr && a.gather != nullptr && gs3d_grad_gather_words(a) > 0) {
+        const hipError_t e = run_grad_gather(gather_args(a), stream);
+        if (e != hipSuccess) {
+            return e;
+        }
+    } else if (a.dx != nullptr) {
         const int64_t bands = (vol + p.band_px - 1) / p.band_px;
         // 8 bytes of gradient per band voxel: 4 channels of a 16-bit type, 2 of fp32 (96 KB of LDS with the election
         // tags); fewer channels than that run one per workgroup
@@ -435,6 +464,42 @@ int64_t gs3d_grad_range_words(const GridSampler3DGradArgs& a)
     }
     const int64_t per_core = a.items_per_core > 0 ? a.items_per_core : 1;
     return a.N * 2 * (int64_t)chunk_count(a.Dout * a.Hout * a.Wout, per_core);
+}
+
+int64_t gs3d_grad_gather_words(const GridSampler3DGradArgs& a)
+{
+    if (a.force_variant == kGs3dGradSorted) {
+        return grad_gather_words(gather_args(a));
+    }
+    if (a.force_variant != kGs3dGradAuto) {
+        return 0;
+    }
+    const int64_t points = a.Dout * a.Hout * a.Wout, vol = a.Din * a.Hin * a.Win;
+    // Device time of a call with both gradients, fp16 or fp32, four channels: ordered kernel / slots / sorting variant.
+    // Volumes sampled at few points: the sorting variant visits every voxel, the ordered kernel every chunk of points
+    // (vol : points 22 : 1 with 46080 points 77 / - / 71 us, 32 : 1 with 8192 points 60 / - / 95, 128 : 1 with 16384
+    // points 67 / - / 102; 16 : 1 with 16384 points 39 / - / 34).  Beyond 65536 points the slots kernels do not run and a chunk of the ordered kernel costs
+    // the same for every band (2 x 64x128x128 from 81920 points 125 / - / 76, 8 x 32x64x64 one to one 362 / - / 119).
+    if (points <= 65536 && (vol > 16 * points || (vol > 8 * points && points <= 32 * kChunkPoints3))) {
+        return 0;
+    }
+    if (a.interp == 1) {
+        // 16 chunks: 21 / - / 20 us, 8 chunks 15 / - / 20, 256 chunks 99 / - / 36
+        return points > 16 * kChunkPoints3 ? grad_gather_words(gather_args(a)) : 0;
+    }
+    if (gs3d_grad_list_words(a) > 0) {
+        // Border and reflection padding gather points on the faces; an item with a crowded voxel is left by the slots
+        // kernels to the ordered kernel (4 x 16x32x32 border: 17 us without such an item, 214 with one, sorting variant
+        // 55; 8 x 16x40x40 307 / 72).  Smaller grids seldom have one and cost half as much in slots (19 / 35 us).
+        const bool piles = a.pad != 0 && points >= 8192;
+        // the slots kernels keep an item on one XCD: one or two large items leave most of the chip idle (one item of
+        // 65536 points: 39 / 30 us, with 16 channels 94 / 42; two items 41 / 37; four 39 / 45; one of 36864 27 / 30)
+        const bool few_items = a.N <= 2 && points >= 49152;
+        if (!piles && !few_items) {
+            return 0;
+        }
+    }
+    return grad_gather_words(gather_args(a));
 }
 
 hipError_t launch_grid_sampler3d_grad(const GridSampler3DGradArgs& a, hipStream_t stream)

@@ -1,0 +1,956 @@
+// Backward of the grid samplers for gfx950: gradient of the input as a gather over lists of contributions, for planes
+// and volumes of any size, every interpolation mode and any number of grid points.
+//
+// The sum that reaches an element of the gradient is a fixed sequence (gs2d_grad.hip, gs3d_grad.hip): its contributions
+// ordered by (chunk of 256 grid points, tap, point), every add rounded to the element type.  The kernels there walk the
+// chunks in order and elect, round after round, who may add to an element; every band of a plane looks at every chunk,
+// so their time grows with points times plane elements.  Here the order is restored per element by sorting:
+//
+//   clear   the counts of every cell
+//   count   one lane per grid point: an atomic count per cell gives the point its rank in the cell (which rank depends
+//           on timing, which points a cell holds does not); the source coordinates go to scratch
+//   place   one lane per four cells: every cell gets a run of the item's list (a prefix sum per workgroup, one atomic
+//           add per workgroup for its base: the order of the runs does not matter)
+//   fill    one lane per grid point: the point's entry goes to its run
+//   gather  one lane per element: the element collects the entries of the cells it is a corner of -- cell (y - ys,
+//           x - xs) holds the points it is corner (ys, xs) of -- keyed (chunk, tap, point), sorts up to 16 or 32 of them in
+//           registers and folds gradOutput times weight in that order with the reference's roundings, every channel
+//           from the same list.  Elements with more contributions (border padding piles points up on the edges) go to a
+//           list of their own; meanwhile spare workgroups sort the runs of more than 64 entries.
+//   crowded one wavefront per listed element: merges the element's runs, 64 entries at a time, in the reference's
+//           order; the lanes compute the 64 contributions of a channel at once and one lane adds them up in order.
+//
+// Input gradient of fp32 8x3x479x637 from as many grid points (rotations of up to 30 degrees): 2568 us with elections;
+// here clear 6, count 43, place 14, fill 13, gather 107, crowded 5 us.  Count is bound by the rate of atomics (55 G/s;
+// four points per lane in flight or one, no difference), gather by the loads it issues per element (about fifty per
+// wavefront: two starts, two counts, two entries per cell, then coordinates and gradOutput per contribution) beside the
+// sorting network's instructions: twice the wavefronts in flight (lists of 16 instead of 32) leave its time as it is.
+//
+// A cell is an element of the lattice of low corners for linear interpolation (one entry per point, 2^DIM runs per
+// element), and the element itself for nearest (one entry per point) and bicubic (sixteen entries per point: padding
+// is applied tap by tap, so a tap's element does not follow from the point's cell).
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "gs2d_grad_math.hpp"
+#include "gs3d_grad_math.hpp"
+#include "gs_grad_gather.hpp"
+#include "kernels.hpp"
+
+namespace opscv {
+
+namespace {
+
+constexpr int kThreads = 256;
+constexpr int kListMost = 32;        // contributions of an element that the gather kernel takes at most
+constexpr uint32_t kSortedRun = 64;  // runs of more entries are sorted in place before the crowded kernel reads them
+constexpr int kPlaceCells = 8;       // cells per lane of the place kernel
+constexpr int kPlaceThreads = 256;
+constexpr int kFoldChans = 16;       // channels whose contributions a crowded element's wavefront computes together
+constexpr int kCtrlWords = 16;       // [0] entries handed out, [1] long runs, [2] crowded elements
+constexpr uint32_t kNoRank = 0xFFFFFFFFu;
+
+struct GatherLayout {  // offsets in 32-bit words within an item's scratch
+    uint32_t counts;   // behind the control words: cleared together with them
+    uint32_t starts;
+    uint32_t ranks;    // [entry of a point][point]
+    uint32_t coords;   // source coordinates of the points: 2 (4 for volumes) values of the element type
+    uint32_t list;     // entries, run after run
+    uint32_t runs;     // cells whose run has more than kSortedRun entries
+    uint32_t crowded;  // elements with more contributions than their list holds
+    uint32_t item_words;
+};
+
+struct GatherParams {
+    int32_t C, D, H, W, points;
+    int32_t pad, align;
+    int32_t items_per_core;
+    int32_t elements, cells;
+    int32_t N;
+    GatherLayout lay;
+};
+
+// Grid points per lane of the count and fill kernels: the atomics and the scattered stores of several are on their way
+// together.
+template <int DIM, int INTERP>
+constexpr int points_per_lane()
+{
+    return (INTERP == 2) ? 1 : 4;
+}
+
+// What depends on the mode: runs an element merges, entries a point makes, how an entry and a run make a sorting key
+// (ascending keys are the reference's order) and back.  An entry is q = point + phase of the item's first chunk, with
+// the tap between chunk and point for bicubic.
+template <int DIM, int INTERP>
+struct Mode {
+    static constexpr int kRuns = (INTERP == 0) ? (1 << DIM) : 1;
+    static constexpr int kEntries = (INTERP == 2) ? 16 : 1;
+    static constexpr int kTapBits = (INTERP == 0) ? DIM : ((INTERP == 2) ? 4 : 0);
+    static __device__ __forceinline__ uint32_t key(uint32_t entry, uint32_t run)
+    {
+        return (INTERP == 0) ? ((entry >> 8) << (8 + DIM)) | (run << 8) | (entry & 255u) : entry;
+    }
+    static __device__ __forceinline__ uint32_t entry(uint32_t q, uint32_t tap)
+    {
+        return (INTERP == 2) ? ((q >> 8) << 12) | (tap << 8) | (q & 255u) : q;
+    }
+    static __device__ __forceinline__ uint32_t tap_of(uint32_t key)
+    {
+        return (kTapBits > 0) ? (key >> 8) & ((1u << kTapBits) - 1u) : 0u;
+    }
+    static __device__ __forceinline__ uint32_t q_of(uint32_t key)
+    {
+        return (kTapBits > 0) ? ((key >> (8 + kTapBits)) << 8) | (key & 255u) : key;
+    }
+};
+
+// source coordinates of a point as they lie in scratch
+template <typename T, int DIM>
+struct Coords {
+    T v[DIM == 3 ? 4 : 2];
+};
+
+__device__ __forceinline__ int32_t phase_of(int64_t n, const GatherParams& p)
+{
+    return (int32_t)(((n % p.items_per_core) * (int64_t)p.points) % kChunkPoints3);
+}
+
+// The source coordinates of a grid point, as the tap decisions of gs2d_grad_math.hpp and gs3d_grad_math.hpp form them
+// (values of the element type).
+template <typename T, int DIM, int INTERP>
+__device__ __forceinline__ Coords<T, DIM> coords_of(const T* __restrict__ g, const GatherParams& p)
+{
+    Coords<T, DIM> c;
+    float m;
+    auto axis = [&](int i, int32_t size) {
+        const float v = ElemIO<T>::load(g + i);
+        const float f = (INTERP == 2) ? unnormalize_set_grad<T>(v, size, p.align, &m)
+                                      : source_index_set_grad<T>(v, size, p.pad, p.align, &m);
+        ElemIO<T>::store(&c.v[i], f);
+    };
+    axis(0, p.W);
+    axis(1, p.H);
+    if constexpr (DIM == 3) {
+        axis(2, p.D);
+        c.v[3] = c.v[2];
+    }
+    return c;
+}
+
+// Calls f(entry number, tap, cell) for every entry that the point makes.
+template <typename T, int DIM, int INTERP, typename F>
+__device__ __forceinline__ void for_entries(const Coords<T, DIM>& c, const GatherParams& p, F&& f)
+{
+    const float fx = ElemIO<T>::load(&c.v[0]), fy = ElemIO<T>::load(&c.v[1]);
+    if constexpr (INTERP == 2) {
+        const float xf = __builtin_floorf(fx), yf = __builtin_floorf(fy);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int32_t off = bicubic_bounded_offset(xf - 1.0f + (float)i, yf - 1.0f + (float)j, p.W, p.H, p.pad,
+                                                           p.align);
+                f(i * 4 + j, off);
+            }
+        }
+    } else if constexpr (INTERP == 1) {
+        const int32_t x = float_to_i32(__builtin_rintf(fx)), y = float_to_i32(__builtin_rintf(fy));
+        int32_t z = 0;
+        if constexpr (DIM == 3) {
+            z = float_to_i32(__builtin_rintf(ElemIO<T>::load(&c.v[2])));
+        }
+        const bool in = (uint32_t)x < (uint32_t)p.W && (uint32_t)y < (uint32_t)p.H && (uint32_t)z < (uint32_t)p.D;
+        f(0, in ? (z * p.H + y) * p.W + x : -1);
+    } else {
+        const int32_t x = float_to_i32(__builtin_floorf(fx)), y = float_to_i32(__builtin_floorf(fy));
+        int32_t z = -1;
+        if constexpr (DIM == 3) {
+            z = float_to_i32(__builtin_floorf(ElemIO<T>::load(&c.v[2])));
+        }
+        // a point none of whose corners is inside has no cell
+        const bool in = x >= -1 && x < p.W && y >= -1 && y < p.H && z >= -1 && z < p.D;
+        f(0, in ? ((z + 1) * (p.H + 1) + (y + 1)) * (p.W + 1) + (x + 1) : -1);
+    }
+}
+
+// The weight of a contribution (unused for nearest): the products of gs2d_grad_math.hpp / gs3d_grad_math.hpp.
+template <typename T, int DIM, int INTERP>
+__device__ __forceinline__ float weight_of(const Coords<T, DIM>& c, uint32_t tap, int32_t x, int32_t y, int32_t z)
+{
+    const float fx = ElemIO<T>::load(&c.v[0]), fy = ElemIO<T>::load(&c.v[1]);
+    if constexpr (INTERP == 1) {
+        return 1.0f;
+    } else if constexpr (INTERP == 2) {
+        auto coefficient = [](uint32_t i, float t) {
+            // the i-th of cubic_coefficients()
+            const float u = (i >= 2) ? 1.0f - t : t;
+            const float outer = cubic_convolution2((i == 0) ? t + 1.0f : 2.0f - t, -0.75f);
+            const float inner = cubic_convolution1(u, -0.75f);
+            return (i == 0 || i == 3) ? outer : inner;
+        };
+        return coefficient(tap >> 2, fx - __builtin_floorf(fx)) * coefficient(tap & 3u, fy - __builtin_floorf(fy));
+    } else {
+        // corner (xs, ys, zs) of the cell is element (x, y, z): the low corner is that much below it
+        const bool xs = tap & 1u, ys = tap & 2u, zs = tap & 4u;
+        const float wx = xs ? fx - (float)(x - 1) : (float)(x + 1) - fx;
+        const float wy = ys ? fy - (float)(y - 1) : (float)(y + 1) - fy;
+        if constexpr (DIM == 3) {
+            const float fz = ElemIO<T>::load(&c.v[2]);
+            const float wz = zs ? fz - (float)(z - 1) : (float)(z + 1) - fz;
+            return rt<T>(as_fp32_value(wx * wy * wz));
+        } else {
+            return rt<T>(as_fp32_value(wx * wy));
+        }
+    }
+}
+
+// One more contribution, added with the reference's roundings (contribution() of gs2d_grad.hip, contribution3()).
+template <typename T, int INTERP>
+__device__ __forceinline__ float value_of(float go, float w)
+{
+    return (INTERP == 1) ? rt<T>(go) : rt<T>(as_fp32_value(w * go));
+}
+
+// Work of a launch cut into `per_item` pieces per batch item, dealt out so that neighbouring pieces run on one XCD
+// (workgroups go to the eight XCDs in turn): XCD k takes the k-th eighth of all pieces.  Pieces beyond the last: false.
+__device__ __forceinline__ bool piece_of_block(uint32_t block, uint32_t pieces, uint32_t per_item, uint32_t* n,
+                                               uint32_t* local)
+{
+    const uint32_t per_xcd = (pieces + 7u) >> 3;
+    const uint32_t piece = (block & 7u) * per_xcd + (block >> 3);
+    *n = piece / per_item;
+    *local = piece - *n * per_item;
+    return (block >> 3) < per_xcd && piece < pieces;
+}
+
+__global__ __launch_bounds__(kThreads) void gs_gather_clear_kernel(uint32_t* __restrict__ ws, uint32_t words,
+                                                                    uint32_t item_words)
+{
+    uint32_t* wsn = ws + (size_t)blockIdx.y * item_words;
+    const uint32_t i = (blockIdx.x * kThreads + threadIdx.x) * 4u;
+    if (i < words) {  // whole units: the words behind the counts are written later anyway
+        *reinterpret_cast<uint4*>(wsn + i) = make_uint4(0u, 0u, 0u, 0u);
+    }
+}
+
+template <typename T, int DIM, int INTERP>
+__global__ __launch_bounds__(kThreads) void gs_gather_count_kernel(const T* __restrict__ grid, uint32_t* __restrict__ ws,
+                                                                    GatherParams p, uint32_t pieces, uint32_t per_item)
+{
+    constexpr int PPL = points_per_lane<DIM, INTERP>();
+    constexpr int NE = Mode<DIM, INTERP>::kEntries;
+    uint32_t n, local;
+    if (!piece_of_block(blockIdx.x, pieces, per_item, &n, &local)) {
+        return;
+    }
+    const int32_t first = (int32_t)(local * kThreads * PPL + threadIdx.x);
+    uint32_t* wsn = ws + (size_t)n * p.lay.item_words;
+    Coords<T, DIM> c[PPL];
+#pragma unroll
+    for (int u = 0; u < PPL; u++) {
+        const int32_t pt = first + u * kThreads;
+        c[u] = coords_of<T, DIM, INTERP>(grid + ((int64_t)n * p.points + (pt < p.points ? pt : 0)) * DIM, p);
+    }
+    uint32_t rank[PPL][NE];
+#pragma unroll
+    for (int u = 0; u < PPL; u++) {
+        const bool have = first + u * kThreads < p.points;
+        for_entries<T, DIM, INTERP>(c[u], p, [&](int i, int32_t cell) {
+            rank[u][i] = (have && cell >= 0) ? atomicAdd(&wsn[p.lay.counts + cell], 1u) : kNoRank;
+        });
+    }
+#pragma unroll
+    for (int u = 0; u < PPL; u++) {
+        const int32_t pt = first + u * kThreads;
+        if (pt < p.points) {
+            reinterpret_cast<Coords<T, DIM>*>(wsn + p.lay.coords)[pt] = c[u];
+#pragma unroll
+            for (int i = 0; i < NE; i++) {
+                wsn[p.lay.ranks + (size_t)i * p.points + pt] = rank[u][i];
+            }
+        }
+    }
+}
+
+__global__ __launch_bounds__(kPlaceThreads) void gs_gather_place_kernel(uint32_t* __restrict__ ws, GatherParams p)
+{
+    __shared__ uint32_t s_sum[kPlaceThreads / 64];
+    __shared__ uint32_t s_base;
+    uint32_t* wsn = ws + (size_t)blockIdx.y * p.lay.item_words;
+    const int t = threadIdx.x;
+    const int32_t first = (int32_t)((blockIdx.x * kPlaceThreads + t) * kPlaceCells);
+    uint32_t cnt[kPlaceCells], sum = 0;
+#pragma unroll
+    for (int i = 0; i < kPlaceCells; i++) {
+        cnt[i] = (first + i < p.cells) ? wsn[p.lay.counts + first + i] : 0u;
+        sum += cnt[i];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t up = __shfl_up(incl, d);
+        incl += ((t & 63) >= d) ? up : 0u;
+    }
+    if ((t & 63) == 63) {
+        s_sum[t >> 6] = incl;
+    }
+    __syncthreads();
+    if (t == 0) {
+        uint32_t total = 0;
+        for (int w = 0; w < kPlaceThreads / 64; w++) {
+            const uint32_t s = s_sum[w];
+            s_sum[w] = total;
+            total += s;
+        }
+        s_base = atomicAdd(&wsn[0], total);
+    }
+    __syncthreads();
+    uint32_t at = s_base + s_sum[t >> 6] + incl - sum;
+#pragma unroll
+    for (int i = 0; i < kPlaceCells; i++) {
+        if (first + i < p.cells) {
+            wsn[p.lay.starts + first + i] = at;
+            at += cnt[i];
+            if (cnt[i] > kSortedRun) {
+                wsn[p.lay.runs + atomicAdd(&wsn[1], 1u)] = (uint32_t)(first + i);
+            }
+        }
+    }
+}
+
+template <typename T, int DIM, int INTERP>
+__global__ __launch_bounds__(kThreads) void gs_gather_fill_kernel(uint32_t* __restrict__ ws, GatherParams p,
+                                                                   uint32_t pieces, uint32_t per_item)
+{
+    constexpr int PPL = points_per_lane<DIM, INTERP>();
+    constexpr int NE = Mode<DIM, INTERP>::kEntries;
+    uint32_t n, local;
+    if (!piece_of_block(blockIdx.x, pieces, per_item, &n, &local)) {
+        return;
+    }
+    const int32_t first = (int32_t)(local * kThreads * PPL + threadIdx.x);
+    uint32_t* wsn = ws + (size_t)n * p.lay.item_words;
+    Coords<T, DIM> c[PPL];
+    uint32_t rank[PPL][NE];
+#pragma unroll
+    for (int u = 0; u < PPL; u++) {
+        const int32_t pt = first + u * kThreads < p.points ? first + u * kThreads : 0;
+        c[u] = reinterpret_cast<const Coords<T, DIM>*>(wsn + p.lay.coords)[pt];
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            rank[u][i] = wsn[p.lay.ranks + (size_t)i * p.points + pt];
+        }
+    }
+    uint32_t start[PPL][NE];
+#pragma unroll
+    for (int u = 0; u < PPL; u++) {
+        for_entries<T, DIM, INTERP>(c[u], p, [&](int i, int32_t cell) {
+            start[u][i] = wsn[p.lay.starts + (cell >= 0 ? cell : 0)];
+        });
+    }
+    const uint32_t phase = (uint32_t)phase_of(n, p);
+#pragma unroll
+    for (int u = 0; u < PPL; u++) {
+        const int32_t pt = first + u * kThreads;
+#pragma unroll
+        for (int i = 0; i < NE; i++) {
+            if (pt < p.points && rank[u][i] != kNoRank) {
+                wsn[p.lay.list + start[u][i] + rank[u][i]] = Mode<DIM, INTERP>::entry((uint32_t)pt + phase, (uint32_t)i);
+            }
+        }
+    }
+}
+
+// Sorts one run (ascending entries, all distinct) into `out` with all threads of the workgroup: a bitmap of the entries
+// that lie in a window of values, then every thread writes out the entries of its words behind those of the threads
+// before it.  A run costs a pass over it per window of 32 * kBitWords values that it spans.
+template <int kBitWords>
+__device__ __forceinline__ void sort_run(const uint32_t* run, uint32_t len, uint32_t* out, uint32_t* bits,
+                                         uint32_t* s_part)
+{
+    const int t = threadIdx.x;
+    uint32_t lo = 0xFFFFFFFFu, hi = 0u;
+    for (uint32_t i = t; i < len; i += kThreads) {
+        const uint32_t v = run[i];
+        lo = v < lo ? v : lo;
+        hi = v > hi ? v : hi;
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        const uint32_t olo = __shfl_xor(lo, d), ohi = __shfl_xor(hi, d);
+        lo = olo < lo ? olo : lo;
+        hi = ohi > hi ? ohi : hi;
+    }
+    __syncthreads();  // the bitmap and s_part of the run before this one are done with
+    if ((t & 63) == 0) {
+        s_part[t >> 6] = lo;
+        s_part[4 + (t >> 6)] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kThreads / 64; w++) {
+        lo = s_part[w] < lo ? s_part[w] : lo;
+        hi = s_part[4 + w] > hi ? s_part[4 + w] : hi;
+    }
+    uint32_t done = 0;
+    while (done < len && lo <= hi) {  // lo: the first value of this window; every entry below it is written
+        const uint32_t left = (hi - lo) / 32u + 1u;
+        const uint32_t words = left < (uint32_t)kBitWords ? left : (uint32_t)kBitWords;
+        const uint32_t each = (words + kThreads - 1u) / kThreads;
+        for (uint32_t i = t; i < each * kThreads; i += kThreads) {
+            bits[i] = 0u;
+        }
+        __syncthreads();
+        for (uint32_t i = t; i < len; i += kThreads) {
+            const uint32_t v = run[i] - lo;  // entries of earlier windows wrap round to huge values
+            if (v < words * 32u) {
+                atomicOr(&bits[v >> 5], 1u << (v & 31u));
+            }
+        }
+        __syncthreads();
+        uint32_t mine = 0;
+        for (uint32_t i = 0; i < each; i++) {
+            mine += (uint32_t)__builtin_popcount(bits[t * each + i]);
+        }
+        uint32_t incl = mine;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t up = __shfl_up(incl, d);
+            incl += ((t & 63) >= d) ? up : 0u;
+        }
+        if ((t & 63) == 63) {
+            s_part[t >> 6] = incl;
+        }
+        __syncthreads();
+        uint32_t at = done + incl - mine;
+        uint32_t total = 0;
+#pragma unroll
+        for (int w = 0; w < kThreads / 64; w++) {
+            at += (w < (t >> 6)) ? s_part[w] : 0u;
+            total += s_part[w];
+        }
+        for (uint32_t i = 0; i < each; i++) {
+            uint32_t b = bits[t * each + i];
+            while (b != 0u) {
+                out[at++] = lo + (t * each + i) * 32u + (uint32_t)__builtin_ctz(b);
+                b &= b - 1u;
+            }
+        }
+        done += total;
+        lo += words * 32u;
+        __syncthreads();
+    }
+}
+
+// The first NK entries of a lane's list (every kThreads-th word from `mine`), sorted ascending through registers.
+template <int NK>
+__device__ __forceinline__ void sort_list(uint32_t* mine, uint32_t len)
+{
+    uint32_t key[NK];
+#pragma unroll
+    for (int i = 0; i < NK; i++) {
+        const uint32_t v = mine[i * kThreads];
+        key[i] = ((uint32_t)i < len) ? v : 0xFFFFFFFFu;
+    }
+#pragma unroll
+    for (int size = 2; size <= NK; size *= 2) {
+#pragma unroll
+        for (int stride = size / 2; stride > 0; stride /= 2) {
+#pragma unroll
+            for (int i = 0; i < NK; i++) {
+                const int l = i ^ stride;
+                if (l > i) {
+                    const uint32_t lo = key[i] < key[l] ? key[i] : key[l];
+                    const uint32_t hi = key[i] < key[l] ? key[l] : key[i];
+                    const bool ascending = (i & size) == 0;
+                    key[i] = ascending ? lo : hi;
+                    key[l] = ascending ? hi : lo;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < NK; i++) {
+        mine[i * kThreads] = key[i];
+    }
+}
+
+// The run (start, length) of each cell that element (x, y, z) is a corner of, in corner order.
+template <int DIM, int INTERP>
+__device__ __forceinline__ void runs_of(const uint32_t* __restrict__ wsn, const GatherParams& p, int32_t e, int32_t x,
+                                        int32_t y, int32_t z, uint32_t* start, uint32_t* count)
+{
+    constexpr int R = Mode<DIM, INTERP>::kRuns;
+    const uint32_t* starts = wsn + p.lay.starts;
+    const uint32_t* counts = wsn + p.lay.counts;
+    if constexpr (R == 1) {
+        start[0] = starts[e];
+        count[0] = counts[e];
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r += 2) {
+            const int ys = (r >> 1) & 1, zs = r >> 2;
+            const int32_t row = (DIM == 3) ? (z + 1 - zs) * (p.H + 1) + (y + 1 - ys) : y + 1 - ys;
+            const int32_t cell = row * (p.W + 1) + x;  // the cell of corner xs = 1; the next one is that of xs = 0
+            uint2 s, c;
+            __builtin_memcpy(&s, starts + cell, 8);
+            __builtin_memcpy(&c, counts + cell, 8);
+            start[r] = s.y;
+            start[r + 1] = s.x;
+            count[r] = c.y;
+            count[r + 1] = c.x;
+        }
+    }
+}
+
+// LIST: contributions an element's list can hold (16 or 32).
+template <typename T, int DIM, int INTERP, int CB, int LIST>
+__global__ __launch_bounds__(kThreads) void gs_gather_kernel(const T* __restrict__ gout, T* __restrict__ dx,
+                                                              uint32_t* __restrict__ ws, GatherParams p, uint32_t pieces,
+                                                              uint32_t gather_blocks, uint32_t tiles,
+                                                              int32_t chans_per_block, uint32_t sorters)
+{
+    typedef Mode<DIM, INTERP> M;
+    constexpr int R = M::kRuns;
+    constexpr int kBitWords = LIST * kThreads;  // the list memory, and the bitmap of a workgroup that sorts runs
+    __shared__ uint32_t list[kBitWords];  // entry i of lane t at [i * kThreads + t]: a bank of its own
+    __shared__ uint32_t s_part[2 * kThreads / 64];
+    const int t = threadIdx.x;
+    if (blockIdx.x >= gather_blocks) {
+        // a spare workgroup: sorts long runs (of elements that the lanes below leave to the crowded kernel)
+        const uint32_t i = blockIdx.x - gather_blocks;
+        uint32_t* wsn = ws + (size_t)(i / sorters) * p.lay.item_words;
+        const uint32_t runs = wsn[1];
+        for (uint32_t r = i % sorters; r < runs; r += sorters) {
+            const uint32_t cell = wsn[p.lay.runs + r];
+            const uint32_t start = wsn[p.lay.starts + cell];
+            sort_run<kBitWords>(wsn + p.lay.list + start, wsn[p.lay.counts + cell], wsn + p.lay.ranks + start, list, s_part);
+        }
+        return;
+    }
+    uint32_t n, local;
+    if (!piece_of_block(blockIdx.x, pieces, pieces / (uint32_t)p.N, &n, &local)) {
+        return;
+    }
+    uint32_t* wsn = ws + (size_t)n * p.lay.item_words;
+    const uint32_t cblock = local / tiles;
+    const int32_t e = (int32_t)((local - cblock * tiles) * kThreads + t);
+    if (e >= p.elements) {
+        return;
+    }
+    const int32_t x = e % p.W, yz = e / p.W;
+    const int32_t y = (DIM == 3) ? yz % p.H : yz, z = (DIM == 3) ? yz / p.H : 0;
+    uint32_t start[R], count[R], len = 0;
+    runs_of<DIM, INTERP>(wsn, p, e, x, y, z, start, count);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        len += count[r];
+    }
+    if (len > (uint32_t)LIST) {
+        if (cblock == 0) {
+            wsn[p.lay.crowded + atomicAdd(&wsn[2], 1u)] = (uint32_t)e;
+        }
+        return;
+    }
+    uint32_t* mine = list + t;
+    const uint32_t* entries = wsn + p.lay.list;
+    // the first two entries of every run without a loop (as many as a smooth grid has)
+    uint32_t first[R], second[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        first[r] = count[r] > 0u ? entries[start[r]] : 0u;
+        second[r] = count[r] > 1u ? entries[start[r] + 1u] : 0u;
+    }
+    uint32_t at = 0;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        if (count[r] > 0u) {
+            mine[at * kThreads] = M::key(first[r], r);
+        }
+        if (count[r] > 1u) {
+            mine[(at + 1u) * kThreads] = M::key(second[r], r);
+        }
+        for (uint32_t i = 2; i < count[r]; i++) {
+            mine[(at + i) * kThreads] = M::key(entries[start[r] + i], r);
+        }
+        at += count[r];
+    }
+    if (__builtin_amdgcn_ballot_w64(len > 8u) == 0) {
+        sort_list<8>(mine, len);
+    } else if (LIST <= 16 || __builtin_amdgcn_ballot_w64(len > 16u) == 0) {
+        sort_list<16>(mine, len);
+    } else {
+        sort_list<LIST>(mine, len);
+    }
+    const Coords<T, DIM>* coords = reinterpret_cast<const Coords<T, DIM>*>(wsn + p.lay.coords);
+    const uint32_t phase = (uint32_t)phase_of(n, p);
+    const int32_t c_begin = (int32_t)cblock * chans_per_block;
+    const int32_t c_end = (c_begin + chans_per_block < p.C) ? c_begin + chans_per_block : p.C;
+    for (int32_t c0 = c_begin; c0 < c_end; c0 += CB) {
+        const int32_t nc = (c_end - c0 < CB) ? c_end - c0 : CB;
+        const T* go = gout + ((int64_t)n * p.C + c0) * (int64_t)p.points;
+        float acc[CB];
+#pragma unroll
+        for (int j = 0; j < CB; j++) {
+            acc[j] = 0.0f;
+        }
+        // two entries in flight: the operands of the entry after this one are asked for before this one is folded in
+        struct Operands {
+            Coords<T, DIM> at;
+            uint32_t tap;
+            T go[CB];
+        };
+        auto fetch = [&](uint32_t i, Operands& o) {
+            const uint32_t key = mine[i * kThreads];
+            const uint32_t pt = M::q_of(key) - phase;
+            o.tap = M::tap_of(key);
+            if (INTERP != 1) {
+                o.at = coords[pt];
+            }
+#pragma unroll
+            for (int j = 0; j < CB; j++) {
+                if (j < nc) {
+                    o.go[j] = go[(int64_t)j * p.points + pt];
+                }
+            }
+        };
+        auto fold = [&](const Operands& o) {
+            const float w = weight_of<T, DIM, INTERP>(o.at, o.tap, x, y, z);
+#pragma unroll
+            for (int j = 0; j < CB; j++) {
+                acc[j] = rt<T>(acc[j] + value_of<T, INTERP>(ElemIO<T>::load(&o.go[j]), w));
+            }
+        };
+        Operands a{}, b{};
+        if (len > 0u) {
+            const uint32_t last = len - 1u;
+            fetch(0u, a);
+            for (uint32_t i = 0; i < len; i += 2) {
+                fetch(i + 1u < len ? i + 1u : last, b);
+                fold(a);
+                fetch(i + 2u < len ? i + 2u : last, a);
+                if (i + 1u < len) {
+                    fold(b);
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < CB; j++) {
+            if (j < nc) {
+                store_streaming<T>(dx + ((int64_t)n * p.C + c0 + j) * (int64_t)p.elements + e, acc[j]);
+            }
+        }
+    }
+}
+
+// Elements with more contributions than the gather kernel takes: a wavefront per element and 64 channels.
+template <typename T, int DIM, int INTERP>
+__global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __restrict__ gout, T* __restrict__ dx,
+                                                                      const uint32_t* __restrict__ ws, GatherParams p)
+{
+    typedef Mode<DIM, INTERP> M;
+    constexpr int R = M::kRuns;
+    constexpr int kWaves = kThreads / 64;
+    __shared__ uint32_t s_window[kWaves][R][64];  // the next 64 entries of every run
+    __shared__ uint32_t s_key[kWaves][64];        // the next 64 keys in order
+    __shared__ float s_val[kWaves][kFoldChans][65];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t n = blockIdx.y;
+    const uint32_t* wsn = ws + (size_t)n * p.lay.item_words;
+    const uint32_t chan_blocks = (uint32_t)(p.C + 63) / 64u;
+    const uint32_t jobs = wsn[2] * chan_blocks;
+    const uint32_t phase = (uint32_t)phase_of(n, p);
+    const Coords<T, DIM>* coords = reinterpret_cast<const Coords<T, DIM>*>(wsn + p.lay.coords);
+    uint32_t(*window)[64] = s_window[wave];
+    uint32_t* keys = s_key[wave];
+    float(*val)[65] = s_val[wave];
+    // the wavefronts of a workgroup share nothing: what a wavefront writes to LDS it reads back itself, in order
+    auto landed = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
+    for (uint32_t job = blockIdx.x * kWaves + wave; job < jobs; job += gridDim.x * kWaves) {
+        const int32_t e = (int32_t)wsn[p.lay.crowded + job / chan_blocks];
+        const int32_t c_first = (int32_t)(job % chan_blocks) * 64;
+        const int32_t nc = (p.C - c_first < 64) ? p.C - c_first : 64;
+        const int32_t x = e % p.W, yz = e / p.W;
+        const int32_t y = (DIM == 3) ? yz % p.H : yz, z = (DIM == 3) ? yz / p.H : 0;
+        uint32_t start[R], left[R];
+        runs_of<DIM, INTERP>(wsn, p, e, x, y, z, start, left);
+        uint32_t total = 0;
+        const uint32_t* from[R];  // where the rest of a run is read from
+        bool whole[R];            // the run is short: sorted here, once, and kept
+        uint32_t skip[R];         // entries of a short run already taken
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            total += left[r];
+            whole[r] = left[r] <= kSortedRun;
+            skip[r] = 0u;
+            from[r] = wsn + (whole[r] ? p.lay.list : p.lay.ranks) + start[r];
+            if (whole[r] && left[r] > 0u) {
+                const bool have = (uint32_t)lane < left[r];
+                const uint32_t v = have ? from[r][lane] : 0xFFFFFFFFu;
+                uint32_t rank = 0;
+                for (uint32_t i = 0; i < left[r]; i++) {
+                    const uint32_t other = (uint32_t)__shfl((int)v, (int)i);
+                    rank += (other < v) ? 1u : 0u;
+                }
+                if (have) {
+                    window[r][rank] = v;
+                }
+            }
+        }
+        float acc = 0.0f;  // of channel c_first + lane
+        while (total > 0u) {
+            // the next entries of every run
+            uint32_t mine[R], held[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                held[r] = left[r] < 64u ? left[r] : 64u;
+                if (!whole[r]) {
+                    landed();
+                    if ((uint32_t)lane < held[r]) {
+                        window[r][lane] = from[r][lane];
+                    }
+                }
+            }
+            landed();
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                mine[r] = ((uint32_t)lane < held[r]) ? window[r][skip[r] + lane] : 0xFFFFFFFFu;
+            }
+            // the rank of every one of them among all: entries of another run come first when their chunk is
+            // earlier, or the same and their corner's number lower
+            const uint32_t batch = total < 64u ? total : 64u;
+            uint32_t taken[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                uint32_t rank = (uint32_t)lane;
+#pragma unroll
+                for (int o = 0; o < R; o++) {
+                    if (o != r) {
+                        const uint32_t chunk = (mine[r] >> 8) + ((o < r) ? 1u : 0u);
+                        uint32_t lo = 0, hi = held[o];  // the first entry of run o whose chunk is not below `chunk`
+                        while (lo < hi) {
+                            const uint32_t mid = (lo + hi) >> 1;
+                            if ((window[o][skip[o] + mid] >> 8) < chunk) {
+                                lo = mid + 1u;
+                            } else {
+                                hi = mid;
+                            }
+                        }
+                        rank += lo;
+                    }
+                }
+                const bool take = (uint32_t)lane < held[r] && rank < batch;
+                if (take) {
+                    keys[rank] = M::key(mine[r], r);
+                }
+                taken[r] = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(take));
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                left[r] -= taken[r];
+                if (whole[r]) {
+                    skip[r] += taken[r];
+                } else {
+                    from[r] += taken[r];
+                }
+            }
+            total -= batch;
+            landed();
+            const uint32_t key = keys[(uint32_t)lane < batch ? lane : 0];
+            const uint32_t pt = M::q_of(key) - phase;
+            const float w = weight_of<T, DIM, INTERP>(coords[pt], M::tap_of(key), x, y, z);
+            for (int32_t g = 0; g < nc; g += kFoldChans) {
+                const T* go = gout + (n * p.C + c_first + g) * (int64_t)p.points + pt;
+                landed();
+#pragma unroll
+                for (int j = 0; j < kFoldChans; j++) {
+                    if (g + j < nc) {
+                        val[j][lane] = value_of<T, INTERP>(ElemIO<T>::load(go + (int64_t)j * p.points), w);
+                    }
+                }
+                landed();
+                if (lane >= g && lane < g + kFoldChans && lane < nc) {
+                    const float* v = val[lane - g];
+                    for (uint32_t i = 0; i < batch; i++) {
+                        acc = rt<T>(acc + v[i]);
+                    }
+                }
+            }
+            landed();
+        }
+        if (lane < nc) {
+            store_streaming<T>(dx + (n * p.C + c_first + lane) * (int64_t)p.elements + e, acc);
+        }
+    }
+}
+
+struct GatherPlan {
+    bool ok = false;
+    GatherParams p{};
+    uint32_t tiles = 0, cblocks = 0;
+    int32_t chans_per_block = 0;
+    int cb = 1;
+    int list = kListMost;
+};
+
+inline uint32_t align4(uint64_t v) { return (uint32_t)((v + 3u) & ~(uint64_t)3u); }
+
+GatherPlan make_plan(const GradGatherArgs& a)
+{
+    GatherPlan pl;
+    const int64_t esz = elem_size(a.elem);
+    const int64_t elements = a.D * a.H * a.W;
+    const int64_t cells = (a.interp != 0) ? elements : (a.W + 1) * (a.H + 1) * (a.dim == 3 ? a.D + 1 : 1);
+    const int64_t entries = a.points * (a.interp == 2 ? 16 : 1);
+    const int64_t runs = a.interp == 0 ? ((int64_t)1 << a.dim) : 1;
+    // keys of 32 bits hold an entry and a corner; counts of 32 bits hold an item's entries
+    const int64_t most_points = (int64_t)1 << (a.dim == 3 || a.interp == 2 ? 27 : 28);
+    if (a.points > most_points || elements > INT32_MAX / 2 || cells > INT32_MAX / 2 || a.N > 65535 || a.N < 1) {
+        return pl;
+    }
+    // A list of 16 leaves LDS and registers for twice the wavefronts; of 32 where a smooth grid has more than six
+    // contributions per element on average (scaled by 0.8 along every axis they are ten)
+    pl.list = (entries * runs <= 6 * elements) ? 16 : kListMost;
+    const int64_t crowded_elements = entries * runs / (pl.list + 1) + 1;
+    const int64_t words = kCtrlWords + 2 * cells + 2 * entries + a.points * (a.dim == 3 ? 4 : 2) * esz / 4 +
+                          entries / kSortedRun + crowded_elements + 64;
+    if (words > ((int64_t)1 << 31) || words * 4 * a.N > kGatherMaxScratch) {
+        return pl;
+    }
+    GatherLayout& l = pl.p.lay;
+    l.counts = kCtrlWords;
+    l.starts = align4((uint64_t)l.counts + (uint64_t)cells);
+    l.ranks = align4((uint64_t)l.starts + (uint64_t)cells);
+    l.coords = align4((uint64_t)l.ranks + (uint64_t)entries);
+    l.list = align4((uint64_t)l.coords + (uint64_t)(a.points * (a.dim == 3 ? 4 : 2) * esz / 4));
+    l.runs = align4((uint64_t)l.list + (uint64_t)entries);
+    l.crowded = align4((uint64_t)l.runs + (uint64_t)(entries / kSortedRun) + 1u);
+    l.item_words = align4((uint64_t)l.crowded + (uint64_t)crowded_elements);
+    pl.p.C = (int32_t)a.C;
+    pl.p.D = (int32_t)a.D;
+    pl.p.H = (int32_t)a.H;
+    pl.p.W = (int32_t)a.W;
+    pl.p.points = (int32_t)a.points;
+    pl.p.pad = a.pad;
+    pl.p.align = a.align;
+    pl.p.items_per_core = (int32_t)(a.items_per_core > 0 ? a.items_per_core : 1);
+    pl.p.elements = (int32_t)elements;
+    pl.p.cells = (int32_t)cells;
+    pl.p.N = (int32_t)a.N;
+    pl.cb = (a.C >= 8) ? 8 : ((a.C >= 3) ? 4 : (int)a.C);
+    pl.tiles = (uint32_t)((elements + kThreads - 1) / kThreads);
+    const int64_t base = a.N * pl.tiles;
+    const int64_t max_cblocks = (a.C + pl.cb - 1) / pl.cb;
+    int64_t cblocks = (2048 + base - 1) / base;
+    cblocks = cblocks > max_cblocks ? max_cblocks : cblocks;
+    int64_t cpb = (a.C + cblocks - 1) / cblocks;
+    cpb = (cpb + pl.cb - 1) / pl.cb * pl.cb;
+    cblocks = (a.C + cpb - 1) / cpb;
+    pl.cblocks = (uint32_t)cblocks;
+    pl.chans_per_block = (int32_t)cpb;
+    if (base * cblocks > INT32_MAX / 2 || a.N * ((a.points + kThreads - 1) / kThreads) > INT32_MAX / 2) {
+        return pl;
+    }
+    pl.ok = true;
+    return pl;
+}
+
+inline uint32_t swizzled_blocks(int64_t pieces) { return (uint32_t)((pieces + 7) / 8 * 8); }
+
+template <typename T, int DIM, int INTERP, int CB, int LIST>
+hipError_t launch_gather(const GradGatherArgs& a, const GatherPlan& pl, hipStream_t stream)
+{
+    const uint32_t pieces = (uint32_t)a.N * pl.tiles * pl.cblocks;
+    const uint32_t blocks = swizzled_blocks(pieces);
+    // workgroups that sort long runs: a turn of the chip at most, and none an item could not use
+    const int64_t most_runs = a.points * Mode<DIM, INTERP>::kEntries / (kSortedRun + 1);
+    int64_t sorters = 512 / a.N > 0 ? 512 / a.N : 1;
+    sorters = sorters < most_runs ? sorters : most_runs;
+    hipLaunchKernelGGL((gs_gather_kernel<T, DIM, INTERP, CB, LIST>), dim3(blocks + (uint32_t)(sorters * a.N)), dim3(kThreads), 0,
+                       stream, (const T*)a.gout, (T*)a.dx, (uint32_t*)a.scratch, pl.p, pieces, blocks, pl.tiles,
+                       pl.chans_per_block, (uint32_t)(sorters > 0 ? sorters : 1));
+    return hipGetLastError();
+}
+
+template <typename T, int DIM, int INTERP>
+hipError_t run_mode(const GradGatherArgs& a, const GatherPlan& pl, hipStream_t stream)
+{
+    const GatherParams& p = pl.p;
+    uint32_t* ws = (uint32_t*)a.scratch;
+    const uint32_t clear_words = p.lay.starts;
+    hipLaunchKernelGGL(gs_gather_clear_kernel, dim3((clear_words / 4 + kThreads - 1) / kThreads, (unsigned)a.N),
+                       dim3(kThreads), 0, stream, ws, clear_words, p.lay.item_words);
+    constexpr int kPoints = kThreads * points_per_lane<DIM, INTERP>();
+    const uint32_t per_item = (uint32_t)((a.points + kPoints - 1) / kPoints);
+    const uint32_t pieces = (uint32_t)a.N * per_item;
+    hipLaunchKernelGGL((gs_gather_count_kernel<T, DIM, INTERP>), dim3(swizzled_blocks(pieces)), dim3(kThreads), 0, stream,
+                       (const T*)a.grid, ws, p, pieces, per_item);
+    hipLaunchKernelGGL(gs_gather_place_kernel,
+                       dim3((unsigned)((p.cells + kPlaceThreads * kPlaceCells - 1) / (kPlaceThreads * kPlaceCells)),
+                            (unsigned)a.N),
+                       dim3(kPlaceThreads), 0, stream, ws, p);
+    hipLaunchKernelGGL((gs_gather_fill_kernel<T, DIM, INTERP>), dim3(swizzled_blocks(pieces)), dim3(kThreads), 0, stream, ws,
+                       p, pieces, per_item);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        return e;
+    }
+    switch (pl.cb * 64 + pl.list) {
+        case 1 * 64 + 16: e = launch_gather<T, DIM, INTERP, 1, 16>(a, pl, stream); break;
+        case 2 * 64 + 16: e = launch_gather<T, DIM, INTERP, 2, 16>(a, pl, stream); break;
+        case 4 * 64 + 16: e = launch_gather<T, DIM, INTERP, 4, 16>(a, pl, stream); break;
+        case 8 * 64 + 16: e = launch_gather<T, DIM, INTERP, 8, 16>(a, pl, stream); break;
+        case 1 * 64 + 32: e = launch_gather<T, DIM, INTERP, 1, 32>(a, pl, stream); break;
+        case 2 * 64 + 32: e = launch_gather<T, DIM, INTERP, 2, 32>(a, pl, stream); break;
+        case 4 * 64 + 32: e = launch_gather<T, DIM, INTERP, 4, 32>(a, pl, stream); break;
+        default: e = launch_gather<T, DIM, INTERP, 8, 32>(a, pl, stream); break;
+    }
+    if (e != hipSuccess) {
+        return e;
+    }
+    const int64_t most = a.points * Mode<DIM, INTERP>::kEntries * Mode<DIM, INTERP>::kRuns / (pl.list + 1);
+    if (most > 0) {  // else no element can be crowded
+        const int64_t per = 1024 / a.N > 1 ? 1024 / a.N : 1;
+        hipLaunchKernelGGL((gs_gather_crowded_kernel<T, DIM, INTERP>), dim3((unsigned)per, (unsigned)a.N), dim3(kThreads),
+                           0, stream, (const T*)a.gout, (T*)a.dx, ws, p);
+    }
+    return hipGetLastError();
+}
+
+template <typename T>
+hipError_t run_typed(const GradGatherArgs& a, const GatherPlan& pl, hipStream_t stream)
+{
+    switch (a.dim * 4 + a.interp) {
+        case 2 * 4 + 0: return run_mode<T, 2, 0>(a, pl, stream);
+        case 2 * 4 + 1: return run_mode<T, 2, 1>(a, pl, stream);
+        case 2 * 4 + 2: return run_mode<T, 2, 2>(a, pl, stream);
+        case 3 * 4 + 0: return run_mode<T, 3, 0>(a, pl, stream);
+        case 3 * 4 + 1: return run_mode<T, 3, 1>(a, pl, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace
+
+int64_t grad_gather_words(const GradGatherArgs& a)
+{
+    const GatherPlan pl = make_plan(a);
+    return pl.ok ? (int64_t)pl.p.lay.item_words * a.N : 0;
+}
+
+hipError_t run_grad_gather(const GradGatherArgs& a, hipStream_t stream)
+{
+    const GatherPlan pl = make_plan(a);
+    if (!pl.ok || a.dx == nullptr || a.gout == nullptr || a.grid == nullptr || a.scratch == nullptr) {
+        return hipErrorInvalidValue;
+    }
+    switch (a.elem) {
+        case Elem::F32: return run_typed<float>(a, pl, stream);
+        case Elem::F16: return run_typed<_Float16>(a, pl, stream);
+        case Elem::BF16: return run_typed<__bf16>(a, pl, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+}  // namespace opscv

@@ -78,6 +78,8 @@ int64_t gs2d_grad_csr_words(const GridSamplerGradArgs& a);
 // on the stream has done that, else it launches a kernel of its own for it
 bool gs2d_grad_csr_clear(const GridSamplerGradArgs& a, GradClear* clear);
 hipError_t run_gs2d_grad_input_csr(const GridSamplerGradArgs& a, hipStream_t stream, bool* handled, bool cleared);
+// ... and of the variant that sorts every element's contributions (gs_grad_gather.hip) where that one does not run
+int64_t gs2d_grad_gather_words(const GridSamplerGradArgs& a);
 hipError_t launch_grid_sampler3d(const GridSampler3DArgs& a, hipStream_t stream);
 hipError_t launch_grid_sampler3d_grad(const GridSampler3DGradArgs& a, hipStream_t stream);
 // 32-bit words of GridSampler3DGradArgs::chunk_ranges that make the input gradient faster; 0 when it would not help
@@ -85,6 +87,9 @@ int64_t gs3d_grad_range_words(const GridSampler3DGradArgs& a);
 // 32-bit words of GridSampler3DGradArgs::lists that the gather variant of the input gradient needs; 0 when the shape
 // does not qualify (gs3d_grad_lists.hip)
 int64_t gs3d_grad_list_words(const GridSampler3DGradArgs& a);
+// 32-bit words of GridSampler3DGradArgs::gather that the sorting variant of the input gradient (gs_grad_gather.hip)
+// needs; 0 where another variant runs
+int64_t gs3d_grad_gather_words(const GridSampler3DGradArgs& a);
 // one scratch region holds both: the chunk spans at its start, the lists from this byte offset
 inline uint64_t gs3d_grad_lists_offset(int64_t range_words) { return ((uint64_t)range_words * 4 + 255) / 256 * 256; }
 

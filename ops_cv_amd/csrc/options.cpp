@@ -56,7 +56,7 @@ Store& store()
             s.reference_ub_bytes = n;
         }
         if (const char* v = getenv("OPSCV_GS3D_GRAD_VARIANT")) {
-            s.gs3d_grad_variant = (v[0] == 'o') ? kGs3dGradOrdered : (v[0] == 'g' ? kGs3dGradGather : kGs3dGradAuto);
+            s.gs3d_grad_variant = (v[0] == 'o') ? kGs3dGradOrdered : (v[0] == 'g' ? kGs3dGradGather : (v[0] == 's' ? kGs3dGradSorted : kGs3dGradAuto));
         }
         if (const char* v = getenv("OPSCV_GRID_SAMPLER2D_RULE")) {
             s.grid_sampler2d_rule = (strcmp(v, "arch35") == 0 || strcmp(v, "1") == 0) ? kRuleGridSampleArch35
@@ -79,7 +79,7 @@ const Entry kEntries[] = {
     {"reference_cores", &Store::reference_cores, 1, INT64_MAX},
     {"reference_ub_bytes", &Store::reference_ub_bytes, 1, INT64_MAX},
     {"grid_sampler2d_rule", &Store::grid_sampler2d_rule, kRuleGridSampler2D, kRuleGridSampleArch35},
-    {"gs3d_grad_variant", &Store::gs3d_grad_variant, kGs3dGradAuto, kGs3dGradGather},
+    {"gs3d_grad_variant", &Store::gs3d_grad_variant, kGs3dGradAuto, kGs3dGradSorted},
 };
 
 const Entry* find(const char* name)

@@ -358,31 +358,33 @@ def _stream_handle(stream):
     return ctypes.c_void_p(s.cuda_stream)
 
 
+_helpers = None
+
+
+def _native():
+    """The native side of the helpers below (csrc/torch_helpers.cpp), which runs both phases on torch tensors."""
+    global _helpers
+    if _helpers is None:
+        _torch()  # the extension needs PyTorch's libraries in the process
+        load_library()
+        try:
+            from . import _torch_helpers
+        except ImportError as e:
+            raise RuntimeError("_torch_helpers.so is not built: run `python -m ops_cv_amd.build`") from e
+        _torch_helpers.set_error_class(AclnnError)
+        _helpers = _torch_helpers
+    return _helpers
+
+
+def _raw(stream):
+    return None if stream is None else stream.cuda_stream
+
+
 def grid_sampler2d(inp, grid, interpolation_mode=0, padding_mode=0, align_corners=False, out=None, stream=None,
                    workspace=None):
     """Both phases of aclnnGridSampler2D on torch CUDA tensors; returns `out` (N,C,Hout,Wout)."""
-    torch = _torch()
-    L = load_library()
-    if out is None:
-        out = torch.empty((inp.shape[0], inp.shape[1], grid.shape[1], grid.shape[2]), dtype=inp.dtype,
-                          device=inp.device)
-    hs = [tensor_handle(inp), tensor_handle(grid), tensor_handle(out)]
-    try:
-        st, ws, ex = get_workspace_size_grid_sampler2d(hs[0], hs[1], interpolation_mode, padding_mode,
-                                                       align_corners, hs[2])
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler2DGetWorkspaceSize", st)
-        if ws > 0 and (workspace is None or workspace.numel() * workspace.element_size() < ws):
-            workspace = torch.empty(ws, dtype=torch.uint8, device=inp.device)
-        wptr = ctypes.c_void_p(workspace.data_ptr()) if ws > 0 else None
-        wsize = workspace.numel() * workspace.element_size() if ws > 0 else 0
-        st = L.aclnnGridSampler2D(wptr, wsize, ex, _stream_handle(stream))
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler2D", st)
-    finally:
-        for h in hs:
-            destroy_tensor(h)
-    return out
+    return (_helpers or _native()).grid_sampler2d(inp, grid, interpolation_mode, padding_mode, align_corners, out,
+                                                  workspace, _raw(stream))
 
 
 NOALLOC_SCRATCH_BYTES = 16 << 20  # OPSCV_NOALLOC_SCRATCH_BYTES (include/opscv_ext.h)
@@ -405,31 +407,9 @@ def grid_sampler2d_backward(grad_out, inp, grid, interpolation_mode=0, padding_m
                             output_mask=(True, True), input_grad=None, grid_grad=None, stream=None, workspace=None):
     """Both phases of aclnnGridSampler2DBackward on torch CUDA tensors; returns (input_grad, grid_grad).  A gradient
     whose mask flag is false is left untouched."""
-    torch = _torch()
-    L = load_library()
-    if input_grad is None:
-        input_grad = torch.empty_like(inp)
-    if grid_grad is None:
-        grid_grad = torch.empty_like(grid)
-    hs = [tensor_handle(t) for t in (grad_out, inp, grid, input_grad, grid_grad)]
-    mask = create_bool_array(list(output_mask))
-    try:
-        st, ws, ex = get_workspace_size_grid_sampler2d_backward(hs[0], hs[1], hs[2], interpolation_mode, padding_mode,
-                                                                align_corners, mask, hs[3], hs[4])
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler2DBackwardGetWorkspaceSize", st)
-        if ws > 0 and (workspace is None or workspace.numel() * workspace.element_size() < ws):
-            workspace = torch.empty(ws, dtype=torch.uint8, device=inp.device)
-        wptr = ctypes.c_void_p(workspace.data_ptr()) if ws > 0 else None
-        wsize = workspace.numel() * workspace.element_size() if ws > 0 else 0
-        st = L.aclnnGridSampler2DBackward(wptr, wsize, ex, _stream_handle(stream))
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler2DBackward", st)
-    finally:
-        for h in hs:
-            destroy_tensor(h)
-        destroy_bool_array(mask)
-    return input_grad, grid_grad
+    return (_helpers or _native()).grid_sampler2d_backward(grad_out, inp, grid, interpolation_mode, padding_mode,
+                                                           align_corners, output_mask, input_grad, grid_grad, workspace,
+                                                           _raw(stream), False)
 
 
 def grid_sampler3d_backward(grad_out, inp, grid, interpolation_mode=0, padding_mode=0, align_corners=False,
@@ -437,33 +417,9 @@ def grid_sampler3d_backward(grad_out, inp, grid, interpolation_mode=0, padding_m
                             channels_last=False):
     """Both phases of aclnnGridSampler3DBackward on torch CUDA tensors; returns (input_grad, grid_grad).  A gradient
     whose mask flag is false is left untouched.  With channels_last, grad_out, inp and input_grad are (N,D,H,W,C)."""
-    torch = _torch()
-    L = load_library()
-    if input_grad is None:
-        input_grad = torch.empty_like(inp)
-    if grid_grad is None:
-        grid_grad = torch.empty_like(grid)
-    fmt = ACL_FORMAT_NDHWC if channels_last else ACL_FORMAT_NCDHW
-    hs = [tensor_handle(grad_out, fmt), tensor_handle(inp, fmt), tensor_handle(grid), tensor_handle(input_grad, fmt),
-          tensor_handle(grid_grad)]
-    mask = create_bool_array(list(output_mask))
-    try:
-        st, ws, ex = get_workspace_size_grid_sampler3d_backward(hs[0], hs[1], hs[2], interpolation_mode, padding_mode,
-                                                                align_corners, mask, hs[3], hs[4])
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler3DBackwardGetWorkspaceSize", st)
-        if ws > 0 and (workspace is None or workspace.numel() * workspace.element_size() < ws):
-            workspace = torch.empty(ws, dtype=torch.uint8, device=inp.device)
-        wptr = ctypes.c_void_p(workspace.data_ptr()) if ws > 0 else None
-        wsize = workspace.numel() * workspace.element_size() if ws > 0 else 0
-        st = L.aclnnGridSampler3DBackward(wptr, wsize, ex, _stream_handle(stream))
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler3DBackward", st)
-    finally:
-        for h in hs:
-            destroy_tensor(h)
-        destroy_bool_array(mask)
-    return input_grad, grid_grad
+    return (_helpers or _native()).grid_sampler3d_backward(grad_out, inp, grid, interpolation_mode, padding_mode,
+                                                           align_corners, output_mask, input_grad, grid_grad, workspace,
+                                                           _raw(stream), channels_last)
 
 
 def grid_sampler3d(inp, grid, interpolation_mode=0, padding_mode=0, align_corners=False, out=None, stream=None,
@@ -473,129 +429,31 @@ def grid_sampler3d(inp, grid, interpolation_mode=0, padding_mode=0, align_corner
     inp is (N,C,D,H,W) and the result (N,C,Do,Ho,Wo); with channels_last inp is (N,D,H,W,C) and the result
     (N,Do,Ho,Wo,C) (format NDHWC).  grid is (N,Do,Ho,Wo,3).
     """
-    torch = _torch()
-    L = load_library()
-    fmt = ACL_FORMAT_NDHWC if channels_last else ACL_FORMAT_NCDHW
-    if out is None:
-        if channels_last:
-            shape = (inp.shape[0], grid.shape[1], grid.shape[2], grid.shape[3], inp.shape[4])
-        else:
-            shape = (inp.shape[0], inp.shape[1], grid.shape[1], grid.shape[2], grid.shape[3])
-        out = torch.empty(shape, dtype=inp.dtype, device=inp.device)
-    hs = [tensor_handle(inp, fmt), tensor_handle(grid), tensor_handle(out, fmt)]
-    try:
-        st, ws, ex = get_workspace_size_grid_sampler3d(hs[0], hs[1], interpolation_mode, padding_mode,
-                                                       align_corners, hs[2])
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler3DGetWorkspaceSize", st)
-        if ws > 0 and (workspace is None or workspace.numel() * workspace.element_size() < ws):
-            workspace = torch.empty(ws, dtype=torch.uint8, device=inp.device)
-        wptr = ctypes.c_void_p(workspace.data_ptr()) if ws > 0 else None
-        wsize = workspace.numel() * workspace.element_size() if ws > 0 else 0
-        st = L.aclnnGridSampler3D(wptr, wsize, ex, _stream_handle(stream))
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnGridSampler3D", st)
-    finally:
-        for h in hs:
-            destroy_tensor(h)
-    return out
+    return (_helpers or _native()).grid_sampler3d(inp, grid, interpolation_mode, padding_mode, align_corners, out,
+                                                  workspace, _raw(stream), channels_last)
 
 
 def upsample_bilinear2d(self_t, output_size, align_corners=False, scales_h=0.0, scales_w=0.0, out=None, stream=None,
                         channels_last=False, workspace=None):
     """Both phases of aclnnUpsampleBilinear2d; tensors are NCHW views, or NHWC views when channels_last."""
-    torch = _torch()
-    L = load_library()
-    fmt = ACL_FORMAT_NHWC if channels_last else ACL_FORMAT_NCHW
-    if out is None:
-        if channels_last:
-            shape = (self_t.shape[0], output_size[0], output_size[1], self_t.shape[3])
-        else:
-            shape = (self_t.shape[0], self_t.shape[1], output_size[0], output_size[1])
-        out = torch.empty(shape, dtype=self_t.dtype, device=self_t.device)
-    hs = [tensor_handle(self_t, fmt), tensor_handle(out, fmt)]
-    size = create_int_array(list(output_size))
-    try:
-        st, ws, ex = get_workspace_size_upsample_bilinear2d(hs[0], size, align_corners, scales_h, scales_w, hs[1])
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnUpsampleBilinear2dGetWorkspaceSize", st)
-        if ws > 0 and (workspace is None or workspace.numel() * workspace.element_size() < ws):
-            workspace = torch.empty(ws, dtype=torch.uint8, device=self_t.device)
-        wptr = ctypes.c_void_p(workspace.data_ptr()) if ws > 0 else None
-        wsize = workspace.numel() * workspace.element_size() if ws > 0 else 0
-        st = L.aclnnUpsampleBilinear2d(wptr, wsize, ex, _stream_handle(stream))
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnUpsampleBilinear2d", st)
-    finally:
-        for h in hs:
-            destroy_tensor(h)
-        destroy_int_array(size)
-    return out
+    return (_helpers or _native()).upsample_bilinear2d(self_t, output_size, align_corners, scales_h, scales_w, out,
+                                                       workspace, _raw(stream), channels_last)
 
 
 def resize(self_t, scales, mode="bilinear", out=None, stream=None, channels_last=False, workspace=None):
     """Both phases of aclnnResize.  `scales` holds four floats in the order of the tensor's dimensions; the output
     extents are trunc(in * scale).  Tensors are NCHW views, or NHWC views when channels_last."""
-    torch = _torch()
-    L = load_library()
-    fmt = ACL_FORMAT_NHWC if channels_last else ACL_FORMAT_NCHW
-    if out is None:
-        shape = list(self_t.shape)
-        for d in ((1, 2) if channels_last else (2, 3)):
-            shape[d] = int(float(self_t.shape[d]) * float(scales[d]))
-        out = torch.empty(shape, dtype=self_t.dtype, device=self_t.device)
-    hs = [tensor_handle(self_t, fmt), tensor_handle(out, fmt)]
-    sc = create_float_array(list(scales))
-    try:
-        st, ws, ex = get_workspace_size_resize(hs[0], sc, mode.encode(), hs[1])
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnResizeGetWorkspaceSize", st)
-        if ws > 0 and (workspace is None or workspace.numel() * workspace.element_size() < ws):
-            workspace = torch.empty(ws, dtype=torch.uint8, device=self_t.device)
-        wptr = ctypes.c_void_p(workspace.data_ptr()) if ws > 0 else None
-        wsize = workspace.numel() * workspace.element_size() if ws > 0 else 0
-        st = L.aclnnResize(wptr, wsize, ex, _stream_handle(stream))
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnResize", st)
-    finally:
-        for h in hs:
-            destroy_tensor(h)
-        destroy_float_array(sc)
-    return out
+    return (_helpers or _native()).resize(self_t, scales, mode, out, workspace, _raw(stream), channels_last)
 
 
 def upsample_bilinear2d_backward(grad_out, input_size, align_corners=False, scales_h=0.0, scales_w=0.0, out=None,
                                  stream=None, channels_last=False, out_dtype=None, workspace=None):
     """Both phases of aclnnUpsampleBilinear2dBackward.  `input_size` holds the four extents of the tensor that was
     upsampled, in the order of the tensors' layout (NCHW, or NHWC when channels_last)."""
-    torch = _torch()
-    L = load_library()
-    fmt = ACL_FORMAT_NHWC if channels_last else ACL_FORMAT_NCHW
-    if out is None:
-        out = torch.empty(tuple(input_size), dtype=grad_out.dtype if out_dtype is None else out_dtype,
-                          device=grad_out.device)
-    hw = (1, 2) if channels_last else (2, 3)
-    hs = [tensor_handle(grad_out, fmt), tensor_handle(out, fmt)]
-    osz = create_int_array([grad_out.shape[hw[0]], grad_out.shape[hw[1]]])
-    isz = create_int_array(list(input_size))
-    try:
-        st, ws, ex = get_workspace_size_upsample_bilinear2d_backward(hs[0], osz, isz, align_corners, scales_h,
-                                                                     scales_w, hs[1])
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnUpsampleBilinear2dBackwardGetWorkspaceSize", st)
-        if ws > 0 and (workspace is None or workspace.numel() * workspace.element_size() < ws):
-            workspace = torch.empty(ws, dtype=torch.uint8, device=grad_out.device)
-        wptr = ctypes.c_void_p(workspace.data_ptr()) if ws > 0 else None
-        wsize = workspace.numel() * workspace.element_size() if ws > 0 else 0
-        st = L.aclnnUpsampleBilinear2dBackward(wptr, wsize, ex, _stream_handle(stream))
-        if st != ACLNN_SUCCESS:
-            raise AclnnError("aclnnUpsampleBilinear2dBackward", st)
-    finally:
-        for h in hs:
-            destroy_tensor(h)
-        destroy_int_array(osz)
-        destroy_int_array(isz)
-    return out
+    if out is None and out_dtype is not None:
+        out = _torch().empty(tuple(input_size), dtype=out_dtype, device=grad_out.device)
+    return (_helpers or _native()).upsample_bilinear2d_backward(grad_out, input_size, align_corners, scales_h, scales_w,
+                                                                out, workspace, _raw(stream), channels_last)
 
 
 def grid_sampler2d_taps(grid, h_in, w_in, interpolation_mode=0, padding_mode=0, align_corners=False, stream=None):

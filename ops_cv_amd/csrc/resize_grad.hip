@@ -271,6 +271,7 @@ __device__ __forceinline__ float tile_sum_fixed(const float* lane_rows, int32_t 
 }
 
 constexpr int kTileCols = 128;
+constexpr int64_t kWantBlocks = 8192;
 constexpr int32_t kGradCapWords = 12288;  // at most 48 KB of LDS per workgroup (fp32 words, one per tile element)
 constexpr int kTileGroups = kGradThreads / kTileCols;  // row groups of a workgroup
 
@@ -517,10 +518,329 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
     }
 }
 
+// Planes whose elements grow by up to four a side (at most eight visited rows and columns): the rectangle stays in the
+// element type and comes by asynchronous copies.
+//
+// A workgroup owns 64 outgoing columns by 16 or 8 outgoing rows, a wavefront every fourth of the rows.  The row segments
+// the tile visits are copied from the 16-byte boundary before their first byte to the one after their last (the bytes
+// outside share an aligned unit with bytes inside, so they are readable), so rows may have any length and start at any
+// element; where a row then starts in LDS is uniform, and a lane reads its run of columns from the 4-byte word its first
+// one lies in.  16-bit columns are shifted into place pair by pair: the reads never straddle a word, and a run takes
+// half the LDS traffic of fp32 words, whose lanes meet in one bank in four where the columns grow by four.
+// Same visits, products and order of the sum as resize_grad_kernel.
+//
+// What bounds it: vector instructions, three per visit plus the shifts, and the set-up of a tile where it serves few
+// planes.  bf16 8x64x65x129 from 257x513: 72.6 us, where rows of odd length were left to resize_grad_kernel before (189
+// us).  4x32x160x240 against resize_grad_lds_kernel (fp16 even rows / fp32) and the gather (bf16 odd rows), before ->
+// after: growth by 0.6 24 -> 16 / 24 -> 16 / 28 -> 17 us, by two 38 -> 29 / 40 -> 28 / 63 -> 31, by three 95 -> 51 /
+// 105 -> 47 / 118 -> 45, by four 136 -> 57 / 174 -> 109 (a growth above four: the gather as before).
+constexpr int kPlaneCols = 64;
+constexpr int kPlaneVisits = 8;                 // most rows, and most columns, an outgoing element may visit
+constexpr int kPlaneRows = 16;                  // most outgoing rows of a tile
+constexpr int32_t kPlaneTallBytes = 24 * 1024;  // tiles of 16 rows up to here: six workgroups and more fit a CU
+constexpr int32_t kPlaneMostBytes = 48 * 1024;  // tiles of 8 rows up to here
+constexpr int32_t kPlanePad = 64;               // bytes behind the last row that a lane's last columns may be read from
+
+typedef __attribute__((address_space(1))) const void* rg_global_cptr_t;
+typedef __attribute__((address_space(3))) void* rg_lds_ptr_t;
+
+// Columns 0 .. KX - 1 of the run that starts at LDS byte `off`, times y_lerp (fma(g, w, -0) is g * w bit for bit).
+template <typename TI, int KX>
+__device__ __forceinline__ void weighted_columns(const char* lds, uint32_t off, float y_lerp, float neg_zero, float* t)
+{
+    if constexpr (sizeof(TI) == 4) {
+        const float* w = reinterpret_cast<const float*>(lds + off);
+#pragma unroll
+        for (int k = 0; k < KX; k++) {
+            t[k] = w[k] * y_lerp;
+        }
+    } else {
+        constexpr int PAIRS = (KX + 1) / 2;
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(lds + (off & ~3u));
+        const uint32_t bits = off << 3;  // alignbit takes its low five bits: 0 or 16
+        uint32_t word[PAIRS + 1];
+#pragma unroll
+        for (int k = 0; k <= PAIRS; k++) {
+            word[k] = w[k];
+        }
+#pragma unroll
+        for (int k = 0; k < PAIRS; k++) {
+            const uint32_t both = __builtin_amdgcn_alignbit(word[k + 1], word[k], bits);
+            TI pair[2];
+            __builtin_memcpy(pair, &both, 4);
+            t[2 * k] = __builtin_fmaf(ElemIO<TI>::load(&pair[0]), y_lerp, neg_zero);
+            if (2 * k + 1 < KX) {
+                t[2 * k + 1] = __builtin_fmaf(ElemIO<TI>::load(&pair[1]), y_lerp, neg_zero);
+            }
+        }
+    }
+}
+
+template <typename TI, typename TO, bool HALF_PIXEL>
+__global__ __launch_bounds__(kGradThreads) void resize_grad_planes_kernel(
+    const TI* __restrict__ g, TO* __restrict__ y, int64_t planes, int32_t Hs, int32_t Ws, int32_t Hd, int32_t Wd,
+    float scale_h, float scale_w, float inv_scale_h, float inv_scale_w, int32_t tile_rows, int32_t lds_bytes,
+    float neg_zero, uint32_t tiles_x, uint32_t tiles_y, uint32_t plane_slots)
+{
+    // tiles go to the XCDs as in resize_grad_lds_kernel
+    const uint32_t per_xcd = gridDim.x / 8u;
+    const uint32_t tile_id = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
+    if (tile_id >= tiles_x * tiles_y * plane_slots) {
+        return;
+    }
+    const uint32_t block_x = tile_id % tiles_x, block_y = (tile_id / tiles_x) % tiles_y;
+    const uint32_t block_z = tile_id / (tiles_x * tiles_y);
+    constexpr int NWAVES = kGradThreads / 64;
+    constexpr int HQ = kPlaneRows / NWAVES;  // outgoing rows of a wavefront at the largest tile height
+    static_assert(HQ * kPlaneVisits <= 64, "the row weights of a wavefront are packed one per lane");
+    extern __shared__ __attribute__((aligned(16))) uint32_t tile_words[];
+    __shared__ int32_t s_x1, s_y1, s_nx, s_nx_min;
+    char* lds = reinterpret_cast<char*>(tile_words);
+    const int32_t lane = (int32_t)threadIdx.x & 63;
+    const int32_t wave = __builtin_amdgcn_readfirstlane((int32_t)threadIdx.x >> 6);
+    const int32_t W0 = (int32_t)block_x * kPlaneCols, H0 = (int32_t)block_y * tile_rows;
+    const float offset = HALF_PIXEL ? 0.5f : 0.0f;
+    const float last_y = (float)Hs - 1.0f, last_x = (float)Ws - 1.0f;
+    auto first_visit = [&](int32_t i, float inv_scale, int32_t len_dst) {
+        const float f = __builtin_ceilf(((float)i - 1.0f + offset) * inv_scale - offset);
+        // a start at or beyond the end visits nothing, whatever its exact value
+        return (f > 0.0f) ? ((f < (float)len_dst) ? (int32_t)f : len_dst) : 0;
+    };
+    const int32_t W = W0 + lane;
+    const bool col_ok = W < Ws;
+    const int32_t col = col_ok ? W : W0;
+    const float fw = (float)col;
+    const int32_t in_x_start = first_visit(col, inv_scale_w, Wd);
+    const int32_t tile_x0 = first_visit(W0, inv_scale_w, Wd);
+    const int32_t tile_y0 = first_visit(H0, inv_scale_h, Hd);
+    const float out_x_start = ((float)in_x_start + offset) * scale_w - offset;
+    if (threadIdx.x == 0) {
+        s_y1 = 0;
+    }
+    __syncthreads();
+
+    // The columns this lane visits and their weights, by the loop of resize_grad_kernel; the rows each of the wavefront's
+    // outgoing rows visits and theirs, one per lane (the row is the same for all lanes).
+    int32_t nx = 0;
+    float xl[kPlaneVisits];
+    {
+        float out_x = out_x_start;
+#pragma unroll
+        for (int k = 0; k < kPlaneVisits; k++) {
+            xl[k] = 1.0f - __builtin_fabsf(__builtin_fmaxf(0.0f, __builtin_fminf(out_x, last_x)) - fw);
+            out_x += scale_w;
+        }
+        out_x = out_x_start;
+        for (int32_t in_x = in_x_start; out_x < fw + 1.0f && in_x < Wd; in_x++) {
+            nx++;
+            out_x += scale_w;
+        }
+    }
+    float lerp_pack = 0.0f;  // lane q * kPlaneVisits + j: weight of visited row j of outgoing row q
+    int32_t meta_pack = -1;  // lane q: rows outgoing row q visits (-1: no such row in this tile); lane 8 + q: the first
+    bool fits = true;
+    int32_t y_end = 0;
+    static_assert(HQ <= 8, "counts in lanes 0 to 7, first rows in lanes 8 to 15");
+    for (int q = 0; q < HQ; q++) {
+        const int32_t H = H0 + wave + q * NWAVES;
+        if (H < H0 + tile_rows && H < Hs) {
+            const int32_t start = first_visit(H, inv_scale_h, Hd);
+            float out_y = ((float)start + offset) * scale_h - offset;
+            const float fh = (float)H;
+            int32_t n = 0;
+            for (int32_t in_y = start; out_y < fh + 1.0f && in_y < Hd; in_y++) {
+                const float w = 1.0f - __builtin_fabsf(__builtin_amdgcn_fmed3f(out_y, 0.0f, last_y) - fh);
+                lerp_pack = (n < kPlaneVisits && lane == q * kPlaneVisits + n) ? w : lerp_pack;
+                n++;
+                out_y += scale_h;
+            }
+            n = __builtin_amdgcn_readfirstlane(n);
+            meta_pack = (lane == q) ? n : ((lane == 8 + q) ? start : meta_pack);
+            fits = fits && n <= kPlaneVisits;
+            y_end = (start + n > y_end) ? start + n : y_end;
+        }
+    }
+    {
+        // largest end and visit counts over the wavefront's columns, which are the workgroup's
+        int32_t m_end = col_ok ? in_x_start + nx : 0, m_nx = col_ok ? nx : 0, m_min = col_ok ? nx : INT32_MAX;
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) {
+            const int32_t o_end = __shfl_xor(m_end, d), o_nx = __shfl_xor(m_nx, d), o_min = __shfl_xor(m_min, d);
+            m_end = (o_end > m_end) ? o_end : m_end;
+            m_nx = (o_nx > m_nx) ? o_nx : m_nx;
+            m_min = (o_min < m_min) ? o_min : m_min;
+        }
+        if (threadIdx.x == 0) {
+            s_x1 = m_end;
+            s_nx = m_nx;
+            s_nx_min = m_min;
+        }
+        if (lane == 0) {
+            atomicMax(&s_y1, fits ? y_end : INT32_MAX);  // a row of too many visits: no rectangle is large enough
+        }
+    }
+    __syncthreads();
+    const int32_t tile_x1 = __builtin_amdgcn_readfirstlane(s_x1), tile_y1 = __builtin_amdgcn_readfirstlane(s_y1);
+    const int32_t nx_max = __builtin_amdgcn_readfirstlane(s_nx), nx_min = __builtin_amdgcn_readfirstlane(s_nx_min);
+    const int32_t rows = (tile_y1 > tile_y0) ? tile_y1 - tile_y0 : 0;
+    const uint32_t seg_bytes = (tile_x1 > tile_x0) ? (uint32_t)(tile_x1 - tile_x0) * (uint32_t)sizeof(TI) : 0u;
+    const uint32_t pitch = (seg_bytes + 30u) & ~15u;
+    const bool use_lds = nx_max <= kPlaneVisits && (int64_t)rows * pitch + kPlanePad <= lds_bytes;
+    const uint32_t lane_off = (nx > 0) ? (uint32_t)(in_x_start - tile_x0) * (uint32_t)sizeof(TI) : 0u;
+    const uint32_t row_low = ((uint32_t)Wd * (uint32_t)sizeof(TI)) & 15u;
+    const float neg_zero_v = as_fp32_value(neg_zero);
+
+    for (int64_t pl = block_z; pl < planes; pl += plane_slots) {
+        const TI* gp = g + pl * (int64_t)Hd * Wd;
+        TO* yp = y + pl * (int64_t)Hs * Ws + W;
+        if (!use_lds) {
+            for (int32_t H = H0 + wave; col_ok && H < H0 + tile_rows && H < Hs; H += NWAVES) {
+                const int32_t in_y_start = first_visit(H, inv_scale_h, Hd);
+                const float out_y_start = ((float)in_y_start + offset) * scale_h - offset;
+                store_streaming<TO>(yp + (int64_t)H * Ws,
+                                    visit_sum<TI>(gp, Wd, 0, 0, in_y_start, in_x_start, out_y_start, out_x_start, (float)H,
+                                                  fw, scale_h, scale_w, last_y, last_x, Hd, Wd));
+            }
+            continue;
+        }
+        const char* src0 = reinterpret_cast<const char*>(gp + (int64_t)tile_y0 * Wd + tile_x0);
+        const uint32_t src0_low = (uint32_t)(reinterpret_cast<uintptr_t>(src0) & 15u);
+        // bytes by which the copy of staged row r starts before the row's segment
+        auto row_shift = [&](uint32_t r) -> uint32_t { return (src0_low + r * row_low) & 15u; };
+        for (uint32_t r = (uint32_t)wave; r < (uint32_t)rows; r += NWAVES) {
+            const uint32_t shift = row_shift(r);
+            const uint32_t limit = (seg_bytes + shift + 15u) & ~15u;
+            const char* row = src0 + (int64_t)r * Wd * (int64_t)sizeof(TI) - shift;
+            for (uint32_t cb = 0; cb < limit; cb += 1024u) {
+                const uint32_t at = cb + (uint32_t)lane * 16u;
+                if (at < limit) {
+                    __builtin_amdgcn_global_load_lds((rg_global_cptr_t)(row + at), (rg_lds_ptr_t)(lds + r * pitch + cb), 16,
+                                                     0, 0);
+                }
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();
+        // KX: columns read, at least as many as any lane visits; every lane visits at least KMIN
+        auto sums = [&](auto kx, auto kmin) {
+            constexpr int KX = decltype(kx)::value, KMIN = decltype(kmin)::value;
+            for (int q = 0; q < HQ; q++) {
+                const int32_t n_rows = __builtin_amdgcn_readlane(meta_pack, q);
+                if (n_rows < 0) {
+                    break;
+                }
+                uint32_t r = (uint32_t)(__builtin_amdgcn_readlane(meta_pack, 8 + q) - tile_y0);
+                float acc = 0.0f;
+#pragma unroll 2
+                for (int j = 0; j < n_rows; j++, r++) {
+                    const float y_lerp = __builtin_bit_cast(
+                        float, __builtin_amdgcn_readlane(__builtin_bit_cast(int32_t, lerp_pack), q * kPlaneVisits + j));
+                    float t[KX + 1];
+                    weighted_columns<TI, KX>(lds, lane_off + (r * pitch + row_shift(r)), y_lerp, neg_zero_v, t);
+#pragma unroll
+                    for (int k = 0; k < KX; k++) {
+                        const float v = t[k] * xl[k];
+                        acc = (k < KMIN || k < nx) ? acc + v : acc;
+                    }
+                }
+                if (col_ok) {
+                    store_streaming<TO>(yp + (int64_t)(H0 + wave + q * NWAVES) * Ws, acc);
+                }
+            }
+        };
+        typedef std::integral_constant<int, 0> k0;
+        typedef std::integral_constant<int, 4> k4;
+        if (nx_max <= 2) {
+            sums(std::integral_constant<int, 2>{}, k0{});
+        } else if (nx_max <= 4) {
+            (nx_min >= 4) ? sums(k4{}, k4{}) : sums(k4{}, k0{});
+        } else if (nx_max <= 5) {
+            (nx_min >= 4) ? sums(std::integral_constant<int, 5>{}, k4{}) : sums(std::integral_constant<int, 5>{}, k0{});
+        } else if (nx_max <= 6) {
+            (nx_min >= 4) ? sums(std::integral_constant<int, 6>{}, k4{}) : sums(std::integral_constant<int, 6>{}, k0{});
+        } else {
+            (nx_min >= 6) ? sums(std::integral_constant<int, 8>{}, std::integral_constant<int, 6>{})
+                          : sums(std::integral_constant<int, 8>{}, k0{});
+        }
+        __syncthreads();  // the tile is overwritten by the next plane
+    }
+}
+
+struct PlaneTile {
+    int32_t rows = 0;  // 0: the variant does not apply
+    int32_t lds_bytes = 0;
+};
+
+template <typename TI>
+int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t* need_words = nullptr);
+
+// Eight visits a side at most (growth by up to four), elements anywhere.  The estimate of the rectangle sizes the
+// launch; the kernel measures it and reads a larger one from global memory.
+template <typename TI>
+PlaneTile plane_tile(const ResizeGradArgs& a)
+{
+    PlaneTile t;
+    if (a.user_scales || (a.channels_last && a.C != 1) || !(a.scale_h >= 0.25f) || !(a.scale_w >= 0.25f) ||
+        reinterpret_cast<uintptr_t>(a.x) % sizeof(TI) != 0) {
+        return t;
+    }
+    // resize_grad_lds_kernel spends fewer instructions on a visit and its set-up pays off over eight planes and more:
+    // fp16 64 planes of 1080x1920 from 2160x3840 405 us there, 452 here.  It takes rows on the word grid; above growth
+    // by about 2.6 its tiles get lower than 8 x 128 and read too much twice.
+    const int64_t wide_tiles = ((a.Ws + kTileCols - 1) / kTileCols) * ((a.Hs + 7) / 8);
+    if (wide_tiles * a.N * a.C >= 8 * kWantBlocks && lds_tile_rows<TI>(a, kGradCapWords) == 8) {
+        return t;
+    }
+    const double per_col = 1.0 / (double)a.scale_w, per_row = 1.0 / (double)a.scale_h;
+    // a tile visits per_col incoming columns for each of its own and two more a side, and a segment is rounded out
+    const double pitch = ((kPlaneCols + 2.0) * per_col + 2.0) * sizeof(TI) + 30.0;
+    for (const int32_t rows : {16, 8}) {
+        const double bytes = ((rows + 2.0) * per_row + 2.0) * pitch + kPlanePad;
+        const int64_t tiles = ((a.Hs + rows - 1) / rows) * ((a.Ws + kPlaneCols - 1) / kPlaneCols) * a.N * a.C;
+        if (bytes <= (rows == 16 ? kPlaneTallBytes : kPlaneMostBytes) && (rows == 8 || tiles >= 1024)) {
+            t.rows = rows;
+            t.lds_bytes = ((int32_t)bytes + 64) / 64 * 64;
+            break;
+        }
+    }
+    return t;
+}
+
+template <typename TI, typename TO>
+hipError_t run_planes(const ResizeGradArgs& a, const PlaneTile& t, hipStream_t stream, bool* handled)
+{
+    const int64_t planes = a.N * a.C;
+    const int64_t tiles_x = (a.Ws + kPlaneCols - 1) / kPlaneCols, tiles_y = (a.Hs + t.rows - 1) / t.rows;
+    const int64_t tiles = tiles_x * tiles_y;
+    // a workgroup walks over several planes, all of them as many, with the geometry and weights it computed once
+    const int64_t want_blocks = 4096;  // 2048: within 2 us; 8192: 6 us slower where planes are small
+    int64_t slots = (want_blocks + tiles - 1) / tiles;
+    slots = slots < planes ? slots : planes;
+    const int64_t walk = (planes + slots - 1) / slots;
+    slots = (planes + walk - 1) / walk;
+    const int64_t blocks = (tiles * slots + 7) / 8 * 8;  // padded for the XCD mapping of the kernel
+    if (blocks > (int64_t)INT32_MAX) {
+        return hipSuccess;
+    }
+    *handled = true;
+#define OPSCV_RGP(HP)                                                                                                \
+    hipLaunchKernelGGL((resize_grad_planes_kernel<TI, TO, HP>), dim3((unsigned)blocks), dim3(kGradThreads), t.lds_bytes, \
+                       stream, (const TI*)a.x, (TO*)a.y, planes, (int32_t)a.Hs, (int32_t)a.Ws, (int32_t)a.Hd,         \
+                       (int32_t)a.Wd, a.scale_h, a.scale_w, a.inv_scale_h, a.inv_scale_w, t.rows, t.lds_bytes, -0.0f, \
+                       (uint32_t)tiles_x, (uint32_t)tiles_y, (uint32_t)slots)
+    if (a.half_pixel) {
+        OPSCV_RGP(true);
+    } else {
+        OPSCV_RGP(false);
+    }
+#undef OPSCV_RGP
+    return hipGetLastError();
+}
+
 // Output rows per workgroup for the LDS variant (0: use the gather kernel).  The estimate only sizes the launch;
 // the kernel measures the rectangle itself.
 template <typename TI>
-int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t* need_words = nullptr)
+int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t* need_words)
 {
     constexpr int EPW = 4 / (int)sizeof(TI);
     const int64_t ci = a.channels_last ? a.C : 1;  // row elements per pixel
@@ -546,6 +866,14 @@ int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t* need_
 template <typename TI, typename TO>
 hipError_t run(const ResizeGradArgs& a, hipStream_t stream)
 {
+    const PlaneTile planes_tile = plane_tile<TI>(a);
+    if (planes_tile.rows > 0) {
+        bool handled = false;
+        const hipError_t e = run_planes<TI, TO>(a, planes_tile, stream, &handled);
+        if (handled) {
+            return e;
+        }
+    }
     constexpr int32_t kCapWords = kGradCapWords;
     int32_t lds_words = kCapWords;
     const int32_t tile_rows = lds_tile_rows<TI>(a, kCapWords, &lds_words);
@@ -558,10 +886,9 @@ hipError_t run(const ResizeGradArgs& a, hipStream_t stream)
         const int64_t planes = a.channels_last ? a.N : a.N * a.C;
         const int64_t row_elems = a.Ws * ci;
         // A workgroup walks over several planes with the tile geometry and column weights it computed once; enough
-        // workgroups are launched to keep every CU supplied (want_blocks), the rest of the planes are looped over.
+        // workgroups are launched to keep every CU supplied (kWantBlocks), the rest of the planes are looped over.
         const int64_t tiles = ((row_elems + kTileCols - 1) / kTileCols) * ((a.Hs + tile_rows - 1) / tile_rows);
-        const int64_t want_blocks = 8192;
-        int64_t zdim = (want_blocks + tiles - 1) / tiles;
+        int64_t zdim = (kWantBlocks + tiles - 1) / tiles;
         zdim = zdim < planes ? zdim : planes;
         zdim = zdim < 65535 ? zdim : 65535;
         const int64_t tiles_x = (row_elems + kTileCols - 1) / kTileCols, tiles_y = (a.Hs + tile_rows - 1) / tile_rows;
@@ -628,6 +955,9 @@ const char* resize_grad_variant(const ResizeGradArgs& a)
 {
     if (a.user_scales) {
         return "resize_grad_gather_scales";
+    }
+    if ((a.elem_in == Elem::F32 ? plane_tile<float>(a) : plane_tile<uint16_t>(a)).rows > 0) {
+        return "resize_grad_lds";
     }
     constexpr int32_t kCapWords = kGradCapWords;
     const int32_t rows = (a.elem_in == Elem::F32) ? lds_tile_rows<float>(a, kCapWords)

@@ -1,0 +1,87 @@
+"""Tiled kernels at the edges of their tiles, bit for bit against the oracle: the direct sampler's tiles
+(gs2d_kernels.hip), the row groups of the flat resize (resize_flat_lds_kernel.hpp) and the planes variant of the resize
+gradient (resize_grad.hip)."""
+import numpy as np
+import pytest
+
+import inputs as I
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(a, b):
+    return np.array_equal(np.ascontiguousarray(a).view(np.uint8), np.ascontiguousarray(b).view(np.uint8))
+
+
+# (input, output): one tile of 32 x 16 and its remainders; channel runs of 4 + 1, 3, 2 and 1; planes above 32 KiB that
+# no LDS variant takes (odd widths of 16-bit elements, large fp32 planes); two columns
+PICTURES = [((1, 5, 301, 211), (16, 32)), ((2, 3, 301, 211), (33, 65)), ((1, 2, 401, 203), (17, 63)),
+            ((1, 1, 70001, 2), (40, 37)), ((1, 9, 301, 211), (31, 97))]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("interp", [0, 1])
+@pytest.mark.parametrize("pad", [0, 1, 2])
+@pytest.mark.parametrize("align", [False, True])
+def test_direct_tiles(oracle, device, aclnn, dtype, interp, pad, align):
+    import torch
+    rng = np.random.default_rng(5000 + 10 * interp + 2 * pad + align)
+    for xs, out in PICTURES:
+        x = I.cast_np(rng.standard_normal(xs).astype(np.float32), dtype)
+        g32 = rng.uniform(-1.3, 1.3, (xs[0],) + out + (2,)).astype(np.float32)
+        if interp == 0:  # what a non-finite coordinate gives: the whole pixel NaN
+            g32[0, 0, :3, 0] = [np.inf, -np.inf, np.nan]
+            g32[0, -1, -3:, 1] = [np.inf, -np.inf, np.nan]
+        g32[0, 1, :2] = [[3e38, 0.1], [0.1, -3e38]] if dtype != "fp16" else [[6e4, 0.1], [0.1, -6e4]]
+        g = I.cast_np(g32, dtype)
+        ref = oracle.grid_sampler2d(x, g, interp, pad, align, dtype=I.oracle_code(dtype))
+        with aclnn.option("gs_variant", 1):
+            got = aclnn.grid_sampler2d(I.to_torch(x, dtype, device), I.to_torch(g, dtype, device), interp, pad, align)
+        torch.cuda.synchronize()
+        a, b = I.as_f32(I.from_torch(got, dtype), dtype), I.as_f32(ref, dtype)
+        assert np.array_equal(np.isnan(a), np.isnan(b)), (xs, out)
+        assert np.array_equal(a[~np.isnan(a)], b[~np.isnan(b)]), (xs, out)
+
+
+# (gradient's planes, size it is reduced to): growth by four (eight visits), three, two, none and a half; one column and
+# one row more than a tile of 64 x 16; tiles of 16 rows (1024 of them and more) and of 8; rows of one element
+GROWTH = [((1, 3, 257, 513), (65, 129)), ((300, 1, 67, 259), (17, 65)), ((1, 2, 51, 195), (17, 65)),
+          ((2, 3, 33, 129), (16, 64)), ((1, 4, 17, 66), (17, 65)), ((1, 4, 9, 33), (17, 65)), ((1, 1, 4, 1), (3, 1)),
+          ((1, 2, 64, 255), (16, 64)), ((1, 2, 31, 511), (16, 128))]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("align", [False, True])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_resize_gradient_planes(oracle, device, aclnn, dtype, align, offset):
+    import torch
+    rng = np.random.default_rng(5100 + align)
+    for gs, small in GROWTH:
+        g = I.cast_np(rng.standard_normal(gs).astype(np.float32), dtype)
+        ref = oracle.upsample_bilinear2d_backward(g, small, align, dtype=I.oracle_code(dtype))
+        t = I.to_torch(g, dtype, device)
+        base = torch.empty(t.numel() + offset, dtype=t.dtype, device=device)  # a view that starts off the 4-byte grid
+        view = base[offset:].view(t.shape)
+        view.copy_(t)
+        got = aclnn.upsample_bilinear2d_backward(view, gs[:2] + small, align)
+        torch.cuda.synchronize()
+        assert _same(I.from_torch(got, dtype), ref), (gs, small)
+
+
+# (input, output): groups of consecutive rows with a short last group, a last band of one row, more groups than rows;
+# rows that shrink take the groups in turn
+FLAT = [((1, 3, 65, 129), (257, 513)), ((2, 40, 7, 9), (29, 31)), ((1, 1, 3, 5), (4, 1000)), ((3, 2, 11, 40), (12, 41)),
+        ((1, 7, 33, 50), (20, 77)), ((1, 600, 5, 6), (9, 8))]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("align", [False, True])
+def test_flat_resize_groups(oracle, device, aclnn, dtype, align):
+    import torch
+    rng = np.random.default_rng(5200 + align)
+    for xs, out in FLAT:
+        x = I.cast_np(rng.standard_normal(xs).astype(np.float32), dtype)
+        ref = oracle.upsample_bilinear2d(x, out, align, dtype=I.oracle_code(dtype))
+        got = aclnn.upsample_bilinear2d(I.to_torch(x, dtype, device), out, align)
+        torch.cuda.synchronize()
+        assert _same(I.from_torch(got, dtype), ref), (xs, out)

@@ -29,7 +29,9 @@ struct FlatLdsParams {
     int32_t band_rows;  // output rows per workgroup
     int32_t cl;         // column lanes = ceil(Wd / V)
     int32_t rg;         // row groups at work: at most THREADS / cl
+    int32_t group_rows;  // 0: the groups take a band's rows in turn; else consecutive rows of a group
     int32_t gran;       // bytes per lane of the asynchronous copy: 16 or 4; 1: 16 in the shifted layout (kernel)
+    int32_t streaming;  // 1: mark the output stores non-temporal
     int32_t raw_lambda;  // fraction from the unclamped source coordinate (see axis_tap)
     float neg_zero;     // -0.0f, passed in so that fma(v, w, -0) is not folded back into a multiply
 };
@@ -114,29 +116,60 @@ __global__ __launch_bounds__(THREADS) void resize_flat_lds_kernel(const T* __res
 
         const __amdgpu_buffer_rsrc_t rsrc =
             __builtin_amdgcn_make_buffer_rsrc(y + pl * (int64_t)p.Hd * p.Wd, 0, out_plane_bytes, kRsBufferFlags);
-        for (int32_t h = active ? h_begin + group : h_end; h < h_end; h += p.rg) {
-            const AxisTap t = axis_tap<HALF_PIXEL>(h, p.scale_h, p.Hs, p.raw_lambda);
-            const char* r0 = lds + shift + (uint32_t)(t.i0 - ys_lo) * src_row_bytes;
-            const char* r1 = lds + shift + (uint32_t)(t.i1 - ys_lo) * src_row_bytes;
-            T tl[V], tr[V], bl[V], br[V];
+        // Consecutive rows of a group reuse the blended source rows they share, as in resize_band_lds_kernel.hpp: same
+        // operations in the same order.  The row index of a lane's group may differ from its wavefront's other group.
+        const bool runs = p.group_rows > 0;
+        const int32_t step = runs ? 1 : p.rg;
+        int32_t h = runs ? h_begin + group * p.group_rows : h_begin + group;
+        int32_t h_stop = (runs && h + p.group_rows < h_end) ? h + p.group_rows : h_end;
+        h_stop = active ? h_stop : h;
+        float ha[V], hb[V];  // blended source rows ya and yb
+        int32_t ya = -1, yb = -1;
+        auto blend_row = [&](float* hrow, int32_t ys) {
+            const char* row = lds + shift + (uint32_t)(ys - ys_lo) * src_row_bytes;
+            T l[V], r[V];
 #pragma unroll
             for (int i = 0; i < V; i++) {
-                tl[i] = *reinterpret_cast<const T*>(r0 + to0[i]);
-                tr[i] = *reinterpret_cast<const T*>(r0 + to1[i]);
-                bl[i] = *reinterpret_cast<const T*>(r1 + to0[i]);
-                br[i] = *reinterpret_cast<const T*>(r1 + to1[i]);
+                l[i] = *reinterpret_cast<const T*>(row + to0[i]);
+                r[i] = *reinterpret_cast<const T*>(row + to1[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < V; i++) {
+                // fma(v, w, -0) is v * w bit for bit; see resize_band_lds_kernel.hpp
+                hrow[i] = __builtin_fmaf(ElemIO<T>::load(&l[i]), omdx[i], neg_zero) +
+                          __builtin_fmaf(ElemIO<T>::load(&r[i]), dx[i], neg_zero);
+            }
+        };
+        for (; h < h_stop; h += step) {
+            const AxisTap t = axis_tap<HALF_PIXEL>(h, p.scale_h, p.Hs, p.raw_lambda);
+            if (t.i0 != ya) {
+                if (t.i0 == yb) {
+#pragma unroll
+                    for (int i = 0; i < V; i++) {
+                        ha[i] = hb[i];
+                    }
+                } else {
+                    blend_row(ha, t.i0);
+                }
+                ya = t.i0;
+            }
+            if (t.i1 != yb) {
+                if (t.i1 == ya) {
+#pragma unroll
+                    for (int i = 0; i < V; i++) {
+                        hb[i] = ha[i];
+                    }
+                } else {
+                    blend_row(hb, t.i1);
+                }
+                yb = t.i1;
             }
             const float dy = t.lambda;
             const float omdy = 1.0f - dy;
             T outv[V];
 #pragma unroll
             for (int i = 0; i < V; i++) {
-                // fma(v, w, -0) is v * w bit for bit; see resize_band_lds_kernel.hpp
-                const float top = __builtin_fmaf(ElemIO<T>::load(&tl[i]), omdx[i], neg_zero) +
-                                  __builtin_fmaf(ElemIO<T>::load(&tr[i]), dx[i], neg_zero);
-                const float bot = __builtin_fmaf(ElemIO<T>::load(&bl[i]), omdx[i], neg_zero) +
-                                  __builtin_fmaf(ElemIO<T>::load(&br[i]), dx[i], neg_zero);
-                ElemIO<T>::store(&outv[i], omdy * top + dy * bot);
+                ElemIO<T>::store(&outv[i], omdy * ha[i] + dy * hb[i]);
             }
             typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
             u32x4 packed;
@@ -144,7 +177,11 @@ __global__ __launch_bounds__(THREADS) void resize_flat_lds_kernel(const T* __res
             const uint32_t out_off = (uint32_t)h * out_row_bytes + col_off;
             if (nvalid == V) {
                 // rows of a width that is not a multiple of V start anywhere: the store is element-aligned
-                __builtin_amdgcn_raw_buffer_store_b128(packed, rsrc, (int)out_off, 0, 2);
+                if (p.streaming) {
+                    __builtin_amdgcn_raw_buffer_store_b128(packed, rsrc, (int)out_off, 0, 2);
+                } else {
+                    __builtin_amdgcn_raw_buffer_store_b128(packed, rsrc, (int)out_off, 0, 0);
+                }
             } else {
                 // the lane that holds the ragged end of the row stores its elements singly
 #pragma unroll
@@ -152,10 +189,10 @@ __global__ __launch_bounds__(THREADS) void resize_flat_lds_kernel(const T* __res
                     if (i < nvalid) {
                         if constexpr (sizeof(T) == 4) {
                             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, outv[i]), rsrc,
-                                                                  (int)(out_off + i * 4), 0, 2);
+                                                                  (int)(out_off + i * 4), 0, 0);
                         } else {
                             __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(uint16_t, outv[i]), rsrc,
-                                                                  (int)(out_off + i * 2), 0, 2);
+                                                                  (int)(out_off + i * 2), 0, 0);
                         }
                     }
                 }

@@ -168,7 +168,13 @@ void launch(const char* api, aclnnStatus (*phase2)(void*, uint64_t, aclOpExecuto
         aclDestroyAclOpExecutor(ex);
         throw;
     }
-    const aclnnStatus st = phase2(bytes > 0 ? ws.data_ptr() : nullptr, bytes > 0 ? (uint64_t)ws.nbytes() : 0u, ex, queue);
+    void* const at = bytes > 0 ? ws.data_ptr() : nullptr;
+    const uint64_t size = bytes > 0 ? (uint64_t)ws.nbytes() : 0u;
+    aclnnStatus st;
+    // a launch may wait for room in the stream's queue: other Python threads go on meanwhile
+    Py_BEGIN_ALLOW_THREADS
+    st = phase2(at, size, ex, queue);
+    Py_END_ALLOW_THREADS
     if (st != ACLNN_SUCCESS) {
         raise_status(api, st);
     }

@@ -85,3 +85,22 @@ def test_flat_resize_groups(oracle, device, aclnn, dtype, align):
         got = aclnn.upsample_bilinear2d(I.to_torch(x, dtype, device), out, align)
         torch.cuda.synchronize()
         assert _same(I.from_torch(got, dtype), ref), (xs, out)
+
+
+# channels-last images whose rows shrink: units of 4 to 16 bytes, a last band of one, two and three rows, an output row
+# longer than a workgroup; a factor just below the rule and one far above it
+SHRINK = [((2, 31, 45, 3), (9, 20)), ((1, 24, 1000, 3), (15, 401)), ((1, 40, 30, 1), (10, 13)), ((1, 21, 18, 5), (14, 9)),
+          ((2, 50, 33, 2), (6, 33)), ((1, 97, 40, 12), (11, 9)), ((1, 13, 700, 20), (3, 301))]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("align", [False, True])
+def test_shrinking_images(oracle, device, aclnn, dtype, align):
+    import torch
+    rng = np.random.default_rng(5300 + align)
+    for xs, out in SHRINK:
+        x = I.cast_np(rng.standard_normal(xs).astype(np.float32), dtype)
+        ref = oracle.upsample_bilinear2d_nhwc(x, out, align, dtype=I.oracle_code(dtype))
+        got = aclnn.upsample_bilinear2d(I.to_torch(x, dtype, device), out, align, channels_last=True)
+        torch.cuda.synchronize()
+        assert _same(I.from_torch(got, dtype), ref), (xs, out)

@@ -218,7 +218,8 @@ __global__ __launch_bounds__(kDirectThreads) void gs2d_direct_kernel(const T* __
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Direct variant in tiles: bilinear and nearest samples of planes that no LDS variant takes (fp32 pictures, odd sizes).
+// Direct variant in tiles: samples of planes that no LDS variant takes (fp32 pictures, odd sizes); bicubic unless padded
+// with zeros (run_direct).
 //
 // A run of 64 output pixels along a row crosses 32 input rows under a rotation of 30 degrees and touches as many cache
 // lines with every load; a patch of 16 x 4 pixels about 14.  A wavefront takes two such patches, one below the other, a
@@ -248,6 +249,28 @@ __device__ __forceinline__ PairBits load_pair(__amdgpu_buffer_rsrc_t plane, uint
 }
 
 template <typename T>
+__device__ __forceinline__ void load_quad(__amdgpu_buffer_rsrc_t plane, uint32_t at, T* q)
+{
+    if constexpr (sizeof(T) == 2) {
+        const auto bits = __builtin_amdgcn_raw_buffer_load_b64(plane, (int)at, 0, 0);
+        __builtin_memcpy(q, &bits, 8);
+    } else {
+        const auto bits = __builtin_amdgcn_raw_buffer_load_b128(plane, (int)at, 0, 0);
+        __builtin_memcpy(q, &bits, 16);
+    }
+}
+
+template <typename T>
+__device__ __forceinline__ T load_one(__amdgpu_buffer_rsrc_t plane, uint32_t at)
+{
+    if constexpr (sizeof(T) == 2) {
+        return __builtin_bit_cast(T, (uint16_t)__builtin_amdgcn_raw_buffer_load_b16(plane, (int)at, 0, 0));
+    } else {
+        return __builtin_bit_cast(T, (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(plane, (int)at, 0, 0));
+    }
+}
+
+template <typename T>
 __device__ __forceinline__ void store_at(__amdgpu_buffer_rsrc_t plane, uint32_t at, float v)
 {
     T e;
@@ -266,7 +289,6 @@ __global__ __launch_bounds__(kDirectThreads) void gs2d_direct_tile_kernel(const 
                                                                           int32_t Wout, int32_t chan_chunk, uint32_t tiles_x,
                                                                           uint32_t tiles_y)
 {
-    static_assert(INTERP == 0 || INTERP == 1, "bilinear or nearest");
     const int32_t c_first = (int32_t)blockIdx.y * chan_chunk;
     const int32_t C = (c_first + chan_chunk < C_all) ? chan_chunk : C_all - c_first;
     const uint32_t per_xcd = gridDim.x >> 3, xcd = blockIdx.x & 7u, turn = blockIdx.x >> 3;
@@ -368,6 +390,70 @@ __global__ __launch_bounds__(kDirectThreads) void gs2d_direct_tile_kernel(const 
             channels(std::integral_constant<int, 2>{});
         } else if (left == 1) {
             channels(std::integral_constant<int, 1>{});
+        }
+    } else if constexpr (INTERP == 2) {
+        // one patch after the other: a channel's sixteen taps are loads enough
+#pragma unroll
+        for (int j = 0; j < kPatches; j++) {
+            const BicubicTap b = decide_bicubic<PAD, ALIGN>(gx[j], gy[j], H, W);
+            const bool nan = b.flag != 0;  // every channel NaN
+            bool row_in[4], col_in[4];
+            uint32_t row_at[4], col_at[4];  // bytes
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                row_in[k] = !nan && b.by[k] >= 0 && b.by[k] < H;
+                col_in[k] = !nan && b.bx[k] >= 0 && b.bx[k] < W;
+                row_at[k] = row_in[k] ? (uint32_t)b.by[k] * (uint32_t)W * (uint32_t)sizeof(T) : 0u;
+                col_at[k] = col_in[k] ? (uint32_t)b.bx[k] * (uint32_t)sizeof(T) : 0u;
+            }
+            // four neighbouring columns inside the image for every lane of the wavefront: one load a row
+            const bool in_a_row = !nan && b.bx[0] >= 0 && b.bx[3] < W && b.bx[1] == b.bx[0] + 1 &&
+                                  b.bx[2] == b.bx[0] + 2 && b.bx[3] == b.bx[0] + 3;
+            auto channels = [&](auto quads) {
+                const T* xc = xp;
+                T* yc = yp;
+#pragma unroll 2
+                for (int32_t c = 0; c < C; c++) {
+                    const __amdgpu_buffer_rsrc_t plane =
+                        __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(xc), 0, in_bytes, kTileBufferFlags);
+                    T q[4][4];
+                    if constexpr (decltype(quads)::value) {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            load_quad<T>(plane, row_at[r] + col_at[0], q[r]);
+                        }
+                    } else {
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+#pragma unroll
+                            for (int k = 0; k < 4; k++) {
+                                q[r][k] = load_one<T>(plane, row_at[r] + col_at[k]);
+                            }
+                        }
+                    }
+                    float row[4];
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        float v[4];
+#pragma unroll
+                        for (int k = 0; k < 4; k++) {
+                            v[k] = (decltype(quads)::value || col_in[k]) ? ElemIO<T>::load(&q[r][k]) : 0.0f;
+                        }
+                        const float sum = bicubic_weighted_sum(b.cx[0], b.cx[1], b.cx[2], b.cx[3], v[0], v[1], v[2], v[3]);
+                        row[r] = row_in[r] ? sum : 0.0f;
+                    }
+                    const float out = bicubic_weighted_sum(b.cy[0], b.cy[1], b.cy[2], b.cy[3], row[0], row[1], row[2], row[3]);
+                    store_at<T>(__builtin_amdgcn_make_buffer_rsrc(yc, 0, out_bytes, kTileBufferFlags), out_at[j],
+                                nan ? __builtin_nanf("") : out);
+                    xc += in_plane;
+                    yc += out_plane;
+                }
+            };
+            if (__builtin_amdgcn_ballot_w64(!in_a_row) == 0) {
+                channels(std::true_type{});
+            } else {
+                channels(std::false_type{});
+            }
         }
     } else {
         uint32_t at[kPatches];
@@ -510,7 +596,10 @@ inline int blocks_for(int64_t items, int threads)
 template <typename T, int INTERP, int PAD, bool ALIGN>
 hipError_t run_direct(const GridSamplerArgs& a, hipStream_t stream)
 {
-    if constexpr (INTERP != 2) {
+    // Bicubic under zeros padding stays with the kernel below, which leaves the loads of rows outside the image out:
+    // scattered points on fp32 4x64x200x200 284 us there, 306 in tiles; under border padding 364 and 314, turned by 25
+    // degrees 111 and 71, 8x3x720x1280 164 and 135, fp16 8x3x719x1279 179 and 164 (scattered 1690 and 687).
+    if constexpr (INTERP != 2 || PAD != 0) {
         // Tiles where lines are shared between the rows of an output: planes beyond the 32 KiB of a CU's first-level
         // cache.  Counts that fit the launch, offsets in a plane that fit 32 bits.
         const int64_t tx = (a.Wout + kTileCols - 1) / kTileCols, ty = (a.Hout + kTileLines - 1) / kTileLines;

@@ -784,11 +784,12 @@ PlaneTile plane_tile(const ResizeGradArgs& a)
         reinterpret_cast<uintptr_t>(a.x) % sizeof(TI) != 0) {
         return t;
     }
-    // resize_grad_lds_kernel spends fewer instructions on a visit and its set-up pays off over eight planes and more:
-    // fp16 64 planes of 1080x1920 from 2160x3840 405 us there, 452 here.  It takes rows on the word grid; above growth
+    // resize_grad_lds_kernel spends fewer instructions on a visit and its set-up pays off over four planes and more: fp16
+    // 64 planes of 1080x1920 from 2160x3840 (sixteen planes a workgroup) 405 us there, 452 here; 128 of 160x240 from
+    // 320x480 (less than one) 38 and 29, which puts equal times at about four.  It takes rows on the word grid; above growth
     // by about 2.6 its tiles get lower than 8 x 128 and read too much twice.
     const int64_t wide_tiles = ((a.Ws + kTileCols - 1) / kTileCols) * ((a.Hs + 7) / 8);
-    if (wide_tiles * a.N * a.C >= 8 * kWantBlocks && lds_tile_rows<TI>(a, kGradCapWords) == 8) {
+    if (wide_tiles * a.N * a.C >= 4 * kWantBlocks && lds_tile_rows<TI>(a, kGradCapWords) == 8) {
         return t;
     }
     const double per_col = 1.0 / (double)a.scale_w, per_row = 1.0 / (double)a.scale_h;

@@ -229,10 +229,15 @@ FlatPlan make_flat_plan(const ResizeArgs& a)
     // fp16 8x512x200x200 (328 MB) 121 / 92, fp32 8x256x112x112 (103 MB) 23.7 / 21.0, 8x32x257x516 (136 MB) 41.7 / 30.1;
     // lines of fp32 rows beyond the last-level cache are better written through: 8x64x257x513 (270 MB) 57.2 / 62.2.
     const int64_t out_bytes = planes * a.Hd * a.Wd * (int64_t)sizeof(T);
-    fp.p.streaming = (out_bytes < kFlatPlainBytes || (sizeof(T) == 4 && out_bytes >= kLastLevelBytes)) ? 1 : 0;
+    // Beyond the cache, rows of whole vectors keep rows in turn and non-temporal stores, which then fill shared lines
+    // together: fp16 8x512x200x200 86 us, 92 otherwise, fp32 8x256x200x200 (328 MB) 82 and 92 (ragged rows bf16
+    // 8x256x257x513, 540 MB: 233 and 161).
+    const bool in_turn = out_bytes >= kLastLevelBytes && (a.Wd * (int64_t)sizeof(T)) % 16 == 0;
+    fp.p.streaming =
+        (out_bytes < kFlatPlainBytes || in_turn || (sizeof(T) == 4 && out_bytes >= kLastLevelBytes)) ? 1 : 0;
     // Rows that grow share source rows: a group's rows are consecutive then, and blended rows are kept (half to an eighth
     // of the LDS reads; with plain stores 33 us on bf16 8x64x65x129 to 257x513, 59 before).
-    fp.p.group_rows = (a.Hd > a.Hs) ? (int32_t)((band_rows + rg - 1) / rg) : 0;
+    fp.p.group_rows = (a.Hd > a.Hs && !in_turn) ? (int32_t)((band_rows + rg - 1) / rg) : 0;
     fp.p.gran = gran;
     fp.p.neg_zero = -0.0f;
     fp.p.raw_lambda = a.raw_lambda;

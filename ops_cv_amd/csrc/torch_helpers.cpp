@@ -8,9 +8,12 @@
 // The functions are positional and internal to the package: aclnn.py holds the public signatures and their defaults.
 #include <Python.h>
 
+#include <optional>
+
 #include <ATen/core/Tensor.h>
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
+#include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -118,22 +121,71 @@ aclDataType dtype_of(const at::Tensor& t)
     throw Raised();
 }
 
+// The stream of a call on the device `like`: the caller's, or PyTorch's current one where the caller named none.
+//
+// The caching allocator orders the reuse of a block by the stream that the block was allocated for.  A stream that is not
+// the current one is therefore made current for the call, so that the workspace and the outputs come from its own pool:
+// nothing on another stream still uses them, and they go back to work that runs behind the call's kernels.  The caller's
+// tensors are noted as in use on that stream, the outputs that the call made as in use on the caller's current one.
+class Queue {
+public:
+    Queue(PyObject* stream, const at::Tensor& like)
+    {
+        if (!like.is_cuda()) {
+            return;  // refused by Call::handle
+        }
+        if (stream == Py_None) {
+            raw_ = c10::hip::getCurrentHIPStream().stream();
+            return;
+        }
+        raw_ = (hipStream_t)int_arg(stream);
+        current_ = c10::hip::getCurrentHIPStream(like.device().index());
+        if (raw_ != current_->stream()) {
+            own_ = c10::hip::getStreamFromExternal(raw_, like.device().index());
+            c10::hip::setCurrentHIPStream(*own_);
+        }
+    }
+    ~Queue()
+    {
+        if (own_) {
+            c10::hip::setCurrentHIPStream(*current_);
+        }
+    }
+    Queue(const Queue&) = delete;
+    Queue& operator=(const Queue&) = delete;
+    void* raw() const { return (void*)raw_; }
+    // a tensor that the kernels of the call use; `made`: by the call, else the caller's
+    void uses(const at::Tensor& t, bool made) const
+    {
+        if (own_ && t.is_cuda()) {
+            c10::hip::HIPCachingAllocator::recordStream(t.storage().data_ptr(), made ? *current_ : *own_);
+        }
+    }
+
+private:
+    std::optional<c10::hip::HIPStream> current_, own_;
+    hipStream_t raw_ = nullptr;
+};
+
 // The handles of one call, destroyed at its end.
 class Call {
 public:
+    explicit Call(const Queue& queue) : queue_(queue) {}
     ~Call()
     {
         for (int i = 0; i < count_; i++) {
             aclDestroyTensor(handles_[i]);
         }
     }
-    // aclTensor over the tensor's memory; strides and storage offset of the view are honoured
-    aclTensor* handle(const at::Tensor& t, aclFormat fmt = ACL_FORMAT_ND)
+    // aclTensor over the tensor's memory; strides and storage offset of the view are honoured.  `made`: an output that
+    // the call allocated
+    aclTensor* handle(const at::Tensor& t, aclFormat fmt = ACL_FORMAT_ND, bool made = false)
     {
         if (!t.is_cuda()) {
             PyErr_SetString(PyExc_RuntimeError, "ops_cv_amd needs device tensors: there is no CPU path");
             throw Raised();
         }
+        queue_.uses(t, made);
         const int64_t storage = (int64_t)(t.storage().nbytes() / t.element_size());
         aclTensor* h = aclCreateTensor(t.sizes().data(), (uint64_t)t.dim(), dtype_of(t), t.strides().data(),
                                        t.storage_offset(), fmt, &storage, 1, const_cast<void*>(t.storage().data()));
@@ -144,24 +196,25 @@ public:
     }
 
 private:
+    const Queue& queue_;
     aclTensor* handles_[5];
     int count_ = 0;
 };
 
 // Second phase: the workspace (the caller's where it is large enough) and the launch on the stream.
 void launch(const char* api, aclnnStatus (*phase2)(void*, uint64_t, aclOpExecutor*, aclrtStream), uint64_t bytes,
-            aclOpExecutor* ex, const at::Tensor& like, PyObject* workspace, PyObject* stream)
+            aclOpExecutor* ex, const at::Tensor& like, PyObject* workspace, const Queue& queue)
 {
-    void* queue = nullptr;
     at::Tensor ws;
     try {
-        queue = (stream == Py_None) ? (void*)c10::hip::getCurrentHIPStream().stream() : (void*)int_arg(stream);
         if (bytes > 0) {
             if (workspace != Py_None) {
                 ws = tensor_arg(workspace);
             }
             if (!ws.defined() || (uint64_t)ws.nbytes() < bytes) {
                 ws = at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
+            } else {
+                queue.uses(ws, false);
             }
         }
     } catch (...) {
@@ -173,7 +226,7 @@ void launch(const char* api, aclnnStatus (*phase2)(void*, uint64_t, aclOpExecuto
     aclnnStatus st;
     // a launch may wait for room in the stream's queue: other Python threads go on meanwhile
     Py_BEGIN_ALLOW_THREADS
-    st = phase2(at, size, ex, queue);
+    st = phase2(at, size, ex, queue.raw());
     Py_END_ALLOW_THREADS
     if (st != ACLNN_SUCCESS) {
         raise_status(api, st);
@@ -216,9 +269,10 @@ PyObject* grid_sampler2d(PyObject*, PyObject* const* a, Py_ssize_t n)
     return guarded(n, 8, [&]() -> PyObject* {
         const at::Tensor& x = tensor_arg(a[0]);
         const at::Tensor& g = tensor_arg(a[1]);
+        const Queue queue(a[7], x);
         const at::Tensor y = out_arg(a[5], x, {size_of(x, 0), size_of(x, 1), size_of(g, 1), size_of(g, 2)});
-        Call c;
-        aclTensor *hx = c.handle(x), *hg = c.handle(g), *hy = c.handle(y);
+        Call c(queue);
+        aclTensor *hx = c.handle(x), *hg = c.handle(g), *hy = c.handle(y, ACL_FORMAT_ND, a[5] == Py_None);
         uint64_t ws = 0;
         aclOpExecutor* ex = nullptr;
         const aclnnStatus st = aclnnGridSampler2DGetWorkspaceSize(hx, hg, int_arg(a[2]), int_arg(a[3]), bool_arg(a[4]), hy,
@@ -226,7 +280,7 @@ PyObject* grid_sampler2d(PyObject*, PyObject* const* a, Py_ssize_t n)
         if (st != ACLNN_SUCCESS) {
             raise_status("aclnnGridSampler2DGetWorkspaceSize", st);
         }
-        launch("aclnnGridSampler2D", aclnnGridSampler2D, ws, ex, x, a[6], a[7]);
+        launch("aclnnGridSampler2D", aclnnGridSampler2D, ws, ex, x, a[6], queue);
         return THPVariable_Wrap(y);
     });
 }
@@ -240,10 +294,11 @@ PyObject* grid_sampler3d(PyObject*, PyObject* const* a, Py_ssize_t n)
         const bool last = bool_arg(a[8]);
         const aclFormat fmt = last ? ACL_FORMAT_NDHWC : ACL_FORMAT_NCDHW;
         const int64_t d = size_of(g, 1), h = size_of(g, 2), w = size_of(g, 3);
+        const Queue queue(a[7], x);
         const at::Tensor y = last ? out_arg(a[5], x, {size_of(x, 0), d, h, w, size_of(x, 4)})
                                   : out_arg(a[5], x, {size_of(x, 0), size_of(x, 1), d, h, w});
-        Call c;
-        aclTensor *hx = c.handle(x, fmt), *hg = c.handle(g), *hy = c.handle(y, fmt);
+        Call c(queue);
+        aclTensor *hx = c.handle(x, fmt), *hg = c.handle(g), *hy = c.handle(y, fmt, a[5] == Py_None);
         uint64_t ws = 0;
         aclOpExecutor* ex = nullptr;
         const aclnnStatus st = aclnnGridSampler3DGetWorkspaceSize(hx, hg, int_arg(a[2]), int_arg(a[3]), bool_arg(a[4]), hy,
@@ -251,7 +306,7 @@ PyObject* grid_sampler3d(PyObject*, PyObject* const* a, Py_ssize_t n)
         if (st != ACLNN_SUCCESS) {
             raise_status("aclnnGridSampler3DGetWorkspaceSize", st);
         }
-        launch("aclnnGridSampler3D", aclnnGridSampler3D, ws, ex, x, a[6], a[7]);
+        launch("aclnnGridSampler3D", aclnnGridSampler3D, ws, ex, x, a[6], queue);
         return THPVariable_Wrap(y);
     });
 }
@@ -268,13 +323,14 @@ PyObject* sampler_backward(PyObject* const* a, bool volume, const char* api1, ba
     const at::Tensor& go = tensor_arg(a[0]);
     const at::Tensor& x = tensor_arg(a[1]);
     const at::Tensor& g = tensor_arg(a[2]);
+    const Queue queue(a[10], x);
     const at::Tensor dx = (a[7] == Py_None) ? at::empty_like(x) : tensor_arg(a[7]);
     const at::Tensor dg = (a[8] == Py_None) ? at::empty_like(g) : tensor_arg(a[8]);
     const aclFormat fmt = !volume ? ACL_FORMAT_ND : (bool_arg(a[11]) ? ACL_FORMAT_NDHWC : ACL_FORMAT_NCDHW);
     const auto flags = sequence_arg<bool>(a[6], bool_arg);
-    Call c;
-    aclTensor *hgo = c.handle(go, fmt), *hx = c.handle(x, fmt), *hg = c.handle(g), *hdx = c.handle(dx, fmt),
-              *hdg = c.handle(dg);
+    Call c(queue);
+    aclTensor *hgo = c.handle(go, fmt), *hx = c.handle(x, fmt), *hg = c.handle(g),
+              *hdx = c.handle(dx, fmt, a[7] == Py_None), *hdg = c.handle(dg, ACL_FORMAT_ND, a[8] == Py_None);
     const int64_t interp = int_arg(a[3]), pad = int_arg(a[4]);
     const bool align = bool_arg(a[5]);
     aclBoolArray* mask = aclCreateBoolArray(flags.data(), flags.size());
@@ -285,7 +341,7 @@ PyObject* sampler_backward(PyObject* const* a, bool volume, const char* api1, ba
     if (st != ACLNN_SUCCESS) {
         raise_status(api1, st);
     }
-    launch(api2, phase2, ws, ex, x, a[9], a[10]);
+    launch(api2, phase2, ws, ex, x, a[9], queue);
     PyObject* pair = PyTuple_New(2);
     if (pair == nullptr) {
         throw Raised();
@@ -321,6 +377,7 @@ PyObject* upsample_bilinear2d(PyObject*, PyObject* const* a, Py_ssize_t n)
         const auto size = ints_arg(a[1]);
         const bool last = bool_arg(a[8]);
         const aclFormat fmt = last ? ACL_FORMAT_NHWC : ACL_FORMAT_NCHW;
+        const Queue queue(a[7], x);
         at::Tensor y;
         if (a[5] == Py_None) {
             if (size.size() < 2) {
@@ -332,8 +389,8 @@ PyObject* upsample_bilinear2d(PyObject*, PyObject* const* a, Py_ssize_t n)
         } else {
             y = tensor_arg(a[5]);
         }
-        Call c;
-        aclTensor *hx = c.handle(x, fmt), *hy = c.handle(y, fmt);
+        Call c(queue);
+        aclTensor *hx = c.handle(x, fmt), *hy = c.handle(y, fmt, a[5] == Py_None);
         const bool align = bool_arg(a[2]);
         const double sh = float_arg(a[3]), sw = float_arg(a[4]);
         aclIntArray* hs = aclCreateIntArray(size.data(), size.size());
@@ -344,7 +401,7 @@ PyObject* upsample_bilinear2d(PyObject*, PyObject* const* a, Py_ssize_t n)
         if (st != ACLNN_SUCCESS) {
             raise_status("aclnnUpsampleBilinear2dGetWorkspaceSize", st);
         }
-        launch("aclnnUpsampleBilinear2d", aclnnUpsampleBilinear2d, ws, ex, x, a[6], a[7]);
+        launch("aclnnUpsampleBilinear2d", aclnnUpsampleBilinear2d, ws, ex, x, a[6], queue);
         return THPVariable_Wrap(y);
     });
 }
@@ -361,6 +418,7 @@ PyObject* resize(PyObject*, PyObject* const* a, Py_ssize_t n)
         }
         const bool last = bool_arg(a[6]);
         const aclFormat fmt = last ? ACL_FORMAT_NHWC : ACL_FORMAT_NCHW;
+        const Queue queue(a[5], x);
         at::Tensor y;
         if (a[3] == Py_None) {
             c10::SmallVector<int64_t, 8> sizes(x.sizes().begin(), x.sizes().end());
@@ -375,8 +433,8 @@ PyObject* resize(PyObject*, PyObject* const* a, Py_ssize_t n)
         } else {
             y = tensor_arg(a[3]);
         }
-        Call c;
-        aclTensor *hx = c.handle(x, fmt), *hy = c.handle(y, fmt);
+        Call c(queue);
+        aclTensor *hx = c.handle(x, fmt), *hy = c.handle(y, fmt, a[3] == Py_None);
         c10::SmallVector<float, 8> scales(scales64.begin(), scales64.end());
         aclFloatArray* hs = aclCreateFloatArray(scales.data(), scales.size());
         uint64_t ws = 0;
@@ -386,7 +444,7 @@ PyObject* resize(PyObject*, PyObject* const* a, Py_ssize_t n)
         if (st != ACLNN_SUCCESS) {
             raise_status("aclnnResizeGetWorkspaceSize", st);
         }
-        launch("aclnnResize", aclnnResize, ws, ex, x, a[4], a[5]);
+        launch("aclnnResize", aclnnResize, ws, ex, x, a[4], queue);
         return THPVariable_Wrap(y);
     });
 }
@@ -399,10 +457,11 @@ PyObject* upsample_bilinear2d_backward(PyObject*, PyObject* const* a, Py_ssize_t
         const auto isize = ints_arg(a[1]);
         const bool last = bool_arg(a[8]);
         const aclFormat fmt = last ? ACL_FORMAT_NHWC : ACL_FORMAT_NCHW;
+        const Queue queue(a[7], go);
         const at::Tensor y = out_arg(a[5], go, isize);
         const int64_t osize[2] = {size_of(go, last ? 1 : 2), size_of(go, last ? 2 : 3)};
-        Call c;
-        aclTensor *hgo = c.handle(go, fmt), *hy = c.handle(y, fmt);
+        Call c(queue);
+        aclTensor *hgo = c.handle(go, fmt), *hy = c.handle(y, fmt, a[5] == Py_None);
         const bool align = bool_arg(a[2]);
         const double sh = float_arg(a[3]), sw = float_arg(a[4]);
         aclIntArray* ho = aclCreateIntArray(osize, 2);
@@ -416,7 +475,7 @@ PyObject* upsample_bilinear2d_backward(PyObject*, PyObject* const* a, Py_ssize_t
         if (st != ACLNN_SUCCESS) {
             raise_status("aclnnUpsampleBilinear2dBackwardGetWorkspaceSize", st);
         }
-        launch("aclnnUpsampleBilinear2dBackward", aclnnUpsampleBilinear2dBackward, ws, ex, go, a[6], a[7]);
+        launch("aclnnUpsampleBilinear2dBackward", aclnnUpsampleBilinear2dBackward, ws, ex, go, a[6], queue);
         return THPVariable_Wrap(y);
     });
 }

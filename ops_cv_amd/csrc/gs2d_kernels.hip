@@ -15,6 +15,7 @@
 #include <cstdlib>
 
 #include "gs2d_common.hpp"
+#include "gs2d_direct_plan.hpp"
 #include "kernels.hpp"
 #include "options.hpp"
 #include "sampler_math.hpp"
@@ -22,8 +23,6 @@
 namespace opscv {
 
 namespace {
-
-constexpr int kDirectThreads = 256;
 
 // ---------------------------------------------------------------------------------------------------------
 // Direct variant: taps are read straight from global memory (through L1/L2).  Works for every shape.
@@ -231,10 +230,6 @@ __global__ __launch_bounds__(kDirectThreads) void gs2d_direct_kernel(const T* __
 // (nearest 99 -> 37), 4x64x200x200 49 -> 21, with scattered points 541 -> 429 and 93 -> 80; fp16 8x3x719x1279 64 -> 61
 // (nearest 55 -> 31).
 // ---------------------------------------------------------------------------------------------------------
-constexpr int kPatchW = 16, kPatchH = 4, kPatches = 2;
-constexpr int kTileCols = 2 * kPatchW, kTileLines = 2 * kPatches * kPatchH;
-static_assert(kTileCols * kTileLines == kPatches * kDirectThreads, "four wavefronts, two by two");
-
 constexpr uint32_t kTileBufferFlags = 0x00020000u;  // raw buffer, 32-bit data format
 
 // two neighbouring elements, aligned to one of them
@@ -600,26 +595,14 @@ hipError_t run_direct(const GridSamplerArgs& a, hipStream_t stream)
     // scattered points on fp32 4x64x200x200 284 us there, 306 in tiles; under border padding 364 and 314, turned by 25
     // degrees 111 and 71, 8x3x720x1280 164 and 135, fp16 8x3x719x1279 179 and 164 (scattered 1690 and 687).
     if constexpr (INTERP != 2 || PAD != 0) {
-        // Tiles where lines are shared between the rows of an output: planes beyond the 32 KiB of a CU's first-level
-        // cache.  Counts that fit the launch, offsets in a plane that fit 32 bits.
-        const int64_t tx = (a.Wout + kTileCols - 1) / kTileCols, ty = (a.Hout + kTileLines - 1) / kTileLines;
-        const int64_t limit = INT32_MAX / (int64_t)sizeof(T);
-        if (a.Win >= 2 && a.Hin * a.Win * (int64_t)sizeof(T) > (32 << 10) && a.Hin * a.Win <= limit &&
-            a.Wout >= kTileCols && a.Hout >= kTileLines && a.Hout <= limit / a.Wout && a.N <= INT32_MAX / (tx * ty)) {
-            const int64_t tiles = a.N * tx * ty;
-            // runs of channels to different workgroups where the tiles alone are too few, as below
-            int64_t chunks = (4096 + tiles - 1) / tiles;
-            chunks = chunks < a.C ? chunks : a.C;
-            int64_t run = (a.C + chunks - 1) / chunks;
-            run = (run + 3) / 4 * 4;
-            const int64_t runs = (a.C + run - 1) / run;
-            if (runs <= 65535) {
-                hipLaunchKernelGGL((gs2d_direct_tile_kernel<T, INTERP, PAD, ALIGN>), dim3((unsigned)tiles, (unsigned)runs),
-                                   dim3(kDirectThreads), 0, stream, (const T*)a.x, (const T*)a.grid, (T*)a.y, (int32_t)a.C,
-                                   (int32_t)a.Hin, (int32_t)a.Win, (int32_t)a.Hout, (int32_t)a.Wout, (int32_t)run,
-                                   (uint32_t)tx, (uint32_t)ty);
-                return hipGetLastError();
-            }
+        const DirectTilePlan t = direct_tile_plan(a);
+        if (t.ok) {
+            hipLaunchKernelGGL((gs2d_direct_tile_kernel<T, INTERP, PAD, ALIGN>),
+                               dim3((unsigned)t.tiles, (unsigned)t.chan_runs), dim3(kDirectThreads), 0, stream,
+                               (const T*)a.x, (const T*)a.grid, (T*)a.y, (int32_t)a.C, (int32_t)a.Hin, (int32_t)a.Win,
+                               (int32_t)a.Hout, (int32_t)a.Wout, (int32_t)t.chan_run, (uint32_t)t.tiles_x,
+                               (uint32_t)t.tiles_y);
+            return hipGetLastError();
         }
     }
     const int64_t total = a.N * a.Hout * a.Wout;

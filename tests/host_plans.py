@@ -1,0 +1,34 @@
+"""ctypes view of the kernels' launch plans (host_plans.cpp over the headers of ops_cv_amd/csrc), which need no GPU."""
+import ctypes
+import os
+import subprocess
+import tempfile
+
+_HERE = os.path.dirname(os.path.abspath(__file__))
+_ROOT = os.path.dirname(_HERE)
+ELEM = {"fp32": 0, "fp16": 1, "bf16": 2}
+_lib = None
+
+
+def lib():
+    global _lib
+    if _lib is None:
+        with tempfile.TemporaryDirectory() as d:
+            so = os.path.join(d, "libhost_plans.so")
+            subprocess.check_call(["g++", "-std=c++17", "-O1", "-ftrapv", "-Wall", "-Wextra", "-shared", "-fPIC",
+                                   "-I" + os.path.join(_ROOT, "include"),
+                                   "-I" + os.path.join(_ROOT, "ops_cv_amd", "csrc"),
+                                   os.path.join(_HERE, "host_plans.cpp"), "-o", so])
+            _lib = ctypes.CDLL(so)
+    return _lib
+
+
+def _call(name, count, elem, *args):
+    out = (ctypes.c_int64 * count)()
+    taken = getattr(lib(), name)(ctypes.c_int(ELEM[elem]), *[ctypes.c_int64(a) for a in args], out)
+    return tuple(out) if taken else None
+
+
+def direct_tiles(dtype, n, c, h, w, ho, wo):
+    """(tiles, channel runs) of the direct sampler's tiled kernel, None where it is not taken."""
+    return _call("direct_tiles", 2, dtype, n, c, h, w, ho, wo)

@@ -1,0 +1,29 @@
+"""Launch plans at the limits of a launch: work items along an axis fit 32 bits, so a launch of 256-thread workgroups
+holds fewer than 2^24 of them."""
+import random
+
+import pytest
+
+import host_plans as P
+
+MOST_BLOCKS = (2**32 - 1) // 256
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
+def test_direct_tiles_fit_the_launch(dtype):
+    # 33 x 17 pixels take four tiles: the last batch that fits, and the first that does not
+    assert P.direct_tiles(dtype, MOST_BLOCKS // 4, 1, 301, 211, 17, 33)[0] == MOST_BLOCKS // 4 * 4
+    assert P.direct_tiles(dtype, MOST_BLOCKS // 4 + 1, 1, 301, 211, 17, 33) is None
+    # large planes: 724 x 1448 tiles an item; sixteen items fit and seventeen do not
+    assert P.direct_tiles(dtype, 16, 1, 301, 211, 23168, 23168)[0] < 2**24
+    assert P.direct_tiles(dtype, 17, 1, 301, 211, 23168, 23168) is None
+    # the counts of a batch beyond 32 bits
+    assert P.direct_tiles(dtype, 2**31 - 1, 1, 301, 211, 16000, 16000) is None
+    rng = random.Random(7)
+    for _ in range(2000):
+        n, c = (int(2 ** rng.uniform(0, 31)) for _ in range(2))
+        h, w = (int(2 ** rng.uniform(1, 15)) for _ in range(2))
+        ho, wo = (int(2 ** rng.uniform(0, 15)) for _ in range(2))
+        p = P.direct_tiles(dtype, n, c, h, w, ho, wo)
+        if p is not None:
+            assert 0 < p[0] <= MOST_BLOCKS and p[0] * 512 >= n * ho * wo and 0 < p[1] <= 65535

@@ -16,13 +16,12 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "resize_grad_plan.hpp"
 #include "sampler_math.hpp"
 
 namespace opscv {
 
 namespace {
-
-constexpr int kGradThreads = 256;
 
 // User-scale template (resize_bilinear_v2_grad_simt_determine_scales.h:77-305), for scales that are not the ratio
 // of the sizes.  Same walk, but the source coordinate of every visited row/column is recomputed as
@@ -270,11 +269,6 @@ __device__ __forceinline__ float tile_sum_fixed(const float* lane_rows, int32_t 
     return acc;
 }
 
-constexpr int kTileCols = 128;
-constexpr int64_t kWantBlocks = 8192;
-constexpr int32_t kGradCapWords = 12288;  // at most 48 KB of LDS per workgroup (fp32 words, one per tile element)
-constexpr int kTileGroups = kGradThreads / kTileCols;  // row groups of a workgroup
-
 // IL: channels-last tensors, taken as planes whose rows are W * ci elements (element j of a row is channel j % ci of
 // pixel j / ci); "columns" then count row elements, a lane's visited columns sit ci elements apart, and the column
 // geometry (first visit, count, weights) is that of the lane's pixel.
@@ -304,8 +298,8 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
     constexpr int EPW = 4 / (int)sizeof(TI);  // elements per 4-byte word
     extern __shared__ __attribute__((aligned(16))) uint32_t tile_words[];
     __shared__ int32_t s_x1, s_y1, s_nx, s_nx_min;
-    const int tx = threadIdx.x % kTileCols, ty = threadIdx.x / kTileCols;
-    const int32_t W0 = (int32_t)block_x * kTileCols, H0 = (int32_t)block_y * tile_rows;
+    const int tx = threadIdx.x % kGradTileCols, ty = threadIdx.x / kGradTileCols;
+    const int32_t W0 = (int32_t)block_x * kGradTileCols, H0 = (int32_t)block_y * tile_rows;
     const float offset = HALF_PIXEL ? 0.5f : 0.0f;
     const float last_y = (float)Hs - 1.0f, last_x = (float)Ws - 1.0f;
     auto first_visit = [&](int32_t i, float inv_scale, int32_t len_dst) {
@@ -359,7 +353,7 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
         }
     }
     if (tx == 0) {
-        for (int32_t H = H0 + ty; H < H0 + tile_rows && H < Hs; H += kTileGroups) {
+        for (int32_t H = H0 + ty; H < H0 + tile_rows && H < Hs; H += kGradTileGroups) {
             atomicMax(&s_y1, end_visit(H, first_visit(H, inv_scale_h, Hd), scale_h, Hd));
         }
     }
@@ -396,7 +390,7 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
     const int32_t x_base = (nx > 0) ? in_x_start * ci + ch - tile_x0 : 0;
 
     // rows visited by each of this wavefront's outgoing rows, and their weights (see tile_sum_fixed)
-    constexpr int HQ = 8 / kTileGroups;  // outgoing rows per lane at the largest tile height
+    constexpr int HQ = 8 / kGradTileGroups;  // outgoing rows per lane at the largest tile height
     static_assert(HQ * kRowWeights <= 64, "the row weights of a wavefront are packed one per lane");
     float lerp_pack = 0.0f;  // lane q * kRowWeights + j: weight of visited row j of outgoing row q (a uniform table)
     int32_t meta_pack = -1;  // lane q: rows outgoing row q visits (-1: no such row in this tile); lane 8 + q: the first
@@ -404,7 +398,7 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
     const int32_t lane_id = (int32_t)threadIdx.x & 63;
 #pragma unroll
     for (int q = 0; q < HQ; q++) {
-        const int32_t H = __builtin_amdgcn_readfirstlane(H0 + ty + q * kTileGroups);
+        const int32_t H = __builtin_amdgcn_readfirstlane(H0 + ty + q * kGradTileGroups);
         if (H < H0 + tile_rows && H < Hs) {
             const int32_t start = first_visit(H, inv_scale_h, Hd);
             float out_y = ((float)start + offset) * scale_h - offset;
@@ -476,7 +470,7 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
                         acc = (nx_min >= 4) ? OPSCV_TILE_SUM(6, 4) : OPSCV_TILE_SUM(6, 0);
                     }
 #undef OPSCV_TILE_SUM
-                    store_streaming<TO>(yp + (int64_t)q * kTileGroups * Wse, acc);
+                    store_streaming<TO>(yp + (int64_t)q * kGradTileGroups * Wse, acc);
                 }
             };
             static_assert(HQ == 4, "one call per outgoing row of a lane");
@@ -485,7 +479,7 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
             one_row(std::integral_constant<int, 2>{});
             one_row(std::integral_constant<int, 3>{});
         } else if (col_ok) {
-            for (int32_t H = H0 + ty; H < H0 + tile_rows && H < Hs; H += kTileGroups) {
+            for (int32_t H = H0 + ty; H < H0 + tile_rows && H < Hs; H += kGradTileGroups) {
                 const int32_t in_y_start = first_visit(H, inv_scale_h, Hd);
                 const float out_y_start = ((float)in_y_start + offset) * scale_h - offset;
                 float acc;
@@ -534,13 +528,6 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
 // us).  4x32x160x240 against resize_grad_lds_kernel (fp16 even rows / fp32) and the gather (bf16 odd rows), before ->
 // after: growth by 0.6 24 -> 16 / 24 -> 16 / 28 -> 17 us, by two 38 -> 29 / 40 -> 28 / 63 -> 31, by three 95 -> 51 /
 // 105 -> 47 / 118 -> 45, by four 136 -> 57 / 174 -> 109 (a growth above four: the gather as before).
-constexpr int kPlaneCols = 64;
-constexpr int kPlaneVisits = 8;                 // most rows, and most columns, an outgoing element may visit
-constexpr int kPlaneRows = 16;                  // most outgoing rows of a tile
-constexpr int32_t kPlaneTallBytes = 24 * 1024;  // tiles of 16 rows up to here: six workgroups and more fit a CU
-constexpr int32_t kPlaneMostBytes = 48 * 1024;  // tiles of 8 rows up to here
-constexpr int32_t kPlanePad = 64;               // bytes behind the last row that a lane's last columns may be read from
-
 typedef __attribute__((address_space(1))) const void* rg_global_cptr_t;
 typedef __attribute__((address_space(3))) void* rg_lds_ptr_t;
 
@@ -766,69 +753,15 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_planes_kernel(
     }
 }
 
-struct PlaneTile {
-    int32_t rows = 0;  // 0: the variant does not apply
-    int32_t lds_bytes = 0;
-};
-
-template <typename TI>
-int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t* need_words = nullptr);
-
-// Eight visits a side at most (growth by up to four), elements anywhere.  The estimate of the rectangle sizes the
-// launch; the kernel measures it and reads a larger one from global memory.
-template <typename TI>
-PlaneTile plane_tile(const ResizeGradArgs& a)
-{
-    PlaneTile t;
-    if (a.user_scales || (a.channels_last && a.C != 1) || !(a.scale_h >= 0.25f) || !(a.scale_w >= 0.25f) ||
-        reinterpret_cast<uintptr_t>(a.x) % sizeof(TI) != 0) {
-        return t;
-    }
-    // resize_grad_lds_kernel spends fewer instructions on a visit and its set-up pays off over four planes and more: fp16
-    // 64 planes of 1080x1920 from 2160x3840 (sixteen planes a workgroup) 405 us there, 452 here; 128 of 160x240 from
-    // 320x480 (less than one) 38 and 29, which puts equal times at about four.  It takes rows on the word grid; above growth
-    // by about 2.6 its tiles get lower than 8 x 128 and read too much twice.
-    const int64_t wide_tiles = ((a.Ws + kTileCols - 1) / kTileCols) * ((a.Hs + 7) / 8);
-    if (wide_tiles * a.N * a.C >= 4 * kWantBlocks && lds_tile_rows<TI>(a, kGradCapWords) == 8) {
-        return t;
-    }
-    const double per_col = 1.0 / (double)a.scale_w, per_row = 1.0 / (double)a.scale_h;
-    // a tile visits per_col incoming columns for each of its own and two more a side, and a segment is rounded out
-    const double pitch = ((kPlaneCols + 2.0) * per_col + 2.0) * sizeof(TI) + 30.0;
-    for (const int32_t rows : {16, 8}) {
-        const double bytes = ((rows + 2.0) * per_row + 2.0) * pitch + kPlanePad;
-        const int64_t tiles = ((a.Hs + rows - 1) / rows) * ((a.Ws + kPlaneCols - 1) / kPlaneCols) * a.N * a.C;
-        if (bytes <= (rows == 16 ? kPlaneTallBytes : kPlaneMostBytes) && (rows == 8 || tiles >= 1024)) {
-            t.rows = rows;
-            t.lds_bytes = ((int32_t)bytes + 64) / 64 * 64;
-            break;
-        }
-    }
-    return t;
-}
-
 template <typename TI, typename TO>
-hipError_t run_planes(const ResizeGradArgs& a, const PlaneTile& t, hipStream_t stream, bool* handled)
+hipError_t run_planes(const ResizeGradArgs& a, const PlaneTile& t, hipStream_t stream)
 {
     const int64_t planes = a.N * a.C;
-    const int64_t tiles_x = (a.Ws + kPlaneCols - 1) / kPlaneCols, tiles_y = (a.Hs + t.rows - 1) / t.rows;
-    const int64_t tiles = tiles_x * tiles_y;
-    // a workgroup walks over several planes, all of them as many, with the geometry and weights it computed once
-    const int64_t want_blocks = 4096;  // 2048: within 2 us; 8192: 6 us slower where planes are small
-    int64_t slots = (want_blocks + tiles - 1) / tiles;
-    slots = slots < planes ? slots : planes;
-    const int64_t walk = (planes + slots - 1) / slots;
-    slots = (planes + walk - 1) / walk;
-    const int64_t blocks = (tiles * slots + 7) / 8 * 8;  // padded for the XCD mapping of the kernel
-    if (blocks > (int64_t)INT32_MAX) {
-        return hipSuccess;
-    }
-    *handled = true;
 #define OPSCV_RGP(HP)                                                                                                \
-    hipLaunchKernelGGL((resize_grad_planes_kernel<TI, TO, HP>), dim3((unsigned)blocks), dim3(kGradThreads), t.lds_bytes, \
-                       stream, (const TI*)a.x, (TO*)a.y, planes, (int32_t)a.Hs, (int32_t)a.Ws, (int32_t)a.Hd,         \
-                       (int32_t)a.Wd, a.scale_h, a.scale_w, a.inv_scale_h, a.inv_scale_w, t.rows, t.lds_bytes, -0.0f, \
-                       (uint32_t)tiles_x, (uint32_t)tiles_y, (uint32_t)slots)
+    hipLaunchKernelGGL((resize_grad_planes_kernel<TI, TO, HP>), dim3((unsigned)t.blocks), dim3(kGradThreads),        \
+                       t.lds_bytes, stream, (const TI*)a.x, (TO*)a.y, planes, (int32_t)a.Hs, (int32_t)a.Ws,          \
+                       (int32_t)a.Hd, (int32_t)a.Wd, a.scale_h, a.scale_w, a.inv_scale_h, a.inv_scale_w, t.rows,     \
+                       t.lds_bytes, -0.0f, (uint32_t)t.tiles_x, (uint32_t)t.tiles_y, (uint32_t)t.slots)
     if (a.half_pixel) {
         OPSCV_RGP(true);
     } else {
@@ -838,46 +771,16 @@ hipError_t run_planes(const ResizeGradArgs& a, const PlaneTile& t, hipStream_t s
     return hipGetLastError();
 }
 
-// Output rows per workgroup for the LDS variant (0: use the gather kernel).  The estimate only sizes the launch;
-// the kernel measures the rectangle itself.
-template <typename TI>
-int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t* need_words)
-{
-    constexpr int EPW = 4 / (int)sizeof(TI);
-    const int64_t ci = a.channels_last ? a.C : 1;  // row elements per pixel
-    if (a.user_scales || (a.Wd * ci) % EPW != 0 || reinterpret_cast<uintptr_t>(a.x) % 4 != 0 ||
-        a.Ws * ci > INT32_MAX || a.Wd * ci > INT32_MAX) {
-        return 0;
-    }
-    const double per_col = (double)a.Wd / (double)a.Ws, per_row = (double)a.Hd / (double)a.Hs;
-    // a tile of kTileCols outgoing elements visits that many times per_col incoming ones, plus two pixels either side
-    const double cols = kTileCols * per_col + (2.0 * per_col + 2.0) * (double)ci + EPW;
-    for (int32_t rows = 8; rows >= kTileGroups; rows /= 2) {
-        const double need = (rows * per_row + 2.0 * per_row + 2.0) * cols;  // fp32 words: one per element
-        if (need <= (double)cap_words) {
-            if (need_words != nullptr) {
-                *need_words = (int32_t)need + 1;
-            }
-            return rows;
-        }
-    }
-    return 0;
-}
-
 template <typename TI, typename TO>
 hipError_t run(const ResizeGradArgs& a, hipStream_t stream)
 {
-    const PlaneTile planes_tile = plane_tile<TI>(a);
+    const PlaneTile planes_tile = plane_tile(a);
     if (planes_tile.rows > 0) {
-        bool handled = false;
-        const hipError_t e = run_planes<TI, TO>(a, planes_tile, stream, &handled);
-        if (handled) {
-            return e;
-        }
+        return run_planes<TI, TO>(a, planes_tile, stream);
     }
     constexpr int32_t kCapWords = kGradCapWords;
     int32_t lds_words = kCapWords;
-    const int32_t tile_rows = lds_tile_rows<TI>(a, kCapWords, &lds_words);
+    const int32_t tile_rows = lds_tile_rows(a, kCapWords, &lds_words);
     // the allocation follows the estimate so that more workgroups share a CU (their load and compute phases overlap);
     // a rectangle that turns out larger than the estimate is read from global memory by the kernel
     lds_words = (lds_words + 63) / 64 * 64;
@@ -888,13 +791,13 @@ hipError_t run(const ResizeGradArgs& a, hipStream_t stream)
         const int64_t row_elems = a.Ws * ci;
         // A workgroup walks over several planes with the tile geometry and column weights it computed once; enough
         // workgroups are launched to keep every CU supplied (kWantBlocks), the rest of the planes are looped over.
-        const int64_t tiles = ((row_elems + kTileCols - 1) / kTileCols) * ((a.Hs + tile_rows - 1) / tile_rows);
+        const int64_t tiles = ((row_elems + kGradTileCols - 1) / kGradTileCols) * ((a.Hs + tile_rows - 1) / tile_rows);
         int64_t zdim = (kWantBlocks + tiles - 1) / tiles;
         zdim = zdim < planes ? zdim : planes;
         zdim = zdim < 65535 ? zdim : 65535;
-        const int64_t tiles_x = (row_elems + kTileCols - 1) / kTileCols, tiles_y = (a.Hs + tile_rows - 1) / tile_rows;
+        const int64_t tiles_x = (row_elems + kGradTileCols - 1) / kGradTileCols, tiles_y = (a.Hs + tile_rows - 1) / tile_rows;
         const int64_t blocks = (tiles * zdim + 7) / 8 * 8;  // padded for the XCD mapping of the kernel
-        if (tiles_y <= 65535 && blocks <= (int64_t)INT32_MAX) {
+        if (tiles_y <= 65535 && fits_launch(blocks, kGradThreads)) {
             const dim3 grid((unsigned)blocks);
 #define OPSCV_RGL(HP, IL)                                                                                            \
     hipLaunchKernelGGL((resize_grad_lds_kernel<TI, TO, HP, IL>), grid, dim3(kGradThreads), lds_words * 4, stream,     \
@@ -957,12 +860,11 @@ const char* resize_grad_variant(const ResizeGradArgs& a)
     if (a.user_scales) {
         return "resize_grad_gather_scales";
     }
-    if ((a.elem_in == Elem::F32 ? plane_tile<float>(a) : plane_tile<uint16_t>(a)).rows > 0) {
+    if (plane_tile(a).rows > 0) {
         return "resize_grad_lds";
     }
     constexpr int32_t kCapWords = kGradCapWords;
-    const int32_t rows = (a.elem_in == Elem::F32) ? lds_tile_rows<float>(a, kCapWords)
-                                                  : lds_tile_rows<uint16_t>(a, kCapWords);
+    const int32_t rows = lds_tile_rows(a, kCapWords);
     return (rows > 0 && (a.Hs + rows - 1) / rows <= 65535) ? "resize_grad_lds" : "resize_grad_gather";
 }
 

@@ -1,0 +1,107 @@
+// Launch plans of the resize gradient's LDS kernels (resize_grad.hip): host arithmetic only.
+#pragma once
+
+#include <cstdint>
+
+#include "acl_types.hpp"
+#include "launch_limits.hpp"
+
+namespace opscv {
+
+constexpr int kGradThreads = 256;
+
+// ---- resize_grad_lds_kernel ----
+constexpr int kGradTileCols = 128;
+constexpr int64_t kWantBlocks = 8192;
+constexpr int32_t kGradCapWords = 12288;  // at most 48 KB of LDS per workgroup (fp32 words, one per tile element)
+constexpr int kGradTileGroups = kGradThreads / kGradTileCols;  // row groups of a workgroup
+
+// Output rows per workgroup for the LDS variant (0: use the gather kernel).  The estimate only sizes the launch;
+// the kernel measures the rectangle itself.
+inline int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t* need_words = nullptr)
+{
+    const int epw = 4 / elem_size(a.elem_in);
+    const int64_t ci = a.channels_last ? a.C : 1;  // row elements per pixel
+    if (a.user_scales || (a.Wd * ci) % epw != 0 || reinterpret_cast<uintptr_t>(a.x) % 4 != 0 ||
+        a.Ws * ci > INT32_MAX || a.Wd * ci > INT32_MAX) {
+        return 0;
+    }
+    const double per_col = (double)a.Wd / (double)a.Ws, per_row = (double)a.Hd / (double)a.Hs;
+    // a tile of kGradTileCols outgoing elements visits that many times per_col incoming ones, plus two pixels either side
+    const double cols = kGradTileCols * per_col + (2.0 * per_col + 2.0) * (double)ci + epw;
+    for (int32_t rows = 8; rows >= kGradTileGroups; rows /= 2) {
+        const double need = (rows * per_row + 2.0 * per_row + 2.0) * cols;  // fp32 words: one per element
+        if (need <= (double)cap_words) {
+            if (need_words != nullptr) {
+                *need_words = (int32_t)need + 1;
+            }
+            return rows;
+        }
+    }
+    return 0;
+}
+
+// ---- resize_grad_planes_kernel ----
+constexpr int kPlaneCols = 64;
+constexpr int kPlaneVisits = 8;                 // most rows, and most columns, an outgoing element may visit
+constexpr int kPlaneRows = 16;                  // most outgoing rows of a tile
+constexpr int32_t kPlaneTallBytes = 24 * 1024;  // tiles of 16 rows up to here: six workgroups and more fit a CU
+constexpr int32_t kPlaneMostBytes = 48 * 1024;  // tiles of 8 rows up to here
+constexpr int32_t kPlanePad = 64;               // bytes behind the last row that a lane's last columns may be read from
+
+struct PlaneTile {
+    int32_t rows = 0;  // 0: the variant does not apply
+    int32_t lds_bytes = 0;
+    int64_t tiles_x = 0, tiles_y = 0;
+    int64_t slots = 0;   // workgroups per tile; each takes every slots-th plane
+    int64_t blocks = 0;  // padded for the XCD mapping of the kernel
+};
+
+// Eight visits a side at most (growth by up to four), elements anywhere.  The estimate of the rectangle sizes the
+// launch; the kernel measures it and reads a larger one from global memory.
+inline PlaneTile plane_tile(const ResizeGradArgs& a)
+{
+    PlaneTile t;
+    const int esz = elem_size(a.elem_in);
+    if (a.user_scales || (a.channels_last && a.C != 1) || !(a.scale_h >= 0.25f) || !(a.scale_w >= 0.25f) ||
+        reinterpret_cast<uintptr_t>(a.x) % (uintptr_t)esz != 0) {
+        return t;
+    }
+    // resize_grad_lds_kernel spends fewer instructions on a visit and its set-up pays off over four planes and more: fp16
+    // 64 planes of 1080x1920 from 2160x3840 (sixteen planes a workgroup) 405 us there, 452 here; 128 of 160x240 from
+    // 320x480 (less than one) 38 and 29, which puts equal times at about four.  It takes rows on the word grid; above growth
+    // by about 2.6 its tiles get lower than 8 x 128 and read too much twice.
+    const int64_t wide_tiles = ((a.Ws + kGradTileCols - 1) / kGradTileCols) * ((a.Hs + 7) / 8);
+    if (wide_tiles * a.N * a.C >= 4 * kWantBlocks && lds_tile_rows(a, kGradCapWords) == 8) {
+        return t;
+    }
+    const int64_t planes = a.N * a.C;
+    const double per_col = 1.0 / (double)a.scale_w, per_row = 1.0 / (double)a.scale_h;
+    // a tile visits per_col incoming columns for each of its own and two more a side, and a segment is rounded out
+    const double pitch = ((kPlaneCols + 2.0) * per_col + 2.0) * esz + 30.0;
+    t.tiles_x = (a.Ws + kPlaneCols - 1) / kPlaneCols;
+    for (const int32_t rows : {16, 8}) {
+        const double bytes = ((rows + 2.0) * per_row + 2.0) * pitch + kPlanePad;
+        t.tiles_y = (a.Hs + rows - 1) / rows;
+        if (bytes <= (rows == 16 ? kPlaneTallBytes : kPlaneMostBytes) &&
+            (rows == 8 || t.tiles_x * t.tiles_y * planes >= 1024)) {
+            t.rows = rows;
+            t.lds_bytes = ((int32_t)bytes + 64) / 64 * 64;
+            break;
+        }
+    }
+    // a workgroup walks over several planes, all of them as many, with the geometry and weights it computed once
+    const int64_t want_blocks = 4096;  // 2048: within 2 us; 8192: 6 us slower where planes are small
+    const int64_t tiles = t.tiles_x * t.tiles_y;
+    t.slots = (want_blocks + tiles - 1) / tiles;
+    t.slots = t.slots < planes ? t.slots : planes;
+    const int64_t walk = (planes + t.slots - 1) / t.slots;
+    t.slots = (planes + walk - 1) / walk;
+    t.blocks = (tiles * t.slots + 7) / 8 * 8;
+    if (!fits_launch(t.blocks, kGradThreads)) {  // tall planes of a few columns: the gather walks its elements
+        t.rows = 0;
+    }
+    return t;
+}
+
+}  // namespace opscv

@@ -1,5 +1,6 @@
 // The launch plans of the kernels, which are plain host arithmetic, for the tests (host_plans.py).
 #include "gs2d_direct_plan.hpp"
+#include "resize_grad_plan.hpp"
 
 using namespace opscv;
 
@@ -20,6 +21,31 @@ int direct_tiles(int elem, int64_t N, int64_t C, int64_t Hin, int64_t Win, int64
     out[0] = p.tiles;
     out[1] = p.chan_runs;
     return p.ok ? 1 : 0;
+}
+
+// tile rows, workgroups, planes a workgroup walks at most; 0 where the planes kernel is not taken.  Gradient of (Hs, Ws)
+// from (Hd, Wd), dense planes on a 16-byte boundary.
+int resize_grad_planes(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int align, int64_t* out)
+{
+    ResizeGradArgs a;
+    a.elem_in = a.elem_out = (Elem)elem;
+    a.half_pixel = align ? 0 : 1;
+    a.N = 1;
+    a.C = planes;
+    a.Hs = Hs;
+    a.Ws = Ws;
+    a.Hd = Hd;
+    a.Wd = Wd;
+    auto scale = [&](int64_t s, int64_t d) {
+        return align ? (d > 1 ? (float)(s - 1) / (float)(d - 1) : 0.0f) : (float)s / (float)d;
+    };
+    a.scale_h = scale(Hs, Hd);
+    a.scale_w = scale(Ws, Wd);
+    const PlaneTile t = plane_tile(a);
+    out[0] = t.rows;
+    out[1] = t.blocks;
+    out[2] = (planes + t.slots - 1) / (t.slots > 0 ? t.slots : 1);
+    return t.rows > 0 ? 1 : 0;
 }
 
 }  // extern "C"

@@ -32,3 +32,9 @@ def _call(name, count, elem, *args):
 def direct_tiles(dtype, n, c, h, w, ho, wo):
     """(tiles, channel runs) of the direct sampler's tiled kernel, None where it is not taken."""
     return _call("direct_tiles", 2, dtype, n, c, h, w, ho, wo)
+
+
+def resize_grad_planes(dtype, planes, small, large, align=False):
+    """(tile rows, workgroups, planes a workgroup walks at most) of the resize gradient's planes kernel, None where it
+    is not taken; the gradient of `small` from `large`, both (rows, columns)."""
+    return _call("resize_grad_planes", 3, dtype, planes, *small, *large, int(align))

@@ -27,3 +27,22 @@ def test_direct_tiles_fit_the_launch(dtype):
         p = P.direct_tiles(dtype, n, c, h, w, ho, wo)
         if p is not None:
             assert 0 < p[0] <= MOST_BLOCKS and p[0] * 512 >= n * ho * wo and 0 < p[1] <= 65535
+
+
+@pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
+def test_resize_gradient_planes_fit_the_launch(dtype):
+    # planes of one column: tiles of sixteen rows fill a launch at 2^28 rows
+    rows = 16 * (MOST_BLOCKS // 8 * 8)
+    if dtype != "fp32":  # which leaves that many tiles to resize_grad_lds_kernel, or its gather
+        assert P.resize_grad_planes(dtype, 1, (rows, 1), (rows + 1, 1))[1] == MOST_BLOCKS // 8 * 8
+    assert P.resize_grad_planes(dtype, 1, (rows + 1, 1), (rows + 2, 1)) is None
+    assert P.resize_grad_planes(dtype, 1, (2**31 - 2, 1), (2**31 - 1, 1)) is None
+    # many small planes: workgroups walk over them
+    assert P.resize_grad_planes(dtype, 2**31 - 1, (20, 30), (23, 31))[1] < 2**14
+    rng = random.Random(8)
+    for _ in range(2000):
+        h, w = (int(2 ** rng.uniform(0, 30)) for _ in range(2))
+        large = [max(1, int(v * 2 ** rng.uniform(-1, 2))) for v in (h, w)]
+        p = P.resize_grad_planes(dtype, int(2 ** rng.uniform(0, 12)), (h, w), large, rng.random() < 0.5)
+        if p is not None:
+            assert p[0] in (8, 16) and 0 < p[1] <= MOST_BLOCKS and p[1] % 8 == 0 and p[2] > 0

@@ -35,10 +35,10 @@ def test_resize_gradient_planes_fit_the_launch(dtype):
     rows = 16 * (MOST_BLOCKS // 8 * 8)
     if dtype != "fp32":  # which leaves that many tiles to resize_grad_lds_kernel, or its gather
         assert P.resize_grad_planes(dtype, 1, (rows, 1), (rows + 1, 1))[1] == MOST_BLOCKS // 8 * 8
+        # many small planes: workgroups walk over them
+        assert P.resize_grad_planes(dtype, 2**31 - 1, (20, 30), (23, 31))[1] < 2**14
     assert P.resize_grad_planes(dtype, 1, (rows + 1, 1), (rows + 2, 1)) is None
     assert P.resize_grad_planes(dtype, 1, (2**31 - 2, 1), (2**31 - 1, 1)) is None
-    # many small planes: workgroups walk over them
-    assert P.resize_grad_planes(dtype, 2**31 - 1, (20, 30), (23, 31))[1] < 2**14
     rng = random.Random(8)
     for _ in range(2000):
         h, w = (int(2 ** rng.uniform(0, 30)) for _ in range(2))

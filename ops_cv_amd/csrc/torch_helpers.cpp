@@ -185,10 +185,13 @@ public:
             PyErr_SetString(PyExc_RuntimeError, "ops_cv_amd needs device tensors: there is no CPU path");
             throw Raised();
         }
+        // a copy-on-write tensor gets memory of its own first: an output must not be written through into the tensor it
+        // was cloned from, and memory shared that way is not the allocator's to note as in use
+        void* const base = t.storage().mutable_data();
         queue_.uses(t, made);
         const int64_t storage = (int64_t)(t.storage().nbytes() / t.element_size());
         aclTensor* h = aclCreateTensor(t.sizes().data(), (uint64_t)t.dim(), dtype_of(t), t.strides().data(),
-                                       t.storage_offset(), fmt, &storage, 1, const_cast<void*>(t.storage().data()));
+                                       t.storage_offset(), fmt, &storage, 1, base);
         if (h != nullptr) {
             handles_[count_++] = h;
         }
@@ -206,6 +209,7 @@ void launch(const char* api, aclnnStatus (*phase2)(void*, uint64_t, aclOpExecuto
             aclOpExecutor* ex, const at::Tensor& like, PyObject* workspace, const Queue& queue)
 {
     at::Tensor ws;
+    void* at = nullptr;
     try {
         if (bytes > 0) {
             if (workspace != Py_None) {
@@ -213,7 +217,9 @@ void launch(const char* api, aclnnStatus (*phase2)(void*, uint64_t, aclOpExecuto
             }
             if (!ws.defined() || (uint64_t)ws.nbytes() < bytes) {
                 ws = at::empty({(int64_t)bytes}, like.options().dtype(at::kByte));
+                at = ws.mutable_data_ptr();
             } else {
+                at = ws.mutable_data_ptr();  // before it is noted, as in Call::handle
                 queue.uses(ws, false);
             }
         }
@@ -221,7 +227,6 @@ void launch(const char* api, aclnnStatus (*phase2)(void*, uint64_t, aclOpExecuto
         aclDestroyAclOpExecutor(ex);
         throw;
     }
-    void* const at = bytes > 0 ? ws.data_ptr() : nullptr;
     const uint64_t size = bytes > 0 ? (uint64_t)ws.nbytes() : 0u;
     aclnnStatus st;
     // a launch may wait for room in the stream's queue: other Python threads go on meanwhile

@@ -113,3 +113,24 @@ def test_memory_dropped_while_the_call_waits_on_its_stream(device, aclnn):
     del got
     assert _block(torch, ptr)[1] == "active_pending_free"
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", CALLS)
+def test_copy_on_write_outputs_leave_their_source_alone(device, aclnn, name):
+    """A lazily cloned tensor that is handed in as an output, or as the workspace, is written into memory of its own."""
+    import torch
+    call, outputs, needs_workspace = _calls(torch, aclnn, device)[name]
+    want = call()
+    want = want if isinstance(want, tuple) else (want,)
+    sources = {k: torch.full_like(t, 7.0) for k, t in zip(outputs, want)}
+    mine = {k: torch._lazy_clone(t) for k, t in sources.items()}
+    if needs_workspace:
+        sources["workspace"] = torch.full((4 << 20,), 7, dtype=torch.uint8, device=device)
+        mine["workspace"] = torch._lazy_clone(sources["workspace"])
+    got = call(**mine)
+    torch.cuda.synchronize()
+    for k, a, b in zip(outputs, want, got if isinstance(got, tuple) else (got,)):
+        assert b is mine[k] and torch.equal(a, b)
+    for k, t in sources.items():
+        assert bool((t == 7).all()), k

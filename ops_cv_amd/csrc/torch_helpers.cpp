@@ -61,13 +61,46 @@ int64_t int_arg(PyObject* o)
     return v;
 }
 
-double float_arg(PyObject* o)
+// int(o): what the extents of an array are made from where no tensor is allocated by them
+int64_t whole_arg(PyObject* o)
 {
-    const double v = PyFloat_AsDouble(o);
-    if (v == -1.0 && PyErr_Occurred() != nullptr) {
+    PyObject* whole = PyNumber_Long(o);
+    if (whole == nullptr) {
+        throw Raised();
+    }
+    const int64_t v = PyLong_AsLongLong(whole);
+    Py_DECREF(whole);
+    if (v == -1 && PyErr_Occurred() != nullptr) {
         throw Raised();
     }
     return v;
+}
+
+// float(o)
+double float_arg(PyObject* o)
+{
+    PyObject* number = PyNumber_Float(o);
+    if (number == nullptr) {
+        throw Raised();
+    }
+    const double v = PyFloat_AS_DOUBLE(number);
+    Py_DECREF(number);
+    return v;
+}
+
+// int(v); not a number or infinite: ValueError, OverflowError
+int64_t truncated(double v)
+{
+    PyObject* whole = PyLong_FromDouble(v);
+    if (whole == nullptr) {
+        throw Raised();
+    }
+    const int64_t t = PyLong_AsLongLong(whole);
+    Py_DECREF(whole);
+    if (t == -1 && PyErr_Occurred() != nullptr) {
+        throw Raised();
+    }
+    return t;
 }
 
 bool bool_arg(PyObject* o)
@@ -100,7 +133,12 @@ c10::SmallVector<T, 8> sequence_arg(PyObject* o, F&& one)
     return v;
 }
 
-c10::SmallVector<int64_t, 8> ints_arg(PyObject* o) { return sequence_arg<int64_t>(o, int_arg); }
+// the extents of a tensor; `allocates`: those of an output that the call allocates, which have to be integers, while
+// those of one that the caller brings may be any numbers
+c10::SmallVector<int64_t, 8> extents_arg(PyObject* o, bool allocates)
+{
+    return sequence_arg<int64_t>(o, allocates ? int_arg : whole_arg);
+}
 
 aclDataType dtype_of(const at::Tensor& t)
 {
@@ -238,9 +276,23 @@ void launch(const char* api, aclnnStatus (*phase2)(void*, uint64_t, aclOpExecuto
     }
 }
 
-at::Tensor out_arg(PyObject* out, const at::Tensor& like, at::IntArrayRef sizes)
+int64_t size_of(const at::Tensor& t, int64_t dim)
 {
-    return (out == Py_None) ? at::empty(sizes, like.options().memory_format(at::MemoryFormat::Contiguous)) : tensor_arg(out);
+    if (dim >= t.dim()) {
+        PyErr_SetString(PyExc_IndexError, "tuple index out of range");
+        throw Raised();
+    }
+    return t.sizes()[dim];
+}
+
+typedef c10::SmallVector<int64_t, 8> Sizes;
+
+// The caller's output, or one of the sizes that `sizes` gives.  They are asked for only then: operands of too few
+// dimensions beside a given output are the library's to refuse.
+template <typename F>
+at::Tensor out_arg(PyObject* out, const at::Tensor& like, F&& sizes)
+{
+    return (out == Py_None) ? at::empty(sizes(), like.options().memory_format(at::MemoryFormat::Contiguous)) : tensor_arg(out);
 }
 
 template <typename F>
@@ -259,15 +311,6 @@ PyObject* guarded(Py_ssize_t nargs, Py_ssize_t want, F&& body)
     END_HANDLE_TH_ERRORS
 }
 
-int64_t size_of(const at::Tensor& t, int64_t dim)
-{
-    if (dim >= t.dim()) {
-        PyErr_SetString(PyExc_IndexError, "tuple index out of range");
-        throw Raised();
-    }
-    return t.sizes()[dim];
-}
-
 // (inp, grid, interpolation, padding, align, out, workspace, stream)
 PyObject* grid_sampler2d(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
@@ -275,7 +318,9 @@ PyObject* grid_sampler2d(PyObject*, PyObject* const* a, Py_ssize_t n)
         const at::Tensor& x = tensor_arg(a[0]);
         const at::Tensor& g = tensor_arg(a[1]);
         const Queue queue(a[7], x);
-        const at::Tensor y = out_arg(a[5], x, {size_of(x, 0), size_of(x, 1), size_of(g, 1), size_of(g, 2)});
+        const at::Tensor y = out_arg(a[5], x, [&] {
+            return Sizes{size_of(x, 0), size_of(x, 1), size_of(g, 1), size_of(g, 2)};
+        });
         Call c(queue);
         aclTensor *hx = c.handle(x), *hg = c.handle(g), *hy = c.handle(y, ACL_FORMAT_ND, a[5] == Py_None);
         uint64_t ws = 0;
@@ -298,10 +343,11 @@ PyObject* grid_sampler3d(PyObject*, PyObject* const* a, Py_ssize_t n)
         const at::Tensor& g = tensor_arg(a[1]);
         const bool last = bool_arg(a[8]);
         const aclFormat fmt = last ? ACL_FORMAT_NDHWC : ACL_FORMAT_NCDHW;
-        const int64_t d = size_of(g, 1), h = size_of(g, 2), w = size_of(g, 3);
         const Queue queue(a[7], x);
-        const at::Tensor y = last ? out_arg(a[5], x, {size_of(x, 0), d, h, w, size_of(x, 4)})
-                                  : out_arg(a[5], x, {size_of(x, 0), size_of(x, 1), d, h, w});
+        const at::Tensor y = out_arg(a[5], x, [&] {
+            const int64_t n = size_of(x, 0), d = size_of(g, 1), h = size_of(g, 2), w = size_of(g, 3);
+            return last ? Sizes{n, d, h, w, size_of(x, 4)} : Sizes{n, size_of(x, 1), d, h, w};
+        });
         Call c(queue);
         aclTensor *hx = c.handle(x, fmt), *hg = c.handle(g), *hy = c.handle(y, fmt, a[5] == Py_None);
         uint64_t ws = 0;
@@ -379,21 +425,18 @@ PyObject* upsample_bilinear2d(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
     return guarded(n, 9, [&]() -> PyObject* {
         const at::Tensor& x = tensor_arg(a[0]);
-        const auto size = ints_arg(a[1]);
+        const auto size = extents_arg(a[1], a[5] == Py_None);
         const bool last = bool_arg(a[8]);
         const aclFormat fmt = last ? ACL_FORMAT_NHWC : ACL_FORMAT_NCHW;
         const Queue queue(a[7], x);
-        at::Tensor y;
-        if (a[5] == Py_None) {
+        const at::Tensor y = out_arg(a[5], x, [&] {
             if (size.size() < 2) {
                 PyErr_SetString(PyExc_IndexError, "output_size holds two extents");
                 throw Raised();
             }
-            y = last ? out_arg(a[5], x, {size_of(x, 0), size[0], size[1], size_of(x, 3)})
-                     : out_arg(a[5], x, {size_of(x, 0), size_of(x, 1), size[0], size[1]});
-        } else {
-            y = tensor_arg(a[5]);
-        }
+            return last ? Sizes{size_of(x, 0), size[0], size[1], size_of(x, 3)}
+                        : Sizes{size_of(x, 0), size_of(x, 1), size[0], size[1]};
+        });
         Call c(queue);
         aclTensor *hx = c.handle(x, fmt), *hy = c.handle(y, fmt, a[5] == Py_None);
         const bool align = bool_arg(a[2]);
@@ -424,20 +467,17 @@ PyObject* resize(PyObject*, PyObject* const* a, Py_ssize_t n)
         const bool last = bool_arg(a[6]);
         const aclFormat fmt = last ? ACL_FORMAT_NHWC : ACL_FORMAT_NCHW;
         const Queue queue(a[5], x);
-        at::Tensor y;
-        if (a[3] == Py_None) {
-            c10::SmallVector<int64_t, 8> sizes(x.sizes().begin(), x.sizes().end());
+        const at::Tensor y = out_arg(a[3], x, [&] {
+            Sizes sizes(x.sizes().begin(), x.sizes().end());
             for (const int64_t d : {last ? 1 : 2, last ? 2 : 3}) {
                 if (d >= x.dim() || d >= (int64_t)scales64.size()) {
                     PyErr_SetString(PyExc_IndexError, "list index out of range");
                     throw Raised();
                 }
-                sizes[d] = (int64_t)((double)sizes[d] * scales64[d]);
+                sizes[d] = truncated((double)sizes[d] * scales64[d]);
             }
-            y = out_arg(a[3], x, sizes);
-        } else {
-            y = tensor_arg(a[3]);
-        }
+            return sizes;
+        });
         Call c(queue);
         aclTensor *hx = c.handle(x, fmt), *hy = c.handle(y, fmt, a[3] == Py_None);
         c10::SmallVector<float, 8> scales(scales64.begin(), scales64.end());
@@ -459,11 +499,11 @@ PyObject* upsample_bilinear2d_backward(PyObject*, PyObject* const* a, Py_ssize_t
 {
     return guarded(n, 9, [&]() -> PyObject* {
         const at::Tensor& go = tensor_arg(a[0]);
-        const auto isize = ints_arg(a[1]);
+        const auto isize = extents_arg(a[1], a[5] == Py_None);
         const bool last = bool_arg(a[8]);
         const aclFormat fmt = last ? ACL_FORMAT_NHWC : ACL_FORMAT_NCHW;
         const Queue queue(a[7], go);
-        const at::Tensor y = out_arg(a[5], go, isize);
+        const at::Tensor y = out_arg(a[5], go, [&] { return isize; });
         const int64_t osize[2] = {size_of(go, last ? 1 : 2), size_of(go, last ? 2 : 3)};
         Call c(queue);
         aclTensor *hgo = c.handle(go, fmt), *hy = c.handle(y, fmt, a[5] == Py_None);

@@ -134,3 +134,60 @@ def test_copy_on_write_outputs_leave_their_source_alone(device, aclnn, name):
         assert b is mine[k] and torch.equal(a, b)
     for k, t in sources.items():
         assert bool((t == 7).all()), k
+
+
+@pytest.mark.gpu
+def test_arguments_taken_and_refused(device, aclnn):
+    """Operands beside a given output are the library's to refuse, with a status; an output that the call would allocate
+    needs operands and integers that give its sizes."""
+    import numpy as np
+    import torch
+
+    def rand(*shape):
+        return torch.rand(shape, device=device)
+    x, grid, y = rand(1, 2, 9, 10), rand(1, 4, 5, 2), rand(1, 2, 4, 5)
+    v, vgrid, vy = rand(1, 2, 3, 9, 10), rand(1, 2, 4, 5, 3), rand(1, 2, 2, 4, 5)
+    up = rand(1, 2, 18, 20)
+
+    def status(call):
+        with pytest.raises(aclnn.AclnnError) as e:
+            call()
+        return e.value.status
+    INV = aclnn.ACLNN_ERR_PARAM_INVALID
+    for few in (x[0], x[0, 0, 0]):
+        assert status(lambda: aclnn.grid_sampler2d(few, grid, out=y)) == INV
+        assert status(lambda: aclnn.grid_sampler2d(x, few[..., :2], out=y)) == INV
+        assert status(lambda: aclnn.grid_sampler3d(few, vgrid, out=vy)) == INV
+        assert status(lambda: aclnn.grid_sampler3d(v, few[..., :3], out=vy)) == INV
+        assert status(lambda: aclnn.grid_sampler3d(few, vgrid, out=vy, channels_last=True)) == INV
+        assert status(lambda: aclnn.upsample_bilinear2d(few, (18, 20), out=up)) == INV
+        assert status(lambda: aclnn.resize(few, (1.0, 1.0, 2.0, 2.0), "nearest", out=up)) == INV
+    row = x[0, 0, 0]
+    for call in (lambda: aclnn.grid_sampler2d(row, grid), lambda: aclnn.grid_sampler2d(x, row),
+                 lambda: aclnn.grid_sampler3d(row, vgrid), lambda: aclnn.grid_sampler3d(v, row),
+                 lambda: aclnn.upsample_bilinear2d(row, (18, 20)),
+                 lambda: aclnn.resize(row, (1.0, 1.0, 2.0, 2.0), "nearest"),
+                 lambda: aclnn.upsample_bilinear2d_backward(row, (1, 2, 9, 10))):
+        with pytest.raises(IndexError):
+            call()
+    assert status(lambda: aclnn.upsample_bilinear2d(x, (18,), out=up)) == INV
+    assert status(lambda: aclnn.upsample_bilinear2d_backward(up, (1, 2, 9), out=x)) == INV
+    # numbers of any kind beside a given output
+    want = aclnn.upsample_bilinear2d(x, (18, 20))
+    for size in ((18.0, 20.0), [np.int64(18), np.float32(20.5)], np.array([18, 20]), torch.tensor([18, 20]), iter((18, 20))):
+        assert torch.equal(aclnn.upsample_bilinear2d(x, size, out=up), want)
+    want = aclnn.upsample_bilinear2d_backward(up, (1, 2, 9, 10))
+    assert torch.equal(aclnn.upsample_bilinear2d_backward(up, (1, 2.0, np.float64(9), 10.5), out=torch.empty_like(x)), want)
+    # integers where they size an allocation
+    assert aclnn.upsample_bilinear2d(x, (np.int64(18), 20)).shape == (1, 2, 18, 20)
+    for call in (lambda: aclnn.upsample_bilinear2d(x, (18.0, 20)),
+                 lambda: aclnn.upsample_bilinear2d_backward(up, (1, 2, 9.0, 10))):
+        with pytest.raises(TypeError):
+            call()
+    with pytest.raises(ValueError):
+        aclnn.resize(x, (1.0, 1.0, float("nan"), 2.0), "nearest")
+    with pytest.raises(OverflowError):
+        aclnn.resize(x, (1.0, 1.0, 2.0, float("inf")), "nearest")
+    assert aclnn.resize(x, ("1", 1, np.float32(2), "2.0"), "nearest").shape == (1, 2, 18, 20)
+    assert torch.equal(aclnn.upsample_bilinear2d(x, (18, 20), False, "2.0", 2), aclnn.upsample_bilinear2d(x, (18, 20)))
+    torch.cuda.synchronize()

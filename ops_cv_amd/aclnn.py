@@ -450,10 +450,8 @@ def upsample_bilinear2d_backward(grad_out, input_size, align_corners=False, scal
                                  stream=None, channels_last=False, out_dtype=None, workspace=None):
     """Both phases of aclnnUpsampleBilinear2dBackward.  `input_size` holds the four extents of the tensor that was
     upsampled, in the order of the tensors' layout (NCHW, or NHWC when channels_last)."""
-    if out is None and out_dtype is not None:
-        out = _torch().empty(tuple(input_size), dtype=out_dtype, device=grad_out.device)
     return (_helpers or _native()).upsample_bilinear2d_backward(grad_out, input_size, align_corners, scales_h, scales_w,
-                                                                out, workspace, _raw(stream), channels_last)
+                                                                out, workspace, _raw(stream), channels_last, out_dtype)
 
 
 def grid_sampler2d_taps(grid, h_in, w_in, interpolation_mode=0, padding_mode=0, align_corners=False, stream=None):

@@ -15,6 +15,7 @@
 #include <ATen/ops/empty_like.h>
 #include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Dtype.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -290,9 +291,20 @@ typedef c10::SmallVector<int64_t, 8> Sizes;
 // The caller's output, or one of the sizes that `sizes` gives.  They are asked for only then: operands of too few
 // dimensions beside a given output are the library's to refuse.
 template <typename F>
-at::Tensor out_arg(PyObject* out, const at::Tensor& like, F&& sizes)
+at::Tensor out_arg(PyObject* out, const at::Tensor& like, F&& sizes, PyObject* dtype = Py_None)
 {
-    return (out == Py_None) ? at::empty(sizes(), like.options().memory_format(at::MemoryFormat::Contiguous)) : tensor_arg(out);
+    if (out != Py_None) {
+        return tensor_arg(out);
+    }
+    at::TensorOptions options = like.options().memory_format(at::MemoryFormat::Contiguous);
+    if (dtype != Py_None) {
+        if (!THPDtype_Check(dtype)) {
+            PyErr_Format(PyExc_TypeError, "expected a torch.dtype, got %s", Py_TYPE(dtype)->tp_name);
+            throw Raised();
+        }
+        options = options.dtype(reinterpret_cast<THPDtype*>(dtype)->scalar_type);
+    }
+    return at::empty(sizes(), options);
 }
 
 template <typename F>
@@ -494,16 +506,16 @@ PyObject* resize(PyObject*, PyObject* const* a, Py_ssize_t n)
     });
 }
 
-// (grad_out, input_size, align, scales_h, scales_w, out, workspace, stream, channels_last)
+// (grad_out, input_size, align, scales_h, scales_w, out, workspace, stream, channels_last, out_dtype)
 PyObject* upsample_bilinear2d_backward(PyObject*, PyObject* const* a, Py_ssize_t n)
 {
-    return guarded(n, 9, [&]() -> PyObject* {
+    return guarded(n, 10, [&]() -> PyObject* {
         const at::Tensor& go = tensor_arg(a[0]);
         const auto isize = extents_arg(a[1], a[5] == Py_None);
         const bool last = bool_arg(a[8]);
         const aclFormat fmt = last ? ACL_FORMAT_NHWC : ACL_FORMAT_NCHW;
         const Queue queue(a[7], go);
-        const at::Tensor y = out_arg(a[5], go, [&] { return isize; });
+        const at::Tensor y = out_arg(a[5], go, [&] { return isize; }, a[9]);
         const int64_t osize[2] = {size_of(go, last ? 1 : 2), size_of(go, last ? 2 : 3)};
         Call c(queue);
         aclTensor *hgo = c.handle(go, fmt), *hy = c.handle(y, fmt, a[5] == Py_None);

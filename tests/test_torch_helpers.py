@@ -37,12 +37,14 @@ def _calls(torch, aclnn, device):
         "sample3d_grad": (lambda **k: aclnn.grid_sampler3d_backward(vgo, v, vgrid, **k), GRADS, True),
         "upsample": (lambda **k: aclnn.upsample_bilinear2d(x, (80, 99), **k), ("out",), False),
         "upsample_grad": (lambda **k: aclnn.upsample_bilinear2d_backward(go, (2, 3, 22, 25), **k), ("out",), False),
+        "upsample_grad_dtype": (lambda **k: aclnn.upsample_bilinear2d_backward(go, (2, 3, 22, 25), out_dtype=torch.float16,
+                                                                               **k), ("out",), False),
         "nearest": (lambda **k: aclnn.resize(x, (1.0, 1.0, 1.5, 1.5), "nearest", **k), ("out",), False),
     }
 
 
 CALLS = ["sample2d", "sample2d_strided", "sample2d_grad", "sample3d", "sample3d_grad", "upsample", "upsample_grad",
-         "nearest"]
+         "upsample_grad_dtype", "nearest"]
 
 
 @pytest.mark.gpu
@@ -184,6 +186,8 @@ def test_arguments_taken_and_refused(device, aclnn):
                  lambda: aclnn.upsample_bilinear2d_backward(up, (1, 2, 9.0, 10))):
         with pytest.raises(TypeError):
             call()
+    with pytest.raises(TypeError):
+        aclnn.upsample_bilinear2d_backward(up, (1, 2, 9, 10), out_dtype="float16")
     with pytest.raises(ValueError):
         aclnn.resize(x, (1.0, 1.0, float("nan"), 2.0), "nearest")
     with pytest.raises(OverflowError):

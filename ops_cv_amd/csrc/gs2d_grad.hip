@@ -501,14 +501,8 @@ int64_t gs2d_grad_gather_words(const GridSamplerGradArgs& a)
     if (gs2d_grad_csr_words(a) > 0) {
         return 0;
     }
-    // The elections take about 3 us per chunk of 256 grid points (bilinear; 1.2 us nearest, 6 us bicubic) and once more
-    // for every turn of bands over the chip, the sorting variant 20 us (bicubic 40) at the least.  Device time of a call
-    // with both gradients, elections / sorting, fp32 N1 C3: bilinear 4 chunks 17 / 20 us, 9 chunks 32 / 22, 64 chunks
-    // 126 / 23; nearest 9 chunks 13 / 19, 16 chunks 21 / 19; bicubic 1 chunk 24 / 36, 3 chunks 50 / 41, 9 chunks
-    // 135 / 45.  From 24 tap passes over a chunk on the sorting variant is taken.
-    const int64_t chunks = (a.Hout * a.Wout + kThreads - 1) / kThreads;
-    const int64_t taps = (a.interp == 0) ? 4 : ((a.interp == 1) ? 1 : 16);
-    return chunks * taps > 24 ? grad_gather_words(gather_args(a)) : 0;
+    const GradGatherArgs g = gather_args(a);
+    return sorting_takes_planes(g) ? grad_gather_words(g) : 0;
 }
 
 hipError_t launch_grid_sampler2d_grad(const GridSamplerGradArgs& a, hipStream_t stream)

@@ -42,34 +42,11 @@ namespace opscv {
 
 namespace {
 
-constexpr int kThreads = 256;
-constexpr int kListMost = 32;        // contributions of an element that the gather kernel takes at most
-constexpr uint32_t kSortedRun = 64;  // runs of more entries are sorted in place before the crowded kernel reads them
+constexpr int kThreads = kGatherThreads;
 constexpr int kPlaceCells = 8;       // cells per lane of the place kernel
 constexpr int kPlaceThreads = 256;
 constexpr int kFoldChans = 16;       // channels whose contributions a crowded element's wavefront computes together
-constexpr int kCtrlWords = 16;       // [0] entries handed out, [1] long runs, [2] crowded elements
 constexpr uint32_t kNoRank = 0xFFFFFFFFu;
-
-struct GatherLayout {  // offsets in 32-bit words within an item's scratch
-    uint32_t counts;   // behind the control words: cleared together with them
-    uint32_t starts;
-    uint32_t ranks;    // [entry of a point][point]
-    uint32_t coords;   // source coordinates of the points: 2 (4 for volumes) values of the element type
-    uint32_t list;     // entries, run after run
-    uint32_t runs;     // cells whose run has more than kSortedRun entries
-    uint32_t crowded;  // elements with more contributions than their list holds
-    uint32_t item_words;
-};
-
-struct GatherParams {
-    int32_t C, D, H, W, points;
-    int32_t pad, align;
-    int32_t items_per_core;
-    int32_t elements, cells;
-    int32_t N;
-    GatherLayout lay;
-};
 
 // Grid points per lane of the count and fill kernels: the atomics and the scattered stores of several are on their way
 // together.
@@ -785,77 +762,6 @@ __global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __
     }
 }
 
-struct GatherPlan {
-    bool ok = false;
-    GatherParams p{};
-    uint32_t tiles = 0, cblocks = 0;
-    int32_t chans_per_block = 0;
-    int cb = 1;
-    int list = kListMost;
-};
-
-inline uint32_t align4(uint64_t v) { return (uint32_t)((v + 3u) & ~(uint64_t)3u); }
-
-GatherPlan make_plan(const GradGatherArgs& a)
-{
-    GatherPlan pl;
-    const int64_t esz = elem_size(a.elem);
-    const int64_t elements = a.D * a.H * a.W;
-    const int64_t cells = (a.interp != 0) ? elements : (a.W + 1) * (a.H + 1) * (a.dim == 3 ? a.D + 1 : 1);
-    const int64_t entries = a.points * (a.interp == 2 ? 16 : 1);
-    const int64_t runs = a.interp == 0 ? ((int64_t)1 << a.dim) : 1;
-    // keys of 32 bits hold an entry and a corner; counts of 32 bits hold an item's entries
-    const int64_t most_points = (int64_t)1 << (a.dim == 3 || a.interp == 2 ? 27 : 28);
-    if (a.points > most_points || elements > INT32_MAX / 2 || cells > INT32_MAX / 2 || a.N > 65535 || a.N < 1) {
-        return pl;
-    }
-    // A list of 16 leaves LDS and registers for twice the wavefronts; of 32 where a smooth grid has more than six
-    // contributions per element on average (scaled by 0.8 along every axis they are ten)
-    pl.list = (entries * runs <= 6 * elements) ? 16 : kListMost;
-    const int64_t crowded_elements = entries * runs / (pl.list + 1) + 1;
-    const int64_t words = kCtrlWords + 2 * cells + 2 * entries + a.points * (a.dim == 3 ? 4 : 2) * esz / 4 +
-                          entries / kSortedRun + crowded_elements + 64;
-    if (words > ((int64_t)1 << 31) || words * 4 * a.N > kGatherMaxScratch) {
-        return pl;
-    }
-    GatherLayout& l = pl.p.lay;
-    l.counts = kCtrlWords;
-    l.starts = align4((uint64_t)l.counts + (uint64_t)cells);
-    l.ranks = align4((uint64_t)l.starts + (uint64_t)cells);
-    l.coords = align4((uint64_t)l.ranks + (uint64_t)entries);
-    l.list = align4((uint64_t)l.coords + (uint64_t)(a.points * (a.dim == 3 ? 4 : 2) * esz / 4));
-    l.runs = align4((uint64_t)l.list + (uint64_t)entries);
-    l.crowded = align4((uint64_t)l.runs + (uint64_t)(entries / kSortedRun) + 1u);
-    l.item_words = align4((uint64_t)l.crowded + (uint64_t)crowded_elements);
-    pl.p.C = (int32_t)a.C;
-    pl.p.D = (int32_t)a.D;
-    pl.p.H = (int32_t)a.H;
-    pl.p.W = (int32_t)a.W;
-    pl.p.points = (int32_t)a.points;
-    pl.p.pad = a.pad;
-    pl.p.align = a.align;
-    pl.p.items_per_core = (int32_t)(a.items_per_core > 0 ? a.items_per_core : 1);
-    pl.p.elements = (int32_t)elements;
-    pl.p.cells = (int32_t)cells;
-    pl.p.N = (int32_t)a.N;
-    pl.cb = (a.C >= 8) ? 8 : ((a.C >= 3) ? 4 : (int)a.C);
-    pl.tiles = (uint32_t)((elements + kThreads - 1) / kThreads);
-    const int64_t base = a.N * pl.tiles;
-    const int64_t max_cblocks = (a.C + pl.cb - 1) / pl.cb;
-    int64_t cblocks = (2048 + base - 1) / base;
-    cblocks = cblocks > max_cblocks ? max_cblocks : cblocks;
-    int64_t cpb = (a.C + cblocks - 1) / cblocks;
-    cpb = (cpb + pl.cb - 1) / pl.cb * pl.cb;
-    cblocks = (a.C + cpb - 1) / cpb;
-    pl.cblocks = (uint32_t)cblocks;
-    pl.chans_per_block = (int32_t)cpb;
-    if (base * cblocks > INT32_MAX / 2 || a.N * ((a.points + kThreads - 1) / kThreads) > INT32_MAX / 2) {
-        return pl;
-    }
-    pl.ok = true;
-    return pl;
-}
-
 inline uint32_t swizzled_blocks(int64_t pieces) { return (uint32_t)((pieces + 7) / 8 * 8); }
 
 template <typename T, int DIM, int INTERP, int CB, int LIST>
@@ -935,13 +841,13 @@ hipError_t run_typed(const GradGatherArgs& a, const GatherPlan& pl, hipStream_t 
 
 int64_t grad_gather_words(const GradGatherArgs& a)
 {
-    const GatherPlan pl = make_plan(a);
+    const GatherPlan pl = gather_plan(a);
     return pl.ok ? (int64_t)pl.p.lay.item_words * a.N : 0;
 }
 
 hipError_t run_grad_gather(const GradGatherArgs& a, hipStream_t stream)
 {
-    const GatherPlan pl = make_plan(a);
+    const GatherPlan pl = gather_plan(a);
     if (!pl.ok || a.dx == nullptr || a.gout == nullptr || a.grid == nullptr || a.scratch == nullptr) {
         return hipErrorInvalidValue;
     }

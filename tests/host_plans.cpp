@@ -1,5 +1,6 @@
 // The launch plans of the kernels, which are plain host arithmetic, for the tests (host_plans.py).
 #include "gs2d_direct_plan.hpp"
+#include "gs_grad_gather_plan.hpp"
 #include "resize_grad_plan.hpp"
 
 using namespace opscv;
@@ -46,6 +47,23 @@ int resize_grad_planes(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t
     out[1] = t.blocks;
     out[2] = (planes + t.slots - 1) / (t.slots > 0 ? t.slots : 1);
     return t.rows > 0 ? 1 : 0;
+}
+
+// estimates of the input gradient of planes (nanoseconds): elections, sorting; 0 where the elections run
+int sorting_takes_planes(int elem, int64_t interp, int64_t N, int64_t C, int64_t H, int64_t W, int64_t points, int64_t* out)
+{
+    GradGatherArgs a;
+    a.elem = (Elem)elem;
+    a.interp = (int)interp;
+    a.N = N;
+    a.C = C;
+    a.H = H;
+    a.W = W;
+    a.points = points;
+    const PlaneGradTimes t = plane_grad_times(a);
+    out[0] = (int64_t)(t.elections * 1e3);
+    out[1] = (int64_t)(t.sorting * 1e3);
+    return sorting_takes_planes(a) && gather_plan(a).ok ? 1 : 0;
 }
 
 }  // extern "C"

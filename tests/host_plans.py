@@ -38,3 +38,9 @@ def resize_grad_planes(dtype, planes, small, large, align=False):
     """(tile rows, workgroups, planes a workgroup walks at most) of the resize gradient's planes kernel, None where it
     is not taken; the gradient of `small` from `large`, both (rows, columns)."""
     return _call("resize_grad_planes", 3, dtype, planes, *small, *large, int(align))
+
+
+def sorting_takes_planes(dtype, interp, shape, points):
+    """(elections, sorting): estimated nanoseconds of the input gradient of (N, C, H, W) planes sampled at `points` points
+    an item, None where the elections run."""
+    return _call("sorting_takes_planes", 2, dtype, interp, *shape, points)

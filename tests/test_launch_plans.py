@@ -46,3 +46,26 @@ def test_resize_gradient_planes_fit_the_launch(dtype):
         p = P.resize_grad_planes(dtype, int(2 ** rng.uniform(0, 12)), (h, w), large, rng.random() < 0.5)
         if p is not None:
             assert p[0] in (8, 16) and 0 < p[1] <= MOST_BLOCKS and p[1] % 8 == 0 and p[2] > 0
+
+
+# (type, mode, input, points per item, microseconds by elections and by sorting): measured, grids turned or scattered
+GRADIENTS = [
+    # pictures and feature maps
+    ("fp32", 0, (8, 3, 479, 637), 479 * 637, 2493, 220), ("fp32", 0, (7, 4, 341, 510), 341 * 510, 2127, 133),
+    ("fp32", 0, (1, 3, 64, 64), 9 * 256, 32, 22), ("fp32", 0, (1, 3, 64, 64), 64 * 256, 126, 23),
+    ("fp32", 2, (1, 3, 64, 64), 3 * 256, 50, 41), ("fp32", 2, (1, 3, 64, 64), 9 * 256, 135, 45),
+    # few tap passes
+    ("fp32", 0, (1, 3, 64, 64), 4 * 256, 17, 20), ("fp32", 1, (1, 3, 64, 64), 9 * 256, 13, 19),
+    ("fp32", 2, (1, 3, 64, 64), 256, 24, 36),
+    # large batches, few points on large planes, many on small ones
+    ("fp32", 0, (512, 3, 64, 64), 1600, 24.9, 75.6), ("fp16", 0, (1000, 3, 48, 48), 2304, 74.7, 132.9),
+    ("fp32", 0, (1, 3, 1080, 1920), 1600, 18.3, 57.6), ("fp16", 0, (8, 3, 512, 512), 1600, 20.6, 55.0),
+    ("fp32", 0, (1024, 1, 16, 16), 4096, 99.9, 1014), ("fp32", 0, (512, 1, 16, 16), 2304, 52.4, 194),
+    ("fp32", 1, (512, 3, 64, 64), 6561, 44.6, 211), ("fp32", 1, (256, 64, 32, 32), 6561, 191, 593),
+    ("fp32", 2, (512, 3, 64, 64), 4096, 340, 1682), ("fp32", 2, (512, 3, 32, 32), 512, 55, 183),
+    ("fp16", 2, (1024, 8, 32, 32), 1024, 220, 758)]
+
+
+@pytest.mark.parametrize("dtype,interp,shape,points,elections,sorting", GRADIENTS)
+def test_input_gradient_takes_the_faster_of_two_variants(dtype, interp, shape, points, elections, sorting):
+    assert (P.sorting_takes_planes(dtype, interp, shape, points) is not None) == (sorting < elections)

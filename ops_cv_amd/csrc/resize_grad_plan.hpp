@@ -57,6 +57,26 @@ struct PlaneTile {
     int64_t blocks = 0;  // padded for the XCD mapping of the kernel
 };
 
+// Rows off the word grid go to the planes kernel or to the gather, whichever is estimated to be faster.  The gather's time
+// follows the elements and the bytes; the planes kernel's the tiles, whole ones also where planes are narrower than 64
+// columns or lower than the tile, and a set-up per turn of the chip: fp16 131072 planes of 3x3 from 7x7 19 us in the
+// gather, 142 in tiles; 16384 of 20x5 from 41x11 25 / 136; 16384 of 14x14 from 29x29 46 / 73; bf16 512 of 65x129 from
+// 257x513 189 / 72.  Fitted to 1777 launches (1 to 60000 planes of 2 to 2000 columns, 4 to 450 us): of these, 958 were
+// slower in tiles than in the gather, by up to 11 times; 92 are with the estimates, by 1.7 at most, and 10 that are left
+// to the gather would have been faster in tiles, by 1.2 at most.
+inline bool gather_takes_planes(const ResizeGradArgs& a, const PlaneTile& t)
+{
+    const double planes = (double)(a.N * a.C), elements = planes * (double)a.Hs * (double)a.Ws * 1e-6;
+    const double megabytes = elem_size(a.elem_in) * (elements + planes * (double)a.Hd * (double)a.Wd * 1e-6);
+    const double tiles = (double)(t.tiles_x * t.tiles_y) * planes * 1e-3;
+    const double turns = t.blocks > 1500 ? (double)t.blocks / 1500.0 : 1.0;
+    const double rows_visited = 2.0 / (double)a.scale_h, columns = 2.0 / (double)a.scale_w;
+    const double visits = t.rows * rows_visited * (columns < kPlaneVisits ? columns : (double)kPlaneVisits);
+    const double gather_us = 5.0 + 1.0 * elements + 1.14 * megabytes;
+    const double tiles_us = 3.1 + 4.1 * turns + tiles * (0.47 + 0.0038 * visits) + 0.33 * megabytes;
+    return gather_us < tiles_us;
+}
+
 // Eight visits a side at most (growth by up to four), elements anywhere.  The estimate of the rectangle sizes the
 // launch; the kernel measures it and reads a larger one from global memory.
 inline PlaneTile plane_tile(const ResizeGradArgs& a)
@@ -67,10 +87,11 @@ inline PlaneTile plane_tile(const ResizeGradArgs& a)
         reinterpret_cast<uintptr_t>(a.x) % (uintptr_t)esz != 0) {
         return t;
     }
-    // resize_grad_lds_kernel spends fewer instructions on a visit and its set-up pays off over four planes and more: fp16
-    // 64 planes of 1080x1920 from 2160x3840 (sixteen planes a workgroup) 405 us there, 452 here; 128 of 160x240 from
-    // 320x480 (less than one) 38 and 29, which puts equal times at about four.  It takes rows on the word grid; above growth
-    // by about 2.6 its tiles get lower than 8 x 128 and read too much twice.
+    // resize_grad_lds_kernel spends fewer instructions on a visit and sets a tile up once for many planes: fp16 64 planes
+    // of 1080x1920 from 2160x3840 (sixteen planes a workgroup) 405 us there, 452 here.  Below four planes a workgroup this
+    // kernel takes 0.60 to 0.78 of that one's time (medians of 576 launches; 1.2 at worst), from four on 0.74 to 0.82 and
+    // 1.4 at worst: those launches stay there.  It takes rows on the word grid; above growth by about 2.6 its tiles get
+    // lower than 8 x 128 and read too much twice.
     const int64_t wide_tiles = ((a.Ws + kGradTileCols - 1) / kGradTileCols) * ((a.Hs + 7) / 8);
     if (wide_tiles * a.N * a.C >= 4 * kWantBlocks && lds_tile_rows(a, kGradCapWords) == 8) {
         return t;
@@ -99,6 +120,9 @@ inline PlaneTile plane_tile(const ResizeGradArgs& a)
     t.slots = (planes + walk - 1) / walk;
     t.blocks = (tiles * t.slots + 7) / 8 * 8;
     if (!fits_launch(t.blocks, kGradThreads)) {  // tall planes of a few columns: the gather walks its elements
+        t.rows = 0;
+    }
+    if (t.rows > 0 && lds_tile_rows(a, kGradCapWords) == 0 && gather_takes_planes(a, t)) {
         t.rows = 0;
     }
     return t;

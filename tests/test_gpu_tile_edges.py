@@ -4,6 +4,7 @@ gradient (resize_grad.hip)."""
 import numpy as np
 import pytest
 
+import host_plans
 import inputs as I
 
 pytestmark = pytest.mark.gpu
@@ -44,7 +45,8 @@ def test_direct_tiles(oracle, device, aclnn, dtype, interp, pad, align):
 
 
 # (gradient's planes, size it is reduced to): growth by four (eight visits), three, two, none and a half; one column and
-# one row more than a tile of 64 x 16; tiles of 16 rows (1024 of them and more) and of 8; rows of one element
+# one row more than a tile of 64 x 16; rows of one element.  Few planes: tiles of 8 rows, each workgroup one plane, and
+# 16-bit rows of odd length in the gather; WALKS has the other forms
 GROWTH = [((1, 3, 257, 513), (65, 129)), ((300, 1, 67, 259), (17, 65)), ((1, 2, 51, 195), (17, 65)),
           ((2, 3, 33, 129), (16, 64)), ((1, 4, 17, 66), (17, 65)), ((1, 4, 9, 33), (17, 65)), ((1, 1, 4, 1), (3, 1)),
           ((1, 2, 64, 255), (16, 64)), ((1, 2, 31, 511), (16, 128))]
@@ -66,6 +68,32 @@ def test_resize_gradient_planes(oracle, device, aclnn, dtype, align, offset):
         got = aclnn.upsample_bilinear2d_backward(view, gs[:2] + small, align)
         torch.cuda.synchronize()
         assert _same(I.from_torch(got, dtype), ref), (gs, small)
+
+
+# (planes, small, large, rows of a tile): workgroups that walk over several planes, the last ones over fewer; tiles of 16
+# rows and of 8, cut off at the right and at the bottom; rows of odd length; growth by 1.4, four, 0.6 and two
+WALKS = [(701, (40, 70), (57, 101), 16), (211, (65, 129), (257, 513), 8), (905, (70, 131), (45, 79), 16),
+         (901, (33, 65), (65, 129), 16)]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("align", [False, True])
+@pytest.mark.parametrize("planes,small,large,rows", WALKS)
+def test_resize_gradient_planes_in_turn(oracle, device, aclnn, dtype, align, planes, small, large, rows):
+    import torch
+    tile_rows, blocks, walk = host_plans.resize_grad_planes(dtype, planes, small, large, align)
+    assert tile_rows == rows and walk > 1 and planes % walk != 0
+    rng = np.random.default_rng(5150 + align)
+    g = I.cast_np(rng.standard_normal((1, planes) + large).astype(np.float32), dtype)
+    ref = oracle.upsample_bilinear2d_backward(g, small, align, dtype=I.oracle_code(dtype))
+    t = I.to_torch(g, dtype, device)
+    for offset in (0, 1):  # a view that starts off the 4-byte grid
+        base = torch.empty(t.numel() + offset, dtype=t.dtype, device=device)
+        view = base[offset:].view(t.shape)
+        view.copy_(t)
+        got = aclnn.upsample_bilinear2d_backward(view, (1, planes) + small, align)
+        torch.cuda.synchronize()
+        assert _same(I.from_torch(got, dtype), ref), offset
 
 
 # (input, output): groups of consecutive rows with a short last group, a last band of one row, more groups than rows;

@@ -31,13 +31,11 @@ def test_direct_tiles_fit_the_launch(dtype):
 
 @pytest.mark.parametrize("dtype", ["fp32", "fp16", "bf16"])
 def test_resize_gradient_planes_fit_the_launch(dtype):
-    # planes of one column: tiles of sixteen rows fill a launch at 2^28 rows
-    rows = 16 * (MOST_BLOCKS // 8 * 8)
-    if dtype != "fp32":  # which leaves that many tiles to resize_grad_lds_kernel, or its gather
-        assert P.resize_grad_planes(dtype, 1, (rows, 1), (rows + 1, 1))[1] == MOST_BLOCKS // 8 * 8
-        # many small planes: workgroups walk over them
-        assert P.resize_grad_planes(dtype, 2**31 - 1, (20, 30), (23, 31))[1] < 2**14
-    assert P.resize_grad_planes(dtype, 1, (rows + 1, 1), (rows + 2, 1)) is None
+    # growth by four: tiles of 64 columns by eight rows fill a launch at 2^27 rows
+    rows = 8 * (MOST_BLOCKS // 8 * 8)
+    assert P.resize_grad_planes(dtype, 1, (rows, 64), (4 * rows, 256)) == (8, MOST_BLOCKS // 8 * 8, 1)
+    assert P.resize_grad_planes(dtype, 1, (rows + 1, 64), (4 * rows + 4, 256)) is None
+    # planes of one column
     assert P.resize_grad_planes(dtype, 1, (2**31 - 2, 1), (2**31 - 1, 1)) is None
     rng = random.Random(8)
     for _ in range(2000):
@@ -69,3 +67,16 @@ GRADIENTS = [
 @pytest.mark.parametrize("dtype,interp,shape,points,elections,sorting", GRADIENTS)
 def test_input_gradient_takes_the_faster_of_two_variants(dtype, interp, shape, points, elections, sorting):
     assert (P.sorting_takes_planes(dtype, interp, shape, points) is not None) == (sorting < elections)
+
+
+# (planes, small, large, microseconds by the gather and by the planes kernel): measured, 16-bit rows off the word grid
+RESIZES = [(131072, (3, 3), (7, 7), 19.4, 142), (16384, (20, 5), (41, 11), 24.9, 136), (64, (500, 3), (1001, 7), 5.1, 19.6),
+           (4096, (40, 9), (81, 19), 21.6, 61), (65536, (7, 7), (15, 15), 48.5, 134), (1, (5000, 5), (10001, 11), 4.4, 7.3),
+           (16384, (14, 14), (29, 29), 46.4, 72.7), (32768, (13, 13), (27, 27), 79.9, 123),
+           (512, (65, 129), (257, 513), 189, 72), (128, (160, 240), (320, 481), 63, 31), (128, (160, 240), (480, 721), 118, 45)]
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "bf16"])
+@pytest.mark.parametrize("planes,small,large,gather,tiles", RESIZES)
+def test_resize_gradient_of_odd_rows_takes_the_faster_of_two_kernels(dtype, planes, small, large, gather, tiles):
+    assert (P.resize_grad_planes(dtype, planes, small, large) is not None) == (tiles < gather)

@@ -14,8 +14,11 @@ def _same(a, b):
     return np.array_equal(np.ascontiguousarray(a).view(np.uint8), np.ascontiguousarray(b).view(np.uint8))
 
 
-# (input, output): one tile of 32 x 16 and its remainders; channel runs of 4 + 1, 3, 2 and 1; planes above 32 KiB that
-# no LDS variant takes (odd widths of 16-bit elements, large fp32 planes); two columns
+# (input, output): planes above 32 KiB that no LDS variant takes (odd widths of 16-bit elements, large fp32 planes), few
+# output pixels: the row order.  MANY has the tiles: one of 32 x 16 and its remainders; channel runs of 1, 3, 4 + 1 and 18
+# times four; two columns
+MANY = [((256, 1, 91, 183), (16, 32)), ((43, 3, 91, 183), (33, 65)), ((65, 5, 91, 183), (17, 63)),
+        ((2, 70, 91, 183), (31, 97)), ((64, 1, 8201, 2), (40, 37))]
 PICTURES = [((1, 5, 301, 211), (16, 32)), ((2, 3, 301, 211), (33, 65)), ((1, 2, 401, 203), (17, 63)),
             ((1, 1, 70001, 2), (40, 37)), ((1, 9, 301, 211), (31, 97))]
 
@@ -34,6 +37,32 @@ def test_direct_tiles(oracle, device, aclnn, dtype, interp, pad, align):
             g32[0, 0, :3, 0] = [np.inf, -np.inf, np.nan]
             g32[0, -1, -3:, 1] = [np.inf, -np.inf, np.nan]
         g32[0, 1, :2] = [[3e38, 0.1], [0.1, -3e38]] if dtype != "fp16" else [[6e4, 0.1], [0.1, -6e4]]
+        g = I.cast_np(g32, dtype)
+        ref = oracle.grid_sampler2d(x, g, interp, pad, align, dtype=I.oracle_code(dtype))
+        with aclnn.option("gs_variant", 1):
+            got = aclnn.grid_sampler2d(I.to_torch(x, dtype, device), I.to_torch(g, dtype, device), interp, pad, align)
+        torch.cuda.synchronize()
+        a, b = I.as_f32(I.from_torch(got, dtype), dtype), I.as_f32(ref, dtype)
+        assert np.array_equal(np.isnan(a), np.isnan(b)), (xs, out)
+        assert np.array_equal(a[~np.isnan(a)], b[~np.isnan(b)]), (xs, out)
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("interp,pad", [(0, 0), (0, 1), (0, 2), (1, 0), (1, 1), (1, 2), (2, 1), (2, 2)])
+@pytest.mark.parametrize("align", [False, True])
+def test_direct_tiles_of_many_pixels(oracle, device, aclnn, dtype, interp, pad, align):
+    import torch
+    rng = np.random.default_rng(5050 + 10 * interp + 2 * pad + align)
+    for xs, out in MANY:
+        assert host_plans.direct_tiles(dtype, *xs, *out) is not None
+        x = I.cast_np(rng.standard_normal(xs, np.float32), dtype)
+        g32 = rng.uniform(-1.3, 1.3, (xs[0],) + out + (2,)).astype(np.float32)
+        if interp != 1:  # what a non-finite coordinate gives: the whole pixel NaN
+            g32[0, 0, :3, 0] = [np.inf, -np.inf, np.nan]
+            g32[-1, -1, -3:, 1] = [np.inf, -np.inf, np.nan]
+        # far outside: beyond what an int32 holds, and for 16-bit coordinates as far as they go
+        far = {"fp32": 1e10, "bf16": 1e10, "fp16": 6e4}[dtype]
+        g32[0, 1, :2] = [[far, 0.1], [0.1, -far]]
         g = I.cast_np(g32, dtype)
         ref = oracle.grid_sampler2d(x, g, interp, pad, align, dtype=I.oracle_code(dtype))
         with aclnn.option("gs_variant", 1):

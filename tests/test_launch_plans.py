@@ -17,6 +17,10 @@ def test_direct_tiles_fit_the_launch(dtype):
     # large planes: 724 x 1448 tiles an item; sixteen items fit and seventeen do not
     assert P.direct_tiles(dtype, 16, 1, 301, 211, 23168, 23168)[0] < 2**24
     assert P.direct_tiles(dtype, 17, 1, 301, 211, 23168, 23168) is None
+    # a workgroup per CU at least: tiles, or tiles times runs of four channels
+    assert P.direct_tiles(dtype, 255, 1, 301, 211, 16, 32) is None
+    assert P.direct_tiles(dtype, 256, 1, 301, 211, 16, 32) == (256, 1)
+    assert P.direct_tiles(dtype, 4, 253, 301, 211, 16, 32) == (4, 64) and P.direct_tiles(dtype, 4, 252, 301, 211, 16, 32) is None
     # the counts of a batch beyond 32 bits
     assert P.direct_tiles(dtype, 2**31 - 1, 1, 301, 211, 16000, 16000) is None
     rng = random.Random(7)

@@ -17,6 +17,7 @@
 #include "options.hpp"
 #include "resize_band_lds_kernel.hpp"
 #include "resize_math.hpp"
+#include "resize_nhwc_plan.hpp"
 #include "sampler_math.hpp"
 
 namespace opscv {
@@ -431,12 +432,11 @@ __global__ __launch_bounds__(kThreads) void resize_nhwc_unit_kernel(const T* __r
     }
 }
 
-// The unit kernel's counterpart for rows that shrink by half as much again or more: an output row then shares a source
-// row with its neighbour at most every other time, so nothing is kept, and two output rows' eight units are on their way
+// The unit kernel's counterpart for rows that shrink by half as much again or more (shrinking_rows_go_in_pairs): an output
+// row then shares a source row with its neighbour at most every other time, so nothing is kept, and two output rows' eight units are on their way
 // together, where the kernel above waits for one source row's two after the other.  Bands of four rows: with eight, a
 // picture's bands fill the chip once and a bit.  Same operations in the same order.
-// fp32 16x720x1280x3 to 384x640: 51.6 -> 45.0 us with operands from memory (36.4 -> 35.1 from the last-level cache); no
-// size slower among units of 2 to 16 bytes and factors of 1.5 to 3.
+// fp32 16x720x1280x3 to 384x640: 51.6 -> 45.0 us with operands from memory (36.4 -> 35.1 from the last-level cache).
 constexpr int kShrinkBand = 4;
 
 template <typename T, bool HALF_PIXEL, int VB>
@@ -1103,9 +1103,8 @@ hipError_t run_resize(const ResizeArgs& a, hipStream_t stream)
             // the lanes' loads coalesce better with one unit each.
             const int upl = (vb > 4 || a.Wd < a.Ws) ? 1 : 16 / vb;
             const int64_t row_lanes = (a.Wd * (a.C * (int64_t)sizeof(T) / vb) + upl - 1) / upl;
-            // below a factor of 1.5 most output rows share a source row with the next: the unit kernel keeps it
             const int64_t shrink_bands = (a.Hd + kShrinkBand - 1) / kShrinkBand;
-            if (upl == 1 && a.scale_h >= 1.5f && shrink_bands <= 65535) {
+            if (upl == 1 && shrinking_rows_go_in_pairs(a, (int)vb) && shrink_bands <= 65535) {
                 dim3 grid((unsigned)((row_lanes + kThreads - 1) / kThreads), (unsigned)shrink_bands,
                           (unsigned)(a.N < 65535 ? a.N : 65535));
 #define OPSCV_NHWC_SHRINK(HP, VB)                                                                                    \

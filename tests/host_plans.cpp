@@ -2,6 +2,7 @@
 #include "gs2d_direct_plan.hpp"
 #include "gs_grad_gather_plan.hpp"
 #include "resize_grad_plan.hpp"
+#include "resize_nhwc_plan.hpp"
 
 using namespace opscv;
 
@@ -64,6 +65,15 @@ int sorting_takes_planes(int elem, int64_t interp, int64_t N, int64_t C, int64_t
     out[0] = (int64_t)(t.elections * 1e3);
     out[1] = (int64_t)(t.sorting * 1e3);
     return sorting_takes_planes(a) && gather_plan(a).ok ? 1 : 0;
+}
+
+// 1: channels-last rows that shrink from Hs to Hd go in pairs
+int shrink_in_pairs(int64_t unit, int64_t Hs, int64_t Hd, int align)
+{
+    ResizeArgs a;
+    a.half_pixel = align ? 0 : 1;
+    a.scale_h = align ? (float)(Hs - 1) / (float)(Hd - 1) : (float)Hs / (float)Hd;
+    return shrinking_rows_go_in_pairs(a, (int)unit) ? 1 : 0;
 }
 
 }  // extern "C"

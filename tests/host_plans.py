@@ -44,3 +44,9 @@ def sorting_takes_planes(dtype, interp, shape, points):
     """(elections, sorting): estimated nanoseconds of the input gradient of (N, C, H, W) planes sampled at `points` points
     an item, None where the elections run."""
     return _call("sorting_takes_planes", 2, dtype, interp, *shape, points)
+
+
+def shrink_in_pairs(unit, rows, shrunk, align=False):
+    """Whether channels-last rows of `unit`-byte units shrink two together (resize_nhwc_shrink_kernel)."""
+    return bool(lib().shrink_in_pairs(ctypes.c_int64(unit), ctypes.c_int64(rows), ctypes.c_int64(shrunk),
+                                      ctypes.c_int(int(align))))

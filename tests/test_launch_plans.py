@@ -84,3 +84,17 @@ RESIZES = [(131072, (3, 3), (7, 7), 19.4, 142), (16384, (20, 5), (41, 11), 24.9,
 @pytest.mark.parametrize("planes,small,large,gather,tiles", RESIZES)
 def test_resize_gradient_of_odd_rows_takes_the_faster_of_two_kernels(dtype, planes, small, large, gather, tiles):
     assert (P.resize_grad_planes(dtype, planes, small, large) is not None) == (tiles < gather)
+
+
+# (bytes of a unit, rows, shrunk, align corners, in pairs): microseconds with kept rows / in pairs
+SHRUNK = [(12, 720, 384, False, True),    # 51.6 / 45.0
+          (6, 720, 480, False, False),    # 33.3 / 39.0
+          (6, 2160, 720, False, False),   # 6.8 / 8.9: every row falls on a source row
+          (6, 1974, 658, False, False), (4, 1305, 435, False, False), (2, 1932, 644, False, False),  # 22 / 35, 8.3 / 12, 25 / 35
+          (12, 7 * 89 + 1, 90, True, False), (12, 7 * 89 + 2, 90, True, True),  # align corners: a factor of 7, and beside it
+          (2, 1000, 400, False, True), (6, 1440, 720, False, True), (12, 750, 500, False, True), (12, 700, 500, False, False)]
+
+
+@pytest.mark.parametrize("unit,rows,shrunk,align,pairs", SHRUNK)
+def test_shrinking_rows_take_the_faster_of_two_kernels(unit, rows, shrunk, align, pairs):
+    assert P.shrink_in_pairs(unit, rows, shrunk, align) == pairs

@@ -483,6 +483,14 @@ int64_t gs3d_grad_gather_words(const GridSampler3DGradArgs& a)
     if (points <= 65536 && (vol > 16 * points || (vol > 8 * points && points <= 32 * kChunkPoints3))) {
         return 0;
     }
+    // Large batches of small volumes sampled densely: the ordered kernel's workgroups fill the chip, while the sorting
+    // variant folds elements of many contributions one wavefront each (bilinear 64x2x8x16x16 from 17x64x64 border 1932 / - /
+    // 6296 us, 222x1x3x16x29 from 7x38x70 607 / 868 / 3703, nearest 463x1x7x9x7 from 15x20x15 32 / - / 104, 543x14x36x4x4
+    // from 65x7x7 87 / - / 211; below the lines sorting is the faster one or close to it, 34x2x13x50x36 from 25x99x71 nearest
+    // 343 / - / 239, 96x1x15x30x49 from 20x40x66 bilinear 696 / - / 338).
+    if (a.interp == 1 ? (a.N >= 192 && points > 2 * vol) : (a.N >= 64 && points > 3 * vol)) {
+        return 0;
+    }
     if (a.interp == 1) {
         // 16 chunks: 21 / - / 20 us, 8 chunks 15 / - / 20, 256 chunks 99 / - / 36
         return points > 16 * kChunkPoints3 ? grad_gather_words(gather_args(a)) : 0;
@@ -490,8 +498,10 @@ int64_t gs3d_grad_gather_words(const GridSampler3DGradArgs& a)
     if (gs3d_grad_list_words(a) > 0) {
         // Border and reflection padding gather points on the faces; an item with a crowded voxel is left by the slots
         // kernels to the ordered kernel (4 x 16x32x32 border: 17 us without such an item, 214 with one, sorting variant
-        // 55; 8 x 16x40x40 307 / 72).  Smaller grids seldom have one and cost half as much in slots (19 / 35 us).
-        const bool piles = a.pad != 0 && points >= 8192;
+        // 55; 8 x 16x40x40 307 / 72).  Smaller grids seldom have one and cost half as much in slots (19 / 35 us), nor do
+        // grids of less than a point per two voxels (13x2x13x41x52 from 9x30x39 28 / 50, 15 of 24 such calls slower sorted;
+        // from 0.8 points per voxel on 192 of 243 are faster sorted, on average by 2.7 times).
+        const bool piles = a.pad != 0 && points >= 8192 && 2 * points >= vol;
         // the slots kernels keep an item on one XCD: one or two large items leave most of the chip idle (one item of
         // 65536 points: 39 / 30 us, with 16 channels 94 / 42; two items 41 / 37; four 39 / 45; one of 36864 27 / 30)
         const bool few_items = a.N <= 2 && points >= 49152;

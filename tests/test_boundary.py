@@ -722,3 +722,34 @@ def test_second_phase_refuses_a_misaligned_workspace(aclnn):
     assert L.aclnnGridSampler2D(None, ws, ex, None) == 161001
     for h in hs:
         aclnn.destroy_tensor(h)
+
+
+# (input, grid, mode, padding, what runs): microseconds of the ordered kernel / slots / sorting
+VOLUMES = [((22, 4, 16, 64, 64), (16, 64, 64), 0, 0, "slots"), ((8, 4, 16, 40, 40), (16, 40, 40), 0, 1, "sorting"),  # - / 307 / 72
+           ((13, 2, 13, 41, 52), (9, 30, 39), 0, 1, "slots"), ((2, 3, 57, 30, 21), (44, 23, 16), 0, 2, "slots"),  # 28 / 50, 23 / 47
+           ((222, 1, 3, 16, 29), (7, 38, 70), 0, 1, "slots"), ((64, 2, 8, 16, 16), (17, 64, 64), 0, 1, "ordered"),  # 1932 / - / 6296
+           ((24, 2, 8, 16, 16), (17, 64, 64), 0, 1, "sorting"), ((2, 1, 64, 128, 128), (10, 128, 64), 0, 0, "sorting"),
+           ((463, 1, 7, 9, 7), (15, 20, 15), 1, 0, "ordered"), ((543, 14, 36, 4, 4), (65, 7, 7), 1, 1, "ordered"),  # 32 / 104, 87 / 211
+           ((34, 2, 13, 50, 36), (25, 99, 71), 1, 0, "sorting"), ((4, 2, 8, 16, 16), (8, 16, 16), 1, 0, "ordered")]
+
+
+@pytest.mark.parametrize("inp,out,interp,pad,runs", VOLUMES)
+def test_grid_sampler3d_backward_variant_by_size(aclnn, inp, out, interp, pad, runs):
+    """which variant of the input gradient phase 1 plans: the sorting variant is the one whose workspace holds the points'
+    entries, 20 bytes and more per point and item"""
+    f32 = aclnn.ACL_FLOAT
+    hs = [aclnn.create_tensor(inp[:2] + out, f32, aclnn.ACL_FORMAT_NCDHW), aclnn.create_tensor(inp, f32, aclnn.ACL_FORMAT_NCDHW),
+          aclnn.create_tensor(inp[:1] + out + (3,), f32), aclnn.create_tensor(inp, f32, aclnn.ACL_FORMAT_NCDHW),
+          aclnn.create_tensor(inp[:1] + out + (3,), f32)]
+    mask = aclnn.create_bool_array([True, True])
+    st, ws, ex = aclnn.get_workspace_size_grid_sampler3d_backward(hs[0], hs[1], hs[2], interp, pad, False, mask, hs[3], hs[4])
+    assert st == 0
+    name = aclnn.executor_variant(ex)
+    aclnn.destroy_executor(ex)
+    aclnn.destroy_bool_array(mask)
+    for h in hs:
+        aclnn.destroy_tensor(h)
+    points = inp[0] * out[0] * out[1] * out[2]
+    assert name == ("gs3d_grad_lists" if runs == "slots" else "gs3d_grad_ordered")
+    if runs != "slots":
+        assert (ws >= 20 * points) == (runs == "sorting")

@@ -8,6 +8,7 @@
 #include "options.hpp"
 #include "resize_band_lds_kernel.hpp"
 #include "resize_flat_lds_kernel.hpp"
+#include "resize_flat_plan.hpp"
 
 namespace opscv {
 
@@ -134,8 +135,6 @@ constexpr int kFlatThreads = 256;
 constexpr int kFlatMaxColumnLanes = 128;   // wider rows keep at least half of the band variant's lanes busy
 constexpr int kFlatLdsBudget = 32 * 1024;  // per workgroup: several workgroups per CU hide the staging latency
 constexpr int64_t kFlatWantBlocks = 1024;
-constexpr int64_t kFlatPlainBytes = 64ll << 20;   // outputs from here on leave by plain stores (make_flat_plan)
-constexpr int64_t kLastLevelBytes = 256ll << 20;  // the chip's last-level cache
 
 struct FlatPlan {
     bool ok = false;
@@ -223,21 +222,9 @@ FlatPlan make_flat_plan(const ResizeArgs& a)
     fp.p.band_rows = (int32_t)band_rows;
     fp.p.cl = (int32_t)cl;
     fp.p.rg = rg;
-    // Non-temporal stores keep small outputs from lying dirty in L2 at the kernel's end, but write a row's first and last
-    // line, which it shares with its neighbours, in pieces.  Non-temporal / plain: fp32 8x64x112x112 (26 MB) 7.0 / 8.9
-    // us, bf16 8x256x112x112 (51 MB) 17.4 / 18.6; 8x40x257x513 (84 MB) 26.6 / 23.4, 8x64x257x513 (135 MB) 45.1 / 32.6,
-    // fp16 8x512x200x200 (328 MB) 121 / 92, fp32 8x256x112x112 (103 MB) 23.7 / 21.0, 8x32x257x516 (136 MB) 41.7 / 30.1;
-    // lines of fp32 rows beyond the last-level cache are better written through: 8x64x257x513 (270 MB) 57.2 / 62.2.
-    const int64_t out_bytes = planes * a.Hd * a.Wd * (int64_t)sizeof(T);
-    // Beyond the cache, rows of whole vectors keep rows in turn and non-temporal stores, which then fill shared lines
-    // together: fp16 8x512x200x200 86 us, 92 otherwise, fp32 8x256x200x200 (328 MB) 82 and 92 (ragged rows bf16
-    // 8x256x257x513, 540 MB: 233 and 161).
-    const bool in_turn = out_bytes >= kLastLevelBytes && (a.Wd * (int64_t)sizeof(T)) % 16 == 0;
-    fp.p.streaming =
-        (out_bytes < kFlatPlainBytes || in_turn || (sizeof(T) == 4 && out_bytes >= kLastLevelBytes)) ? 1 : 0;
-    // Rows that grow share source rows: a group's rows are consecutive then, and blended rows are kept (half to an eighth
-    // of the LDS reads; with plain stores 33 us on bf16 8x64x65x129 to 257x513, 59 before).
-    fp.p.group_rows = (a.Hd > a.Hs && !in_turn) ? (int32_t)((band_rows + rg - 1) / rg) : 0;
+    const FlatStores stores = flat_stores(a);
+    fp.p.streaming = stores.streaming ? 1 : 0;
+    fp.p.group_rows = stores.runs ? (int32_t)((band_rows + rg - 1) / rg) : 0;
     fp.p.gran = gran;
     fp.p.neg_zero = -0.0f;
     fp.p.raw_lambda = a.raw_lambda;

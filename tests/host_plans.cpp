@@ -1,6 +1,7 @@
 // The launch plans of the kernels, which are plain host arithmetic, for the tests (host_plans.py).
 #include "gs2d_direct_plan.hpp"
 #include "gs_grad_gather_plan.hpp"
+#include "resize_flat_plan.hpp"
 #include "resize_grad_plan.hpp"
 #include "resize_nhwc_plan.hpp"
 
@@ -74,6 +75,23 @@ int shrink_in_pairs(int64_t unit, int64_t Hs, int64_t Hd, int align)
     a.half_pixel = align ? 0 : 1;
     a.scale_h = align ? (float)(Hs - 1) / (float)(Hd - 1) : (float)Hs / (float)Hd;
     return shrinking_rows_go_in_pairs(a, (int)unit) ? 1 : 0;
+}
+
+// flat resize: non-temporal stores, rows of a group in runs
+int flat_resize(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int64_t* out)
+{
+    ResizeArgs a;
+    a.elem = (Elem)elem;
+    a.N = 1;
+    a.C = planes;
+    a.Hs = Hs;
+    a.Ws = Ws;
+    a.Hd = Hd;
+    a.Wd = Wd;
+    const FlatStores s = flat_stores(a);
+    out[0] = s.streaming;
+    out[1] = s.runs;
+    return 1;
 }
 
 }  // extern "C"

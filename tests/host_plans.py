@@ -50,3 +50,8 @@ def shrink_in_pairs(unit, rows, shrunk, align=False):
     """Whether channels-last rows of `unit`-byte units shrink two together (resize_nhwc_shrink_kernel)."""
     return bool(lib().shrink_in_pairs(ctypes.c_int64(unit), ctypes.c_int64(rows), ctypes.c_int64(shrunk),
                                       ctypes.c_int(int(align))))
+
+
+def flat_resize(dtype, planes, small, large):
+    """(non-temporal stores, consecutive rows per group) of the flat resize from `small` to `large`."""
+    return tuple(bool(v) for v in _call("flat_resize", 2, dtype, planes, *small, *large))

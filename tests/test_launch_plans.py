@@ -98,3 +98,17 @@ SHRUNK = [(12, 720, 384, False, True),    # 51.6 / 45.0
 @pytest.mark.parametrize("unit,rows,shrunk,align,pairs", SHRUNK)
 def test_shrinking_rows_take_the_faster_of_two_kernels(unit, rows, shrunk, align, pairs):
     assert P.shrink_in_pairs(unit, rows, shrunk, align) == pairs
+
+
+# (type, planes, small, large, non-temporal stores, rows in runs): outputs of 26, 103, 135, 270 and 328 MB; fp32 of which input
+# and output together are beyond the last-level cache; rows that shrink
+FLAT = [("fp32", 512, (56, 56), (112, 112), True, True), ("fp32", 2048, (56, 56), (112, 112), False, True),
+        ("bf16", 512, (65, 129), (257, 513), False, True), ("fp32", 512, (65, 129), (257, 513), True, True),
+        ("fp16", 4096, (100, 100), (200, 200), True, False), ("fp32", 2048, (100, 100), (200, 200), True, False),
+        ("fp32", 5869, (42, 65), (88, 114), True, False), ("fp32", 4273, (56, 71), (112, 113), True, False),
+        ("fp16", 11595, (54, 79), (75, 110), False, True), ("fp32", 64, (112, 112), (56, 56), True, False)]
+
+
+@pytest.mark.parametrize("dtype,planes,small,large,streaming,runs", FLAT)
+def test_flat_resize_rows_and_stores(dtype, planes, small, large, streaming, runs):
+    assert P.flat_resize(dtype, planes, small, large) == (streaming, runs)

@@ -90,7 +90,7 @@ struct Coords {
 
 __device__ __forceinline__ int32_t phase_of(int64_t n, const GatherParams& p)
 {
-    return (int32_t)(((n % p.items_per_core) * (int64_t)p.points) % kChunkPoints3);
+    return (int32_t)((((p.first_item + n) % p.items_per_core) * (int64_t)p.points) % kChunkPoints3);
 }
 
 // The source coordinates of a grid point, as the tap decisions of gs2d_grad_math.hpp and gs3d_grad_math.hpp form them
@@ -842,21 +842,36 @@ hipError_t run_typed(const GradGatherArgs& a, const GatherPlan& pl, hipStream_t 
 int64_t grad_gather_words(const GradGatherArgs& a)
 {
     const GatherPlan pl = gather_plan(a);
-    return pl.ok ? (int64_t)pl.p.lay.item_words * a.N : 0;
+    return pl.ok ? (int64_t)pl.p.lay.item_words * pl.group : 0;
 }
 
 hipError_t run_grad_gather(const GradGatherArgs& a, hipStream_t stream)
 {
-    const GatherPlan pl = gather_plan(a);
+    GatherPlan pl = gather_plan(a);
     if (!pl.ok || a.dx == nullptr || a.gout == nullptr || a.grid == nullptr || a.scratch == nullptr) {
         return hipErrorInvalidValue;
     }
-    switch (a.elem) {
-        case Elem::F32: return run_typed<float>(a, pl, stream);
-        case Elem::F16: return run_typed<_Float16>(a, pl, stream);
-        case Elem::BF16: return run_typed<__bf16>(a, pl, stream);
+    // the items are independent: a group of them after the other, each in all of the scratch
+    const int64_t esz = elem_size(a.elem);
+    for (int64_t first = 0; first < a.N; first += pl.group) {
+        GradGatherArgs g = a;
+        g.N = (a.N - first < pl.group) ? a.N - first : pl.group;
+        g.gout = (const char*)a.gout + first * a.C * a.points * esz;
+        g.grid = (const char*)a.grid + first * a.points * a.dim * esz;
+        g.dx = (char*)a.dx + first * a.C * (a.D * a.H * a.W) * esz;
+        pl.p.N = (int32_t)g.N;
+        pl.p.first_item = (int32_t)first;
+        hipError_t e = hipErrorInvalidValue;
+        switch (a.elem) {
+            case Elem::F32: e = run_typed<float>(g, pl, stream); break;
+            case Elem::F16: e = run_typed<_Float16>(g, pl, stream); break;
+            case Elem::BF16: e = run_typed<__bf16>(g, pl, stream); break;
+        }
+        if (e != hipSuccess) {
+            return e;
+        }
     }
-    return hipErrorInvalidValue;
+    return hipSuccess;
 }
 
 }  // namespace opscv

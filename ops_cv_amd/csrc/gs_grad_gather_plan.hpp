@@ -5,10 +5,16 @@
 #include <cstdint>
 
 #include "acl_types.hpp"
+#include "launch_limits.hpp"
 
 namespace opscv {
 
-constexpr int64_t kGatherMaxScratch = (int64_t)4 << 30;  // bytes of a call, of the 288 GB of the device
+// Bytes of scratch.  A batch whose items need more than the first together is run some items at a time, in the same scratch;
+// an item that needs more than the second is left to the elections.  The first is the last-level cache's size: fp32
+// 64x3x720x1280 in one go (1.4 GiB) 3696 us, in groups of 512 MiB 3798, 256 MiB 3627, 128 MiB 3837, 64 MiB 4380; 16x3x
+// 1080x1920 2119 (0.8 GiB), 1969 in groups of 256 MiB; bicubic 8x3x1080x1920 7997 (2.3 GiB), 7662 an item at a time (290 MiB).
+constexpr int64_t kGatherGroupScratch = (int64_t)256 << 20;
+constexpr int64_t kGatherMostScratch = (int64_t)4 << 30;
 
 struct GradGatherArgs {
     Elem elem = Elem::F32;
@@ -44,13 +50,15 @@ struct GatherParams {
     int32_t pad, align;
     int32_t items_per_core;
     int32_t elements, cells;
-    int32_t N;
+    int32_t N;           // items of this launch, and the batch's number of the first one
+    int32_t first_item;
     GatherLayout lay;
 };
 
 struct GatherPlan {
     bool ok = false;
-    GatherParams p{};
+    GatherParams p{};    // of the first group of items
+    int64_t group = 0;   // items run at a time
     uint32_t tiles = 0, cblocks = 0;
     int32_t chans_per_block = 0;
     int cb = 1;
@@ -83,9 +91,12 @@ inline GatherPlan gather_plan(const GradGatherArgs& a)
     const int64_t crowded_elements = entries * runs / (pl.list + 1) + 1;
     const int64_t words = kCtrlWords + 2 * cells + 2 * entries + a.points * (a.dim == 3 ? 4 : 2) * esz / 4 +
                           entries / kSortedRun + crowded_elements + 64;
-    if (words > ((int64_t)1 << 31) || words * 4 * a.N > kGatherMaxScratch) {
+    if (words > ((int64_t)1 << 31) || words * 4 > kGatherMostScratch) {
         return pl;
     }
+    const int64_t fit = kGatherGroupScratch / (words * 4);
+    const int64_t group = fit < 1 ? 1 : (fit < a.N ? fit : a.N);
+    pl.group = (a.N + (a.N + group - 1) / group - 1) / ((a.N + group - 1) / group);  // as many items in every group
     GatherLayout& l = pl.p.lay;
     l.counts = kCtrlWords;
     l.starts = align4((uint64_t)l.counts + (uint64_t)cells);
@@ -105,10 +116,11 @@ inline GatherPlan gather_plan(const GradGatherArgs& a)
     pl.p.items_per_core = (int32_t)(a.items_per_core > 0 ? a.items_per_core : 1);
     pl.p.elements = (int32_t)elements;
     pl.p.cells = (int32_t)cells;
-    pl.p.N = (int32_t)a.N;
+    pl.p.N = (int32_t)pl.group;
+    pl.p.first_item = 0;
     pl.cb = (a.C >= 8) ? 8 : ((a.C >= 3) ? 4 : (int)a.C);
     pl.tiles = (uint32_t)((elements + kGatherThreads - 1) / kGatherThreads);
-    const int64_t base = a.N * pl.tiles;
+    const int64_t base = pl.group * pl.tiles;
     const int64_t max_cblocks = (a.C + pl.cb - 1) / pl.cb;
     int64_t cblocks = (2048 + base - 1) / base;
     cblocks = cblocks > max_cblocks ? max_cblocks : cblocks;
@@ -117,10 +129,8 @@ inline GatherPlan gather_plan(const GradGatherArgs& a)
     cblocks = (a.C + cpb - 1) / cpb;
     pl.cblocks = (uint32_t)cblocks;
     pl.chans_per_block = (int32_t)cpb;
-    if (base * cblocks > INT32_MAX / 2 || a.N * ((a.points + kGatherThreads - 1) / kGatherThreads) > INT32_MAX / 2) {
-        return pl;
-    }
-    pl.ok = true;
+    pl.ok = fits_launch(base * cblocks + 8 + 65536, kGatherThreads) &&  // padded to the XCDs, and the sorting workgroups
+            fits_launch(pl.group * ((a.points + kGatherThreads - 1) / kGatherThreads) + 8, kGatherThreads);
     return pl;
 }
 

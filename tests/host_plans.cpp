@@ -94,4 +94,23 @@ int flat_resize(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, in
     return 1;
 }
 
+// sorting variant of the input gradient: items run at a time, 32-bit words of an item; 0 where it cannot run
+int gather_groups(int elem, int64_t interp, int64_t N, int64_t C, int64_t D, int64_t H, int64_t W, int64_t points, int64_t* out)
+{
+    GradGatherArgs a;
+    a.elem = (Elem)elem;
+    a.dim = D > 0 ? 3 : 2;
+    a.interp = (int)interp;
+    a.N = N;
+    a.C = C;
+    a.D = D > 0 ? D : 1;
+    a.H = H;
+    a.W = W;
+    a.points = points;
+    const GatherPlan p = gather_plan(a);
+    out[0] = p.group;
+    out[1] = p.p.lay.item_words;
+    return p.ok ? 1 : 0;
+}
+
 }  // extern "C"

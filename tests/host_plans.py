@@ -55,3 +55,10 @@ def shrink_in_pairs(unit, rows, shrunk, align=False):
 def flat_resize(dtype, planes, small, large):
     """(non-temporal stores, consecutive rows per group) of the flat resize from `small` to `large`."""
     return tuple(bool(v) for v in _call("flat_resize", 2, dtype, planes, *small, *large))
+
+
+def gather_groups(dtype, interp, shape, points):
+    """(items run at a time, 32-bit words of an item) of the sorting input gradient of (N, C, [D,] H, W), None where it
+    cannot run."""
+    shape = shape if len(shape) == 5 else shape[:2] + (0,) + shape[2:]
+    return _call("gather_groups", 2, dtype, interp, *shape, points)

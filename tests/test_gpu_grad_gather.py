@@ -2,6 +2,7 @@
 import numpy as np
 import pytest
 
+import host_plans
 import inputs as I
 
 pytestmark = pytest.mark.gpu
@@ -65,3 +66,37 @@ def test_volumes(oracle, device, aclnn, dtype, interp, pad):
                                                    False)
         torch.cuda.synchronize()
         assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref)), (xs, out, span)
+
+
+@pytest.mark.parametrize("interp,n,out", [(0, 45, (480, 641)), (2, 9, (500, 641))])
+def test_planes_in_groups_of_items(device, aclnn, interp, n, out):
+    """a batch whose items are run a group at a time, against its items one by one"""
+    import torch
+    xs = (n, 1, 480, 641)
+    group, _ = host_plans.gather_groups("fp16", interp, xs, out[0] * out[1])
+    assert group < n and n % group != 0
+    g = torch.Generator(device=device).manual_seed(4)
+    x = torch.randn(xs, generator=g, device=device).half()
+    go = torch.randn((n, 1) + out, generator=g, device=device).half()
+    grid = (torch.rand((n,) + out + (2,), generator=g, device=device) * 2.4 - 1.2).half()
+    got, _ = aclnn.grid_sampler2d_backward(go, x, grid, interp, 1, False, (True, False))
+    for i in range(n):
+        one, _ = aclnn.grid_sampler2d_backward(go[i:i + 1], x[i:i + 1], grid[i:i + 1], interp, 1, False, (True, False))
+        assert torch.equal(one[0], got[i]), i
+
+
+def test_volumes_in_groups_of_items(device, aclnn):
+    """the chunks of a volume start at a shift that its number in the batch gives, whatever group it is run in"""
+    import torch
+    xs, out = (300, 1, 9, 20, 21), (39, 32, 31)
+    group, _ = host_plans.gather_groups("fp32", 0, xs, out[0] * out[1] * out[2])
+    assert group < 300 and out[0] * out[1] * out[2] % 256 != 0
+    g = torch.Generator(device=device).manual_seed(5)
+    x = torch.randn(xs, generator=g, device=device)
+    go = torch.randn((300, 1) + out, generator=g, device=device)
+    grid = torch.rand((300,) + out + (3,), generator=g, device=device) * 2.2 - 1.1
+    grads = []
+    for variant in (1, 3):
+        with aclnn.option("gs3d_grad_variant", variant):
+            grads.append(aclnn.grid_sampler3d_backward(go, x, grid, 0, 0, False, (True, False))[0])
+    assert torch.equal(*grads)

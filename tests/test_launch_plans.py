@@ -112,3 +112,24 @@ FLAT = [("fp32", 512, (56, 56), (112, 112), True, True), ("fp32", 2048, (56, 56)
 @pytest.mark.parametrize("dtype,planes,small,large,streaming,runs", FLAT)
 def test_flat_resize_rows_and_stores(dtype, planes, small, large, streaming, runs):
     assert P.flat_resize(dtype, planes, small, large) == (streaming, runs)
+
+
+def test_sorting_scratch_holds_a_group_of_items():
+    """a batch's scratch is that of as many items as 256 MiB hold, of one at least; items beyond 4 GiB are left alone"""
+    cache = 256 << 20
+    assert P.gather_groups("fp32", 0, (8, 3, 479, 637), 479 * 637)[0] == 8  # 58 MiB
+    for dtype, interp, shape, points, groups in [("fp32", 2, (16, 3, 1080, 1920), 1080 * 1920, 16),
+                                                 ("fp32", 0, (64, 3, 720, 1280), 720 * 1280, 6),
+                                                 ("fp16", 0, (45, 1, 480, 641), 480 * 641, 2),
+                                                 ("fp32", 0, (300, 1, 9, 20, 21), 39 * 32 * 31, 2)]:
+        group, words = P.gather_groups(dtype, interp, shape, points)
+        assert -(-shape[0] // group) == groups and (group == 1 or group * words * 4 <= cache), (shape, group, words)
+    assert P.gather_groups("fp32", 2, (1, 1, 5300, 5300), 5300 * 5300) is not None  # 3.9 GiB
+    assert P.gather_groups("fp32", 2, (1, 1, 5800, 5800), 5800 * 5800) is None
+    assert P.gather_groups("fp32", 0, (65536, 1, 9, 9), 2000) is None
+    rng = random.Random(9)
+    for _ in range(2000):
+        n, c, h, w = (int(2 ** rng.uniform(0, k)) for k in (16, 10, 13, 13))
+        p = P.gather_groups(rng.choice(["fp32", "fp16"]), rng.choice([0, 1, 2]), (n, c, h, w), int(2 ** rng.uniform(8, 25)))
+        if p is not None:
+            assert 1 <= p[0] <= n and (p[0] == 1 or p[0] * p[1] * 4 <= cache) and p[1] * 4 <= 4 << 30

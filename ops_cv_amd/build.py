@@ -1,4 +1,5 @@
-"""Builds libopscv_amd.so in-tree with hipcc for gfx950 (python -m ops_cv_amd.build)."""
+"""Builds libopscv_amd.so in-tree with hipcc for gfx950, and the native side of the torch helpers against the installed
+PyTorch (python -m ops_cv_amd.build)."""
 import os
 import subprocess
 import sys
@@ -7,7 +8,7 @@ _HERE = os.path.dirname(os.path.abspath(__file__))
 
 
 def build(force=True, jobs=8):
-    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), "-j%d" % jobs]
+    cmd = ["make", "-C", os.path.join(_HERE, "csrc"), "-j%d" % jobs, "all", "helpers"]
     if force:
         cmd.append("-B")
     proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)

@@ -370,7 +370,9 @@ def _native():
         try:
             from . import _torch_helpers
         except ImportError as e:
-            raise RuntimeError("_torch_helpers.so is not built: run `python -m ops_cv_amd.build`") from e
+            built = os.path.exists(os.path.join(os.path.dirname(os.path.abspath(__file__)), "_torch_helpers.so"))
+            why = "does not load (%s): built against another PyTorch or Python?" % e if built else "is not built:"
+            raise RuntimeError("_torch_helpers.so %s run `python -m ops_cv_amd.build`" % why) from e
         _torch_helpers.set_error_class(AclnnError)
         _helpers = _torch_helpers
     return _helpers

@@ -1,4 +1,5 @@
-"""Input gradients of the samplers through the sorting variant (gs_grad_gather.hip), bit for bit against the oracle."""
+"""Input gradients of the samplers through the sorting variant (gs_grad_gather.hip), and of planes through the elections
+(gs2d_grad.hip) where these are the faster ones, bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -43,6 +44,44 @@ def test_planes(oracle, device, aclnn, dtype, interp, pad):
         got, _ = aclnn.grid_sampler2d_backward(*(I.to_torch(v, dtype, device) for v in (go, x, g)), interp, pad, False)
         torch.cuda.synchronize()
         assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref)), (xs, out, kind)
+
+
+# What the shapes above leave to other variants: bilinear samples of 8 channels and more (the list variant up to 16384
+# points) and nearest samples below 25 chunks of points.
+SORTED2D = [(0, (1, 70, 20, 31), (130, 140), "random"), (0, (1, 9, 81, 101), (129, 130), "affine"),
+            (0, (1, 70, 20, 31), (130, 140), "far"), (1, (2, 3, 37, 53), (82, 81), "affine"),
+            (1, (1, 2, 20, 31), (90, 75), "random"), (1, (1, 5, 19, 23), (90, 80), "far"), (1, (2, 9, 81, 101), (81, 101), "affine")]
+# Large batches: several chunks of points; planes of two bands, of one and of a few elements that many points share.
+ELECTED2D = [(0, (400, 1, 80, 90), (20, 21), "random"), (0, (300, 2, 12, 12), (30, 40), "affine"),
+             (1, (600, 1, 12, 12), (90, 80), "random"), (1, (130, 3, 70, 80), (82, 81), "affine"),
+             (2, (200, 1, 70, 80), (30, 31), "random"), (2, (300, 2, 16, 16), (45, 50), "affine")]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("interp,xs,out,kind,sorts", [c + (True,) for c in SORTED2D] + [c + (False,) for c in ELECTED2D])
+def test_planes_by_the_variant_that_takes_them(oracle, device, aclnn, dtype, interp, xs, out, kind, sorts):
+    import torch
+    points = out[0] * out[1]
+    lists = interp == 0 and xs[1] >= 8 and points <= 16384 and points * (4 if dtype == "fp32" else 2) <= 32768
+    assert not lists and (host_plans.sorting_takes_planes(dtype, interp, xs, points) is not None) == sorts
+    rng = np.random.default_rng(4050 + interp)
+    x = I.cast_np(rng.standard_normal(xs).astype(np.float32), dtype)
+    g = I.cast_np(_grid2d(rng, kind, xs[0], *out), dtype)
+    go = I.cast_np(rng.standard_normal(xs[:2] + out).astype(np.float32), dtype)
+    tensors = [I.to_torch(v, dtype, device) for v in (go, x, g)]
+    hs = [aclnn.tensor_handle(t) for t in tensors + tensors[1:]]
+    mask = aclnn.create_bool_array([True, False])
+    st, ws, ex = aclnn.get_workspace_size_grid_sampler2d_backward(*hs[:3], interp, 1, False, mask, *hs[3:])
+    assert st == 0 and (ws > 0) == sorts  # the elections need no workspace
+    aclnn.destroy_executor(ex)
+    aclnn.destroy_bool_array(mask)
+    for h in hs:
+        aclnn.destroy_tensor(h)
+    for pad in (0, 1, 2):
+        ref, _ = oracle.grid_sampler2d_backward(go, x, g, interp, pad, False, dtype=I.oracle_code(dtype))
+        got, _ = aclnn.grid_sampler2d_backward(*tensors, interp, pad, False)
+        torch.cuda.synchronize()
+        assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref)), pad
 
 
 # the last: more items than the reference device has cores, so that the chunks of every other item start at a shift

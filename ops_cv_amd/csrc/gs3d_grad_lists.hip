@@ -29,6 +29,7 @@
 #include <type_traits>
 
 #include "gs3d_grad_math.hpp"
+#include "gs_grad_sort_list.hpp"
 #include "kernels.hpp"
 #include "options.hpp"
 
@@ -232,39 +233,6 @@ struct Fold3<_Float16> {
     static __device__ __forceinline__ void store(_Float16* p, acc_t acc) { __builtin_nontemporal_store(acc, p); }
 };
 
-// The first NK entries of a lane's list (every kLThreads-th word from `mine`), sorted ascending through registers.
-template <int NK>
-__device__ __forceinline__ void sort_list(uint32_t* mine, uint32_t len)
-{
-    uint32_t key[NK];
-#pragma unroll
-    for (int i = 0; i < NK; i++) {
-        const uint32_t v = mine[i * kLThreads];
-        key[i] = ((uint32_t)i < len) ? v : 0xFFFFFFFFu;
-    }
-#pragma unroll
-    for (int size = 2; size <= NK; size *= 2) {
-#pragma unroll
-        for (int stride = size / 2; stride > 0; stride /= 2) {
-#pragma unroll
-            for (int i = 0; i < NK; i++) {
-                const int l = i ^ stride;
-                if (l > i) {
-                    const uint32_t lo = key[i] < key[l] ? key[i] : key[l];
-                    const uint32_t hi = key[i] < key[l] ? key[l] : key[i];
-                    const bool ascending = (i & size) == 0;
-                    key[i] = ascending ? lo : hi;
-                    key[l] = ascending ? hi : lo;
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NK; i++) {
-        mine[i * kLThreads] = key[i];
-    }
-}
-
 template <typename T>
 __global__ __launch_bounds__(kLThreads) void gs3d_lists_gather_kernel(T* __restrict__ dx,
                                                                        uint32_t* __restrict__ ws, Grad3Params p,
@@ -362,9 +330,9 @@ __global__ __launch_bounds__(kLThreads) void gs3d_lists_gather_kernel(T* __restr
     // or of 32 where a lane of the wavefront has more (past its end a list is padded with the largest key).  An
     // insertion sort in LDS, chains of dependent reads and writes, took three times as long as everything else here.
     if (__builtin_amdgcn_ballot_w64(len > 16u) == 0) {
-        sort_list<16>(mine, len);
+        sort_list<16, kLThreads>(mine, len);
     } else {
-        sort_list<32>(mine, len);
+        sort_list<32, kLThreads>(mine, len);
     }
     // Walk the list once per group of channels, two entries in flight: the operands of the entry after this one are
     // asked for before this one is folded in.  No branches in the loop -- past the end of the list or of the channels

@@ -9,7 +9,7 @@
 //   clear   the counts of every cell
 //   count   one lane per grid point: an atomic count per cell gives the point its rank in the cell (which rank depends
 //           on timing, which points a cell holds does not); the source coordinates go to scratch
-//   place   one lane per four cells: every cell gets a run of the item's list (a prefix sum per workgroup, one atomic
+//   place   one lane per eight cells: every cell gets a run of the item's list (a prefix sum per workgroup, one atomic
 //           add per workgroup for its base: the order of the runs does not matter)
 //   fill    one lane per grid point: the point's entry goes to its run
 //   gather  one lane per element: the element collects the entries of the cells it is a corner of -- cell (y - ys,
@@ -36,6 +36,7 @@
 #include "gs2d_grad_math.hpp"
 #include "gs3d_grad_math.hpp"
 #include "gs_grad_gather.hpp"
+#include "gs_grad_sort_list.hpp"
 #include "kernels.hpp"
 
 namespace opscv {
@@ -420,39 +421,6 @@ __device__ __forceinline__ void sort_run(const uint32_t* run, uint32_t len, uint
     }
 }
 
-// The first NK entries of a lane's list (every kThreads-th word from `mine`), sorted ascending through registers.
-template <int NK>
-__device__ __forceinline__ void sort_list(uint32_t* mine, uint32_t len)
-{
-    uint32_t key[NK];
-#pragma unroll
-    for (int i = 0; i < NK; i++) {
-        const uint32_t v = mine[i * kThreads];
-        key[i] = ((uint32_t)i < len) ? v : 0xFFFFFFFFu;
-    }
-#pragma unroll
-    for (int size = 2; size <= NK; size *= 2) {
-#pragma unroll
-        for (int stride = size / 2; stride > 0; stride /= 2) {
-#pragma unroll
-            for (int i = 0; i < NK; i++) {
-                const int l = i ^ stride;
-                if (l > i) {
-                    const uint32_t lo = key[i] < key[l] ? key[i] : key[l];
-                    const uint32_t hi = key[i] < key[l] ? key[l] : key[i];
-                    const bool ascending = (i & size) == 0;
-                    key[i] = ascending ? lo : hi;
-                    key[l] = ascending ? hi : lo;
-                }
-            }
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NK; i++) {
-        mine[i * kThreads] = key[i];
-    }
-}
-
 // The run (start, length) of each cell that element (x, y, z) is a corner of, in corner order.
 template <int DIM, int INTERP>
 __device__ __forceinline__ void runs_of(const uint32_t* __restrict__ wsn, const GatherParams& p, int32_t e, int32_t x,
@@ -554,11 +522,11 @@ __global__ __launch_bounds__(kThreads) void gs_gather_kernel(const T* __restrict
         at += count[r];
     }
     if (__builtin_amdgcn_ballot_w64(len > 8u) == 0) {
-        sort_list<8>(mine, len);
+        sort_list<8, kThreads>(mine, len);
     } else if (LIST <= 16 || __builtin_amdgcn_ballot_w64(len > 16u) == 0) {
-        sort_list<16>(mine, len);
+        sort_list<16, kThreads>(mine, len);
     } else {
-        sort_list<LIST>(mine, len);
+        sort_list<LIST, kThreads>(mine, len);
     }
     const Coords<T, DIM>* coords = reinterpret_cast<const Coords<T, DIM>*>(wsn + p.lay.coords);
     const uint32_t phase = (uint32_t)phase_of(n, p);

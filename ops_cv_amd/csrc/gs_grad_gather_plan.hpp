@@ -188,8 +188,10 @@ inline PlaneGradTimes plane_grad_times(const GradGatherArgs& a)
 
 // Whether the sorting variant takes the input gradient of planes (where the list variant does not).
 //
-// Up to 24 tap passes over a chunk the elections take 10 to 30 us and sorting no less (fp32 N1 C3: bilinear 4 chunks 17
-// us against 20, 9 chunks 32 / 22; nearest 16 chunks 21 / 19; bicubic 1 chunk 24 / 36, 3 chunks 50 / 41).  Beyond, sorting
+// Up to 24 tap passes over a chunk (6 chunks bilinear, 24 nearest, 1 bicubic) the elections take 10 to 30 us and sorting as
+// much or more.  Sorting against elections over grids and planes of up to eight items, medians: bilinear 5 and 6 chunks
+// 0.95, 7 and 8 0.52; nearest 13 to 16 1.05, 17 to 24 0.90, 25 to 30 0.82; bicubic 1 chunk 1.69, 2 0.95, 3 0.74 (fp32 N1 C3:
+// bilinear 4 chunks 17 us against 20, 9 chunks 32 / 22; bicubic 1 chunk 24 / 36, 3 chunks 50 / 41).  Beyond, sorting
 // wins unless batches are large (every item costs its passes over the plane, the elections of a thousand workgroups run
 // side by side) or points are few on large planes, or many on small ones: fp32 512 x 3 x 64x64 from 40x40 points 24.9 us
 // against 75.6, 1 x 3 x 1080x1920 from 40x40 18.3 / 57.6, 1024 x 1 x 16x16 from 64x64 100 / 1014; bicubic 512 x 3 x

@@ -139,3 +139,32 @@ def test_volumes_in_groups_of_items(device, aclnn):
         with aclnn.option("gs3d_grad_variant", variant):
             grads.append(aclnn.grid_sampler3d_backward(go, x, grid, 0, 0, False, (True, False))[0])
     assert torch.equal(*grads)
+
+
+def test_groups_of_items_in_a_graph(device, aclnn):
+    """replays of a captured call whose groups share their scratch, with eager work between them"""
+    import torch
+    xs, out = (45, 1, 480, 641), (480, 641)
+    assert host_plans.gather_groups("fp16", 0, xs, out[0] * out[1])[0] < 45
+    g = torch.Generator(device=device).manual_seed(6)
+    x, go = (torch.randn(xs, generator=g, device=device).half() for _ in range(2))
+    grid = torch.empty((45,) + out + (2,), dtype=torch.float16, device=device)
+    dx, dg = torch.empty_like(x), torch.empty_like(grid)
+    grids = [(torch.rand(grid.shape, generator=g, device=device) * 2.4 - 1.2).half() for _ in range(3)]
+    want = [aclnn.grid_sampler2d_backward(go, x, v) for v in grids]
+    grid.copy_(grids[0])
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        aclnn.grid_sampler2d_backward(go, x, grid, input_grad=dx, grid_grad=dg)
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            aclnn.grid_sampler2d_backward(go, x, grid, input_grad=dx, grid_grad=dg)
+    torch.cuda.synchronize()
+    for i in (0, 1, 2, 1):
+        grid.copy_(grids[i])
+        dx.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(dx, want[i][0]) and torch.equal(dg, want[i][1]), i

@@ -196,10 +196,10 @@ inline PlaneGradTimes plane_grad_times(const GradGatherArgs& a)
 // side by side) or points are few on large planes, or many on small ones: fp32 512 x 3 x 64x64 from 40x40 points 24.9 us
 // against 75.6, 1 x 3 x 1080x1920 from 40x40 18.3 / 57.6, 1024 x 1 x 16x16 from 64x64 100 / 1014; bicubic 512 x 3 x
 // 64x64 340 / 1682.  The elections' time follows the grid more than sorting does (a chunk of a turned grid on a small
-// plane can take three times the rounds of a scattered one), less so in large batches: hence the margins.  Of the 1970
-// calls that sorting would take by tap passes alone, 237 were slower than elections, the worst 8.7 times; with the
-// estimates 75, the worst but one (7.6 times: long runs of scattered bicubic points) 2.4, and 44 of those left to the
-// elections would have been faster sorted, by 2.9 at most.
+// plane can take three times the rounds of a scattered one), nearest samples' most: hence the margins, which leave a launch
+// to sorting unless the elections are clearly faster.  Of the 1970 calls that sorting would take by tap passes alone, 237 were
+// slower than elections, the worst 8.7 times; with the estimates 93, the worst but one (7.6 times: long runs of scattered
+// bicubic points) 3.1, and 23 of those left to the elections would have been faster sorted, by 2.9 at most.
 inline bool sorting_takes_planes(const GradGatherArgs& a)
 {
     const int64_t chunks = (a.points + 255) / 256;
@@ -208,7 +208,7 @@ inline bool sorting_takes_planes(const GradGatherArgs& a)
         return false;
     }
     const PlaneGradTimes t = plane_grad_times(a);
-    const double margin = a.N >= 64 ? 0.9 : (a.interp == 1 ? 0.5 : 0.7);
+    const double margin = (a.interp == 1 && a.N < 64) ? 0.5 : 0.7;
     return t.elections >= margin * t.sorting;
 }
 

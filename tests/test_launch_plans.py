@@ -63,7 +63,7 @@ GRADIENTS = [
     ("fp32", 0, (512, 3, 64, 64), 1600, 24.9, 75.6), ("fp16", 0, (1000, 3, 48, 48), 2304, 74.7, 132.9),
     ("fp32", 0, (1, 3, 1080, 1920), 1600, 18.3, 57.6), ("fp16", 0, (8, 3, 512, 512), 1600, 20.6, 55.0),
     ("fp32", 0, (1024, 1, 16, 16), 4096, 99.9, 1014), ("fp32", 0, (512, 1, 16, 16), 2304, 52.4, 194),
-    ("fp32", 1, (512, 3, 64, 64), 6561, 44.6, 211), ("fp32", 1, (256, 64, 32, 32), 6561, 191, 593),
+    ("fp32", 1, (512, 3, 64, 64), 6561, 44.6, 211), ("fp16", 0, (128, 7, 32, 32), 1600, 64.1, 41.9),
     ("fp32", 2, (512, 3, 64, 64), 4096, 340, 1682), ("fp32", 2, (512, 3, 32, 32), 512, 55, 183),
     ("fp16", 2, (1024, 8, 32, 32), 1024, 220, 758)]
 

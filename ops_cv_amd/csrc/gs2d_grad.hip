@@ -23,6 +23,7 @@
 
 #include <type_traits>
 
+#include "fast_div.hpp"
 #include "gs2d_grad_math.hpp"
 #include "gs_grad_gather.hpp"
 #include "kernels.hpp"
@@ -34,6 +35,7 @@ namespace {
 constexpr int kThreads = 256;         // also the chunk length of the accumulation order
 constexpr uint32_t kKeyBits = 8;      // 256 points of a chunk
 constexpr uint32_t kEpochMax = (1u << (32 - kKeyBits)) - 1;
+constexpr int kGridTile = 16;         // the grid kernel's tiles are square: a lane per grid point
 constexpr int kTagsMax = 1024;        // election tags of a band
 
 // Tag of a band element.  Elements that share a tag are elected as if they were one; folding the high bits in keeps
@@ -60,6 +62,8 @@ struct GradParams {
     int32_t pad, align;
     int32_t band_px;  // plane elements per workgroup (dx kernel)
     int32_t tags;     // election tags of the dx kernel, a power of two (tag_of)
+    uint32_t pieces;  // tiles of the grid kernel, and how they are numbered
+    FastDiv by_item, by_tiles_x;
 };
 
 // CB channels of one batch item per workgroup: the grid points, their taps and the election of a round are the
@@ -224,28 +228,55 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_input_kernel(const T* __re
     }
 }
 
-template <typename T, int INTERP>
+// One lane per grid point.  TILED: a workgroup takes 16 x 16 points of an item, a wavefront 16 x 4 of them, so that under a
+// turned grid the corners of its points share cache lines in both directions: 64 points of a row lie in up to 64 lines of a
+// plane.  XCD k takes the k-th eighth of the workgroups, so that neighbouring tiles share an L2.
+//
+// Bound by the lines that the gathers touch and their latency: the loads of up to eight channels are on their way together,
+// of fewer channels all of them (fp32 8x3x479x637, rotations of up to 30 degrees: 58 us in rows, a channel after the other;
+// 40 with the three channels' loads together; 33 in tiles).
+template <typename T, int INTERP, bool TILED>
 __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __restrict__ gout, const T* __restrict__ x,
                                                                    const T* __restrict__ grid, T* __restrict__ dgrid,
                                                                    int64_t total, GradParams p, int32_t blocks_per_item)
 {
     using Taps = GradTaps<T, INTERP>;
-    // blocks_per_item > 0: workgroups are handed to the 8 XCDs round-robin by index; all workgroups of one batch item
-    // go to one XCD, so that the planes of that item (every lane walks all of them) are fetched into one L2 once
-    // instead of into all eight (fp16 N16 C256 64x64: 185.6 MB fetched for 67.1 MB of operands otherwise).  The launch
-    // plan asks for it when the items divide evenly among the XCDs and the workgroups evenly among the items.
-    uint32_t block = blockIdx.x;
-    if (blocks_per_item > 0) {
-        const uint32_t xcd = blockIdx.x & 7u, i = blockIdx.x >> 3;
-        block = ((i / (uint32_t)blocks_per_item) * 8u + xcd) * (uint32_t)blocks_per_item + i % (uint32_t)blocks_per_item;
-    }
-    const int64_t idx = (int64_t)block * kThreads + threadIdx.x;
-    if (idx >= total) {
-        return;
-    }
     const int32_t points = p.Ho * p.Wo;
-    const int64_t n = idx / points;
-    const int32_t pt = (int32_t)(idx - n * points);
+    int64_t n, idx;
+    int32_t pt;
+    if constexpr (TILED) {
+        const uint32_t per_xcd = p.pieces / 8u + (p.pieces % 8u != 0u ? 1u : 0u);
+        const uint32_t piece = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
+        if ((blockIdx.x >> 3) >= per_xcd || piece >= p.pieces) {
+            return;
+        }
+        const uint32_t item = fast_div(piece, p.by_item), tile = piece - item * p.by_item.div;
+        const uint32_t ty = fast_div(tile, p.by_tiles_x), tx = tile - ty * p.by_tiles_x.div;
+        const int32_t px = (int32_t)(tx * kGridTile + threadIdx.x % kGridTile);
+        const int32_t py = (int32_t)(ty * kGridTile + threadIdx.x / kGridTile);
+        if (px >= p.Wo || py >= p.Ho) {
+            return;
+        }
+        n = item;
+        pt = py * p.Wo + px;
+        idx = n * points + pt;
+    } else {
+        // blocks_per_item > 0: workgroups are handed to the 8 XCDs round-robin by index; all workgroups of one batch item
+        // go to one XCD, so that the planes of that item (every lane walks all of them) are fetched into one L2 once
+        // instead of into all eight (fp16 N16 C256 64x64: 185.6 MB fetched for 67.1 MB of operands otherwise).  The launch
+        // plan asks for it when the items divide evenly among the XCDs and the workgroups evenly among the items.
+        uint32_t block = blockIdx.x;
+        if (blocks_per_item > 0) {
+            const uint32_t xcd = blockIdx.x & 7u, i = blockIdx.x >> 3;
+            block = ((i / (uint32_t)blocks_per_item) * 8u + xcd) * (uint32_t)blocks_per_item + i % (uint32_t)blocks_per_item;
+        }
+        idx = (int64_t)block * kThreads + threadIdx.x;
+        if (idx >= total) {
+            return;
+        }
+        n = idx / points;
+        pt = (int32_t)(idx - n * points);
+    }
     if (INTERP == 1) {
         ElemIO<T>::store(dgrid + 2 * idx, 0.0f);
         ElemIO<T>::store(dgrid + 2 * idx + 1, 0.0f);
@@ -258,12 +289,27 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __res
     const T* x_n = x + n * p.C * (int64_t)plane_px;
     const T* go_n = gout + n * p.C * (int64_t)points + pt;
     float gix = 0.0f, giy = 0.0f;
+    // f(number of channels, first channel): the sums run over the channels in order; the loads do not depend on them, so
+    // they are issued a group of channels ahead (a lane has one grid point and would otherwise wait out every load in turn)
+    auto for_groups = [&](auto&& f) {
+        int32_t c = 0;
+        for (; c + 8 <= p.C; c += 8) {
+            f(std::integral_constant<int, 8>{}, c);
+        }
+        if (c + 4 <= p.C) {
+            f(std::integral_constant<int, 4>{}, c);
+            c += 4;
+        }
+        switch (p.C - c) {
+            case 3: f(std::integral_constant<int, 3>{}, c); break;
+            case 2: f(std::integral_constant<int, 2>{}, c); break;
+            case 1: f(std::integral_constant<int, 1>{}, c); break;
+            default: break;
+        }
+    };
     if (INTERP == 0) {
         const float dxe = (float)(tp.x0 == INT32_MAX ? tp.x0 : tp.x0 + 1) - tp.fx, dxw = tp.fx - (float)tp.x0;
         const float dys = (float)(tp.y0 == INT32_MAX ? tp.y0 : tp.y0 + 1) - tp.fy, dyn = tp.fy - (float)tp.y0;
-        // The sums run over the channels in order; the loads do not depend on them, so they are issued a group of
-        // channels ahead (a lane has one grid point and would otherwise wait out every load in turn).
-        constexpr int U = 8;
         const bool ok0 = tp.off[0] >= 0, ok1 = tp.off[1] >= 0, ok2 = tp.off[2] >= 0, ok3 = tp.off[3] >= 0;
         const int32_t o0 = ok0 ? tp.off[0] : 0, o1 = ok1 ? tp.off[1] : 0, o2 = ok2 ? tp.off[2] : 0,
                       o3 = ok3 ? tp.off[3] : 0;
@@ -285,7 +331,6 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __res
                 giy += v3 * dxw * go;
             }
         };
-        int32_t c = 0;
         if (p.W >= 2) {
             // The west and east corner of a row are neighbours in memory: one load of two elements (aligned to one
             // element only) per row instead of two loads halves the addresses the gather puts through the memory
@@ -298,7 +343,8 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __res
             const bool lo_w = (x0 == pb), lo_e = (x1 == pb);
             const int32_t r0 = (tp.y0 >= 0 && tp.y0 < p.H) ? tp.y0 * p.W + pb : 0;
             const int32_t r1 = (y1 >= 0 && y1 < p.H) ? y1 * p.W + pb : 0;
-            for (; c + U <= p.C; c += U) {
+            for_groups([&](auto count, int32_t c) {
+                constexpr int U = decltype(count)::value;
                 float go[U];
                 PairBits north[U], south[U];
 #pragma unroll
@@ -317,28 +363,25 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __res
                     const float slo = ElemIO<T>::load(&s2[0]), shi = ElemIO<T>::load(&s2[1]);
                     accumulate(go[u], lo_w ? nlo : nhi, lo_e ? nlo : nhi, lo_w ? slo : shi, lo_e ? slo : shi);
                 }
-            }
-        }
-        for (; c + U <= p.C; c += U) {
-            float go[U], v[U][4];
+            });
+        } else {
+            for_groups([&](auto count, int32_t c) {
+                constexpr int U = decltype(count)::value;
+                float go[U], v[U][4];
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                const T* xc = x_n + (int64_t)(c + u) * plane_px;
-                go[u] = ElemIO<T>::load(go_n + (int64_t)(c + u) * points);
-                v[u][0] = ElemIO<T>::load(xc + o0);
-                v[u][1] = ElemIO<T>::load(xc + o1);
-                v[u][2] = ElemIO<T>::load(xc + o2);
-                v[u][3] = ElemIO<T>::load(xc + o3);
-            }
+                for (int u = 0; u < U; u++) {
+                    const T* xc = x_n + (int64_t)(c + u) * plane_px;
+                    go[u] = ElemIO<T>::load(go_n + (int64_t)(c + u) * points);
+                    v[u][0] = ElemIO<T>::load(xc + o0);
+                    v[u][1] = ElemIO<T>::load(xc + o1);
+                    v[u][2] = ElemIO<T>::load(xc + o2);
+                    v[u][3] = ElemIO<T>::load(xc + o3);
+                }
 #pragma unroll
-            for (int u = 0; u < U; u++) {
-                accumulate(go[u], v[u][0], v[u][1], v[u][2], v[u][3]);
-            }
-        }
-        for (; c < p.C; c++) {
-            const T* xc = x_n + (int64_t)c * plane_px;
-            accumulate(ElemIO<T>::load(go_n + (int64_t)c * points), ElemIO<T>::load(xc + o0),
-                       ElemIO<T>::load(xc + o1), ElemIO<T>::load(xc + o2), ElemIO<T>::load(xc + o3));
+                for (int u = 0; u < U; u++) {
+                    accumulate(go[u], v[u][0], v[u][1], v[u][2], v[u][3]);
+                }
+            });
         }
     } else {
         const float xf = __builtin_floorf(tp.fx), yf = __builtin_floorf(tp.fy);
@@ -348,16 +391,20 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __res
         cubic_coefficients_grad(cyg, tp.fy - yf);
         cubic_coefficients_grad(cxg, tp.fx - xf);
         for (int32_t c = 0; c < p.C; c++) {
-            const float go = ElemIO<T>::load(go_n + (int64_t)c * points);
             const T* xc = x_n + (int64_t)c * plane_px;
+            const float go = ElemIO<T>::load(go_n + (int64_t)c * points);
+            T v[16];  // all on their way together; a tap outside the plane counts as 0
+#pragma unroll
+            for (int k = 0; k < 16; k++) {
+                v[k] = xc[tp.off[k] >= 0 ? tp.off[k] : 0];
+            }
 #pragma unroll
             for (int i = 0; i < 4; i++) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) {
-                    const int32_t o = tp.off[i * 4 + j];
-                    const float v = (o >= 0) ? ElemIO<T>::load(xc + o) : 0.0f;
-                    giy += v * cyg[j] * cx[i] * go;
-                    gix += v * cxg[i] * cy[j] * go;
+                    const float w = (tp.off[i * 4 + j] >= 0) ? ElemIO<T>::load(&v[i * 4 + j]) : 0.0f;
+                    giy += w * cyg[j] * cx[i] * go;
+                    gix += w * cxg[i] * cy[j] * go;
                 }
             }
         }
@@ -387,10 +434,23 @@ GradGatherArgs gather_args(const GridSamplerGradArgs& a)
     return g;
 }
 
+// Tiles of grid points for the grid gradient: planes beyond the first-level cache, where lines are fetched again for every
+// row of points, two workgroups per CU, and few lanes along the edges without a point.  Rows / tiles, both gradients' grid
+// part alone: fp32 8x3x479x637 40.5 / 33.2 us, fp16 6x3x576x472 -> 362x297 15.8 / 11.3, fp32 2x37x132x184 11.7 / 9.6; smaller
+// planes bf16 2x105x90x146 19.4 / 24.4, fp16 19x11x144x120 -> 210x175 22.6 / 23.8; few tiles fp32 3x3x241x369 -> 128x196 7.0 /
+// 7.2.
+bool grid_in_tiles(const GridSamplerGradArgs& a)
+{
+    const int64_t tiles_x = (a.Wout + kGridTile - 1) / kGridTile, tiles_y = (a.Hout + kGridTile - 1) / kGridTile;
+    const int64_t lanes = tiles_x * tiles_y * kGridTile * kGridTile;
+    return a.Hin * a.Win * elem_size(a.elem) > (64 << 10) && a.N * tiles_x * tiles_y >= 512 &&
+           lanes - lanes / 5 <= a.Hout * a.Wout;
+}
+
 template <typename T, int INTERP>
 hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
 {
-    GradParams p;
+    GradParams p{};
     p.C = (int32_t)a.C;
     p.H = (int32_t)a.Hin;
     p.W = (int32_t)a.Win;
@@ -469,6 +529,19 @@ hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
     }
     if (a.dgrid != nullptr && !dgrid_done) {
         const int64_t total = a.N * a.Hout * a.Wout;
+        const int64_t tiles_x = (a.Wout + kGridTile - 1) / kGridTile, tiles_y = (a.Hout + kGridTile - 1) / kGridTile;
+        const int64_t tiles = a.N * tiles_x * tiles_y;
+        if (INTERP != 1 && grid_in_tiles(a) && tiles <= INT32_MAX / 2) {
+            p.pieces = (uint32_t)tiles;
+            p.by_item = make_fast_div((uint32_t)(tiles_x * tiles_y));
+            p.by_tiles_x = make_fast_div((uint32_t)tiles_x);
+            const uint32_t blocks = (uint32_t)((tiles + 7) / 8 * 8);  // as many for every XCD
+            if (fits_launch(blocks, kThreads)) {
+                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, true>), dim3(blocks), dim3(kThreads), 0, stream,
+                                   (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, total, p, 0);
+                return hipGetLastError();
+            }
+        }
         const int64_t blocks = (total + kThreads - 1) / kThreads;
         if (blocks > INT32_MAX) {
             return hipErrorInvalidValue;
@@ -476,7 +549,7 @@ hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
         const int64_t points = a.Hout * a.Wout;
         const int32_t blocks_per_item =
             (points % kThreads == 0 && a.N % 8 == 0 && points / kThreads <= INT32_MAX) ? (int32_t)(points / kThreads) : 0;
-        hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
+        hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, false>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
                            (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, total, p, blocks_per_item);
         return hipGetLastError();
     }

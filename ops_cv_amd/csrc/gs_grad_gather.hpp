@@ -12,4 +12,8 @@ namespace opscv {
 int64_t grad_gather_words(const GradGatherArgs& a);
 hipError_t run_grad_gather(const GradGatherArgs& a, hipStream_t stream);
 
+// the same by tiles of the plane or volume (gs_grad_tiles.hip)
+int64_t grad_tiles_words(const GradGatherArgs& a);
+hipError_t run_grad_tiles(const GradGatherArgs& a, hipStream_t stream);
+
 }  // namespace opscv

@@ -1,0 +1,1152 @@
+// Backward of the grid samplers for gfx950: gradient of the input tile by tile, for planes and volumes, linear and
+// nearest samples, any number of channels.
+//
+// The sum that reaches an element is a fixed sequence (gs2d_grad.hip, gs3d_grad.hip): its contributions ordered by
+// (chunk of 256 grid points, tap, point), every add rounded to the element type.  Two kernels, no global atomics:
+//
+//   bin     a workgroup takes a block of 1024 consecutive grid points (whole chunks) and sorts them by the tile of the
+//           plane that they contribute to, stably: every block leaves, per tile, a segment of 16-bit point numbers in
+//           ascending order.  A point whose corners lie in several tiles is in the segments of all of them.
+//   gather  a workgroup per tile, a lane per element: the tile's segments, block after block, are its points in
+//           ascending order.  The points are counted by cell in LDS, every lane finds the runs of the cells that its
+//           element is a corner of, keys them (chunk, tap, number in LDS), sorts the keys in registers and folds
+//           weight times gradOutput, both from LDS, with the reference's roundings.  Elements with more contributions
+//           than keys are merged, run by run, a lane each, or where a single element holds hundreds by the whole
+//           wavefront; more points than LDS holds are taken a run of segments after the other, which are whole chunks
+//           in ascending order.
+//
+// Every operand is read once and a point's gradOutput once per tile that it reaches; all that is scattered happens in LDS.
+//
+// fp32 8x3x479x637 from as many points (rotations of up to 30 degrees), operands from memory: lists through global memory
+// (gs_grad_gather.hip) 188 us in six kernels, here bin 21 and gather 71.  Bin: 34 us with an LDS atomic a point, which the
+// 64 lanes of a wavefront on one tile take in turn, 20 with a run of lanes entered at once.  Gather is bound by its chain of
+// steps, not by a unit: 450 vector and 350 scalar instructions a wavefront (28 us of issue), and seven waits for memory or
+// the other wavefronts (segments, records, points; counts, starts, lists, keys) at two workgroups per CU.  Without fetching,
+// sorting and folding keys it takes 47 us, without gradOutput 63, without stores 64; three workgroups per CU (80 registers)
+// are no faster, tiles of 32 x 8 take 92 us (and bin 61), half as many points a round 97.  Weights in LDS instead of
+// coordinates took 82 to 80 us, loads of all of a lane's points together and divisions by multiplication 74, a reflection's
+// constants out of the other paddings' way 69.
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "gs_grad_gather.hpp"
+#include "gs_grad_points.hpp"
+#include "gs_grad_tiles_plan.hpp"
+#include "kernels.hpp"
+
+namespace opscv {
+
+namespace {
+
+constexpr int kPosBits = 11;           // a point's number in LDS, or kRecords: none
+constexpr int kTapBits = 3;
+constexpr uint32_t kNoKey = 0xFFFFFFFFu;
+constexpr uint32_t kNoPlace = 0xFFFFFFFFu;
+constexpr uint32_t kCountedRun = 32;   // runs of up to as many points are put in order by counting, longer ones by ballots
+constexpr uint32_t kSerialMost = 192;  // contributions that a lane merges by itself, and adds by itself where
+constexpr int kFewCrowded = 6;         // more lanes than this of its wavefront have as many as that to do
+
+__device__ __forceinline__ void landed()
+{
+    // what a wavefront writes to LDS it reads back itself, in order
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+__device__ __forceinline__ uint32_t bits_below(uint64_t mask)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// Inclusive sum over the wavefront: within rows of 16 lanes, then from row to row.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v)
+{
+    int s = (int)v;
+    s += __builtin_amdgcn_update_dpp(0, s, 0x111, 0xf, 0xf, false);  // row_shr:1
+    s += __builtin_amdgcn_update_dpp(0, s, 0x112, 0xf, 0xf, false);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xf, 0xf, false);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xf, 0xf, false);
+    s += __builtin_amdgcn_update_dpp(0, s, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
+    s += __builtin_amdgcn_update_dpp(0, s, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
+    return (uint32_t)s;
+}
+
+// The cell of a point: the lattice of low corners for linear interpolation, the element for nearest.  False: no corner
+// is inside (or the coordinate is not a number; sizes are exact in single precision: launch plan).
+template <typename T, int DIM, int INTERP>
+__device__ __forceinline__ bool low_corner(const Coords<T, DIM>& c, const TilesParams& p, int32_t* x, int32_t* y, int32_t* z)
+{
+    constexpr float least = (INTERP == 1) ? 0.0f : -1.0f;
+    auto axis = [&](int i, int32_t size, int32_t* cell) {
+        const float v = ElemIO<T>::load(&c.v[i]);
+        const float f = (INTERP == 1) ? __builtin_rintf(v) : __builtin_floorf(v);
+        const bool in = f >= least && f < (float)size;
+        *cell = (int32_t)(in ? f : 0.0f);
+        return in;
+    };
+    bool in = axis(0, p.W, x);
+    in = axis(1, p.H, y) && in;
+    *z = 0;
+    if constexpr (DIM == 3) {
+        in = axis(2, p.D, z) && in;
+    }
+    return in;
+}
+
+// workgroups go to the eight XCDs in turn: XCD k takes the k-th eighth of all pieces, so that neighbours share an L2
+__device__ __forceinline__ bool piece_of(uint32_t block, uint32_t pieces, const FastDiv& per_item, uint32_t* n, uint32_t* local)
+{
+    const uint32_t per_xcd = (pieces + 7u) >> 3;
+    const uint32_t piece = (block & 7u) * per_xcd + (block >> 3);
+    *n = fast_div(piece, per_item);
+    *local = piece - *n * per_item.div;
+    return (block >> 3) < per_xcd && piece < pieces;
+}
+
+template <typename T, int DIM, int INTERP>
+__global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __restrict__ grid, uint32_t* __restrict__ ws,
+                                                                   TilesParams p, uint32_t pieces)
+{
+    typedef GradTile<DIM> S;
+    constexpr int kWaves = kBinThreads / 64;
+    constexpr int kSteps = kBinPoints / kBinThreads;
+    constexpr int K = (INTERP == 0) ? (1 << DIM) : 1;  // tiles a point reaches at most
+    extern __shared__ __align__(16) uint32_t smem[];
+    __shared__ uint32_t s_total;
+    uint32_t* counts = smem;                      // [wave][tile]
+    unsigned long long* masks = reinterpret_cast<unsigned long long*>(smem + kWaves * p.tiles);  // [wave][tile]
+    uint32_t n, block;
+    if (!piece_of(blockIdx.x, pieces, p.by_blocks, &n, &block)) {
+        return;
+    }
+    const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int32_t phase = (DIM == 3 && p.items_per_core > 1) ? phase_of(n, p) : 0;
+    T raw[kSteps][DIM];  // all loads on their way before the first is looked at
+    bool have[kSteps];
+#pragma unroll
+    for (int u = 0; u < kSteps; u++) {
+        const int32_t pt = (int32_t)(block * kBinPoints) + wave * 256 + u * 64 + lane - phase;
+        have[u] = pt >= 0 && pt < p.points;
+        __builtin_memcpy(raw[u], grid + ((int64_t)n * p.points + (have[u] ? pt : 0)) * DIM, sizeof(raw[u]));
+    }
+    for (int i = t; i < kWaves * p.tiles * 3 / 4; i += kBinThreads) {
+        reinterpret_cast<uint4*>(smem)[i] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    if (t == 0) {
+        s_total = 0u;
+    }
+    // The tiles of a point, -1 where it has no k-th one: that of its low corner, then those that the high corner lies in
+    // along x, along y and so on; `any`: the k of which any lane of the wavefront has one.
+    auto tiles_of = [&](int u, int32_t (&tile)[K], uint32_t* any) {
+        int32_t x, y, z;
+        const bool in = low_corner<T, DIM, INTERP>(coords_of<T, DIM, INTERP>(raw[u], p), p, &x, &y, &z) && have[u];
+        auto low_of = [](int32_t v, int32_t edge) { return (int32_t)((uint32_t)(v < 0 ? 0 : v) / (uint32_t)edge); };
+        auto next = [](int32_t v, int32_t size, int32_t edge) {  // the high corner lies in the next tile
+            return v >= 0 && (v & (edge - 1)) == edge - 1 && v + 1 < size;
+        };
+        int32_t low = low_of(y, S::kY) * p.tiles_x + low_of(x, S::kX);
+        if constexpr (DIM == 3) {
+            low += low_of(z, S::kZ) * p.tiles_x * p.tiles_y;
+        }
+        const bool nx = next(x, p.W, S::kX), ny = next(y, p.H, S::kY), nz = DIM == 3 && next(z, p.D, S::kZ);
+        *any = 1u;
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const bool is = in && (!(k & 1) || nx) && (!(k & 2) || ny) && (!(k & 4) || nz);
+            tile[k] = is ? low + (k & 1) + ((k & 2) ? p.tiles_x : 0) + ((k & 4) ? p.tiles_x * p.tiles_y : 0) : -1;
+            if (k > 0) {
+                *any |= __builtin_amdgcn_ballot_w64(is) != 0 ? 1u << k : 0u;
+            }
+        }
+    };
+    // The rank of a point among those of its tile in earlier lanes and steps of the wavefront, from a mask of the tile's
+    // lanes.  Neighbouring points share tiles: the first of a run of lanes with one tile enters the whole run (an atomic of
+    // 64 lanes on one address would take 64 turns).
+    uint32_t* mine = counts + wave * p.tiles;
+    unsigned long long* my_masks = masks + wave * p.tiles;
+    uint32_t place[kSteps][K], any[kSteps];  // tile << 8 | rank among the wavefront's 256 points
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kSteps; u++) {
+        int32_t tile[K];
+        tiles_of(u, tile, &any[u]);
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            place[u][k] = kNoPlace;
+            if ((any[u] >> k) & 1u) {
+                const int32_t left = __builtin_amdgcn_update_dpp(-2, tile[k], 0x138, 0xf, 0xf, false);  // of the lane before
+                const bool begins = left != tile[k];
+                const uint64_t bounds = __builtin_amdgcn_ballot_w64(begins);
+                if (begins && tile[k] >= 0) {
+                    const uint64_t from_here = ~0ull << lane, later = bounds & (from_here << 1);
+                    atomicOr(&my_masks[tile[k]], (unsigned long long)(((later & (0ull - later)) - 1ull) & from_here));
+                }
+            }
+        }
+        landed();
+        uint64_t mask[K];
+        uint32_t before[K];
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (((any[u] >> k) & 1u) && tile[k] >= 0) {
+                mask[k] = my_masks[tile[k]];
+                before[k] = mine[tile[k]];
+            }
+        }
+        landed();
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (((any[u] >> k) & 1u) && tile[k] >= 0) {
+                const uint32_t below = bits_below(mask[k]);
+                place[u][k] = ((uint32_t)tile[k] << 8) | (before[k] + below);
+                if (below == 0u) {
+                    mine[tile[k]] = before[k] + (uint32_t)__builtin_popcountll(mask[k]);
+                    my_masks[tile[k]] = 0ull;
+                }
+            }
+        }
+        landed();
+    }
+    __syncthreads();
+    // a run of the block's records per tile (the order of the runs does not matter), and within it one per wavefront
+    uint32_t* wsn = ws + (size_t)n * p.lay.item_words;
+    for (int32_t i0 = 0; i0 < p.tiles; i0 += kBinThreads) {
+        const int32_t i = i0 + t;
+        uint32_t of[kWaves], sum = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; w++) {
+            of[w] = (i < p.tiles) ? counts[w * p.tiles + i] : 0u;
+            sum += of[w];
+        }
+        uint32_t start = 0;
+        if (__builtin_amdgcn_ballot_w64(sum != 0u) != 0) {
+            const uint32_t incl = wave_scan(sum);
+            uint32_t base = 0;
+            if (lane == 63) {
+                base = atomicAdd(&s_total, incl);
+            }
+            start = (uint32_t)__builtin_amdgcn_readlane((int)base, 63) + incl - sum;
+            if (sum != 0u) {
+                uint32_t begin = start;
+#pragma unroll
+                for (int w = 0; w < kWaves; w++) {
+                    counts[w * p.tiles + i] = begin;
+                    begin += of[w];
+                }
+            }
+        }
+        if (i < p.tiles) {
+            wsn[p.lay.segments + (size_t)block * p.tiles + i] = start | (sum << 16);
+        }
+    }
+    __syncthreads();
+    uint16_t* records = reinterpret_cast<uint16_t*>(wsn + p.lay.records + (size_t)block * p.lay.block_words);
+#pragma unroll
+    for (int u = 0; u < kSteps; u++) {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if (((any[u] >> k) & 1u) && place[u][k] != kNoPlace) {
+                records[mine[place[u][k] >> 8] + (place[u][k] & 255u)] = (uint16_t)(wave * 256 + u * 64 + lane);
+            }
+        }
+    }
+}
+
+// Ascending, by Batcher's odd-even merge sort (cut to N keys: the ones past the end would stay there): 12 comparators for
+// 6 keys, 19 for 8, 41 for 12, 63 for 16, 127 for 24.
+template <int N>
+__device__ __forceinline__ void sort_keys(uint32_t* key)
+{
+#pragma unroll
+    for (int p = 1; p < N; p *= 2) {
+#pragma unroll
+        for (int k = p; k >= 1; k /= 2) {
+#pragma unroll
+            for (int j = k % p; j + k < N; j += 2 * k) {
+#pragma unroll
+                for (int i = 0; i < k; i++) {
+                    const int l = i + j, h = i + j + k;
+                    if (h < N && l / (2 * p) == h / (2 * p)) {
+                        const uint32_t a = key[l], b = key[h];
+                        key[l] = a < b ? a : b;
+                        key[h] = a < b ? b : a;
+                    }
+                }
+            }
+        }
+    }
+}
+
+// The network for `most` keys, a multiple of STEP up to N.
+template <int N, int STEP>
+__device__ __forceinline__ void sort_most(uint32_t* key, int most)
+{
+    if (most == N) {
+        sort_keys<N>(key);
+    } else if constexpr (N > STEP) {
+        sort_most<N - STEP, STEP>(key, most);
+    }
+}
+
+// The sums of an element's channels.  A contribution is weight times gradOutput rounded to the element type, added with a
+// rounding to the element type.  For fp16 both steps are the native instructions, two channels at a time: the product of
+// two fp16 values is exact in fp32, so rounding it to fp16 is the fp16 product, and the fp32 sum of two fp16 values rounded
+// to fp16 is the fp16 sum (24 >= 2 x 11 + 2 bits).
+template <typename T, int INTERP, int CB>
+struct Sums {
+    float v[CB];
+    __device__ __forceinline__ void clear()
+    {
+#pragma unroll
+        for (int j = 0; j < CB; j++) {
+            v[j] = 0.0f;
+        }
+    }
+    __device__ __forceinline__ void add(const T* go, float w)
+    {
+#pragma unroll
+        for (int j = 0; j < CB; j++) {
+            v[j] = rt<T>(v[j] + value_of<T, INTERP>(ElemIO<T>::load(go + j), w));
+        }
+    }
+    __device__ __forceinline__ float get(int j) const { return v[j]; }
+    __device__ __forceinline__ void set(int j, float f) { v[j] = f; }
+};
+template <int INTERP, int CB>
+struct Sums<_Float16, INTERP, CB> {
+    typedef _Float16 pair_t __attribute__((ext_vector_type(2)));
+    static constexpr int P = (CB + 1) / 2;
+    pair_t v[P];
+    __device__ __forceinline__ void clear()
+    {
+#pragma unroll
+        for (int j = 0; j < P; j++) {
+            v[j] = (pair_t)((_Float16)0.0f);
+        }
+    }
+    __device__ __forceinline__ void add(const _Float16* go, float w)
+    {
+        const pair_t ww = (pair_t)((_Float16)w);  // exact
+#pragma unroll
+        for (int j = 0; j < P; j++) {
+            pair_t g;
+            g.x = go[2 * j];
+            g.y = (2 * j + 1 < CB) ? go[(2 * j + 1 < CB) ? 2 * j + 1 : 0] : (_Float16)0.0f;
+            const pair_t val = (INTERP == 1) ? g : g * ww;
+            v[j] = v[j] + val;
+        }
+    }
+    __device__ __forceinline__ float get(int j) const { return (float)((j & 1) ? v[j >> 1].y : v[j >> 1].x); }
+    __device__ __forceinline__ void set(int j, float f)
+    {
+        if (j & 1) {
+            v[j >> 1].y = (_Float16)f;
+        } else {
+            v[j >> 1].x = (_Float16)f;
+        }
+    }
+};
+
+// Weights of the points in LDS, plane by plane (a lane reads a weight of some point: neighbours in a plane lie in different
+// banks): every corner's, values of the element type; of volumes in single precision, which would fill LDS, the products
+// of the four corners along x and y and the two distances along z.  The last of a plane is zero.
+template <typename T, int DIM, int CAP>
+struct Weights {
+    static constexpr bool kProducts = DIM == 3 && sizeof(T) == 4;
+    static constexpr int kPlanes = kProducts ? 6 : (1 << DIM);
+    static constexpr uint32_t kStride = CAP + 1;
+    T v[kPlanes * kStride];
+    __device__ __forceinline__ void put(uint32_t i, const Coords<T, DIM>& c)
+    {
+        float d[DIM][2];  // to the high edge and from the low edge of the cell, as the decisions of the taps have them
+#pragma unroll
+        for (int k = 0; k < DIM; k++) {
+            const float f = ElemIO<T>::load(&c.v[k]), low = __builtin_floorf(f);
+            d[k][0] = (low + 1.0f) - f;
+            d[k][1] = f - low;
+        }
+#pragma unroll
+        for (int k = 0; k < kPlanes; k++) {
+            float w;
+            if constexpr (kProducts) {
+                w = (k < 4) ? d[0][k & 1] * d[1][(k >> 1) & 1] : d[DIM - 1][k & 1];
+            } else {
+                w = d[0][k & 1] * d[1][(k >> 1) & 1];
+                if constexpr (DIM == 3) {
+                    w = w * d[DIM - 1][k >> 2];
+                }
+            }
+            ElemIO<T>::store(&v[k * kStride + i], as_fp32_value(w));
+        }
+    }
+    __device__ __forceinline__ float get(uint32_t i, uint32_t tap) const
+    {
+        if constexpr (kProducts) {
+            return v[(tap & 3u) * kStride + i] * v[((tap >> 2) + 4u) * kStride + i];
+        } else {
+            return ElemIO<T>::load(&v[tap * kStride + i]);
+        }
+    }
+    __device__ __forceinline__ void clear_last(int t)
+    {
+        if (t < kPlanes) {
+            ElemIO<T>::store(&v[t * kStride + CAP], 0.0f);
+        }
+    }
+};
+
+template <typename T, int DIM, int INTERP, int CB>
+__global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_kernel(
+    const T* __restrict__ gout, const T* __restrict__ grid, T* __restrict__ dx, const uint32_t* __restrict__ ws, TilesParams p,
+    uint32_t pieces, int32_t chans_per_block)
+{
+    typedef GradTile<DIM> S;
+    constexpr int TH = S::kThreads, CAP = S::kRecords, RPL = (CAP + TH - 1) / TH, kWaves = TH / 64;
+    static_assert(CAP % 64 == 0 && CAP >= kBinPoints && CAP < (1 << kPosBits), "whole segments, numbers that fit a key");
+    static_assert(DIM == 3 || S::kX * kWaves * (64 / S::kX) == TH, "whole rows in a wavefront");
+    static_assert(kWaves <= 16, "totals of the wavefronts in a row of lanes");
+    constexpr int PADC = (INTERP == 0) ? 1 : 0;  // cells beside the first element of a row
+    constexpr int CX = S::kX + PADC, CY = S::kY + PADC, CZ = (DIM == 3) ? S::kZ + PADC : 1;
+    constexpr int CELLS = CX * CY * CZ;
+    constexpr int RR = (INTERP == 0) ? (1 << (DIM - 1)) : 1;  // rows of cells: a row's two cells are neighbours in the list
+    constexpr int R = (INTERP == 0) ? 2 * RR : 1;             // runs
+    constexpr int GS = (CB == 3) ? 4 : CB;                    // of a point's gradOutput in LDS
+    constexpr int NK = (DIM == 3 && INTERP == 0) ? 24 : 16;   // keys of an element, in steps of
+    constexpr int kStep = (DIM == 3 && INTERP == 0) ? 4 : 2;
+    constexpr int kStarts = (CELLS + 1 + 3) / 4 * 4;
+    // a point of a plane is a contribution of four elements: all crowded ones fit; of volumes most do
+    constexpr uint32_t kSorted = (INTERP == 1) ? CAP : ((DIM == 3) ? 3072 : 4 * CAP);
+    constexpr uint32_t kLowBits = (1u << (kPosBits + kTapBits)) - 1u;
+    __shared__ __align__(16) uint32_t s_start[kStarts];  // counts by cell, then the start of every cell's run in s_list
+    __shared__ uint32_t s_list[CAP + 2 * NK];  // keys by cell; lanes read past the end of their runs
+    __shared__ Weights<T, DIM, (INTERP == 0) ? CAP : 0> s_weight;
+    __shared__ __align__(16) T s_go[(CAP + 1) * GS];  // the last: zeros
+    // of crowded elements: while lists are put in order, then while contributions are added
+    struct ByPoint {
+        uint32_t key[CAP];  // chunk, parity of the cell along every axis, the point's number: ascending
+        uint16_t cell[CAP];
+    };
+    struct ByWave {
+        float value[CB][68];
+        uint16_t order[64];
+    };
+    union Rare {
+        ByPoint points;
+        ByWave waves[kWaves];
+    };
+    __shared__ __align__(16) Rare s_rare;
+    __shared__ uint16_t s_long[CAP / kCountedRun + 1];
+    __shared__ uint32_t s_scan[kWaves];
+    __shared__ uint16_t s_sorted[kSorted];  // contributions of crowded elements in order: the low bits of their keys
+    __shared__ uint32_t s_longs, s_crowded, s_sorted_used;
+    extern __shared__ uint32_t s_seg[];  // per segment that is not empty: points before it; block << 14 | first record
+    uint32_t n, local;
+    if (!piece_of(blockIdx.x, pieces, p.by_item, &n, &local)) {
+        return;
+    }
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const uint32_t cblock = fast_div(local, p.by_tiles), tile = local - cblock * (uint32_t)p.tiles;
+    const uint32_t* wsn = ws + (size_t)n * p.lay.item_words;
+    const uint16_t* records = reinterpret_cast<const uint16_t*>(wsn + p.lay.records);
+    const int32_t tile_yz = (int32_t)fast_div(tile, p.by_tiles_x), tile_x = (int32_t)tile - tile_yz * p.tiles_x;
+    const int32_t tile_z = (DIM == 3) ? (int32_t)fast_div((uint32_t)tile_yz, p.by_tiles_y) : 0;
+    const int32_t tile_y = tile_yz - tile_z * p.tiles_y;
+    const int32_t x0 = tile_x * S::kX, y0 = tile_y * S::kY, z0 = tile_z * S::kZ;
+    const int32_t phase = (DIM == 3 && p.items_per_core > 1) ? phase_of(n, p) : 0;
+    // sums of the wavefronts before this one, and of all, from s_scan
+    auto waves_before = [&](uint32_t* all) {
+        const uint32_t incl = wave_scan(lane < kWaves ? s_scan[lane < kWaves ? lane : 0] : 0u);
+        *all = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWaves - 1);
+        return wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)incl, wave - 1) : 0u;
+    };
+
+    // the tile's segments (packed sums: segments that are not empty above 21 bits of points; both fit by launch plan)
+    uint32_t* s_before = s_seg;
+    uint32_t* s_where = s_seg + p.blocks + 1;
+    uint32_t segs = 0, total = 0;
+    for (int32_t b0 = 0; b0 < p.blocks; b0 += TH) {
+        const int32_t b = b0 + t;
+        const uint32_t w = (b < p.blocks) ? wsn[p.lay.segments + (size_t)b * p.tiles + tile] : 0u;
+        const uint32_t count = w >> 16, packed = count | (count > 0u ? 1u << 21 : 0u);
+        uint32_t incl = 0u;
+        if (b0 + wave * 64 < p.blocks) {
+            incl = wave_scan(packed);
+        }
+        if (lane == 63) {
+            s_scan[wave] = incl;
+        }
+        __syncthreads();
+        uint32_t all;
+        const uint32_t before = waves_before(&all) + incl - packed;
+        if (count > 0u) {
+            const uint32_t at = segs + (before >> 21);
+            s_before[at] = total + (before & 0x1FFFFFu);
+            s_where[at] = ((uint32_t)b << 14) | (w & 0xFFFFu);
+        }
+        segs += all >> 21;
+        total += all & 0x1FFFFFu;
+        __syncthreads();
+    }
+    if (t == 0) {
+        s_before[segs] = total;
+    }
+    if (t < GS) {
+        ElemIO<T>::store(&s_go[CAP * GS + t], 0.0f);
+    }
+    if (INTERP == 0) {
+        s_weight.clear_last(t);
+    }
+    for (int i = t; i < CAP + 2 * NK; i += TH) {
+        s_list[i] = 0u;
+    }
+    __syncthreads();
+
+    // rows of a plane to different wavefronts in turn: neighbours on which padding piles points up are then summed side by side
+    const int row = (DIM == 2) ? wave + (lane / S::kX) * kWaves : t / S::kX;
+    const int lx = t % S::kX, ly = row % S::kY, lz = row / S::kY;
+    const int32_t c_begin = (int32_t)cblock * chans_per_block;
+    const int32_t c_end = (c_begin + chans_per_block < p.C) ? c_begin + chans_per_block : p.C;
+    const T* go_n = gout + (int64_t)n * p.C * (int64_t)p.points;
+    const T* grid_n = grid + (int64_t)n * p.points * DIM;
+
+    int32_t pt[RPL];                // the lane's points of this run of segments
+    uint32_t key[NK];
+    uint32_t len = 0, number = 0;   // contributions; points in LDS
+    int most = 0;                   // keys of any lane of the wavefront
+    bool crowded = false;
+    uint32_t sorted = kNoKey;       // where a crowded element's contributions lie in s_sorted, or
+    uint32_t only = kNoKey;         // in s_list: those of a single run
+    // which corner of the element's cells a point is follows from the parity of its cell: 1 for the cell before
+    const uint32_t parity = (INTERP == 1) ? 0u
+                                          : (uint32_t)((lx & 1) | ((ly & 1) << 1) | ((DIM == 3) ? (lz & 1) << 2 : 0)) << kPosBits;
+    constexpr uint32_t kCorners = (INTERP == 1) ? 0u : ((1u << DIM) - 1u) << kPosBits;
+    const uint32_t corner = parity ^ kCorners;
+    // the first cell of a row of an element's cells
+    auto row_of = [&](int r) {
+        if (INTERP == 1) {
+            return (uint32_t)((lz * CY + ly) * CX + lx);
+        }
+        const int ys = r & 1, zs = r >> 1;
+        return (uint32_t)((((DIM == 3) ? (lz + 1 - zs) * CY : 0) + ly + 1 - ys) * CX + lx);
+    };
+    constexpr uint32_t kRowCells = (INTERP == 1) ? 1u : 2u;
+
+    auto lane_points = [&](int k) { return (uint32_t)(k * TH + wave * 64) < number; };  // any in this wavefront
+    auto load_go = [&](int32_t c0, int32_t nc, int k, T (&go)[GS]) {
+        const char* base = reinterpret_cast<const char*>(go_n + (int64_t)c0 * p.points);
+        const uint32_t off = (uint32_t)pt[k] * (uint32_t)sizeof(T);  // an item's grid points fit 32 bits many times over
+        auto load = [&](int j) {
+            return *reinterpret_cast<const T*>(base + (int64_t)j * p.points * (int64_t)sizeof(T) + off);
+        };
+        if (nc == CB) {
+#pragma unroll
+            for (int j = 0; j < CB; j++) {
+                go[j] = load(j);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < CB; j++) {
+                go[j] = load(j < nc ? j : 0);
+            }
+        }
+        if (GS > CB) {
+            ElemIO<T>::store(&go[GS - 1], 0.0f);
+        }
+    };
+    auto stage_go = [&](int k, const T (&go)[GS]) {
+        const uint32_t i = (uint32_t)(k * TH + t);
+        if (i < number) {
+            __builtin_memcpy(__builtin_assume_aligned(&s_go[i * GS], sizeof(T) * GS), go, sizeof(T) * GS);
+        }
+    };
+
+    // run r of the list: the points that corner r of this element comes from
+    auto runs_of_element = [&](uint32_t (&begin)[R], uint32_t (&end)[R]) {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint32_t cell = row_of(r >> 1) + ((INTERP == 1 || (r & 1)) ? 0u : 1u);
+            begin[r] = s_start[cell];
+            end[r] = s_start[cell + 1u];
+        }
+    };
+    // f(key) for the contributions of a lane's element in order: the least of its runs' next keys
+    auto merge_alone = [&](auto&& f) {
+        uint32_t at[R], end[R], head[R];
+        runs_of_element(at, end);
+        auto next = [&](int r) { return (at[r] < end[r]) ? s_list[at[r]] ^ corner : kNoKey; };
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            head[r] = next(r);
+        }
+        for (uint32_t i = 0; i < len; i++) {
+            uint32_t least = head[0];
+#pragma unroll
+            for (int r = 1; r < R; r++) {
+                least = head[r] < least ? head[r] : least;
+            }
+            f(i, least);
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                if (head[r] == least) {
+                    at[r]++;
+                    head[r] = next(r);
+                }
+            }
+        }
+    };
+    // the contributions of lane `owner`'s element by the whole wavefront: the least 64 of its runs' next 64 each are put(place
+    // among them, key), then done(how many)
+    auto merge_together = [&](int owner, int lane, auto&& put, auto&& done) {
+        uint32_t begin[R], left[R], rest = 0;
+        runs_of_element(begin, left);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            begin[r] = (uint32_t)__builtin_amdgcn_readlane((int)begin[r], owner);
+            left[r] = (uint32_t)__builtin_amdgcn_readlane((int)left[r], owner) - begin[r];
+            rest += left[r];
+        }
+        const uint32_t its_corner = (uint32_t)__builtin_amdgcn_readlane((int)corner, owner);
+        while (rest > 0u) {
+            const uint32_t batch = rest < 64u ? rest : 64u;
+            uint32_t head[R], window[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                window[r] = left[r] < 64u ? left[r] : 64u;
+                head[r] = ((uint32_t)lane < window[r]) ? s_list[begin[r] + lane] ^ its_corner : kNoKey;
+            }
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                uint32_t rank = (uint32_t)lane;
+#pragma unroll
+                for (int o = 0; o < R; o++) {
+                    if (o != r && window[o] > 0u && window[r] > 0u) {
+                        // keys of run o below this lane's
+                        uint32_t less = 0;
+#pragma unroll
+                        for (uint32_t d = 32; d > 0u; d >>= 1) {
+                            const uint32_t other = (uint32_t)__shfl((int)head[o], (int)(less + d - 1u));
+                            less += (other < head[r]) ? d : 0u;
+                        }
+                        // the last of 64
+                        less += ((uint32_t)__shfl((int)head[o], (int)less) < head[r]) ? 1u : 0u;
+                        rank += less;
+                    }
+                }
+                const bool take = (uint32_t)lane < window[r] && rank < batch;
+                if (take) {
+                    put(rank, head[r] & kLowBits);
+                }
+                const uint32_t taken = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(take));
+                begin[r] += taken;
+                left[r] -= taken;
+            }
+            rest -= batch;
+            done(batch);
+        }
+    };
+    // The contributions of crowded elements in order to s_sorted, once for all channels: a lane each, or where a single
+    // element has hundreds the wavefront together.
+    auto merge_crowded = [&]() {
+        sorted = kNoKey;
+        if (__builtin_amdgcn_ballot_w64(crowded) == 0) {
+            return;
+        }
+        bool fits = false;
+        if (crowded) {
+            uint32_t begin[R], end[R];
+            runs_of_element(begin, end);
+            only = kNoKey;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                only = (end[r] - begin[r] == len) ? begin[r] : only;
+            }
+            if (only == kNoKey) {
+                const uint32_t to = atomicAdd(&s_sorted_used, len);
+                fits = to + len <= kSorted;
+                sorted = fits ? to : kNoKey;
+            }
+        }
+        if (fits && len <= kSerialMost) {
+            merge_alone([&](uint32_t i, uint32_t k) { s_sorted[sorted + i] = (uint16_t)(k & kLowBits); });
+        }
+        int lane = t & 63;
+        asm volatile("" : "+v"(lane));  // what follows is rare: none of it is worked out ahead
+        uint64_t big = __builtin_amdgcn_ballot_w64(fits && len > kSerialMost);
+        while (big != 0) {
+            const int owner = __builtin_ctzll(big);
+            big &= big - 1u;
+            uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)sorted, owner);
+            merge_together(owner, lane, [&](uint32_t rank, uint32_t k) { s_sorted[to + rank] = (uint16_t)k; },
+                           [&](uint32_t batch) { to += batch; });
+        }
+        landed();
+    };
+
+    // the points of segments [from, to): cells, lists, and this element's keys in order
+    auto build = [&](uint32_t from, uint32_t to, int32_t c0, int32_t nc) {
+        const uint32_t base = s_before[from];
+        number = s_before[to] - base;
+        for (int i = t; i < kStarts / 4; i += TH) {
+            reinterpret_cast<uint4*>(s_start)[i] = make_uint4(0u, 0u, 0u, 0u);
+        }
+        if (t == 0) {
+            s_longs = s_crowded = s_sorted_used = 0u;
+        }
+        uint32_t own_key[RPL], rank[RPL], cell[RPL];
+        T raw[RPL][DIM], go[RPL][GS];
+        // stage by stage for all of the lane's points, so that their loads are on their way together
+        uint32_t steps = 1;
+        while (steps < to - from) {
+            steps <<= 1;
+        }
+        uint32_t block[RPL];
+        uint16_t record[RPL];
+#pragma unroll
+        for (int k = 0; k < RPL; k++) {
+            if (lane_points(k)) {
+                uint32_t i = (uint32_t)(k * TH + t);
+                i = base + (i < number ? i : 0u);
+                uint32_t seg = from;  // the last segment that does not start behind point i
+                for (uint32_t d = steps >> 1; d > 0u; d >>= 1) {
+                    const uint32_t mid = seg + d < to ? seg + d : to;
+                    seg = s_before[mid] <= i ? mid : seg;
+                }
+                const uint32_t where = s_where[seg];
+                block[k] = where >> 14;
+                record[k] = *reinterpret_cast<const uint16_t*>(
+                    reinterpret_cast<const char*>(records) +
+                    (block[k] * (p.lay.block_words * 4u) + ((where & 0x3FFFu) + (i - s_before[seg])) * 2u));
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < RPL; k++) {
+            if (lane_points(k)) {
+                const uint32_t q = block[k] * kBinPoints + record[k];
+                pt[k] = (int32_t)q - phase;
+                own_key[k] = (q >> 8) << (kPosBits + kTapBits);
+                __builtin_memcpy(raw[k], reinterpret_cast<const char*>(grid_n) + (uint32_t)pt[k] * (uint32_t)sizeof(raw[k]), sizeof(raw[k]));
+                load_go(c0, nc, k, go[k]);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < RPL; k++) {
+            if (lane_points(k)) {
+                const uint32_t i = (uint32_t)(k * TH + t);
+                const Coords<T, DIM> at = coords_of<T, DIM, INTERP>(raw[k], p);
+                int32_t cx, cy, cz;
+                low_corner<T, DIM, INTERP>(at, p, &cx, &cy, &cz);
+                cx += PADC - x0;
+                cy += PADC - y0;
+                cz += PADC - z0;
+                cell[k] = (uint32_t)((((DIM == 3) ? cz * CY : 0) + cy) * CX + cx);
+                cell[k] = cell[k] < (uint32_t)CELLS ? cell[k] : 0u;  // never: the point is in this tile's segment
+                const uint32_t odd = (uint32_t)((cx & 1) | ((cy & 1) << 1) | ((DIM == 3) ? (cz & 1) << 2 : 0)) << kPosBits;
+                own_key[k] |= (INTERP == 1 ? 0u : odd) | i;
+                rank[k] = 0u;
+                if (i < number) {
+                    rank[k] = atomicAdd(&s_start[cell[k]], 1u);
+                    s_rare.points.key[i] = own_key[k];
+                    s_rare.points.cell[i] = (uint16_t)cell[k];
+                    if constexpr (INTERP == 0) {
+                        s_weight.put(i, at);
+                    }
+                }
+                stage_go(k, go[k]);
+            }
+        }
+        __syncthreads();
+        // the starts: four cells a lane
+        uint4 four = make_uint4(0u, 0u, 0u, 0u);
+        uint32_t incl = 0, sum = 0;
+        if (t < kStarts / 4) {
+            four = reinterpret_cast<uint4*>(s_start)[t];
+        }
+        if (wave * 64 < kStarts / 4) {
+            sum = four.x + four.y + four.z + four.w;
+            incl = wave_scan(sum);
+        }
+        if (lane == 63) {
+            s_scan[wave] = incl;
+        }
+        __syncthreads();
+        if (wave * 64 < kStarts / 4) {
+            uint32_t all;
+            const uint32_t before = waves_before(&all) + incl - sum;
+            if (t < kStarts / 4) {
+                reinterpret_cast<uint4*>(s_start)[t] =
+                    make_uint4(before, before + four.x, before + four.x + four.y, before + four.x + four.y + four.z);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < RPL; k++) {
+            if ((uint32_t)(k * TH + t) < number) {
+                s_list[s_start[cell[k]] + rank[k]] = own_key[k];
+            }
+        }
+        uint32_t from_row[RR], upto[RR];  // where the row's keys lie in the list, less those of the rows before; contributions
+        len = 0u;
+#pragma unroll
+        for (int r = 0; r < RR; r++) {
+            const uint32_t row = row_of(r), begin = s_start[row];
+            from_row[r] = begin - len;
+            len += s_start[row + kRowCells] - begin;
+            upto[r] = len;
+        }
+        len = (x0 + lx < p.W && y0 + ly < p.H && z0 + lz < p.D) ? len : 0u;
+        crowded = len > (uint32_t)NK;
+        if (crowded) {
+            s_crowded = 1u;
+        }
+        __syncthreads();
+        if (s_crowded != 0u) {
+            // merging wants the points of a cell in order
+            uint32_t place[RPL];
+#pragma unroll
+            for (int k = 0; k < RPL; k++) {
+                const uint32_t i = (uint32_t)(k * TH + t);
+                place[k] = 0xFFFFu;
+                if (i < number) {
+                    const uint32_t begin = s_start[cell[k]], end = s_start[cell[k] + 1u];
+                    if (end - begin <= kCountedRun) {
+                        uint32_t less = 0;
+                        for (uint32_t j = begin; j < end; j++) {
+                            less += (s_list[j] < own_key[k]) ? 1u : 0u;  // of one cell: in the order of their numbers
+                        }
+                        place[k] = begin + less;
+                    } else if (rank[k] == 0u) {
+                        s_long[atomicAdd(&s_longs, 1u)] = (uint16_t)cell[k];
+                    }
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < RPL; k++) {
+                if (place[k] != 0xFFFFu) {
+                    s_list[place[k]] = own_key[k];
+                }
+            }
+            for (uint32_t r = (uint32_t)wave; r < s_longs; r += kWaves) {
+                const uint32_t c = s_long[r];
+                uint32_t to_list = s_start[c];
+                for (uint32_t i0 = 0; i0 < number; i0 += 64u) {
+                    const uint32_t i = i0 + (uint32_t)lane;
+                    const bool member = i < number && s_rare.points.cell[i < number ? i : 0u] == c;
+                    const uint64_t mask = __builtin_amdgcn_ballot_w64(member);
+                    if (member) {
+                        s_list[to_list + bits_below(mask)] = s_rare.points.key[i];
+                    }
+                    to_list += (uint32_t)__builtin_popcountll(mask);
+                }
+            }
+            __syncthreads();
+            merge_crowded();
+        }
+        // Keys of as many contributions as any lane of the wavefront has, rounded up to kStep: beyond its own a lane reads
+        // some key of the list and takes that of the zeros instead.
+        const uint32_t keys = crowded ? 0u : len;
+        most = 0;
+#pragma unroll
+        for (int i = 0; i < NK; i += kStep) {
+            most = (__builtin_amdgcn_ballot_w64(keys > (uint32_t)i) != 0) ? i + kStep : most;
+        }
+#pragma unroll
+        for (int r = 0; r < RR; r++) {
+            from_row[r] = crowded ? 0u : from_row[r];
+        }
+#pragma unroll
+        for (int g = 0; g < NK; g += kStep) {
+            if (g < most) {
+#pragma unroll
+                for (int i = g; i < g + kStep; i++) {
+                    uint32_t row = from_row[0];
+#pragma unroll
+                    for (int r = 1; r < RR; r++) {
+                        row = ((uint32_t)i >= upto[r - 1]) ? from_row[r] : row;
+                    }
+                    const uint32_t k = s_list[row + (uint32_t)i] ^ corner;
+                    key[i] = ((uint32_t)i < keys) ? k : (kNoKey << kPosBits) | (uint32_t)CAP;
+                }
+            }
+        }
+        sort_most<NK, kStep>(key, most);
+    };
+
+    Sums<T, INTERP, CB> sums;
+    auto add = [&](uint32_t k) {
+        const uint32_t i = k & ((1u << kPosBits) - 1u);
+        T go[GS];
+        __builtin_memcpy(go, __builtin_assume_aligned(&s_go[i * GS], sizeof(T) * GS), sizeof(T) * GS);
+        float w = 1.0f;
+        if constexpr (INTERP == 0) {
+            w = s_weight.get(i, (k >> kPosBits) & ((1u << DIM) - 1u));
+        }
+        // a contribution that is not there is zero times zero, which changes no sum that started at +0
+        sums.add(go, w);
+    };
+    auto fold = [&]() {
+#pragma unroll
+        for (int g = 0; g < NK; g += kStep) {
+            if (g < most) {
+#pragma unroll
+                for (int i = g; i < g + kStep; i++) {
+                    add(key[i]);
+                }
+            }
+        }
+        const uint64_t rare = __builtin_amdgcn_ballot_w64(crowded);
+        if (rare == 0) {
+            return;
+        }
+        int lane = t & 63;
+        asm volatile("" : "+v"(lane));  // what follows is rare: none of it is worked out ahead
+        const bool together = crowded && (len > kSerialMost || ((sorted & only) != kNoKey && __builtin_popcountll(rare) <= kFewCrowded));
+        if (crowded && !together) {
+            if (only != kNoKey) {
+                for (uint32_t i = 0; i < len; i++) {
+                    add(s_list[only + i] ^ corner);
+                }
+            } else if (sorted != kNoKey) {
+                for (uint32_t i = 0; i < len; i++) {
+                    add(s_sorted[sorted + i]);
+                }
+            } else {
+                merge_alone([&](uint32_t, uint32_t k) { add(k); });
+            }
+        }
+        // The wavefront together, an element after the other: 64 contributions at a time are computed side by side, and a
+        // lane per channel adds them one by one.
+        ByWave& own = s_rare.waves[wave];
+        uint64_t big = __builtin_amdgcn_ballot_w64(together);
+        while (big != 0) {
+            const int owner = __builtin_ctzll(big);
+            big &= big - 1u;
+            float sum = 0.0f;  // of channel `lane`
+#pragma unroll
+            for (int j = 0; j < CB; j++) {
+                const float s = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sums.get(j)), owner));
+                sum = (lane == j) ? s : sum;
+            }
+            auto add_batch = [&](uint32_t k, uint32_t batch) {  // k: lane's key, of the first where it has none
+                const bool have = (uint32_t)lane < batch;
+                const uint32_t i = k & ((1u << kPosBits) - 1u);
+                float w = 1.0f;
+                if constexpr (INTERP == 0) {
+                    w = s_weight.get(i, (k >> kPosBits) & ((1u << DIM) - 1u));
+                }
+                bool some = false;
+#pragma unroll
+                for (int j = 0; j < CB; j++) {
+                    const float v = have ? value_of<T, INTERP>(ElemIO<T>::load(&s_go[i * GS + j]), w) : 0.0f;
+                    own.value[j][lane] = v;
+                    some = some || v != 0.0f;
+                }
+                landed();
+                // zeros change no sum: padding piles points up with weight 0 on the elements next to an edge
+                if (__builtin_amdgcn_ballot_w64(some) != 0 && lane < CB) {
+                    for (uint32_t s = 0; s < batch; s += 4u) {
+                        const float4 v = *reinterpret_cast<const float4*>(&own.value[lane][s]);
+                        sum = rt<T>(sum + v.x);
+                        sum = rt<T>(sum + v.y);
+                        sum = rt<T>(sum + v.z);
+                        sum = rt<T>(sum + v.w);
+                    }
+                }
+                landed();
+            };
+            const uint32_t from = (uint32_t)__builtin_amdgcn_readlane((int)sorted, owner);
+            const uint32_t run = (uint32_t)__builtin_amdgcn_readlane((int)only, owner);
+            const uint32_t its_corner = (uint32_t)__builtin_amdgcn_readlane((int)corner, owner);
+            const uint32_t its_len = (uint32_t)__builtin_amdgcn_readlane((int)len, owner);
+            if ((from & run) != kNoKey) {
+                for (uint32_t done = 0; done < its_len; done += 64u) {
+                    const uint32_t batch = its_len - done < 64u ? its_len - done : 64u;
+                    const uint32_t i = done + ((uint32_t)lane < batch ? (uint32_t)lane : 0u);
+                    add_batch(run != kNoKey ? s_list[run + i] ^ its_corner : (uint32_t)s_sorted[from + i], batch);
+                }
+            } else {
+                merge_together(owner, lane, [&](uint32_t rank, uint32_t k) { own.order[rank] = (uint16_t)k; },
+                               [&](uint32_t batch) {
+                                   landed();
+                                   add_batch(own.order[(uint32_t)lane < batch ? lane : 0], batch);
+                               });
+            }
+#pragma unroll
+            for (int j = 0; j < CB; j++) {
+                const float s = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, sum), j));
+                if (lane == owner) {
+                    sums.set(j, s);
+                }
+            }
+        }
+    };
+
+    // Runs of segments that fit LDS, in order; the channels in turn for each.  The sums so far are values of the element type
+    // and wait in the gradient itself, where the lane that stored them reads them again.
+    const bool inside = x0 + lx < p.W && y0 + ly < p.H && z0 + lz < p.D;
+    const uint32_t e = (uint32_t)(((z0 + lz) * p.H + y0 + ly) * p.W + x0 + lx) * (uint32_t)sizeof(T);
+    uint32_t from = 0;
+    do {
+        uint32_t to = segs;
+        if (total - s_before[from] > (uint32_t)CAP) {
+            uint32_t lo = from + 1u;  // the last that fits: a segment does
+            while (to - lo > 1u) {
+                const uint32_t mid = (lo + to) >> 1;
+                if (s_before[mid] - s_before[from] <= (uint32_t)CAP) {
+                    lo = mid;
+                } else {
+                    to = mid;
+                }
+            }
+            to = lo;
+        }
+        for (int32_t c0 = c_begin; c0 < c_end; c0 += CB) {
+            const int32_t nc = (c_end - c0 < CB) ? c_end - c0 : CB;
+            char* out = reinterpret_cast<char*>(dx + ((int64_t)n * p.C + c0) * (int64_t)p.elements);
+            auto at = [&](int j) { return reinterpret_cast<T*>(out + (int64_t)j * p.elements * (int64_t)sizeof(T) + e); };
+            sums.clear();
+            if (to > from) {
+                if (c0 == c_begin) {
+                    build(from, to, c0, nc);
+                } else {
+                    T go[RPL][GS];
+#pragma unroll
+                    for (int k = 0; k < RPL; k++) {
+                        if (lane_points(k)) {
+                            load_go(c0, nc, k, go[k]);
+                        }
+                    }
+#pragma unroll
+                    for (int k = 0; k < RPL; k++) {
+                        if (lane_points(k)) {
+                            stage_go(k, go[k]);
+                        }
+                    }
+                    __syncthreads();
+                }
+                if (from > 0u && inside) {
+#pragma unroll
+                    for (int j = 0; j < CB; j++) {
+                        if (j < nc) {
+                            sums.set(j, ElemIO<T>::load(at(j)));
+                        }
+                    }
+                }
+                fold();
+            }
+            if (inside) {
+#pragma unroll
+                for (int j = 0; j < CB; j++) {
+                    if (j < nc) {
+                        ElemIO<T>::store(at(j), sums.get(j));
+                    }
+                }
+            }
+            if (to < segs || c0 + CB < c_end) {
+                __syncthreads();  // LDS is written again
+            }
+        }
+        from = to;
+    } while (from < segs);
+}
+
+inline uint32_t xcd_blocks(int64_t pieces) { return (uint32_t)((pieces + 7) / 8 * 8); }
+
+template <typename T, int DIM, int INTERP, int CB>
+hipError_t launch_tiles(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t stream)
+{
+    typedef GradTile<DIM> S;
+    static std::atomic<uint32_t> bin_allowed{0};
+    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(gs_tiles_bin_kernel<T, DIM, INTERP>),
+                                     (int)kTilesMost * (kBinThreads / 64) * 12, bin_allowed);
+    if (e != hipSuccess) {
+        return e;
+    }
+    static std::atomic<uint32_t> gather_allowed{0};
+    e = allow_dynamic_lds(reinterpret_cast<const void*>(gs_tiles_gather_kernel<T, DIM, INTERP, CB>),
+                          (int)(kTileBlocksMost + 1) * 8, gather_allowed);
+    if (e != hipSuccess) {
+        return e;
+    }
+    const uint32_t bins = (uint32_t)a.N * (uint32_t)pl.p.blocks;
+    hipLaunchKernelGGL((gs_tiles_bin_kernel<T, DIM, INTERP>), dim3(xcd_blocks(bins)), dim3(kBinThreads), (size_t)pl.bin_lds,
+                       stream, (const T*)a.grid, (uint32_t*)a.scratch, pl.p, bins);
+    e = hipGetLastError();
+    if (e != hipSuccess) {
+        return e;
+    }
+    const uint32_t pieces = (uint32_t)a.N * pl.p.by_item.div;
+    hipLaunchKernelGGL((gs_tiles_gather_kernel<T, DIM, INTERP, CB>), dim3(xcd_blocks(pieces)), dim3(S::kThreads),
+                       (size_t)pl.segment_lds, stream, (const T*)a.gout, (const T*)a.grid, (T*)a.dx,
+                       (const uint32_t*)a.scratch, pl.p, pieces, pl.chans_per_block);
+    return hipGetLastError();
+}
+
+template <typename T, int DIM, int INTERP>
+hipError_t run_channels(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t stream)
+{
+    switch (pl.cb) {
+        case 1: return launch_tiles<T, DIM, INTERP, 1>(a, pl, stream);
+        case 2: return launch_tiles<T, DIM, INTERP, 2>(a, pl, stream);
+        case 3: return launch_tiles<T, DIM, INTERP, 3>(a, pl, stream);
+        case 4: return launch_tiles<T, DIM, INTERP, 4>(a, pl, stream);
+        default: break;
+    }
+    if constexpr (sizeof(T) == 2) {
+        return launch_tiles<T, DIM, INTERP, 8>(a, pl, stream);
+    }
+    return hipErrorInvalidValue;
+}
+
+template <typename T>
+hipError_t run_typed(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t stream)
+{
+    switch (a.dim * 2 + a.interp) {
+        case 2 * 2 + 0: return run_channels<T, 2, 0>(a, pl, stream);
+        case 2 * 2 + 1: return run_channels<T, 2, 1>(a, pl, stream);
+        case 3 * 2 + 0: return run_channels<T, 3, 0>(a, pl, stream);
+        case 3 * 2 + 1: return run_channels<T, 3, 1>(a, pl, stream);
+        default: return hipErrorInvalidValue;
+    }
+}
+
+}  // namespace
+
+int64_t grad_tiles_words(const GradGatherArgs& a)
+{
+    const TilesPlan pl = tiles_plan(a);
+    return pl.ok ? (int64_t)pl.p.lay.item_words * pl.group : 0;
+}
+
+hipError_t run_grad_tiles(const GradGatherArgs& a, hipStream_t stream)
+{
+    TilesPlan pl = tiles_plan(a);
+    if (!pl.ok || a.dx == nullptr || a.gout == nullptr || a.grid == nullptr || a.scratch == nullptr) {
+        return hipErrorInvalidValue;
+    }
+    // the items are independent: a group of them after the other, each in all of the scratch
+    const int64_t esz = elem_size(a.elem);
+    for (int64_t first = 0; first < a.N; first += pl.group) {
+        GradGatherArgs g = a;
+        g.N = (a.N - first < pl.group) ? a.N - first : pl.group;
+        g.gout = (const char*)a.gout + first * a.C * a.points * esz;
+        g.grid = (const char*)a.grid + first * a.points * a.dim * esz;
+        g.dx = (char*)a.dx + first * a.C * (a.D * a.H * a.W) * esz;
+        pl.p.N = (int32_t)g.N;
+        pl.p.first_item = (int32_t)first;
+        hipError_t e = hipErrorInvalidValue;
+        switch (a.elem) {
+            case Elem::F32: e = run_typed<float>(g, pl, stream); break;
+            case Elem::F16: e = run_typed<_Float16>(g, pl, stream); break;
+            case Elem::BF16: e = run_typed<__bf16>(g, pl, stream); break;
+        }
+        if (e != hipSuccess) {
+            return e;
+        }
+    }
+    return hipSuccess;
+}
+
+}  // namespace opscv

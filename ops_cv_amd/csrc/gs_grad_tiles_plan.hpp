@@ -1,0 +1,174 @@
+// Plan of the samplers' input gradient by tiles (gs_grad_tiles.hip): host arithmetic only.
+#pragma once
+
+#include <cstdint>
+
+#include "fast_div.hpp"
+#include "gs_grad_gather_plan.hpp"
+
+namespace opscv {
+
+constexpr int kBinThreads = 256;
+constexpr int kBinPoints = 1024;  // grid points of a block: a segment holds the points of a block that fall on a tile
+
+// A tile of the plane or volume, a lane of a workgroup per element, and the points that the workgroup has in LDS at a time:
+// a whole segment at least.
+template <int DIM>
+struct GradTile;
+template <>
+struct GradTile<2> {
+    static constexpr int kX = 32, kY = 16, kZ = 1;
+    static constexpr int kThreads = kX * kY * kZ;
+    static constexpr int kRecords = 1024;
+};
+template <>
+struct GradTile<3> {
+    static constexpr int kX = 16, kY = 8, kZ = 4;
+    static constexpr int kThreads = kX * kY * kZ;
+    static constexpr int kRecords = 1280;
+};
+
+struct TilesLayout {   // offsets in 32-bit words within an item's scratch
+    uint32_t segments; // [block][tile]: first record in the block's records, and how many << 16
+    uint32_t records;  // [block]: 16-bit numbers of points within the block, segment after segment
+    uint32_t block_words;  // of records
+    uint32_t item_words;
+};
+
+struct TilesParams {
+    int32_t C, D, H, W, points;
+    int32_t pad, align;
+    int32_t items_per_core;
+    int32_t elements;
+    int32_t N;  // items of this launch, and the batch's number of the first one
+    int32_t first_item;
+    int32_t tiles_x, tiles_y, tiles;
+    int32_t blocks;  // of points
+    FastDiv by_tiles_x, by_tiles_y, by_tiles, by_blocks, by_item;  // the last: workgroups of the gather kernel per item
+    TilesLayout lay;
+};
+
+struct TilesPlan {
+    bool ok = false;
+    TilesParams p{};
+    int64_t group = 0;  // items run at a time
+    int64_t cblocks = 0;
+    int32_t chans_per_block = 0;
+    int cb = 1;         // channels of a point in LDS together
+    int32_t bin_lds = 0, segment_lds = 0;  // bytes
+};
+
+constexpr int64_t kTilesFewGroups = 256;     // workgroups: one per CU
+constexpr int64_t kTilesMost = 2048;         // per item: counts and masks of every tile in LDS (96 KiB)
+constexpr int64_t kTileBlocksMost = 2047;    // per item: segments of a tile in LDS (16 KiB), counts of 11 and 21 bits
+
+template <int DIM>
+inline TilesPlan tiles_plan_of(const GradGatherArgs& a)
+{
+    typedef GradTile<DIM> S;
+    TilesPlan pl;
+    if (a.interp > 1 || a.N < 1 || a.N > 65535 || a.W > INT32_MAX / 2 || a.H > INT32_MAX / 2 || a.D > INT32_MAX / 2) {
+        return pl;
+    }
+    const int64_t esz = elem_size(a.elem);
+    const int64_t tx = (a.W + S::kX - 1) / S::kX, ty = (a.H + S::kY - 1) / S::kY, tz = (a.D + S::kZ - 1) / S::kZ;
+    if (tx > kTilesMost || ty > kTilesMost || tz > kTilesMost || tx * ty * tz > kTilesMost) {
+        return pl;
+    }
+    const int64_t per_core = a.items_per_core > 0 ? a.items_per_core : 1;
+    // the first block of an item starts at the boundary of the chunk that its first point lies in
+    const int64_t blocks = (a.points + (per_core > 1 ? kBinPoints - 1 + 255 : kBinPoints - 1)) / kBinPoints;
+    if (blocks > kTileBlocksMost) {
+        return pl;
+    }
+    TilesParams& p = pl.p;
+    p.C = (int32_t)a.C;
+    p.D = (int32_t)a.D;
+    p.H = (int32_t)a.H;
+    p.W = (int32_t)a.W;
+    p.points = (int32_t)a.points;
+    p.pad = a.pad;
+    p.align = a.align;
+    p.items_per_core = (int32_t)per_core;
+    p.elements = (int32_t)(a.D * a.H * a.W);
+    p.tiles_x = (int32_t)tx;
+    p.tiles_y = (int32_t)ty;
+    p.tiles = (int32_t)(tx * ty * tz);
+    p.blocks = (int32_t)blocks;
+    // a point's corners lie in one tile or, with linear interpolation, in up to two along every axis
+    p.lay.block_words = (uint32_t)(kBinPoints / 2) << (a.interp == 0 ? DIM : 0);
+    p.lay.segments = 0;
+    p.lay.records = align4((uint64_t)(blocks * p.tiles));
+    p.lay.item_words = p.lay.records + (uint32_t)blocks * p.lay.block_words;
+    const int64_t fit = kGatherGroupScratch / ((int64_t)p.lay.item_words * 4);
+    const int64_t group = fit < 1 ? 1 : (fit < a.N ? fit : a.N);
+    pl.group = (a.N + (a.N + group - 1) / group - 1) / ((a.N + group - 1) / group);  // as many items in every group
+    p.N = (int32_t)pl.group;
+    p.first_item = 0;
+    pl.cb = (esz == 2 && a.C > 4 && DIM == 2) ? 8 : ((a.C > 3) ? 4 : (int)a.C);
+    // fewer channels together where the tiles do not fill the chip
+    while (pl.cb > 1 && pl.group * p.tiles * ((a.C + pl.cb - 1) / pl.cb) < kTilesFewGroups) {
+        pl.cb = (pl.cb == 3) ? 2 : pl.cb / 2;
+    }
+    // channel blocks where the tiles alone do not fill the chip (four workgroups per CU): each makes the lists again
+    const int64_t base = pl.group * p.tiles;
+    const int64_t max_cblocks = (a.C + pl.cb - 1) / pl.cb;
+    int64_t cblocks = (1024 + base - 1) / base;
+    cblocks = cblocks > max_cblocks ? max_cblocks : cblocks;
+    int64_t cpb = (a.C + cblocks - 1) / cblocks;
+    cpb = (cpb + pl.cb - 1) / pl.cb * pl.cb;
+    pl.cblocks = (a.C + cpb - 1) / cpb;
+    pl.chans_per_block = (int32_t)cpb;
+    p.by_tiles_x = make_fast_div((uint32_t)p.tiles_x);
+    p.by_tiles_y = make_fast_div((uint32_t)p.tiles_y);
+    p.by_tiles = make_fast_div((uint32_t)p.tiles);
+    p.by_blocks = make_fast_div((uint32_t)p.blocks);
+    p.by_item = make_fast_div((uint32_t)(p.tiles * pl.cblocks));
+    pl.bin_lds = p.tiles * (kBinThreads / 64) * 12;
+    pl.segment_lds = (p.blocks + 1) * 8;
+    pl.ok = fits_launch(base * pl.cblocks + 8, S::kThreads) && fits_launch(pl.group * blocks + 8, kBinThreads);
+    return pl;
+}
+
+// Whether the tiles are the faster way to sort (elsewhere the lists of gs_grad_gather_plan.hpp).  Input gradient alone, lists /
+// tiles in microseconds.
+//
+// As a rule they are: fp32 8x3x479x637 zeros 178 / 86, fp16 17x3x271x355 101 / 54, fp32 14x3x312x301 -> 388x374 nearest 245 / 96,
+// fp16 1x14x236x198 -> 229x192 32 / 20, volumes bf16 13x5x27x47x57 108 / 86, fp32 10x2x14x26x17 nearest 24 / 15.
+//
+// Not in dense grids, where half of the elements have more contributions than keys and a tile takes several rounds: volumes
+// from 1.25 points a voxel on (1x12x9x81x64 -> 13x117x93 130 / 237, 2x5x19x59x56 -> 27x85x80 169 / 211, 6x6x56x17x60 ->
+// 65x19x70 134 / 164), planes from two an element on with many channels (21x60x40x40 -> 77x77 86 / 156; 10x2x267x440 ->
+// 448x738 314 / 111) or border padding (14x4x33x56 -> 62x106 60 / 93), and bf16 coordinates beyond 64, whose eight bits gather
+// points on whole and half pixels, from one on (2x5x96x192 -> 162x324 31 / 40, 12x5x100x129 -> 163x210 135 / 147; thinner ones
+// 6x12x136x184 -> 115x156 47 / 34).
+// Not where a single tile outlasts the launch: a workgroup adds the points that border padding piles up on a corner (a few in
+// a hundred of an item) a thousand at a time, in lists a wavefront per element does, and with few items and channels nothing
+// else is left to do meanwhile (1x3x480x640 73 / 110, 2x2x200x300 51 / 101; 8x3x479x637 455 / 330, 15x3x200x280 -> 221x309 209 /
+// 157).
+// Nor for many channels of volumes (12x31x18x62x20 142 / 159, 3x26x27x18x31 42 / 46; nearest 23x10x28x67x49 114 / 130,
+// 5x28x9x71x45 35 / 39; 7x19x30x20x91 175 / 151, nearest 9x6x52x46x37 67 / 55).
+inline bool tiles_are_faster(const GradGatherArgs& a)
+{
+    const int64_t elements = a.D * a.H * a.W;
+    if (a.dim == 3) {
+        return a.interp == 1 ? a.C <= 8 : (a.C <= 24 && 4 * a.points <= 5 * elements);
+    }
+    if (a.interp == 0 && a.points > 2 * elements && (a.C > 8 || a.pad == 1)) {
+        return false;
+    }
+    if (a.interp == 0 && a.elem == Elem::BF16 && (a.H > 64 || a.W > 64) && a.points >= elements) {
+        return false;
+    }
+    return a.pad != 1 || a.N * (a.C + 4) >= (a.interp == 1 ? 24 : 48);
+}
+
+inline TilesPlan tiles_plan(const GradGatherArgs& a)
+{
+    if (!tiles_are_faster(a)) {
+        return TilesPlan();
+    }
+    return a.dim == 3 ? tiles_plan_of<3>(a) : tiles_plan_of<2>(a);
+}
+
+}  // namespace opscv

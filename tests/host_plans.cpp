@@ -1,6 +1,7 @@
 // The launch plans of the kernels, which are plain host arithmetic, for the tests (host_plans.py).
 #include "gs2d_direct_plan.hpp"
 #include "gs_grad_gather_plan.hpp"
+#include "gs_grad_tiles_plan.hpp"
 #include "resize_flat_plan.hpp"
 #include "resize_grad_plan.hpp"
 #include "resize_nhwc_plan.hpp"
@@ -110,6 +111,32 @@ int gather_groups(int elem, int64_t interp, int64_t N, int64_t C, int64_t D, int
     const GatherPlan p = gather_plan(a);
     out[0] = p.group;
     out[1] = p.p.lay.item_words;
+    return p.ok ? 1 : 0;
+}
+
+// input gradient by tiles: items run at a time, 32-bit words of an item, tiles, blocks of points, channel blocks; 0 where the
+// lists of gather_groups take it
+int gradient_tiles(int elem, int64_t interp, int64_t pad, int64_t N, int64_t C, int64_t D, int64_t H, int64_t W, int64_t points,
+                   int64_t per_core, int64_t* out)
+{
+    GradGatherArgs a;
+    a.elem = (Elem)elem;
+    a.dim = D > 0 ? 3 : 2;
+    a.interp = (int)interp;
+    a.pad = (int)pad;
+    a.N = N;
+    a.C = C;
+    a.D = D > 0 ? D : 1;
+    a.H = H;
+    a.W = W;
+    a.points = points;
+    a.items_per_core = per_core;
+    const TilesPlan p = tiles_plan(a);
+    out[0] = p.group;
+    out[1] = p.p.lay.item_words;
+    out[2] = p.p.tiles;
+    out[3] = p.p.blocks;
+    out[4] = p.cblocks;
     return p.ok ? 1 : 0;
 }
 

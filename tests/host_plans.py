@@ -62,3 +62,10 @@ def gather_groups(dtype, interp, shape, points):
     cannot run."""
     shape = shape if len(shape) == 5 else shape[:2] + (0,) + shape[2:]
     return _call("gather_groups", 2, dtype, interp, *shape, points)
+
+
+def gradient_tiles(dtype, interp, pad, shape, points, per_core=1):
+    """(items run at a time, 32-bit words of an item, tiles, blocks of points, channel blocks) of the sorting input gradient
+    by tiles, None where the lists of gather_groups take it."""
+    shape = shape if len(shape) == 5 else shape[:2] + (0,) + shape[2:]
+    return _call("gradient_tiles", 5, dtype, interp, pad, *shape, points, per_core)

@@ -1,0 +1,103 @@
+"""Input gradients of the samplers by tiles (gs_grad_tiles.hip), bit for bit against the oracle."""
+import numpy as np
+import pytest
+
+import host_plans
+import inputs as I
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid, rng, variant=None):
+    import torch
+    x = I.cast_np(rng.standard_normal(xs).astype(np.float32), dtype)
+    g = I.cast_np(grid.astype(np.float32), dtype)
+    go = I.cast_np(rng.standard_normal(xs[:2] + out).astype(np.float32), dtype)
+    if len(xs) == 4:
+        ref, _ = oracle.grid_sampler2d_backward(go, x, g, interp, pad, False, dtype=I.oracle_code(dtype))
+        got, _ = aclnn.grid_sampler2d_backward(*(I.to_torch(v, dtype, device) for v in (go, x, g)), interp, pad, False,
+                                               (True, False))
+    else:
+        ref, _ = oracle.grid_sampler3d_backward(go, x, g, interp, pad, False, dtype=I.oracle_code(dtype))
+        with aclnn.option("gs3d_grad_variant", 3):
+            got, _ = aclnn.grid_sampler3d_backward(*(I.to_torch(v, dtype, device) for v in (go, x, g)), interp, pad, False,
+                                                   (True, False))
+    torch.cuda.synchronize()
+    a, b = (np.ascontiguousarray(v).view(np.uint8) for v in (I.from_torch(got, dtype), ref))
+    assert np.array_equal(a, b), (xs, out)
+
+
+def _spots(rng, n, count, dim, spread):
+    """points on a few spots and scattered ones between them: cells of hundreds of points and elements of thousands"""
+    g = rng.uniform(-1.1, 1.1, (n, count, dim))
+    at = rng.uniform(-0.9, 0.9, (n, 5, dim))
+    for i in range(n):
+        some = rng.random(count) < spread
+        g[i, some] = at[i, rng.integers(0, 5, int(some.sum()))]
+    return g
+
+
+# tiles of 32 x 16: one, parts of one, edges on and beside their borders; channels together and in blocks (1 to 4, 8 of a
+# 16-bit type, several blocks); about one point an element, and a round of points more than LDS holds; the third number:
+# points on five spots, so that lanes merge alone (up to 192), the wavefront together, and runs stay single
+PLANES = [((1, 1, 16, 32), (40, 41), 0.0), ((2, 3, 49, 65), (47, 61), 0.0), ((3, 2, 33, 95), (50, 61), 0.0),
+          ((4, 4, 64, 96), (66, 90), 0.0), ((9, 5, 17, 33), (60, 33), 0.0), ((6, 9, 48, 31), (50, 33), 0.0),
+          ((6, 21, 50, 64), (52, 66), 0.0), ((6, 7, 20, 40), (40, 39), 0.9), ((16, 2, 18, 34), (65, 60), 0.5)]
+
+# nearest samples are sorted from 25 chunks of points on
+NEAREST = [((1, 1, 80, 96), (90, 100), 0.0), ((8, 3, 97, 130), (70, 99), 0.0), ((9, 9, 65, 95), (81, 83), 0.0),
+           ((9, 5, 90, 70), (80, 81), 0.5)]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("pad", [0, 1, 2])
+@pytest.mark.parametrize("interp,xs,out,spots", [(0,) + c for c in PLANES] + [(1,) + c for c in NEAREST])
+def test_planes(oracle, device, aclnn, dtype, pad, interp, xs, out, spots):
+    rng = np.random.default_rng(4400 + 10 * interp + pad)
+    points = out[0] * out[1]
+    if spots > 0.0:
+        grid = _spots(rng, xs[0], points, 2, spots).reshape((xs[0],) + out + (2,))
+    else:
+        grid = I.affine_grid(rng, xs[0], *out)
+    lists = interp == 0 and xs[1] >= 8 and points % 8 == 0 and points * (4 if dtype == "fp32" else 2) <= 32768
+    if pad == 0 and not lists and spots == 0.0:
+        assert host_plans.sorting_takes_planes(dtype, interp, xs, points) is not None
+        assert host_plans.gradient_tiles(dtype, interp, pad, xs, points) is not None
+    _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid, rng)
+
+
+# tiles of 16 x 8 x 4; the last two: more items than the reference device has cores, so that the chunks of every other item,
+# and with them its blocks of points, start at a shift
+VOLUMES = [((1, 1, 4, 8, 16), (8, 8, 9), 0.0), ((2, 3, 5, 9, 17), (8, 9, 12), 0.0), ((1, 4, 9, 17, 33), (9, 17, 33), 0.0),
+           ((2, 9, 8, 16, 16), (10, 15, 16), 0.0), ((2, 2, 12, 24, 48), (12, 24, 48), 0.3), ((1, 6, 13, 15, 31), (13, 15, 31), 0.9),
+           ((70, 1, 5, 9, 20), (6, 10, 17), 0.0), ((130, 2, 4, 9, 17), (5, 10, 13), 0.2)]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("pad", [0, 1, 2])
+@pytest.mark.parametrize("interp", [0, 1])
+@pytest.mark.parametrize("xs,out,spots", VOLUMES)
+def test_volumes(oracle, device, aclnn, dtype, pad, interp, xs, out, spots):
+    rng = np.random.default_rng(4500 + 10 * interp + pad)
+    points = out[0] * out[1] * out[2]
+    if xs[1] <= 8 or interp == 0:
+        assert host_plans.gradient_tiles(dtype, interp, pad, xs, points, 1 if xs[0] < 64 else 2) is not None
+    if spots > 0.0:
+        grid = _spots(rng, xs[0], points, 3, spots)
+    else:
+        axes = [(2 * np.arange(k) + 1) / k - 1 for k in out]
+        z, y, x = np.meshgrid(*axes, indexing="ij")
+        grid = np.stack([x, y, z], axis=-1)[None] * rng.uniform(0.9, 1.1, (xs[0], 1, 1, 1, 3)) + rng.normal(0, 0.02, (xs[0],) + out + (3,))
+    _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid.reshape((xs[0],) + out + (3,)), rng)
+
+
+def test_special_grid_values(oracle, device, aclnn):
+    """points that are no numbers, infinite or far outside have no tile; on and beside the edges of tiles and of the plane"""
+    rng = np.random.default_rng(4600)
+    xs, out = (2, 2, 40, 70), (45, 50)
+    px = np.concatenate([np.arange(-2, 72, 0.5), [15.999, 31.9999, 32.0001, 63.9999], [np.nan, np.inf, -np.inf, 1e30, -1e30]])
+    gx = (2 * rng.choice(px, (2,) + out) + 1) / 70 - 1
+    gy = (2 * rng.choice(px, (2,) + out) + 1) / 40 - 1
+    for dtype in I.DTYPES:
+        for interp, pad in ((0, 0), (0, 2)):
+            _check(aclnn, oracle, device, dtype, interp, pad, xs, out, np.stack([gx, gy], axis=-1), rng)

@@ -133,3 +133,45 @@ def test_sorting_scratch_holds_a_group_of_items():
         p = P.gather_groups(rng.choice(["fp32", "fp16"]), rng.choice([0, 1, 2]), (n, c, h, w), int(2 ** rng.uniform(8, 25)))
         if p is not None:
             assert 1 <= p[0] <= n and (p[0] == 1 or p[0] * p[1] * 4 <= cache) and p[1] * 4 <= 4 << 30
+
+
+# (type, mode, padding, input, points per item, microseconds by lists and by tiles): measured
+TILES = [("fp32", 0, 0, (8, 3, 479, 637), 479 * 637, 178, 86), ("fp16", 0, 2, (1, 14, 236, 198), 229 * 192, 32, 20),
+         ("fp32", 0, 1, (8, 3, 479, 637), 479 * 637, 455, 330), ("fp32", 0, 1, (1, 3, 480, 640), 480 * 640, 73, 110),
+         ("fp32", 0, 1, (2, 2, 200, 300), 200 * 300, 51, 101), ("fp32", 0, 0, (21, 60, 40, 40), 77 * 77, 86, 156),
+         ("fp16", 0, 0, (10, 2, 267, 440), 448 * 738, 314, 111), ("fp32", 0, 1, (14, 4, 33, 56), 62 * 106, 60, 93),
+         ("bf16", 0, 0, (2, 5, 96, 192), 162 * 324, 31, 40), ("bf16", 0, 2, (6, 12, 136, 184), 115 * 156, 47, 34),
+         ("bf16", 0, 0, (13, 5, 27, 47, 57), 27 * 47 * 57, 108, 86), ("fp32", 0, 2, (1, 12, 9, 81, 64), 13 * 117 * 93, 130, 237),
+         ("bf16", 0, 2, (12, 31, 18, 62, 20), 18 * 62 * 20, 142, 159), ("fp16", 1, 2, (23, 10, 28, 67, 49), 28 * 67 * 49, 114, 130),
+         ("fp32", 1, 0, (10, 2, 14, 26, 17), 14 * 26 * 17, 24, 15)]
+
+
+@pytest.mark.parametrize("dtype,interp,pad,shape,points,lists,tiles", TILES)
+def test_sorting_takes_the_faster_of_lists_and_tiles(dtype, interp, pad, shape, points, lists, tiles):
+    assert (P.gradient_tiles(dtype, interp, pad, shape, points) is not None) == (tiles < lists)
+
+
+def test_gradient_tiles_fit_lds_and_the_launch():
+    """2048 tiles of 32 x 16 (16 x 8 x 4) and 2047 blocks of 1024 points an item; a block more for chunks that start at a shift"""
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 16 * 2048, 32), 2000)[2] == 2048
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 16 * 2048 + 1, 32), 2000) is None
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 4 * 32, 8 * 8, 16 * 8), 2000)[2] == 2048
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 4 * 32 + 1, 8 * 8, 16 * 8), 2000) is None
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 1024, 1024), 2047 * 1024)[3] == 2047
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 1024, 1024), 2047 * 1024 + 1) is None
+    assert P.gradient_tiles("fp32", 0, 0, (128, 1, 9, 20, 21), 3 * 1024, 2)[3] == 4
+    assert P.gradient_tiles("fp32", 0, 0, (128, 1, 9, 20, 21), 3 * 1024, 1)[3] == 3
+    # bicubic samples have no tiles
+    assert P.gradient_tiles("fp32", 2, 0, (1, 1, 64, 64), 2000) is None
+    rng = random.Random(10)
+    taken = 0
+    for _ in range(4000):
+        n, c, h, w = (int(2 ** rng.uniform(0, k)) for k in (16, 10, 12, 12))
+        shape = (n, c, h, w) if rng.random() < 0.5 else (n, c, int(2 ** rng.uniform(0, 7)), max(1, h // 16), max(1, w // 16))
+        p = P.gradient_tiles(rng.choice(["fp32", "fp16", "bf16"]), rng.choice([0, 1]), rng.choice([0, 1, 2]), shape,
+                             int(2 ** rng.uniform(8, 21)), rng.choice([1, 1, 3]))
+        if p is not None:
+            taken += 1
+            assert 1 <= p[0] <= n and (p[0] == 1 or p[0] * p[1] * 4 <= 256 << 20) and p[1] * 4 <= 1 << 30
+            assert p[2] <= 2048 and p[3] <= 2047 and 1 <= p[4] <= c and p[0] * p[2] * p[4] <= MOST_BLOCKS // 2
+    assert taken > 400

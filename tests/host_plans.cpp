@@ -4,6 +4,7 @@
 #include "gs_grad_tiles_plan.hpp"
 #include "resize_flat_plan.hpp"
 #include "resize_grad_plan.hpp"
+#include "resize_nearest_plan.hpp"
 #include "resize_nhwc_plan.hpp"
 
 using namespace opscv;
@@ -138,6 +139,31 @@ int gradient_tiles(int elem, int64_t interp, int64_t pad, int64_t N, int64_t C, 
     out[3] = p.p.blocks;
     out[4] = p.cblocks;
     return p.ok ? 1 : 0;
+}
+
+// nearest resize by runs of rows: rows of a run, pieces of a row, elements of a piece, bytes of LDS; 0 where another kernel
+// takes it.  `in_chunks`: source rows on the 16-byte grid
+int nearest_rows(int elem, int64_t N, int64_t C, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int64_t last, int64_t in_chunks,
+                 int64_t* out)
+{
+    ResizeArgs a;
+    a.elem = (Elem)elem;
+    a.mode = ResizeMode::Nearest;
+    a.channels_last = (int)last;
+    a.N = N;
+    a.C = C;
+    a.Hs = Hs;
+    a.Ws = Ws;
+    a.Hd = Hd;
+    a.Wd = Wd;
+    a.scale_h = (float)Hs / (float)Hd;
+    a.scale_w = (float)Ws / (float)Wd;
+    const NearestRows p = nearest_rows_plan(a, in_chunks != 0);
+    out[0] = p.run;
+    out[1] = p.chunks;
+    out[2] = p.cols;
+    out[3] = p.lds_bytes;
+    return p.run > 0 ? 1 : 0;
 }
 
 }  // extern "C"

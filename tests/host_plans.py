@@ -69,3 +69,12 @@ def gradient_tiles(dtype, interp, pad, shape, points, per_core=1):
     by tiles, None where the lists of gather_groups take it."""
     shape = shape if len(shape) == 5 else shape[:2] + (0,) + shape[2:]
     return _call("gradient_tiles", 5, dtype, interp, pad, *shape, points, per_core)
+
+
+def nearest_rows(dtype, shape, out, channels_last=False):
+    """(rows of a run, pieces of a row, elements of a piece, bytes of LDS) of the nearest resize of (N, C, H, W) images by runs
+    of rows, None where another kernel takes it."""
+    n, c, h, w = shape
+    unit = 4 if dtype == "fp32" else 8
+    grid = w * (c if channels_last else 1) % unit == 0 and not (channels_last and c % unit == 0)
+    return _call("nearest_rows", 4, dtype, n, c, h, w, *out, int(channels_last), int(grid))

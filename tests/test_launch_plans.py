@@ -175,3 +175,32 @@ def test_gradient_tiles_fit_lds_and_the_launch():
             assert 1 <= p[0] <= n and (p[0] == 1 or p[0] * p[1] * 4 <= 256 << 20) and p[1] * 4 <= 1 << 30
             assert p[2] <= 2048 and p[3] <= 2047 and 1 <= p[4] <= c and p[0] * p[2] * p[4] <= MOST_BLOCKS // 2
     assert taken > 400
+
+
+# (type, image, output, channels last, microseconds before and by runs of rows): measured
+NEAREST = [("fp16", (6, 4, 764, 1263), (1528, 2526), False, 117, 42), ("fp32", (17, 11, 62, 120), (151, 292), False, 20.6, 8.1),
+           ("bf16", (15, 174, 74, 83), (296, 332), False, 291, 121), ("bf16", (12, 145, 92, 116), (184, 232), True, 166, 35),
+           ("fp16", (4, 1, 1004, 1749), (4016, 6996), True, 208, 42), ("fp16", (1, 6, 61, 91), (122, 182), False, 5.0, 6.6),
+           ("bf16", (18, 4, 1010, 936), (1078, 999), False, 61.2, 63.7)]
+
+
+@pytest.mark.parametrize("dtype,shape,out,last,before,runs", NEAREST)
+def test_nearest_rows_where_they_are_faster(dtype, shape, out, last, before, runs):
+    assert (P.nearest_rows(dtype, shape, out, last) is not None) == (runs < before)
+
+
+def test_nearest_rows_fit_lds_and_cover_the_row():
+    rng = random.Random(11)
+    whole = pieces = 0
+    for _ in range(4000):
+        n, c, h, w = (int(2 ** rng.uniform(0, k)) for k in (6, 9, 11, 12))
+        out = tuple(max(v, int(v * rng.uniform(0.9, 5))) for v in (h, w))
+        dtype, last = rng.choice(["fp32", "fp16", "bf16"]), rng.random() < 0.5
+        p = P.nearest_rows(dtype, (n, c, h, w), out, last)
+        if p is not None:
+            row = out[1] * (c if last else 1)
+            unit = 4 if dtype == "fp32" else 8
+            assert p[0] % 8 == 0 and 0 < p[3] <= 64 << 10 and (p[1] - 1) * p[2] < row <= p[1] * p[2]
+            assert p[1] == 1 or p[2] % unit == 0
+            whole, pieces = whole + (p[1] == 1), pieces + (p[1] > 1)
+    assert whole > 300 and pieces > 100

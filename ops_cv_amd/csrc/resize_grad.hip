@@ -524,8 +524,8 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
 // Same visits, products and order of the sum as resize_grad_kernel.
 //
 // What bounds it: vector instructions, three per visit plus the shifts, and the set-up of a tile where it serves few
-// planes.  bf16 8x64x65x129 from 257x513: 72.6 us, where rows of odd length were left to resize_grad_kernel before (189
-// us).  4x32x160x240 against resize_grad_lds_kernel (fp16 even rows / fp32) and the gather (bf16 odd rows), before ->
+// planes.  bf16 8x64x65x129 from 257x513: 55 us, 72 before the one column past whole tiles was taken by strip_element, and 189
+// in resize_grad_kernel, where rows of odd length were left before.  4x32x160x240 against resize_grad_lds_kernel (fp16 even rows / fp32) and the gather (bf16 odd rows), before ->
 // after: growth by 0.6 24 -> 16 / 24 -> 16 / 28 -> 17 us, by two 38 -> 29 / 40 -> 28 / 63 -> 31, by three 95 -> 51 /
 // 105 -> 47 / 118 -> 45, by four 136 -> 57 / 174 -> 109 (a growth above four: the gather as before).
 typedef __attribute__((address_space(1))) const void* rg_global_cptr_t;
@@ -563,15 +563,87 @@ __device__ __forceinline__ void weighted_columns(const char* lds, uint32_t off, 
     }
 }
 
+template <bool HALF_PIXEL>
+__device__ __forceinline__ int32_t first_visited(int32_t i, float inv_scale, int32_t len_dst)
+{
+    const float offset = HALF_PIXEL ? 0.5f : 0.0f;
+    const float f = __builtin_ceilf(((float)i - 1.0f + offset) * inv_scale - offset);
+    // a start at or beyond the end visits nothing, whatever its exact value
+    return (f > 0.0f) ? ((f < (float)len_dst) ? (int32_t)f : len_dst) : 0;
+}
+
+// Element e of the columns past the last whole tile, all planes' one after the other: a lane each, straight from memory, the
+// up to eight loads of a row on their way together.  These workgroups go first, so that their chain of a load a row ends
+// under the tiles'.
+template <typename TI, typename TO, bool HALF_PIXEL>
+__device__ __forceinline__ void strip_element(const TI* __restrict__ g, TO* __restrict__ y, int64_t planes, int32_t Hs,
+                                              int32_t Ws, int32_t Hd, int32_t Wd, float scale_h, float scale_w,
+                                              float inv_scale_h, float inv_scale_w, uint32_t cols, uint32_t e)
+{
+    const uint32_t line = e / cols, pl = line / (uint32_t)Hs;
+    if ((int64_t)pl >= planes) {
+        return;
+    }
+    const int32_t H = (int32_t)(line - pl * (uint32_t)Hs), W = Ws - (int32_t)cols + (int32_t)(e - line * cols);
+    const float offset = HALF_PIXEL ? 0.5f : 0.0f, fh = (float)H, fw = (float)W;
+    const float last_y = (float)Hs - 1.0f, last_x = (float)Ws - 1.0f;
+    const int32_t in_x_start = first_visited<HALF_PIXEL>(W, inv_scale_w, Wd);
+    const int32_t in_y_start = first_visited<HALF_PIXEL>(H, inv_scale_h, Hd);
+    const float out_x_start = ((float)in_x_start + offset) * scale_w - offset;
+    const float out_y_start = ((float)in_y_start + offset) * scale_h - offset;
+    const TI* gp = g + (int64_t)pl * Hd * Wd;
+    int32_t nx = 0;
+    float xl[kPlaneVisits], out_x = out_x_start;
+#pragma unroll
+    for (int k = 0; k < kPlaneVisits; k++) {
+        xl[k] = 1.0f - __builtin_fabsf(__builtin_fmaxf(0.0f, __builtin_fminf(out_x, last_x)) - fw);
+        out_x += scale_w;
+    }
+    out_x = out_x_start;
+    for (int32_t in_x = in_x_start; out_x < fw + 1.0f && in_x < Wd; in_x++) {
+        nx++;
+        out_x += scale_w;
+    }
+    float acc = 0.0f;
+    if (nx > kPlaneVisits) {
+        acc = visit_sum<TI>(gp, Wd, 0, 0, in_y_start, in_x_start, out_y_start, out_x_start, fh, fw, scale_h, scale_w, last_y,
+                            last_x, Hd, Wd);
+    } else if (nx > 0) {
+        float out_y = out_y_start;
+#pragma unroll 2
+        for (int32_t in_y = in_y_start; out_y < fh + 1.0f && in_y < Hd; in_y++) {
+            const float y_lerp = 1.0f - __builtin_fabsf(__builtin_fmaxf(0.0f, __builtin_fminf(out_y, last_y)) - fh);
+            const TI* row = gp + (int64_t)in_y * Wd + in_x_start;
+            TI v[kPlaneVisits];
+#pragma unroll
+            for (int k = 0; k < kPlaneVisits; k++) {
+                v[k] = row[k < nx ? k : 0];
+            }
+#pragma unroll
+            for (int k = 0; k < kPlaneVisits; k++) {
+                const float t = ElemIO<TI>::load(&v[k]) * y_lerp * xl[k];
+                acc = (k < nx) ? acc + t : acc;
+            }
+            out_y += scale_h;
+        }
+    }
+    store_streaming<TO>(y + (int64_t)pl * Hs * Ws + (int64_t)H * Ws + W, acc);
+}
+
 template <typename TI, typename TO, bool HALF_PIXEL>
 __global__ __launch_bounds__(kGradThreads) void resize_grad_planes_kernel(
     const TI* __restrict__ g, TO* __restrict__ y, int64_t planes, int32_t Hs, int32_t Ws, int32_t Hd, int32_t Wd,
     float scale_h, float scale_w, float inv_scale_h, float inv_scale_w, int32_t tile_rows, int32_t lds_bytes,
-    float neg_zero, uint32_t tiles_x, uint32_t tiles_y, uint32_t plane_slots)
+    float neg_zero, uint32_t tiles_x, uint32_t tiles_y, uint32_t plane_slots, uint32_t strip_cols, uint32_t strip_blocks)
 {
-    // tiles go to the XCDs as in resize_grad_lds_kernel
-    const uint32_t per_xcd = gridDim.x / 8u;
-    const uint32_t tile_id = (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u;
+    if (blockIdx.x < strip_blocks) {
+        strip_element<TI, TO, HALF_PIXEL>(g, y, planes, Hs, Ws, Hd, Wd, scale_h, scale_w, inv_scale_h, inv_scale_w, strip_cols,
+                                          blockIdx.x * kGradThreads + threadIdx.x);
+        return;
+    }
+    // tiles go to the XCDs as in resize_grad_lds_kernel; the strip's workgroups are whole eights
+    const uint32_t tile_block = blockIdx.x - strip_blocks, per_xcd = (gridDim.x - strip_blocks) / 8u;
+    const uint32_t tile_id = (tile_block % 8u) * per_xcd + tile_block / 8u;
     if (tile_id >= tiles_x * tiles_y * plane_slots) {
         return;
     }
@@ -589,9 +661,7 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_planes_kernel(
     const float offset = HALF_PIXEL ? 0.5f : 0.0f;
     const float last_y = (float)Hs - 1.0f, last_x = (float)Ws - 1.0f;
     auto first_visit = [&](int32_t i, float inv_scale, int32_t len_dst) {
-        const float f = __builtin_ceilf(((float)i - 1.0f + offset) * inv_scale - offset);
-        // a start at or beyond the end visits nothing, whatever its exact value
-        return (f > 0.0f) ? ((f < (float)len_dst) ? (int32_t)f : len_dst) : 0;
+        return first_visited<HALF_PIXEL>(i, inv_scale, len_dst);
     };
     const int32_t W = W0 + lane;
     const bool col_ok = W < Ws;
@@ -761,7 +831,8 @@ hipError_t run_planes(const ResizeGradArgs& a, const PlaneTile& t, hipStream_t s
     hipLaunchKernelGGL((resize_grad_planes_kernel<TI, TO, HP>), dim3((unsigned)t.blocks), dim3(kGradThreads),        \
                        t.lds_bytes, stream, (const TI*)a.x, (TO*)a.y, planes, (int32_t)a.Hs, (int32_t)a.Ws,          \
                        (int32_t)a.Hd, (int32_t)a.Wd, a.scale_h, a.scale_w, a.inv_scale_h, a.inv_scale_w, t.rows,     \
-                       t.lds_bytes, -0.0f, (uint32_t)t.tiles_x, (uint32_t)t.tiles_y, (uint32_t)t.slots)
+                       t.lds_bytes, -0.0f, (uint32_t)t.tiles_x, (uint32_t)t.tiles_y, (uint32_t)t.slots,       \
+                       (uint32_t)t.strip_cols, (uint32_t)t.strip_blocks)
     if (a.half_pixel) {
         OPSCV_RGP(true);
     } else {

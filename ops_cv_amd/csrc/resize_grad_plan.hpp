@@ -48,6 +48,7 @@ constexpr int kPlaneRows = 16;                  // most outgoing rows of a tile
 constexpr int32_t kPlaneTallBytes = 24 * 1024;  // tiles of 16 rows up to here: six workgroups and more fit a CU
 constexpr int32_t kPlaneMostBytes = 48 * 1024;  // tiles of 8 rows up to here
 constexpr int32_t kPlanePad = 64;               // bytes behind the last row that a lane's last columns may be read from
+constexpr int kStripCols = 4;                   // most columns past the last whole tile that are taken a lane per element
 
 struct PlaneTile {
     int32_t rows = 0;  // 0: the variant does not apply
@@ -55,6 +56,8 @@ struct PlaneTile {
     int64_t tiles_x = 0, tiles_y = 0;
     int64_t slots = 0;   // workgroups per tile; each takes every slots-th plane
     int64_t blocks = 0;  // padded for the XCD mapping of the kernel
+    int32_t strip_cols = 0;    // columns past the last whole tile, 0: they are a tile
+    int64_t strip_blocks = 0;  // workgroups of them, ahead of the tiles' and counted in blocks
 };
 
 // Rows off the word grid go to the planes kernel or to the gather, whichever is estimated to be faster.  The gather's time
@@ -124,6 +127,20 @@ inline PlaneTile plane_tile(const ResizeGradArgs& a)
     }
     if (t.rows > 0 && lds_tile_rows(a, kGradCapWords) == 0 && gather_takes_planes(a, t)) {
         t.rows = 0;
+    }
+    // A tile spends a wavefront on every row of a few columns; read in place they cost a lane per element.  Microseconds as a
+    // tile / a lane per element, 512 planes: bf16 65x129 from 257x513 72 / 56, fp32 111 / 91; one, two, three and four columns
+    // past the first tile, bf16 of 64 rows growing by two, 30.1 / 18.1, 30.2 / 18.1, 30.2 / 18.8, 30.3 / 18.8; past the fourth
+    // tile, one and four, 52.1 / 43.0 and 52.3 / 44.8.  Few planes: fp32 8 of 300x644 from 480x1031 14.2 / 12.5, one of 100x65
+    // from 300x195 7.2 / 7.2.
+    const int64_t rest = a.Ws % kPlaneCols, strip = planes * a.Hs * rest;
+    if (t.rows > 0 && a.Ws > kPlaneCols && rest > 0 && rest <= kStripCols && planes <= INT32_MAX && strip <= INT32_MAX) {
+        PlaneTile s = t;
+        s.strip_cols = (int32_t)rest;
+        s.strip_blocks = ((strip + kGradThreads - 1) / kGradThreads + 7) / 8 * 8;
+        s.tiles_x = a.Ws / kPlaneCols;
+        s.blocks = (s.tiles_x * s.tiles_y * s.slots + 7) / 8 * 8 + s.strip_blocks;
+        t = fits_launch(s.blocks, kGradThreads) ? s : t;
     }
     return t;
 }

@@ -125,6 +125,25 @@ def test_resize_gradient_planes_in_turn(oracle, device, aclnn, dtype, align, pla
         assert _same(I.from_torch(got, dtype), ref), offset
 
 
+# one to five columns past whole tiles (up to four are taken a lane per element), more planes than a workgroup of them;
+# growth by four, 1.4, 0.6 and none along x
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("align", [False, True])
+@pytest.mark.parametrize("small,wide", [((9, 65), 254), ((5, 66), 92), ((17, 67), 40), ((3, 68), 68), ((6, 69), 270), ((7, 132), 522)])
+def test_resize_gradient_columns_past_whole_tiles(oracle, device, aclnn, dtype, align, small, wide):
+    import torch
+    gs = (3, 43, 2 * small[0] + 1, wide)
+    assert host_plans.resize_grad_planes(dtype, 129, small, gs[2:], align) is not None
+    g32 = np.random.default_rng(5180 + align).standard_normal(gs).astype(np.float32)
+    g32[1, 1, 1, -1], g32[2, 5, 2, -2], g32[0, 0, -1, 0] = np.inf, -np.inf, np.nan
+    g = I.cast_np(g32, dtype)
+    ref = oracle.upsample_bilinear2d_backward(g, small, align, dtype=I.oracle_code(dtype))
+    got = aclnn.upsample_bilinear2d_backward(I.to_torch(g, dtype, device), gs[:2] + small, align)
+    torch.cuda.synchronize()
+    a, b = I.as_f32(I.from_torch(got, dtype), dtype), I.as_f32(ref, dtype)
+    assert np.array_equal(np.isnan(a), np.isnan(b)) and np.array_equal(a[~np.isnan(a)], b[~np.isnan(b)])
+
+
 # (input, output): groups of consecutive rows with a short last group, a last band of one row, more groups than rows;
 # rows that shrink take the groups in turn
 FLAT = [((1, 3, 65, 129), (257, 513)), ((2, 40, 7, 9), (29, 31)), ((1, 1, 3, 5), (4, 1000)), ((3, 2, 11, 40), (12, 41)),

@@ -48,7 +48,6 @@ constexpr int kPlaneRows = 16;                  // most outgoing rows of a tile
 constexpr int32_t kPlaneTallBytes = 24 * 1024;  // tiles of 16 rows up to here: six workgroups and more fit a CU
 constexpr int32_t kPlaneMostBytes = 48 * 1024;  // tiles of 8 rows up to here
 constexpr int32_t kPlanePad = 64;               // bytes behind the last row that a lane's last columns may be read from
-constexpr int kStripCols = 4;                   // most columns past the last whole tile that are taken a lane per element
 
 struct PlaneTile {
     int32_t rows = 0;  // 0: the variant does not apply
@@ -128,13 +127,22 @@ inline PlaneTile plane_tile(const ResizeGradArgs& a)
     if (t.rows > 0 && lds_tile_rows(a, kGradCapWords) == 0 && gather_takes_planes(a, t)) {
         t.rows = 0;
     }
-    // A tile spends a wavefront on every row of a few columns; read in place they cost a lane per element.  Microseconds as a
-    // tile / a lane per element, 512 planes: bf16 65x129 from 257x513 72 / 56, fp32 111 / 91; one, two, three and four columns
-    // past the first tile, bf16 of 64 rows growing by two, 30.1 / 18.1, 30.2 / 18.1, 30.2 / 18.8, 30.3 / 18.8; past the fourth
-    // tile, one and four, 52.1 / 43.0 and 52.3 / 44.8.  Few planes: fp32 8 of 300x644 from 480x1031 14.2 / 12.5, one of 100x65
-    // from 300x195 7.2 / 7.2.
+    // Columns past the last whole tile.  A tile spends a wavefront on every row of them, however few; read in place they cost a
+    // lane per element.  Microseconds as a tile / a lane per element, 512 planes of 64 rows:
+    //   past the first tile (half of the launch's tiles): growth by 0.7, 1.4, 2, 3 and 4, 16 columns, bf16 18.1 / 14.6,
+    //   24.9 / 19.9, 30.0 / 24.4, 49.6 / 38.6, 50.1 / 44.4, fp32 17.5 / 14.0, 24.2 / 19.2, 29.2 / 23.7, 43.0 / 38.9,
+    //   87.9 / 79.6; 24 columns, growth by 4 50.3 / 57.4 and 88.8 / 95.1;
+    //   past the fourth: 0.7 and 1.4, 16 columns, bf16 26.7 / 25.5, 41.6 / 38.9, fp32 25.9 / 24.5, 40.4 / 38.2, 24 columns
+    //   41.1 / 42.4; growth by 2, 8 columns, 51.9 / 45.7 and 50.6 / 48.2, 12 columns, fp32 50.8 / 52.0; growth by 3, 6 columns,
+    //   fp32 85.5 / 87.6.
+    // bf16 512 planes of 65x129 from 257x513 72 / 55.  Few planes are 0 to 15 % faster, 24 growing by 2 and one column 6.2 / 5.7,
+    // but for growth by four with few elements, whose chain of eight rows outlasts the tiles: 24 of 64x65 9.0 / 9.5, of 64x257
+    // 12.0 / 12.9, with 64x72 (12288 elements) 8.7 / 8.2.
     const int64_t rest = a.Ws % kPlaneCols, strip = planes * a.Hs * rest;
-    if (t.rows > 0 && a.Ws > kPlaneCols && rest > 0 && rest <= kStripCols && planes <= INT32_MAX && strip <= INT32_MAX) {
+    const double visits = 4.0 / ((double)a.scale_h * (double)a.scale_w);  // of an outgoing element
+    const int64_t most = (a.Ws < 2 * kPlaneCols || visits <= 8.2) ? 16 : (visits <= 16.5 ? 8 : 4);
+    if (t.rows > 0 && a.Ws > kPlaneCols && rest > 0 && rest <= most && planes <= INT32_MAX && strip <= INT32_MAX &&
+        (visits <= 40.0 || strip >= 12288)) {
         PlaneTile s = t;
         s.strip_cols = (int32_t)rest;
         s.strip_blocks = ((strip + kGradThreads - 1) / kGradThreads + 7) / 8 * 8;

@@ -125,11 +125,12 @@ def test_resize_gradient_planes_in_turn(oracle, device, aclnn, dtype, align, pla
         assert _same(I.from_torch(got, dtype), ref), offset
 
 
-# one to five columns past whole tiles (up to four are taken a lane per element), more planes than a workgroup of them;
-# growth by four, 1.4, 0.6 and none along x
+# one to seventeen columns past whole tiles (up to four, eight or sixteen are taken a lane per element), more planes than a
+# workgroup of them; growth by four, 1.4, 0.6 and none along x
 @pytest.mark.parametrize("dtype", I.DTYPES)
 @pytest.mark.parametrize("align", [False, True])
-@pytest.mark.parametrize("small,wide", [((9, 65), 254), ((5, 66), 92), ((17, 67), 40), ((3, 68), 68), ((6, 69), 270), ((7, 132), 522)])
+@pytest.mark.parametrize("small,wide", [((9, 65), 254), ((5, 66), 92), ((17, 67), 40), ((3, 68), 68), ((6, 69), 270), ((7, 132), 522),
+                                        ((5, 80), 310), ((5, 81), 300), ((6, 136), 270), ((4, 144), 130)])
 def test_resize_gradient_columns_past_whole_tiles(oracle, device, aclnn, dtype, align, small, wide):
     import torch
     gs = (3, 43, 2 * small[0] + 1, wide)

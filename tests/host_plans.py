@@ -78,3 +78,10 @@ def nearest_rows(dtype, shape, out, channels_last=False):
     unit = 4 if dtype == "fp32" else 8
     grid = w * (c if channels_last else 1) % unit == 0 and not (channels_last and c % unit == 0)
     return _call("nearest_rows", 4, dtype, n, c, h, w, *out, int(channels_last), int(grid))
+
+
+def nearest_rows_nanoseconds(dtype, shape, out, channels_last=False):
+    """Host time of that plan."""
+    plan = lib().nearest_rows_nanoseconds
+    plan.restype = ctypes.c_int64
+    return plan(ctypes.c_int(ELEM[dtype]), *[ctypes.c_int64(v) for v in (*shape, *out, int(channels_last))])

@@ -204,3 +204,11 @@ def test_nearest_rows_fit_lds_and_cover_the_row():
             assert p[1] == 1 or p[2] % unit == 0
             whole, pieces = whole + (p[1] == 1), pieces + (p[1] > 1)
     assert whole > 300 and pieces > 100
+
+
+@pytest.mark.parametrize("shape,out,last", [((1, 1001, 40, 40), (80, 80), True), ((1, 1, 8, 1000000), (16, 2000000), False),
+                                            ((1, 513, 64, 64), (128, 128), True)])
+def test_nearest_rows_plan_takes_no_time(shape, out, last):
+    """The plan is made on every call: where no piece of a row fits LDS (the first two) it took 9 us, half as much again as the
+    smallest call; 0.1 us, here without optimisation some times that."""
+    assert P.nearest_rows_nanoseconds("fp32", shape, out, last) < 2000

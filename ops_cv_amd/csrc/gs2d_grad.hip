@@ -24,6 +24,7 @@
 #include <type_traits>
 
 #include "fast_div.hpp"
+#include "gs2d_grad_grid_plan.hpp"
 #include "gs2d_grad_math.hpp"
 #include "gs_grad_gather.hpp"
 #include "kernels.hpp"
@@ -35,7 +36,6 @@ namespace {
 constexpr int kThreads = 256;         // also the chunk length of the accumulation order
 constexpr uint32_t kKeyBits = 8;      // 256 points of a chunk
 constexpr uint32_t kEpochMax = (1u << (32 - kKeyBits)) - 1;
-constexpr int kGridTile = 16;         // the grid kernel's tiles are square: a lane per grid point
 constexpr int kTagsMax = 1024;        // election tags of a band
 
 // Tag of a band element.  Elements that share a tag are elected as if they were one; folding the high bits in keeps
@@ -234,7 +234,10 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_input_kernel(const T* __re
 //
 // Bound by the lines that the gathers touch and their latency: the loads of up to eight channels are on their way together,
 // of fewer channels all of them (fp32 8x3x479x637, rotations of up to 30 degrees: 58 us in rows, a channel after the other;
-// 40 with the three channels' loads together; 33 in tiles).
+// 40 with the three channels' loads together; 33 in tiles).  Bicubic samples have the sixteen loads of a channel on their way
+// together, in rows (grid_tile_plan): turned grids, one load after the other / together, fp32 8x3x479x637 114 / 115 us, 2x64x128x128
+// 72 / 62, 8x128x32x32 114 / 116, fp16 134 / 108, 156 / 62, 190 / 101; points at random, whose lines are seldom in the cache, fp32
+// 393 / 395, 118 / 125, 108 / 117, fp16 373 / 370, 154 / 107, 188 / 115.
 template <typename T, int INTERP, bool TILED>
 __global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __restrict__ gout, const T* __restrict__ x,
                                                                    const T* __restrict__ grid, T* __restrict__ dgrid,
@@ -434,19 +437,6 @@ GradGatherArgs gather_args(const GridSamplerGradArgs& a)
     return g;
 }
 
-// Tiles of grid points for the grid gradient: planes beyond the first-level cache, where lines are fetched again for every
-// row of points, two workgroups per CU, and few lanes along the edges without a point.  Rows / tiles, both gradients' grid
-// part alone: fp32 8x3x479x637 40.5 / 33.2 us, fp16 6x3x576x472 -> 362x297 15.8 / 11.3, fp32 2x37x132x184 11.7 / 9.6; smaller
-// planes bf16 2x105x90x146 19.4 / 24.4, fp16 19x11x144x120 -> 210x175 22.6 / 23.8; few tiles fp32 3x3x241x369 -> 128x196 7.0 /
-// 7.2.
-bool grid_in_tiles(const GridSamplerGradArgs& a)
-{
-    const int64_t tiles_x = (a.Wout + kGridTile - 1) / kGridTile, tiles_y = (a.Hout + kGridTile - 1) / kGridTile;
-    const int64_t lanes = tiles_x * tiles_y * kGridTile * kGridTile;
-    return a.Hin * a.Win * elem_size(a.elem) > (64 << 10) && a.N * tiles_x * tiles_y >= 512 &&
-           lanes - lanes / 5 <= a.Hout * a.Wout;
-}
-
 template <typename T, int INTERP>
 hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
 {
@@ -529,15 +519,12 @@ hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
     }
     if (a.dgrid != nullptr && !dgrid_done) {
         const int64_t total = a.N * a.Hout * a.Wout;
-        const int64_t tiles_x = (a.Wout + kGridTile - 1) / kGridTile, tiles_y = (a.Hout + kGridTile - 1) / kGridTile;
-        const int64_t tiles = a.N * tiles_x * tiles_y;
-        if (INTERP != 1 && grid_in_tiles(a) && tiles <= INT32_MAX / 2) {
-            p.pieces = (uint32_t)tiles;
-            p.by_item = make_fast_div((uint32_t)(tiles_x * tiles_y));
-            p.by_tiles_x = make_fast_div((uint32_t)tiles_x);
-            const uint32_t blocks = (uint32_t)((tiles + 7) / 8 * 8);  // as many for every XCD
-            if (fits_launch(blocks, kThreads)) {
-                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, true>), dim3(blocks), dim3(kThreads), 0, stream,
+        if constexpr (INTERP == 0) {
+            if (const GridTilePlan t = grid_tile_plan(a); t.ok) {
+                p.pieces = (uint32_t)t.tiles;
+                p.by_item = make_fast_div((uint32_t)t.per_item);
+                p.by_tiles_x = make_fast_div((uint32_t)t.tiles_x);
+                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, true>), dim3((unsigned)t.blocks), dim3(kThreads), 0, stream,
                                    (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, total, p, 0);
                 return hipGetLastError();
             }

@@ -1,0 +1,48 @@
+// Launch plan of the grid gradient's tiles (gs2d_grad.hip): host arithmetic only.
+#pragma once
+
+#include <cstdint>
+
+#include "acl_types.hpp"
+#include "launch_limits.hpp"
+
+namespace opscv {
+
+constexpr int kGridTile = 16;  // square: a lane per grid point of 256
+constexpr int kGridTileThreads = kGridTile * kGridTile;
+
+struct GridTilePlan {
+    bool ok = false;
+    int64_t tiles_x = 0, per_item = 0, tiles = 0;
+    int64_t blocks = 0;  // as many for every XCD
+};
+
+// Tiles of grid points for the grid gradient: planes beyond the first-level cache, where lines are fetched again for every
+// row of points, two workgroups per CU, and few lanes along the edges without a point.  Rows / tiles, both gradients' grid
+// part alone: fp32 8x3x479x637 40.5 / 33.2 us, fp16 6x3x576x472 -> 362x297 15.8 / 11.3, fp32 2x37x132x184 11.7 / 9.6; smaller
+// planes bf16 2x105x90x146 19.4 / 24.4, fp16 19x11x144x120 -> 210x175 22.6 / 23.8; few tiles fp32 3x3x241x369 -> 128x196 7.0 /
+// 7.2.
+//
+// Not for bicubic samples, whose sixteen taps share lines within a point already: fp32 8x3x479x637 115 / 138 us, fp16 108 / 153,
+// fp32 2x3x720x1280 106 / 120, 1x4x256x256 -> 512x512 18.0 / 23.5, with border padding 19.6 / 32.3, 4x1x300x400 17.2 / 19.4.
+inline GridTilePlan grid_tile_plan(const GridSamplerGradArgs& a)
+{
+    GridTilePlan p;
+    if (a.interp != 0 || a.N < 1 || a.Hout < 1 || a.Wout < 1 || a.Hout > INT32_MAX / 2 || a.Wout > INT32_MAX / 2 || a.N > INT32_MAX / 2) {
+        return p;
+    }
+    const int64_t tiles_y = (a.Hout + kGridTile - 1) / kGridTile;
+    p.tiles_x = (a.Wout + kGridTile - 1) / kGridTile;
+    p.per_item = p.tiles_x * tiles_y;
+    if (p.per_item > INT32_MAX / 2 / a.N) {
+        return p;
+    }
+    p.tiles = a.N * p.per_item;
+    p.blocks = (p.tiles + 7) / 8 * 8;
+    const int64_t lanes = p.per_item * kGridTileThreads;
+    p.ok = a.Hin * a.Win * elem_size(a.elem) > (64 << 10) && p.tiles >= 512 && lanes - lanes / 5 <= a.Hout * a.Wout &&
+           fits_launch(p.blocks, kGridTileThreads);
+    return p;
+}
+
+}  // namespace opscv

@@ -2,6 +2,7 @@
 #include <chrono>
 
 #include "gs2d_direct_plan.hpp"
+#include "gs2d_grad_grid_plan.hpp"
 #include "gs_grad_gather_plan.hpp"
 #include "gs_grad_tiles_plan.hpp"
 #include "resize_flat_plan.hpp"
@@ -140,6 +141,24 @@ int gradient_tiles(int elem, int64_t interp, int64_t pad, int64_t N, int64_t C, 
     out[2] = p.p.tiles;
     out[3] = p.p.blocks;
     out[4] = p.cblocks;
+    return p.ok ? 1 : 0;
+}
+
+// the grid gradient's tiles: tiles, workgroups; 0 where its points are taken in rows
+int grid_gradient_tiles(int elem, int64_t interp, int64_t N, int64_t H, int64_t W, int64_t Ho, int64_t Wo, int64_t* out)
+{
+    GridSamplerGradArgs a;
+    a.elem = (Elem)elem;
+    a.interp = (int)interp;
+    a.N = N;
+    a.C = 1;
+    a.Hin = H;
+    a.Win = W;
+    a.Hout = Ho;
+    a.Wout = Wo;
+    const GridTilePlan p = grid_tile_plan(a);
+    out[0] = p.tiles;
+    out[1] = p.blocks;
     return p.ok ? 1 : 0;
 }
 

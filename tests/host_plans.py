@@ -71,6 +71,11 @@ def gradient_tiles(dtype, interp, pad, shape, points, per_core=1):
     return _call("gradient_tiles", 5, dtype, interp, pad, *shape, points, per_core)
 
 
+def grid_gradient_tiles(dtype, interp, n, plane, out):
+    """(tiles, workgroups) of the 2-D sampler's grid gradient, None where its points are taken in rows."""
+    return _call("grid_gradient_tiles", 2, dtype, interp, n, *plane, *out)
+
+
 def nearest_rows(dtype, shape, out, channels_last=False):
     """(rows of a run, pieces of a row, elements of a piece, bytes of LDS) of the nearest resize of (N, C, H, W) images by runs
     of rows, None where another kernel takes it."""

@@ -177,6 +177,26 @@ def test_gradient_tiles_fit_lds_and_the_launch():
     assert taken > 400
 
 
+# (type, mode, items, plane, points, microseconds in rows and in tiles): measured, bicubic too
+GRID = [("fp32", 0, 8, (479, 637), (479, 637), 40.5, 33.2), ("fp16", 0, 6, (576, 472), (362, 297), 15.8, 11.3),
+        ("bf16", 0, 2, (90, 146), (90, 146), 19.4, 24.4), ("fp32", 0, 3, (241, 369), (128, 196), 7.0, 7.2),
+        ("fp32", 2, 8, (479, 637), (479, 637), 115, 138), ("fp16", 2, 8, (479, 637), (479, 637), 108, 153),
+        ("fp32", 2, 2, (720, 1280), (720, 1280), 106, 120), ("fp32", 2, 1, (256, 256), (512, 512), 19.6, 32.3)]
+
+
+@pytest.mark.parametrize("dtype,interp,n,plane,out,rows,tiles", GRID)
+def test_grid_gradient_in_the_faster_of_rows_and_tiles(dtype, interp, n, plane, out, rows, tiles):
+    assert (P.grid_gradient_tiles(dtype, interp, n, plane, out) is not None) == (tiles < rows)
+
+
+def test_grid_gradient_tiles_fit_the_launch():
+    # 256 x 256 points: 256 tiles an item
+    assert P.grid_gradient_tiles("fp32", 0, 2, (200, 200), (256, 256))[0] == 512
+    assert P.grid_gradient_tiles("fp32", 0, MOST_BLOCKS // 256, (200, 200), (256, 256))[1] <= MOST_BLOCKS
+    assert P.grid_gradient_tiles("fp32", 0, MOST_BLOCKS // 256 + 1, (200, 200), (256, 256)) is None
+    assert P.grid_gradient_tiles("fp32", 0, 2**31 - 1, (200, 200), (40000, 40000)) is None
+
+
 # (type, image, output, channels last, microseconds before and by runs of rows): measured
 NEAREST = [("fp16", (6, 4, 764, 1263), (1528, 2526), False, 117, 42), ("fp32", (17, 11, 62, 120), (151, 292), False, 20.6, 8.1),
            ("bf16", (15, 174, 74, 83), (296, 332), False, 291, 121), ("bf16", (12, 145, 92, 116), (184, 232), True, 166, 35),

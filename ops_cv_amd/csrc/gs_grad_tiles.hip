@@ -32,6 +32,7 @@
 
 #include "gs_grad_gather.hpp"
 #include "gs_grad_points.hpp"
+#include "gs_grad_tiles_kernel.hpp"
 #include "gs_grad_tiles_plan.hpp"
 #include "kernels.hpp"
 
@@ -46,63 +47,6 @@ constexpr uint32_t kNoPlace = 0xFFFFFFFFu;
 constexpr uint32_t kCountedRun = 32;   // runs of up to as many points are put in order by counting, longer ones by ballots
 constexpr uint32_t kSerialMost = 192;  // contributions that a lane merges by itself, and adds by itself where
 constexpr int kFewCrowded = 6;         // more lanes than this of its wavefront have as many as that to do
-
-__device__ __forceinline__ void landed()
-{
-    // what a wavefront writes to LDS it reads back itself, in order
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-__device__ __forceinline__ uint32_t bits_below(uint64_t mask)
-{
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
-// Inclusive sum over the wavefront: within rows of 16 lanes, then from row to row.
-__device__ __forceinline__ uint32_t wave_scan(uint32_t v)
-{
-    int s = (int)v;
-    s += __builtin_amdgcn_update_dpp(0, s, 0x111, 0xf, 0xf, false);  // row_shr:1
-    s += __builtin_amdgcn_update_dpp(0, s, 0x112, 0xf, 0xf, false);
-    s += __builtin_amdgcn_update_dpp(0, s, 0x114, 0xf, 0xf, false);
-    s += __builtin_amdgcn_update_dpp(0, s, 0x118, 0xf, 0xf, false);
-    s += __builtin_amdgcn_update_dpp(0, s, 0x142, 0xa, 0xf, false);  // row_bcast:15 to rows 1 and 3
-    s += __builtin_amdgcn_update_dpp(0, s, 0x143, 0xc, 0xf, false);  // row_bcast:31 to rows 2 and 3
-    return (uint32_t)s;
-}
-
-// The cell of a point: the lattice of low corners for linear interpolation, the element for nearest.  False: no corner
-// is inside (or the coordinate is not a number; sizes are exact in single precision: launch plan).
-template <typename T, int DIM, int INTERP>
-__device__ __forceinline__ bool low_corner(const Coords<T, DIM>& c, const TilesParams& p, int32_t* x, int32_t* y, int32_t* z)
-{
-    constexpr float least = (INTERP == 1) ? 0.0f : -1.0f;
-    auto axis = [&](int i, int32_t size, int32_t* cell) {
-        const float v = ElemIO<T>::load(&c.v[i]);
-        const float f = (INTERP == 1) ? __builtin_rintf(v) : __builtin_floorf(v);
-        const bool in = f >= least && f < (float)size;
-        *cell = (int32_t)(in ? f : 0.0f);
-        return in;
-    };
-    bool in = axis(0, p.W, x);
-    in = axis(1, p.H, y) && in;
-    *z = 0;
-    if constexpr (DIM == 3) {
-        in = axis(2, p.D, z) && in;
-    }
-    return in;
-}
-
-// workgroups go to the eight XCDs in turn: XCD k takes the k-th eighth of all pieces, so that neighbours share an L2
-__device__ __forceinline__ bool piece_of(uint32_t block, uint32_t pieces, const FastDiv& per_item, uint32_t* n, uint32_t* local)
-{
-    const uint32_t per_xcd = (pieces + 7u) >> 3;
-    const uint32_t piece = (block & 7u) * per_xcd + (block >> 3);
-    *n = fast_div(piece, per_item);
-    *local = piece - *n * per_item.div;
-    return (block >> 3) < per_xcd && piece < pieces;
-}
 
 template <typename T, int DIM, int INTERP>
 __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __restrict__ grid, uint32_t* __restrict__ ws,
@@ -348,54 +292,6 @@ struct Sums<_Float16, INTERP, CB> {
     }
 };
 
-// Weights of the points in LDS, plane by plane (a lane reads a weight of some point: neighbours in a plane lie in different
-// banks): every corner's, values of the element type; of volumes in single precision, which would fill LDS, the products
-// of the four corners along x and y and the two distances along z.  The last of a plane is zero.
-template <typename T, int DIM, int CAP>
-struct Weights {
-    static constexpr bool kProducts = DIM == 3 && sizeof(T) == 4;
-    static constexpr int kPlanes = kProducts ? 6 : (1 << DIM);
-    static constexpr uint32_t kStride = CAP + 1;
-    T v[kPlanes * kStride];
-    __device__ __forceinline__ void put(uint32_t i, const Coords<T, DIM>& c)
-    {
-        float d[DIM][2];  // to the high edge and from the low edge of the cell, as the decisions of the taps have them
-#pragma unroll
-        for (int k = 0; k < DIM; k++) {
-            const float f = ElemIO<T>::load(&c.v[k]), low = __builtin_floorf(f);
-            d[k][0] = (low + 1.0f) - f;
-            d[k][1] = f - low;
-        }
-#pragma unroll
-        for (int k = 0; k < kPlanes; k++) {
-            float w;
-            if constexpr (kProducts) {
-                w = (k < 4) ? d[0][k & 1] * d[1][(k >> 1) & 1] : d[DIM - 1][k & 1];
-            } else {
-                w = d[0][k & 1] * d[1][(k >> 1) & 1];
-                if constexpr (DIM == 3) {
-                    w = w * d[DIM - 1][k >> 2];
-                }
-            }
-            ElemIO<T>::store(&v[k * kStride + i], as_fp32_value(w));
-        }
-    }
-    __device__ __forceinline__ float get(uint32_t i, uint32_t tap) const
-    {
-        if constexpr (kProducts) {
-            return v[(tap & 3u) * kStride + i] * v[((tap >> 2) + 4u) * kStride + i];
-        } else {
-            return ElemIO<T>::load(&v[tap * kStride + i]);
-        }
-    }
-    __device__ __forceinline__ void clear_last(int t)
-    {
-        if (t < kPlanes) {
-            ElemIO<T>::store(&v[t * kStride + CAP], 0.0f);
-        }
-    }
-};
-
 template <typename T, int DIM, int INTERP, int CB>
 __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_kernel(
     const T* __restrict__ gout, const T* __restrict__ grid, T* __restrict__ dx, const uint32_t* __restrict__ ws, TilesParams p,
@@ -454,43 +350,12 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
     const int32_t tile_y = tile_yz - tile_z * p.tiles_y;
     const int32_t x0 = tile_x * S::kX, y0 = tile_y * S::kY, z0 = tile_z * S::kZ;
     const int32_t phase = (DIM == 3 && p.items_per_core > 1) ? phase_of(n, p) : 0;
-    // sums of the wavefronts before this one, and of all, from s_scan
-    auto waves_before = [&](uint32_t* all) {
-        const uint32_t incl = wave_scan(lane < kWaves ? s_scan[lane < kWaves ? lane : 0] : 0u);
-        *all = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWaves - 1);
-        return wave > 0 ? (uint32_t)__builtin_amdgcn_readlane((int)incl, wave - 1) : 0u;
-    };
+    auto waves_before = [&](uint32_t* all) { return sums_before<kWaves>(s_scan, wave, lane, all); };
 
-    // the tile's segments (packed sums: segments that are not empty above 21 bits of points; both fit by launch plan)
     uint32_t* s_before = s_seg;
     uint32_t* s_where = s_seg + p.blocks + 1;
-    uint32_t segs = 0, total = 0;
-    for (int32_t b0 = 0; b0 < p.blocks; b0 += TH) {
-        const int32_t b = b0 + t;
-        const uint32_t w = (b < p.blocks) ? wsn[p.lay.segments + (size_t)b * p.tiles + tile] : 0u;
-        const uint32_t count = w >> 16, packed = count | (count > 0u ? 1u << 21 : 0u);
-        uint32_t incl = 0u;
-        if (b0 + wave * 64 < p.blocks) {
-            incl = wave_scan(packed);
-        }
-        if (lane == 63) {
-            s_scan[wave] = incl;
-        }
-        __syncthreads();
-        uint32_t all;
-        const uint32_t before = waves_before(&all) + incl - packed;
-        if (count > 0u) {
-            const uint32_t at = segs + (before >> 21);
-            s_before[at] = total + (before & 0x1FFFFFu);
-            s_where[at] = ((uint32_t)b << 14) | (w & 0xFFFFu);
-        }
-        segs += all >> 21;
-        total += all & 0x1FFFFFu;
-        __syncthreads();
-    }
-    if (t == 0) {
-        s_before[segs] = total;
-    }
+    uint32_t segs, total;
+    tile_segments<TH>(wsn, p, tile, s_before, s_where, s_scan, &segs, &total);
     if (t < GS) {
         ElemIO<T>::store(&s_go[CAP * GS + t], 0.0f);
     }

@@ -13,7 +13,7 @@
 //           weight times gradOutput, both from LDS, with the reference's roundings.  Elements with more contributions
 //           than keys are merged, run by run, a lane each, or where a single element holds hundreds by the whole
 //           wavefront; more points than LDS holds are taken a run of segments after the other, which are whole chunks
-//           in ascending order.
+//           in ascending order.  Tiles that many points fall on are left to a third kernel (gs_grad_tiles_crowded.hip).
 //
 // Every operand is read once and a point's gradOutput once per tile that it reaches; all that is scattered happens in LDS.
 //
@@ -60,6 +60,9 @@ __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __re
     __shared__ uint32_t s_total;
     uint32_t* counts = smem;                      // [wave][tile]
     unsigned long long* masks = reinterpret_cast<unsigned long long*>(smem + kWaves * p.tiles);  // [wave][tile]
+    if (blockIdx.x == 0 && threadIdx.x == 0 && p.list_most > 0) {
+        ws[p.list] = 0u;  // for the gather kernel
+    }
     uint32_t n, block;
     if (!piece_of(blockIdx.x, pieces, p.by_blocks, &n, &block)) {
         return;
@@ -82,7 +85,7 @@ __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __re
     }
     // The tiles of a point, -1 where it has no k-th one: that of its low corner, then those that the high corner lies in
     // along x, along y and so on; `any`: the k of which any lane of the wavefront has one.
-    auto tiles_of = [&](int u, int32_t (&tile)[K], uint32_t* any) {
+    auto tiles_of = [&](int u, int32_t (&tile)[K], uint32_t (&part)[K], uint32_t* any) {
         int32_t x, y, z;
         const bool in = low_corner<T, DIM, INTERP>(coords_of<T, DIM, INTERP>(raw[u], p), p, &x, &y, &z) && have[u];
         auto low_of = [](int32_t v, int32_t edge) { return (int32_t)((uint32_t)(v < 0 ? 0 : v) / (uint32_t)edge); };
@@ -94,11 +97,24 @@ __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __re
             low += low_of(z, S::kZ) * p.tiles_x * p.tiles_y;
         }
         const bool nx = next(x, p.W, S::kX), ny = next(y, p.H, S::kY), nz = DIM == 3 && next(z, p.D, S::kZ);
+        // along an axis where it is the high corner that lies in the tile, that is in the first part
+        uint32_t stride = 1;
+        auto along = [&](int32_t v, int32_t edge, int32_t part_edge, int axis) {
+            const uint32_t in_tile = (uint32_t)(v < 0 ? 0 : v) & (uint32_t)(edge - 1);
+            const bool spills = INTERP == 0 && v >= 0 && (in_tile & (uint32_t)(part_edge - 1)) == (uint32_t)(part_edge - 1) &&
+                                in_tile != (uint32_t)(edge - 1);
+            const uint32_t code = in_tile / (uint32_t)part_edge * stride | (spills ? 1u << (kRecordPartBits + axis) : 0u);
+            stride *= (uint32_t)(edge / part_edge);
+            return code;
+        };
+        const uint32_t part_x = along(x, S::kX, S::kPartX, 0), part_y = along(y, S::kY, S::kPartY, 1);
+        const uint32_t part_z = (DIM == 3) ? along(z, S::kZ, S::kPartZ, 2) : 0u;
         *any = 1u;
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const bool is = in && (!(k & 1) || nx) && (!(k & 2) || ny) && (!(k & 4) || nz);
             tile[k] = is ? low + (k & 1) + ((k & 2) ? p.tiles_x : 0) + ((k & 4) ? p.tiles_x * p.tiles_y : 0) : -1;
+            part[k] = ((k & 1) ? 0u : part_x) + ((k & 2) ? 0u : part_y) + ((k & 4) ? 0u : part_z);
             if (k > 0) {
                 *any |= __builtin_amdgcn_ballot_w64(is) != 0 ? 1u << k : 0u;
             }
@@ -109,12 +125,13 @@ __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __re
     // 64 lanes on one address would take 64 turns).
     uint32_t* mine = counts + wave * p.tiles;
     unsigned long long* my_masks = masks + wave * p.tiles;
-    uint32_t place[kSteps][K], any[kSteps];  // tile << 8 | rank among the wavefront's 256 points
+    uint32_t place[kSteps][K], any[kSteps];  // part << 20 | tile << 8 | rank among the wavefront's 256 points
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kSteps; u++) {
         int32_t tile[K];
-        tiles_of(u, tile, &any[u]);
+        uint32_t part[K];
+        tiles_of(u, tile, part, &any[u]);
 #pragma unroll
         for (int k = 0; k < K; k++) {
             place[u][k] = kNoPlace;
@@ -143,7 +160,7 @@ __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __re
         for (int k = 0; k < K; k++) {
             if (((any[u] >> k) & 1u) && tile[k] >= 0) {
                 const uint32_t below = bits_below(mask[k]);
-                place[u][k] = ((uint32_t)tile[k] << 8) | (before[k] + below);
+                place[u][k] = (part[k] << 20) | ((uint32_t)tile[k] << 8) | (before[k] + below);
                 if (below == 0u) {
                     mine[tile[k]] = before[k] + (uint32_t)__builtin_popcountll(mask[k]);
                     my_masks[tile[k]] = 0ull;
@@ -191,7 +208,8 @@ __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __re
 #pragma unroll
         for (int k = 0; k < K; k++) {
             if (((any[u] >> k) & 1u) && place[u][k] != kNoPlace) {
-                records[mine[place[u][k] >> 8] + (place[u][k] & 255u)] = (uint16_t)(wave * 256 + u * 64 + lane);
+                const uint32_t at = mine[(place[u][k] >> 8) & 0xFFFu] + (place[u][k] & 255u);
+                records[at] = (uint16_t)((place[u][k] >> 20 << kRecordBits) | (uint32_t)(wave * 256 + u * 64 + lane));
             }
         }
     }
@@ -294,8 +312,8 @@ struct Sums<_Float16, INTERP, CB> {
 
 template <typename T, int DIM, int INTERP, int CB>
 __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_kernel(
-    const T* __restrict__ gout, const T* __restrict__ grid, T* __restrict__ dx, const uint32_t* __restrict__ ws, TilesParams p,
-    uint32_t pieces, int32_t chans_per_block)
+    const T* __restrict__ gout, const T* __restrict__ grid, T* __restrict__ dx, const uint32_t* __restrict__ ws,
+    uint32_t* __restrict__ list, TilesParams p, uint32_t pieces, int32_t chans_per_block)
 {
     typedef GradTile<DIM> S;
     constexpr int TH = S::kThreads, CAP = S::kRecords, RPL = (CAP + TH - 1) / TH, kWaves = TH / 64;
@@ -356,6 +374,18 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
     uint32_t* s_where = s_seg + p.blocks + 1;
     uint32_t segs, total;
     tile_segments<TH>(wsn, p, tile, s_before, s_where, s_scan, &segs, &total);
+    // to gs_tiles_crowded_kernel; every tile has room on the list.  One number is all that is kept for it: scalar registers are
+    // what this kernel has too few of
+    const uint32_t entry = cblock == 0u ? (n << kTileBits) | tile : kNoPlace;
+    auto leave = [&]() {
+        if (entry != kNoPlace && t == 0) {
+            list[1u + atomicAdd(list, 1u)] = entry;
+        }
+    };
+    if (total > p.crowded.points) {
+        leave();
+        return;
+    }
     if (t < GS) {
         ElemIO<T>::store(&s_go[CAP * GS + t], 0.0f);
     }
@@ -548,7 +578,7 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
         landed();
     };
 
-    // the points of segments [from, to): cells, lists, and this element's keys in order
+    // the points of segments [from, to): cells, lists, and this element's keys in order; whether the tile is another kernel's
     auto build = [&](uint32_t from, uint32_t to, int32_t c0, int32_t nc) {
         const uint32_t base = s_before[from];
         number = s_before[to] - base;
@@ -587,7 +617,7 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
 #pragma unroll
         for (int k = 0; k < RPL; k++) {
             if (lane_points(k)) {
-                const uint32_t q = block[k] * kBinPoints + record[k];
+                const uint32_t q = block[k] * kBinPoints + (record[k] & (kBinPoints - 1u));
                 pt[k] = (int32_t)q - phase;
                 own_key[k] = (q >> 8) << (kPosBits + kTapBits);
                 __builtin_memcpy(raw[k], reinterpret_cast<const char*>(grid_n) + (uint32_t)pt[k] * (uint32_t)sizeof(raw[k]), sizeof(raw[k]));
@@ -663,10 +693,13 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
         len = (x0 + lx < p.W && y0 + ly < p.H && z0 + lz < p.D) ? len : 0u;
         crowded = len > (uint32_t)NK;
         if (crowded) {
-            s_crowded = 1u;
+            atomicOr(&s_crowded, len > p.crowded.contributions ? 3u : 1u);
         }
         __syncthreads();
         if (s_crowded != 0u) {
+            if (INTERP == 0 && from == 0u && s_crowded == 3u) {
+                return true;
+            }
             // merging wants the points of a cell in order
             uint32_t place[RPL];
 #pragma unroll
@@ -737,6 +770,7 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
             }
         }
         sort_most<NK, kStep>(key, most);
+        return false;
     };
 
     Sums<T, INTERP, CB> sums;
@@ -874,7 +908,10 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
             sums.clear();
             if (to > from) {
                 if (c0 == c_begin) {
-                    build(from, to, c0, nc);
+                    if (build(from, to, c0, nc)) {
+                        leave();
+                        return;
+                    }
                 } else {
                     T go[RPL][GS];
 #pragma unroll
@@ -945,8 +982,9 @@ hipError_t launch_tiles(const GradGatherArgs& a, const TilesPlan& pl, hipStream_
     const uint32_t pieces = (uint32_t)a.N * pl.p.by_item.div;
     hipLaunchKernelGGL((gs_tiles_gather_kernel<T, DIM, INTERP, CB>), dim3(xcd_blocks(pieces)), dim3(S::kThreads),
                        (size_t)pl.segment_lds, stream, (const T*)a.gout, (const T*)a.grid, (T*)a.dx,
-                       (const uint32_t*)a.scratch, pl.p, pieces, pl.chans_per_block);
-    return hipGetLastError();
+                       (const uint32_t*)a.scratch, (uint32_t*)a.scratch + pl.p.list, pl.p, pieces, pl.chans_per_block);
+    e = hipGetLastError();
+    return (e == hipSuccess && pl.p.list_most > 0) ? run_crowded_tiles(a, pl, stream) : e;
 }
 
 template <typename T, int DIM, int INTERP>
@@ -982,7 +1020,7 @@ hipError_t run_typed(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t s
 int64_t grad_tiles_words(const GradGatherArgs& a)
 {
     const TilesPlan pl = tiles_plan(a);
-    return pl.ok ? (int64_t)pl.p.lay.item_words * pl.group : 0;
+    return pl.ok ? pl.words : 0;
 }
 
 hipError_t run_grad_tiles(const GradGatherArgs& a, hipStream_t stream)

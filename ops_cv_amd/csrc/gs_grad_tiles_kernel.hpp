@@ -1,5 +1,5 @@
-// What the kernels of the input gradient by tiles share (gs_grad_tiles.hip): scans, the cell of a point, a tile's segments,
-// weights in LDS.
+// What the kernels of the input gradient by tiles share (gs_grad_tiles.hip, gs_grad_tiles_crowded.hip): scans, the cell of a
+// point, a tile's segments, weights in LDS.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -8,6 +8,9 @@
 #include "gs_grad_tiles_plan.hpp"
 
 namespace opscv {
+
+// the tiles on the list, after the gather kernel (gs_grad_tiles_crowded.hip)
+hipError_t run_crowded_tiles(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t stream);
 
 __device__ __forceinline__ void landed()
 {

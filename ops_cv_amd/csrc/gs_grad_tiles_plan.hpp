@@ -18,22 +18,59 @@ struct GradTile;
 template <>
 struct GradTile<2> {
     static constexpr int kX = 32, kY = 16, kZ = 1;
+    static constexpr int kPartX = 8, kPartY = 4, kPartZ = 1;  // of a crowded tile
     static constexpr int kThreads = kX * kY * kZ;
     static constexpr int kRecords = 1024;
 };
 template <>
 struct GradTile<3> {
     static constexpr int kX = 16, kY = 8, kZ = 4;
+    static constexpr int kPartX = 4, kPartY = 4, kPartZ = 4;
     static constexpr int kThreads = kX * kY * kZ;
     static constexpr int kRecords = 1280;
 };
 
+// A record: the point's number within its block, and above it the part of the tile that its low corner lies in (of the corners
+// inside the tile, along every axis) and along which axes its high corner lies in the next part.
+constexpr int kRecordBits = 10;
+constexpr int kRecordPartBits = 4;  // of the part; an axis a bit each above them
+
 struct TilesLayout {   // offsets in 32-bit words within an item's scratch
     uint32_t segments; // [block][tile]: first record in the block's records, and how many << 16
-    uint32_t records;  // [block]: 16-bit numbers of points within the block, segment after segment
+    uint32_t records;  // [block]: 16-bit records of points, segment after segment
     uint32_t block_words;  // of records
     uint32_t item_words;
 };
+
+// Tiles that are left to gs_tiles_crowded_kernel: of more than `points` points, or with an element of more than
+// `contributions` among the tile's first points.
+//
+// The kernel costs a launch, and 4.6 us where no tile is crowded.  Input gradient alone, as many points as elements on a part of
+// either axis; lists / rounds of the gather kernel alone / here, microseconds.  Half of an axis stays with the rounds: fp32
+// 1x3x480x640 93 / 62 / 64 (112 with every tile beyond one round here), fp16 8x4x256x256 from 360x360 175 / 143 / 146 (225 from
+// 3072 points on), nearest 1x3x480x640 34 / 25 / 27 (84).  A quarter: 1x3x480x640 125 / 335 / 80, 8x3x479x637 758 / 372 / 470,
+// fp16 2x16x200x300 88 / 332 / 90 (127 from 5120 points on), fp32 2x64x200x200 163 / 589 / 228; nearest 60 / 102 / 102 and 233 /
+// 130 / 130 (389 from 4096 on).  An eighth: 167 / 1583 / 151, 820 / 1653 / 388, 120 / 1377 / 124, 218 / 1995 / 184, nearest 86 /
+// 529 / 186 and 394 / 563 / 411.  Volumes: fp16 2x4x32x64x64 half 296 / 236 / 92, quarter 487 / 2197 / 252, eighth 1608 / 35542 /
+// 1249; fp32 4x16x16x64x64 reflection 339 / 360 / 371 (548 by the line of few channels), 553 / 2712 / 770, 1576 / 30692 / 646;
+// nearest 2x4x32x64x64 38 / 33 / 36, 78 / 311 / 194, 119 / 1902 / 633: nearest samples of an eighth of every axis are what the
+// lists remain much faster at.  Nine points of ten on five spots: 1x3x480x640 6156 / 2138 / 1433.
+// Border padding piles points up on few elements, which the gather kernel's wavefronts add together: no limit of contributions
+// (fp16 8x4x256x256 from 360x360 131 / 97 / 100, with the limit 133).
+struct CrowdedTile {
+    uint32_t points, contributions;
+};
+inline CrowdedTile crowded_tile(const GradGatherArgs& a)
+{
+    const uint32_t any = 0xFFFFFFFFu;
+    if (a.interp == 1) {
+        return {a.dim == 3 ? 10240u : 12288u, any};
+    }
+    if (a.dim == 3) {
+        return a.N * a.C <= 48 ? CrowdedTile{1920, 48} : CrowdedTile{6144, 72};
+    }
+    return {a.C > 8 ? 3072u : 5120u, a.pad == 1 ? any : 48u};
+}
 
 struct TilesParams {
     int32_t C, D, H, W, points;
@@ -46,12 +83,17 @@ struct TilesParams {
     int32_t blocks;  // of points
     FastDiv by_tiles_x, by_tiles_y, by_tiles, by_blocks, by_item;  // the last: workgroups of the gather kernel per item
     TilesLayout lay;
+    // crowded tiles: which, how many there can be in the launch, and where in scratch their list is (how many there are, then
+    // item << kTileBits | tile of each)
+    CrowdedTile crowded;
+    uint32_t list_most, list;
 };
 
 struct TilesPlan {
     bool ok = false;
     TilesParams p{};
     int64_t group = 0;  // items run at a time
+    int64_t words = 0;  // of scratch
     int64_t cblocks = 0;
     int32_t chans_per_block = 0;
     int cb = 1;         // channels of a point in LDS together
@@ -60,7 +102,10 @@ struct TilesPlan {
 
 constexpr int64_t kTilesFewGroups = 256;     // workgroups: one per CU
 constexpr int64_t kTilesMost = 2048;         // per item: counts and masks of every tile in LDS (96 KiB)
+constexpr int kTileBits = 11;
 constexpr int64_t kTileBlocksMost = 2047;    // per item: segments of a tile in LDS (16 KiB), counts of 11 and 21 bits
+
+constexpr int kCrowdedGroups = 1024;   // workgroups of that launch at most: with no tile on the list they cost it 2 us
 
 template <int DIM>
 inline TilesPlan tiles_plan_of(const GradGatherArgs& a)
@@ -109,6 +154,10 @@ inline TilesPlan tiles_plan_of(const GradGatherArgs& a)
     pl.group = (a.N + (a.N + group - 1) / group - 1) / ((a.N + group - 1) / group);  // as many items in every group
     p.N = (int32_t)pl.group;
     p.first_item = 0;
+    p.crowded = crowded_tile(a);
+    p.list_most = (uint32_t)(a.points > p.crowded.points || a.points > p.crowded.contributions ? pl.group * p.tiles : 0);
+    p.list = (uint32_t)(pl.group * p.lay.item_words);
+    pl.words = (int64_t)p.list + (p.list_most > 0 ? (int64_t)align4((uint64_t)p.list_most + 1u) : 0);
     pl.cb = (esz == 2 && a.C > 4 && DIM == 2) ? 8 : ((a.C > 3) ? 4 : (int)a.C);
     // fewer channels together where the tiles do not fill the chip
     while (pl.cb > 1 && pl.group * p.tiles * ((a.C + pl.cb - 1) / pl.cb) < kTilesFewGroups) {

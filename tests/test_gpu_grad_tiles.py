@@ -66,6 +66,40 @@ def test_planes(oracle, device, aclnn, dtype, pad, interp, xs, out, spots):
     _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid, rng)
 
 
+def _cropped(rng, n, out, part, spots):
+    """all points on `part` of every axis, some way off the middle, a little turned and jittered; some of them on one spot"""
+    axes = [(2 * np.arange(k) + 1) / k - 1 for k in out]
+    g = np.stack(np.meshgrid(*axes, indexing="ij")[::-1], axis=-1)
+    g[..., 0] += 0.2 * g[..., 1]
+    g = g[None] * part + rng.uniform(-0.4, 0.4, (n,) + (1,) * len(out) + (len(out),)) + rng.normal(0, 0.003, (n,) + out + (len(out),))
+    some = rng.random(g.shape[:-1]) < spots
+    g[some] = 0.3
+    return g
+
+
+# Tiles of many points, which another kernel takes in parts.  Elements with some contributions and with thousands; parts beyond
+# the edge of the plane; channels of one workgroup and of several; all points on few elements; chunks at a shift
+CROPPED = [((1, 3, 60, 64), (120, 131), 0.25, 0.0), ((2, 1, 20, 37), (93, 101), 0.4, 0.0), ((2, 11, 64, 64), (90, 90), 0.03, 0.1),
+           ((3, 2, 100, 90), (93, 96), 0.02, 0.0)]
+CROPPED_VOLUMES = [((1, 3, 13, 31, 33), (20, 28, 29), 0.2, 0.0), ((2, 1, 12, 24, 40), (19, 21, 30), 0.15, 0.0), ((1, 8, 30, 30, 30), (29, 28, 31), 0.1, 0.3),
+                   ((70, 1, 25, 17, 33), (18, 24, 23), 0.03, 0.1), ((1, 2, 32, 32, 32), (29, 30, 31), 0.01, 0.0)]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("interp", [0, 1])
+@pytest.mark.parametrize("xs,out,part,spots", CROPPED + CROPPED_VOLUMES)
+def test_crowded_tiles(oracle, device, aclnn, dtype, interp, xs, out, part, spots):
+    rng = np.random.default_rng(4580 + interp)
+    if interp == 1:
+        out = (2 * out[0],) + out[1:]  # of nearest samples a tile may have more points
+    grid = _cropped(rng, xs[0], out, part, spots)
+    assert host_plans.gradient_tiles(dtype, interp, 0, xs, int(np.prod(out)), 1 if xs[0] < 64 else 2) is not None
+    edges, limit = ((32, 16), (5120, 12288)) if len(out) == 2 else ((16, 8, 4), (1920, 10240))
+    tile = ((grid + 1) * np.array(xs[:1:-1]) - 1) / 2 // np.array(edges)
+    assert any(np.unique(t.reshape(-1, len(out)), axis=0, return_counts=True)[1].max() > limit[interp] for t in tile)
+    _check(aclnn, oracle, device, dtype, interp, 0, xs, out, grid, rng)
+
+
 # tiles of 16 x 8 x 4; the last two: more items than the reference device has cores, so that the chunks of every other item,
 # and with them its blocks of points, start at a shift
 VOLUMES = [((1, 1, 4, 8, 16), (8, 8, 9), 0.0), ((2, 3, 5, 9, 17), (8, 9, 12), 0.0), ((1, 4, 9, 17, 33), (9, 17, 33), 0.0),

@@ -201,9 +201,31 @@ inline TilesPlan tiles_plan_of(const GradGatherArgs& a)
 // 157).
 // Nor for many channels of volumes (12x31x18x62x20 142 / 159, 3x26x27x18x31 42 / 46; nearest 23x10x28x67x49 114 / 130,
 // 5x28x9x71x45 35 / 39; 7x19x30x20x91 175 / 151, nearest 9x6x52x46x37 67 / 55).
+// Not in planes and volumes of many tiles: every block of points clears, sums and writes a count per tile, and from 1706 tiles
+// on a CU has room for one workgroup of that kernel.  fp32 4x3x720x1280 (1800 tiles) 158 / 220, reflection 168 / 269, nearest
+// 113 / 166, 8x3x720x1280 323 / 428, 1x3x720x1280 58 / 66, 1x1x1024x1024 62 / 67, 4x3x1024x1024 -> 512x512 114 / 118; volumes
+// 4x4x64x128x128 (2048) 300 / 461, 1x4 96 / 122.  One item of few points is faster by tiles: 1x1x1024x1024 -> 512x512 44 / 30.
+// Below 1706, planes: one item 1x3x704x1152 (1584) 54 / 50, reflection (whose points lie closer at the edges) 60 / 62,
+// 1x1x640x1120 (1400) 47 / 51; several 4x3x640x1120 125 / 129, nearest 90 / 101, reflection 133 / 157; 4x3x608x1024 (1216) 116 /
+// 114, nearest 84 / 87, reflection 131 / 139; 4x3x600x800 (950) 99 / 77, reflection 107 / 99.  Volumes: 4x4x48x112x128 (1344) 198 /
+// 173, reflection 272 / 242.
+inline bool many_tiles(const GradGatherArgs& a)
+{
+    const int64_t elements = a.D * a.H * a.W;
+    const int64_t tiles = a.dim == 3 ? ((a.W + 15) / 16) * ((a.H + 7) / 8) * ((a.D + 3) / 4) : ((a.W + 31) / 32) * ((a.H + 15) / 16);
+    if (a.N == 1 && 2 * a.points <= elements) {
+        return false;
+    }
+    const int64_t items = (a.dim == 2 && a.N > 1) ? 5 : 4, edges = (a.dim == 2 && a.pad == 2) ? 5 : 4;
+    return tiles * items * edges > 1706 * 16;
+}
+
 inline bool tiles_are_faster(const GradGatherArgs& a)
 {
     const int64_t elements = a.D * a.H * a.W;
+    if (many_tiles(a)) {
+        return false;
+    }
     if (a.dim == 3) {
         return a.interp == 1 ? a.C <= 8 : (a.C <= 24 && 4 * a.points <= 5 * elements);
     }

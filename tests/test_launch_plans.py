@@ -143,7 +143,15 @@ TILES = [("fp32", 0, 0, (8, 3, 479, 637), 479 * 637, 178, 86), ("fp16", 0, 2, (1
          ("bf16", 0, 0, (2, 5, 96, 192), 162 * 324, 31, 40), ("bf16", 0, 2, (6, 12, 136, 184), 115 * 156, 47, 34),
          ("bf16", 0, 0, (13, 5, 27, 47, 57), 27 * 47 * 57, 108, 86), ("fp32", 0, 2, (1, 12, 9, 81, 64), 13 * 117 * 93, 130, 237),
          ("bf16", 0, 2, (12, 31, 18, 62, 20), 18 * 62 * 20, 142, 159), ("fp16", 1, 2, (23, 10, 28, 67, 49), 28 * 67 * 49, 114, 130),
-         ("fp32", 1, 0, (10, 2, 14, 26, 17), 14 * 26 * 17, 24, 15)]
+         ("fp32", 1, 0, (10, 2, 14, 26, 17), 14 * 26 * 17, 24, 15),
+         # many tiles
+         ("fp32", 0, 0, (8, 3, 720, 1280), 720 * 1280, 323, 428), ("fp32", 1, 0, (4, 3, 720, 1280), 720 * 1280, 113, 166),
+         ("fp32", 0, 0, (1, 3, 720, 1280), 720 * 1280, 58, 66), ("fp32", 0, 0, (1, 1, 1024, 1024), 512 * 512, 44, 30),
+         ("fp32", 0, 0, (4, 3, 1024, 1024), 512 * 512, 114, 118), ("fp32", 0, 0, (1, 3, 704, 1152), 704 * 1152, 54, 50),
+         ("fp32", 0, 2, (1, 3, 704, 1152), 704 * 1152, 60, 62), ("fp32", 0, 0, (4, 3, 640, 1120), 640 * 1120, 125, 129),
+         ("fp32", 0, 0, (4, 3, 608, 1024), 608 * 1024, 116, 114), ("fp32", 0, 2, (4, 3, 608, 1024), 608 * 1024, 131, 139),
+         ("fp32", 0, 2, (4, 3, 600, 800), 600 * 800, 107, 99), ("fp32", 0, 0, (4, 4, 64, 128, 128), 64 * 128 * 128, 300, 461),
+         ("fp32", 0, 2, (4, 4, 48, 112, 128), 48 * 112 * 128, 272, 242)]
 
 
 @pytest.mark.parametrize("dtype,interp,pad,shape,points,lists,tiles", TILES)
@@ -157,8 +165,8 @@ def test_gradient_tiles_fit_lds_and_the_launch():
     assert P.gradient_tiles("fp32", 0, 0, (1, 1, 16 * 2048 + 1, 32), 2000) is None
     assert P.gradient_tiles("fp32", 0, 0, (1, 1, 4 * 32, 8 * 8, 16 * 8), 2000)[2] == 2048
     assert P.gradient_tiles("fp32", 0, 0, (1, 1, 4 * 32 + 1, 8 * 8, 16 * 8), 2000) is None
-    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 1024, 1024), 2047 * 1024)[3] == 2047
-    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 1024, 1024), 2047 * 1024 + 1) is None
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 832, 1024), 2047 * 1024)[3] == 2047
+    assert P.gradient_tiles("fp32", 0, 0, (1, 1, 832, 1024), 2047 * 1024 + 1) is None
     assert P.gradient_tiles("fp32", 0, 0, (128, 1, 9, 20, 21), 3 * 1024, 2)[3] == 4
     assert P.gradient_tiles("fp32", 0, 0, (128, 1, 9, 20, 21), 3 * 1024, 1)[3] == 3
     # bicubic samples have no tiles

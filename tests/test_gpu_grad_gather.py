@@ -107,12 +107,21 @@ def test_volumes(oracle, device, aclnn, dtype, interp, pad):
         assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref)), (xs, out, span)
 
 
-@pytest.mark.parametrize("interp,n,out", [(0, 45, (480, 641)), (2, 9, (500, 641))])
-def test_planes_in_groups_of_items(device, aclnn, interp, n, out):
-    """a batch whose items are run a group at a time, against its items one by one"""
+def _group(dtype, interp, pad, xs, points, tiles, per_core=1):
+    """items that the variant which takes the call runs at a time"""
+    by_tiles = host_plans.gradient_tiles(dtype, interp, pad, xs, points, per_core)
+    assert (by_tiles is not None) == tiles
+    return (by_tiles if tiles else host_plans.gather_groups(dtype, interp, xs, points))[0]
+
+
+# by lists, which take planes of more tiles than gs_grad_tiles.hip does, and bicubic samples; by tiles
+@pytest.mark.parametrize("interp,n,plane,out,tiles", [(0, 13, (1100, 1000), (1090, 1001), False), (2, 9, (480, 641), (500, 641), False),
+                                                      (0, 85, (480, 641), (500, 641), True), (1, 97, (700, 700), (701, 699), True)])
+def test_planes_in_groups_of_items(device, aclnn, interp, n, plane, out, tiles):
+    """a batch whose items are run a group at a time, the last group a shorter one, against its items one by one"""
     import torch
-    xs = (n, 1, 480, 641)
-    group, _ = host_plans.gather_groups("fp16", interp, xs, out[0] * out[1])
+    xs = (n, 1) + plane
+    group = _group("fp16", interp, 1, xs, out[0] * out[1], tiles)
     assert group < n and n % group != 0
     g = torch.Generator(device=device).manual_seed(4)
     x = torch.randn(xs, generator=g, device=device).half()
@@ -124,16 +133,17 @@ def test_planes_in_groups_of_items(device, aclnn, interp, n, out):
         assert torch.equal(one[0], got[i]), i
 
 
-def test_volumes_in_groups_of_items(device, aclnn):
+@pytest.mark.parametrize("xs,out,tiles", [((299, 1, 9, 20, 21), (39, 32, 31), False), ((129, 1, 25, 70, 75), (25, 69, 77), True)])
+def test_volumes_in_groups_of_items(device, aclnn, xs, out, tiles):
     """the chunks of a volume start at a shift that its number in the batch gives, whatever group it is run in"""
     import torch
-    xs, out = (300, 1, 9, 20, 21), (39, 32, 31)
-    group, _ = host_plans.gather_groups("fp32", 0, xs, out[0] * out[1] * out[2])
-    assert group < 300 and out[0] * out[1] * out[2] % 256 != 0
+    n, points = xs[0], out[0] * out[1] * out[2]
+    group = _group("fp32", 0, 0, xs, points, tiles, (n + 63) // 64)
+    assert group < n and n % group != 0 and points % 256 != 0
     g = torch.Generator(device=device).manual_seed(5)
     x = torch.randn(xs, generator=g, device=device)
-    go = torch.randn((300, 1) + out, generator=g, device=device)
-    grid = torch.rand((300,) + out + (3,), generator=g, device=device) * 2.2 - 1.1
+    go = torch.randn((n, 1) + out, generator=g, device=device)
+    grid = torch.rand((n,) + out + (3,), generator=g, device=device) * 2.2 - 1.1
     grads = []
     for variant in (1, 3):
         with aclnn.option("gs3d_grad_variant", variant):
@@ -141,14 +151,16 @@ def test_volumes_in_groups_of_items(device, aclnn):
     assert torch.equal(*grads)
 
 
-def test_groups_of_items_in_a_graph(device, aclnn):
+@pytest.mark.parametrize("n,plane,tiles", [(13, (1100, 1000), False), (85, (480, 641), True)])
+def test_groups_of_items_in_a_graph(device, aclnn, n, plane, tiles):
     """replays of a captured call whose groups share their scratch, with eager work between them"""
     import torch
-    xs, out = (45, 1, 480, 641), (480, 641)
-    assert host_plans.gather_groups("fp16", 0, xs, out[0] * out[1])[0] < 45
+    xs, out = (n, 1) + plane, plane
+    group = _group("fp16", 0, 0, xs, out[0] * out[1], tiles)
+    assert group < n and n % group != 0
     g = torch.Generator(device=device).manual_seed(6)
     x, go = (torch.randn(xs, generator=g, device=device).half() for _ in range(2))
-    grid = torch.empty((45,) + out + (2,), dtype=torch.float16, device=device)
+    grid = torch.empty((n,) + out + (2,), dtype=torch.float16, device=device)
     dx, dg = torch.empty_like(x), torch.empty_like(grid)
     grids = [(torch.rand(grid.shape, generator=g, device=device) * 2.4 - 1.2).half() for _ in range(3)]
     want = [aclnn.grid_sampler2d_backward(go, x, v) for v in grids]

@@ -66,6 +66,19 @@ def test_planes(oracle, device, aclnn, dtype, pad, interp, xs, out, spots):
     _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid, rng)
 
 
+# the most tiles, and the most blocks of points, that are taken: counts of all tiles in more than 64 KiB of LDS, and a tile's
+# segments found 512 blocks at a time
+@pytest.mark.parametrize("interp", [0, 1])
+@pytest.mark.parametrize("dtype,xs,out,plan", [("fp32", (1, 1, 1024, 1024), (700, 700), (2048, 479)),
+                                               ("fp16", (1, 1, 832, 1024), (1447, 1448), (1664, 2047))])
+def test_large_planes(oracle, device, aclnn, interp, dtype, xs, out, plan):
+    rng = np.random.default_rng(4550 + interp)
+    points = out[0] * out[1]
+    assert host_plans.sorting_takes_planes(dtype, interp, xs, points) is not None
+    assert host_plans.gradient_tiles(dtype, interp, 0, xs, points)[2:4] == plan
+    _check(aclnn, oracle, device, dtype, interp, 0, xs, out, I.affine_grid(rng, 1, *out), rng)
+
+
 def _cropped(rng, n, out, part, spots):
     """all points on `part` of every axis, some way off the middle, a little turned and jittered; some of them on one spot"""
     axes = [(2 * np.arange(k) + 1) / k - 1 for k in out]

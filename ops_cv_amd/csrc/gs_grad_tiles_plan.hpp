@@ -145,10 +145,6 @@ inline TilesPlan tiles_plan_of(const GradGatherArgs& a)
     p.lay.segments = 0;
     p.lay.records = align4((uint64_t)(blocks * p.tiles));
     p.lay.item_words = p.lay.records + (uint32_t)blocks * p.lay.block_words;
-    if (DIM == 3 && (int64_t)p.lay.item_words < 5 * a.points) {
-        // by the size of its workspace, 20 bytes and more a point, phase 1 of a volume's backward says that it sorts, whichever way
-        p.lay.item_words = align4((uint64_t)(5 * a.points));
-    }
     const int64_t fit = kGatherGroupScratch / ((int64_t)p.lay.item_words * 4);
     const int64_t group = fit < 1 ? 1 : (fit < a.N ? fit : a.N);
     pl.group = (a.N + (a.N + group - 1) / group - 1) / ((a.N + group - 1) / group);  // as many items in every group

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "fast_div.hpp"
 #include "gs2d_grad_math.hpp"
 #include "gs3d_grad_math.hpp"
 
@@ -93,14 +94,31 @@ __device__ __forceinline__ float value_of(float go, float w)
 
 // Work of a launch cut into `per_item` pieces per batch item, dealt out so that neighbouring pieces run on one XCD
 // (workgroups go to the eight XCDs in turn): XCD k takes the k-th eighth of all pieces.  Pieces beyond the last: false.
+__device__ __forceinline__ bool piece_of_block(uint32_t block, uint32_t pieces, uint32_t* piece)
+{
+    const uint32_t per_xcd = (pieces + 7u) >> 3;
+    *piece = (block & 7u) * per_xcd + (block >> 3);
+    return (block >> 3) < per_xcd && *piece < pieces;
+}
+
 __device__ __forceinline__ bool piece_of_block(uint32_t block, uint32_t pieces, uint32_t per_item, uint32_t* n,
                                                uint32_t* local)
 {
-    const uint32_t per_xcd = (pieces + 7u) >> 3;
-    const uint32_t piece = (block & 7u) * per_xcd + (block >> 3);
+    uint32_t piece;
+    const bool have = piece_of_block(block, pieces, &piece);
     *n = piece / per_item;
     *local = piece - *n * per_item;
-    return (block >> 3) < per_xcd && piece < pieces;
+    return have;
+}
+
+__device__ __forceinline__ bool piece_of_block(uint32_t block, uint32_t pieces, const FastDiv& per_item, uint32_t* n,
+                                               uint32_t* local)
+{
+    uint32_t piece;
+    const bool have = piece_of_block(block, pieces, &piece);
+    *n = fast_div(piece, per_item);
+    *local = piece - *n * per_item.div;
+    return have;
 }
 
 }  // namespace opscv

@@ -15,17 +15,20 @@
 //           wavefront; more points than LDS holds are taken a run of segments after the other, which are whole chunks
 //           in ascending order.  Tiles that many points fall on are left to a third kernel (gs_grad_tiles_crowded.hip).
 //
-// Every operand is read once and a point's gradOutput once per tile that it reaches; all that is scattered happens in LDS.
+// The grid is read here and there, by the gather once per tile that a point reaches and block of channels, gradOutput once per
+// tile that a point reaches; all that is scattered happens in LDS.
 //
 // fp32 8x3x479x637 from as many points (rotations of up to 30 degrees), operands from memory: lists through global memory
-// (gs_grad_gather.hip) 188 us in six kernels, here bin 21 and gather 71.  Bin: 34 us with an LDS atomic a point, which the
+// (gs_grad_gather.hip) 188 us in six kernels, here bin 21, gather 73 and 4.6 for a list of crowded tiles that is empty (bin 19
+// and gather 69 before there was one: where a point lies in its tile, and scalar registers that the way out takes).  Bin: 34 us with an LDS atomic a point, which the
 // 64 lanes of a wavefront on one tile take in turn, 20 with a run of lanes entered at once.  Gather is bound by its chain of
-// steps, not by a unit: 450 vector and 350 scalar instructions a wavefront (28 us of issue), and seven waits for memory or
-// the other wavefronts (segments, records, points; counts, starts, lists, keys) at two workgroups per CU.  Without fetching,
+// steps, not by a unit: 550 vector, 400 scalar and 49 LDS instructions a wavefront (34 us of issue), and seven waits for memory
+// or the other wavefronts (segments, records, points; counts, starts, lists, keys) at two workgroups per CU.  Without fetching,
 // sorting and folding keys it takes 47 us, without gradOutput 63, without stores 64; three workgroups per CU (80 registers)
 // are no faster, tiles of 32 x 8 take 92 us (and bin 61), half as many points a round 97.  Weights in LDS instead of
 // coordinates took 82 to 80 us, loads of all of a lane's points together and divisions by multiplication 74, a reflection's
-// constants out of the other paddings' way 69.
+// constants out of the other paddings' way 69.  Volumes of four channels, linear, need more than the 128 registers that two
+// workgroups per CU leave: 40 bytes of scratch a lane in fp32.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -64,7 +67,7 @@ __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __re
         ws[p.list] = 0u;  // for the gather kernel
     }
     uint32_t n, block;
-    if (!piece_of(blockIdx.x, pieces, p.by_blocks, &n, &block)) {
+    if (!piece_of_block(blockIdx.x, pieces, p.by_blocks, &n, &block)) {
         return;
     }
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
@@ -356,7 +359,7 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
     __shared__ uint32_t s_longs, s_crowded, s_sorted_used;
     extern __shared__ uint32_t s_seg[];  // per segment that is not empty: points before it; block << 14 | first record
     uint32_t n, local;
-    if (!piece_of(blockIdx.x, pieces, p.by_item, &n, &local)) {
+    if (!piece_of_block(blockIdx.x, pieces, p.by_item, &n, &local)) {
         return;
     }
     const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -997,7 +1000,7 @@ hipError_t run_channels(const GradGatherArgs& a, const TilesPlan& pl, hipStream_
         case 4: return launch_tiles<T, DIM, INTERP, 4>(a, pl, stream);
         default: break;
     }
-    if constexpr (sizeof(T) == 2) {
+    if constexpr (sizeof(T) == 2 && DIM == 2) {
         return launch_tiles<T, DIM, INTERP, 8>(a, pl, stream);
     }
     return hipErrorInvalidValue;

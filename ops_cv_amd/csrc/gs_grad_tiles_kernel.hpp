@@ -59,16 +59,6 @@ __device__ __forceinline__ bool low_corner(const Coords<T, DIM>& c, const TilesP
     return in;
 }
 
-// workgroups go to the eight XCDs in turn: XCD k takes the k-th eighth of all pieces, so that neighbours share an L2
-__device__ __forceinline__ bool piece_of(uint32_t block, uint32_t pieces, const FastDiv& per_item, uint32_t* n, uint32_t* local)
-{
-    const uint32_t per_xcd = (pieces + 7u) >> 3;
-    const uint32_t piece = (block & 7u) * per_xcd + (block >> 3);
-    *n = fast_div(piece, per_item);
-    *local = piece - *n * per_item.div;
-    return (block >> 3) < per_xcd && piece < pieces;
-}
-
 // Sums of the wavefronts before this one, and of all, from every wavefront's in LDS.
 template <int WAVES>
 __device__ __forceinline__ uint32_t sums_before(const uint32_t* s_scan, int wave, int lane, uint32_t* all)

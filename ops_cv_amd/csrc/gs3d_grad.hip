@@ -475,7 +475,9 @@ int64_t gs3d_grad_gather_words(const GridSampler3DGradArgs& a)
         return 0;
     }
     const int64_t points = a.Dout * a.Hout * a.Wout, vol = a.Din * a.Hin * a.Win;
-    // Device time of a call with both gradients, fp16 or fp32, four channels: ordered kernel / slots / sorting variant.
+    // Device time of a call with both gradients, fp16 or fp32, four channels: ordered kernel / slots / sorting variant, by lists
+    // (gs_grad_gather.hip).  By tiles (gs_grad_tiles.hip), which take most of these calls now, sorting is up to twice as fast:
+    // the lines lie on the side of the other two.
     // Volumes sampled at few points: the sorting variant visits every voxel, the ordered kernel every chunk of points
     // (vol : points 22 : 1 with 46080 points 77 / - / 71 us, 32 : 1 with 8192 points 60 / - / 95, 128 : 1 with 16384
     // points 67 / - / 102; 16 : 1 with 16384 points 39 / - / 34).  Beyond 65536 points the slots kernels do not run and a chunk of the ordered kernel costs

@@ -186,7 +186,9 @@ inline PlaneGradTimes plane_grad_times(const GradGatherArgs& a)
     return t;
 }
 
-// Whether the sorting variant takes the input gradient of planes (where the list variant does not).
+// Whether the sorting variant takes the input gradient of planes (where the list variant does not).  The rates above and the
+// figures below are of sorting by lists (gs_grad_gather.hip).  Where the tiles of gs_grad_tiles.hip take the call sorting is up
+// to twice as fast, so the lines lie on the elections' side there: some calls near them would be faster sorted.
 //
 // Up to 24 tap passes over a chunk (6 chunks bilinear, 24 nearest, 1 bicubic) the elections take 10 to 30 us and sorting as
 // much or more.  Sorting against elections over grids and planes of up to eight items, medians: bilinear 5 and 6 chunks

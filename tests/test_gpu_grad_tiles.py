@@ -100,17 +100,50 @@ CROPPED_VOLUMES = [((1, 3, 13, 31, 33), (20, 28, 29), 0.2, 0.0), ((2, 1, 12, 24,
 
 @pytest.mark.parametrize("dtype", I.DTYPES)
 @pytest.mark.parametrize("interp", [0, 1])
+@pytest.mark.parametrize("pad", [0, 2])
 @pytest.mark.parametrize("xs,out,part,spots", CROPPED + CROPPED_VOLUMES)
-def test_crowded_tiles(oracle, device, aclnn, dtype, interp, xs, out, part, spots):
+def test_crowded_tiles(oracle, device, aclnn, dtype, interp, pad, xs, out, part, spots):
     rng = np.random.default_rng(4580 + interp)
     if interp == 1:
         out = (2 * out[0],) + out[1:]  # of nearest samples a tile may have more points
     grid = _cropped(rng, xs[0], out, part, spots)
-    assert host_plans.gradient_tiles(dtype, interp, 0, xs, int(np.prod(out)), 1 if xs[0] < 64 else 2) is not None
+    assert host_plans.gradient_tiles(dtype, interp, pad, xs, int(np.prod(out)), 1 if xs[0] < 64 else 2) is not None
     edges, limit = ((32, 16), (5120, 12288)) if len(out) == 2 else ((16, 8, 4), (1920, 10240))
     tile = ((grid + 1) * np.array(xs[:1:-1]) - 1) / 2 // np.array(edges)
     assert any(np.unique(t.reshape(-1, len(out)), axis=0, return_counts=True)[1].max() > limit[interp] for t in tile)
-    _check(aclnn, oracle, device, dtype, interp, 0, xs, out, grid, rng)
+    _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid, rng)
+
+
+@pytest.mark.parametrize("n,plane", [(3, (100, 120)), (420, (240, 321))])  # the last: two groups of items, one list after the other
+def test_crowded_tiles_in_a_graph(device, aclnn, n, plane):
+    """replays of a captured call on grids with crowded tiles and without, with eager work between them"""
+    import torch
+    rng = np.random.default_rng(4590)
+    xs, points = (n, 1) + plane, plane[0] * plane[1]
+    group = host_plans.gradient_tiles("fp16", 0, 0, xs, points)[0]
+    assert (group < n) == (n == 420) and host_plans.sorting_takes_planes("fp16", 0, xs, points) is not None
+    x, go = (torch.from_numpy(rng.standard_normal(xs).astype(np.float16)).to(device) for _ in range(2))
+    base = [_cropped(rng, 3, plane, part, 0.0) for part in (0.2, 1.0, 0.05)]
+    grids = [torch.from_numpy(g.astype(np.float16)).to(device).repeat(n // 3, 1, 1, 1).contiguous() for g in base]
+    want = [aclnn.grid_sampler2d_backward(go, x, g)[0] for g in grids]
+    grid, dx, dg = grids[0].clone(), torch.empty_like(x), torch.empty_like(grids[0])
+    one, _ = aclnn.grid_sampler2d_backward(go[n - 1:], x[n - 1:], grids[0][n - 1:])
+    assert torch.equal(one[0], want[0][n - 1])
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(s):
+        aclnn.grid_sampler2d_backward(go, x, grid, input_grad=dx, grid_grad=dg)
+        s.synchronize()
+        with torch.cuda.graph(graph, stream=s):
+            aclnn.grid_sampler2d_backward(go, x, grid, input_grad=dx, grid_grad=dg)
+    torch.cuda.synchronize()
+    for i in (0, 1, 2, 1, 0):
+        grid.copy_(grids[i])
+        dx.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(dx, want[i]), i
 
 
 # tiles of 16 x 8 x 4; the last two: more items than the reference device has cores, so that the chunks of every other item,

@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "kernels.hpp"
+#include "resize_grad_math.hpp"
 #include "resize_grad_plan.hpp"
 #include "sampler_math.hpp"
 
@@ -182,32 +183,6 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_kernel(const TI* __r
 // copied into LDS with independent 4-byte loads -- all in flight together, where the gather variant waits for one
 // two-byte load per visit -- and the lanes then run the unchanged visiting loops on LDS.  A rectangle that does not
 // fit the LDS capacity is read from global memory instead (same loops, same result).
-// The visiting loops of resize_grad_kernel over a row-major array whose element (y0, x0) is base[0].
-template <typename TI>
-__device__ __forceinline__ float visit_sum(const TI* base, int32_t pitch, int32_t y0, int32_t x0, int32_t in_y_start,
-                                           int32_t in_x_start, float out_y_start, float out_x_start, float fh,
-                                           float fw, float scale_h, float scale_w, float last_y, float last_x,
-                                           int32_t Hd, int32_t Wd, int32_t ci = 1, int32_t ch = 0)
-{
-    // ci, ch: channels-last rows hold ci elements per pixel, this lane's channel is ch (x0 counts elements)
-    float acc = 0.0f;
-    float out_y = out_y_start;
-    for (int32_t in_y = in_y_start; out_y < fh + 1.0f && in_y < Hd; in_y++) {
-        const float yc = __builtin_fmaxf(0.0f, __builtin_fminf(out_y, last_y));
-        const float y_lerp = 1.0f - __builtin_fabsf(yc - fh);
-        const TI* row = base + (int64_t)(in_y - y0) * pitch;
-        float out_x = out_x_start;
-        for (int32_t in_x = in_x_start; out_x < fw + 1.0f && in_x < Wd; in_x++) {
-            const float xc = __builtin_fmaxf(0.0f, __builtin_fminf(out_x, last_x));
-            const float x_lerp = 1.0f - __builtin_fabsf(xc - fw);
-            acc += ElemIO<TI>::load(row + ((int64_t)in_x * ci + ch - x0)) * y_lerp * x_lerp;
-            out_x += scale_w;
-        }
-        out_y += scale_h;
-    }
-    return acc;
-}
-
 // The same sum with the column part of the loop taken out: a lane keeps the weights of the (at most KX) columns it
 // visits -- computed once, by the same repeated additions -- and a row costs one LDS read, two products and an add
 // per column.  Column k of a lane with fewer than k + 1 visits leaves the sum alone.
@@ -512,8 +487,8 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
     }
 }
 
-// Planes whose elements grow by up to four a side (at most eight visited rows and columns): the rectangle stays in the
-// element type and comes by asynchronous copies.
+// Planes whose elements grow by up to four a side (at most eight visited rows and columns) and that resize_grad_rows.hip leaves
+// (planes of 1 GiB, 2^18 rows): the rectangle stays in the element type and comes by asynchronous copies.
 //
 // A workgroup owns 64 outgoing columns by 16 or 8 outgoing rows, a wavefront every fourth of the rows.  The row segments
 // the tile visits are copied from the 16-byte boundary before their first byte to the one after their last (the bytes
@@ -561,15 +536,6 @@ __device__ __forceinline__ void weighted_columns(const char* lds, uint32_t off, 
             }
         }
     }
-}
-
-template <bool HALF_PIXEL>
-__device__ __forceinline__ int32_t first_visited(int32_t i, float inv_scale, int32_t len_dst)
-{
-    const float offset = HALF_PIXEL ? 0.5f : 0.0f;
-    const float f = __builtin_ceilf(((float)i - 1.0f + offset) * inv_scale - offset);
-    // a start at or beyond the end visits nothing, whatever its exact value
-    return (f > 0.0f) ? ((f < (float)len_dst) ? (int32_t)f : len_dst) : 0;
 }
 
 // Element e of the columns past the last whole tile, all planes' one after the other: a lane each, straight from memory, the
@@ -845,6 +811,10 @@ hipError_t run_planes(const ResizeGradArgs& a, const PlaneTile& t, hipStream_t s
 template <typename TI, typename TO>
 hipError_t run(const ResizeGradArgs& a, hipStream_t stream)
 {
+    const RowsPlan rows = rows_plan(a);
+    if (rows.ok) {
+        return run_resize_grad_rows(a, rows, stream);
+    }
     const PlaneTile planes_tile = plane_tile(a);
     if (planes_tile.rows > 0) {
         return run_planes<TI, TO>(a, planes_tile, stream);

@@ -4,6 +4,7 @@
 #include <cstdint>
 
 #include "acl_types.hpp"
+#include "fast_div.hpp"
 #include "launch_limits.hpp"
 
 namespace opscv {
@@ -151,6 +152,77 @@ inline PlaneTile plane_tile(const ResizeGradArgs& a)
         t = fits_launch(s.blocks, kGradThreads) ? s : t;
     }
     return t;
+}
+
+// ---- resize_grad_rows_kernel ----
+constexpr int kRowsColumns = 10;         // most columns, and most rows, an outgoing element may visit
+constexpr float kRowsLeastScale = 0.2f;  // 2 / scale columns and rows
+
+constexpr int64_t kRowsMost = 1 << 18;    // outgoing rows: single precision tells which of them visit a row, but for neighbours
+
+struct RowsPlan {
+    bool ok = false;
+    uint32_t columns = 0;  // of all planes, side by side
+    FastDiv by_ws, by_groups;
+    bool two = false;      // a row of a wavefront's columns may have more than 64 units of 16 bytes
+    bool tall = false;     // an element may visit more than eight rows
+    int32_t rows = 0;      // outgoing rows of a wavefront
+    int64_t blocks = 0;    // padded for the XCD mapping of the kernel
+};
+
+// Taken wherever it can: growth by up to five, planes (rows from 2^18 on and planes of 1 GiB are left to the kernels above).
+// Against them, medians of three runs, device time in microseconds before / with it: bf16 8x64x65x129 from 257x513 58 / 44, fp32 81 / 57,
+// fp16 64x128 from 256x512 53 / 41; growth by two fp32 4x16x270x480 43 / 32, fp16 16x64x56x56 29 / 17, 4x16x1080x1920 437 / 415, bf16
+// 512x32x14x14 43 / 17; growth by 1.1 fp32 2000 planes of 82x424 315 / 164, fp16 182 / 143; shrunk by 0.5 120 / 104 and 30 / 29 (64
+// planes of 400x600), by 0.35 28 / 28.  Growth by four with aligned corners, where an element visits nine rows and columns, had no
+// kernel but the gather: fp16 85 planes of 539x108 206 / 54.8.  Over 260 random shapes (1 to 20000 planes of 2 to 1500 columns, growth by
+// 0.25 to 4) 1.57 times as fast, none slower by more than a microsecond.
+inline RowsPlan rows_plan(const ResizeGradArgs& a)
+{
+    RowsPlan r;
+    const int esz = elem_size(a.elem_in);
+    const int64_t planes = a.N * a.C;
+    if (a.user_scales || (a.channels_last && a.C != 1) || !(a.scale_h >= kRowsLeastScale) || !(a.scale_w >= kRowsLeastScale) ||
+        reinterpret_cast<uintptr_t>(a.x) % (uintptr_t)esz != 0 || planes <= 0 || a.Ws <= 0 || a.Hs <= 0 ||
+        planes > INT32_MAX / a.Ws || a.Hs > kRowsMost) {
+        return r;
+    }
+    // Few elements of planes of a column or two spend longer on finding their runs than the gather does on all of it.
+    if (a.Ws < 4 && planes * a.Hs * a.Ws < (int64_t)1 << 19) {
+        return r;
+    }
+    // a lane's plane lies up to that far behind the first lane's: 32 bits
+    const int64_t span = a.Ws >= 64 ? 2 : 63 / a.Ws + 2;
+    if (a.Hd * a.Wd > INT32_MAX / (span * esz)) {
+        return r;
+    }
+    // units of a row: of whole planes, or of a run that the end of a plane may cut
+    const int64_t units = a.Ws < 64 ? (a.Wd * esz + 30) / 16 * (64 % a.Ws == 0 ? 64 / a.Ws : span)
+                                    : (int64_t)((64.0 / a.scale_w + 12.0) * esz + 60.0) / 16;
+    if (units > 128) {
+        return r;
+    }
+    r.two = units > 64;
+    r.columns = (uint32_t)(planes * a.Ws);
+    r.by_ws = make_fast_div((uint32_t)a.Ws);
+    const int64_t tiles = ((int64_t)r.columns + kGradThreads - 1) / kGradThreads;
+    r.tall = a.scale_h < 0.2501f;
+    r.rows = 8;
+    while (r.rows > 2 && tiles * ((a.Hs + r.rows - 1) / r.rows) < 512) {
+        r.rows /= 2;
+    }
+    // Rows of a wavefront: few enough to fill the chip, as many as leave its workgroups turns to even out (64 and 18 rows of 82
+    // took 155 us where 41 and 41 take 104), more of them where a row is soon done (64 planes of 400x600 by 0.5 31 / 29)
+    const int64_t enough = a.scale_h > 1.2f ? 1536 : 4096;
+    while (r.rows < 64 && r.rows < a.Hs && tiles * ((a.Hs + 2 * r.rows - 1) / (2 * r.rows)) >= enough) {
+        r.rows *= 2;
+    }
+    const int64_t groups = (a.Hs + r.rows - 1) / r.rows;
+    r.rows = (int32_t)((a.Hs + groups - 1) / groups);
+    r.by_groups = make_fast_div((uint32_t)groups);
+    r.blocks = (tiles * groups + 7) / 8 * 8;
+    r.ok = fits_launch(r.blocks, kGradThreads);
+    return r;
 }
 
 }  // namespace opscv

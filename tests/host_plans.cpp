@@ -33,7 +33,7 @@ int direct_tiles(int elem, int64_t N, int64_t C, int64_t Hin, int64_t Win, int64
 
 // tile rows, workgroups, planes a workgroup walks at most; 0 where the planes kernel is not taken.  Gradient of (Hs, Ws)
 // from (Hd, Wd), dense planes on a 16-byte boundary.
-int resize_grad_planes(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int align, int64_t* out)
+static ResizeGradArgs resize_grad_args(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int align)
 {
     ResizeGradArgs a;
     a.elem_in = a.elem_out = (Elem)elem;
@@ -49,11 +49,27 @@ int resize_grad_planes(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t
     };
     a.scale_h = scale(Hs, Hd);
     a.scale_w = scale(Ws, Wd);
-    const PlaneTile t = plane_tile(a);
+    return a;
+}
+
+int resize_grad_planes(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int align, int64_t* out)
+{
+    const PlaneTile t = plane_tile(resize_grad_args(elem, planes, Hs, Ws, Hd, Wd, align));
     out[0] = t.rows;
     out[1] = t.blocks;
     out[2] = (planes + t.slots - 1) / (t.slots > 0 ? t.slots : 1);
     return t.rows > 0 ? 1 : 0;
+}
+
+// rows of a wavefront, whether a lane moves two units of a row, whether an element may visit more than eight rows; 0 where the
+// rows kernel is not taken
+int resize_grad_rows(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int align, int64_t* out)
+{
+    const RowsPlan p = rows_plan(resize_grad_args(elem, planes, Hs, Ws, Hd, Wd, align));
+    out[0] = p.rows;
+    out[1] = p.two ? 1 : 0;
+    out[2] = p.tall ? 1 : 0;
+    return p.ok ? 1 : 0;
 }
 
 // estimates of the input gradient of planes (nanoseconds): elections, sorting; 0 where the elections run

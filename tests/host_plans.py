@@ -40,6 +40,12 @@ def resize_grad_planes(dtype, planes, small, large, align=False):
     return _call("resize_grad_planes", 3, dtype, planes, *small, *large, int(align))
 
 
+def resize_grad_rows(dtype, planes, small, large, align=False):
+    """(outgoing rows of a wavefront, whether a lane moves two units of a row, whether an element may visit more than eight
+    rows) of the resize gradient's rows kernel, None where it is not taken."""
+    return _call("resize_grad_rows", 3, dtype, planes, *small, *large, int(align))
+
+
 def sorting_takes_planes(dtype, interp, shape, points):
     """(elections, sorting): estimated nanoseconds of the input gradient of (N, C, H, W) planes sampled at `points` points
     an item, None where the elections run."""

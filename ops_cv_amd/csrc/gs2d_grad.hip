@@ -24,9 +24,9 @@
 #include <type_traits>
 
 #include "fast_div.hpp"
-#include "gs2d_grad_grid_plan.hpp"
 #include "gs2d_grad_math.hpp"
 #include "gs_grad_gather.hpp"
+#include "gs_grad_grid.hpp"
 #include "kernels.hpp"
 
 namespace opscv {
@@ -62,8 +62,6 @@ struct GradParams {
     int32_t pad, align;
     int32_t band_px;  // plane elements per workgroup (dx kernel)
     int32_t tags;     // election tags of the dx kernel, a power of two (tag_of)
-    uint32_t pieces;  // tiles of the grid kernel, and how they are numbered
-    FastDiv by_item, by_tiles_x;
 };
 
 // CB channels of one batch item per workgroup: the grid points, their taps and the election of a round are the
@@ -228,193 +226,12 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_input_kernel(const T* __re
     }
 }
 
-// One lane per grid point.  TILED: a workgroup takes 16 x 16 points of an item, a wavefront 16 x 4 of them, so that under a
-// turned grid the corners of its points share cache lines in both directions: 64 points of a row lie in up to 64 lines of a
-// plane.  XCD k takes the k-th eighth of the workgroups, so that neighbouring tiles share an L2.
-//
-// Bound by the lines that the gathers touch and their latency: the loads of up to eight channels are on their way together,
-// of fewer channels all of them (fp32 8x3x479x637, rotations of up to 30 degrees: 58 us in rows, a channel after the other;
-// 40 with the three channels' loads together; 33 in tiles).  Bicubic samples have the sixteen loads of a channel on their way
-// together, in rows (grid_tile_plan): turned grids, one load after the other / together, fp32 8x3x479x637 114 / 115 us, 2x64x128x128
-// 72 / 62, 8x128x32x32 114 / 116, fp16 134 / 108, 156 / 62, 190 / 101; points at random, whose lines are seldom in the cache, fp32
-// 393 / 395, 118 / 125, 108 / 117, fp16 373 / 370, 154 / 107, 188 / 115.
 template <typename T, int INTERP, bool TILED>
-__global__ __launch_bounds__(kThreads) void gs2d_grad_grid_kernel(const T* __restrict__ gout, const T* __restrict__ x,
-                                                                   const T* __restrict__ grid, T* __restrict__ dgrid,
-                                                                   int64_t total, GradParams p, int32_t blocks_per_item)
+__global__ __launch_bounds__(kGridTileThreads) void gs2d_grad_grid_kernel(const T* __restrict__ gout, const T* __restrict__ x,
+                                                                          const T* __restrict__ grid, T* __restrict__ dgrid,
+                                                                          Grid2Params p)
 {
-    using Taps = GradTaps<T, INTERP>;
-    const int32_t points = p.Ho * p.Wo;
-    int64_t n, idx;
-    int32_t pt;
-    if constexpr (TILED) {
-        const uint32_t per_xcd = p.pieces / 8u + (p.pieces % 8u != 0u ? 1u : 0u);
-        const uint32_t piece = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
-        if ((blockIdx.x >> 3) >= per_xcd || piece >= p.pieces) {
-            return;
-        }
-        const uint32_t item = fast_div(piece, p.by_item), tile = piece - item * p.by_item.div;
-        const uint32_t ty = fast_div(tile, p.by_tiles_x), tx = tile - ty * p.by_tiles_x.div;
-        const int32_t px = (int32_t)(tx * kGridTile + threadIdx.x % kGridTile);
-        const int32_t py = (int32_t)(ty * kGridTile + threadIdx.x / kGridTile);
-        if (px >= p.Wo || py >= p.Ho) {
-            return;
-        }
-        n = item;
-        pt = py * p.Wo + px;
-        idx = n * points + pt;
-    } else {
-        // blocks_per_item > 0: workgroups are handed to the 8 XCDs round-robin by index; all workgroups of one batch item
-        // go to one XCD, so that the planes of that item (every lane walks all of them) are fetched into one L2 once
-        // instead of into all eight (fp16 N16 C256 64x64: 185.6 MB fetched for 67.1 MB of operands otherwise).  The launch
-        // plan asks for it when the items divide evenly among the XCDs and the workgroups evenly among the items.
-        uint32_t block = blockIdx.x;
-        if (blocks_per_item > 0) {
-            const uint32_t xcd = blockIdx.x & 7u, i = blockIdx.x >> 3;
-            block = ((i / (uint32_t)blocks_per_item) * 8u + xcd) * (uint32_t)blocks_per_item + i % (uint32_t)blocks_per_item;
-        }
-        idx = (int64_t)block * kThreads + threadIdx.x;
-        if (idx >= total) {
-            return;
-        }
-        n = idx / points;
-        pt = (int32_t)(idx - n * points);
-    }
-    if (INTERP == 1) {
-        ElemIO<T>::store(dgrid + 2 * idx, 0.0f);
-        ElemIO<T>::store(dgrid + 2 * idx + 1, 0.0f);
-        return;
-    }
-    Taps tp;
-    decide_grad_taps<T, INTERP>(tp, ElemIO<T>::load(grid + 2 * idx), ElemIO<T>::load(grid + 2 * idx + 1), p.H, p.W,
-                                p.pad, p.align);
-    const int32_t plane_px = p.H * p.W;
-    const T* x_n = x + n * p.C * (int64_t)plane_px;
-    const T* go_n = gout + n * p.C * (int64_t)points + pt;
-    float gix = 0.0f, giy = 0.0f;
-    // f(number of channels, first channel): the sums run over the channels in order; the loads do not depend on them, so
-    // they are issued a group of channels ahead (a lane has one grid point and would otherwise wait out every load in turn)
-    auto for_groups = [&](auto&& f) {
-        int32_t c = 0;
-        for (; c + 8 <= p.C; c += 8) {
-            f(std::integral_constant<int, 8>{}, c);
-        }
-        if (c + 4 <= p.C) {
-            f(std::integral_constant<int, 4>{}, c);
-            c += 4;
-        }
-        switch (p.C - c) {
-            case 3: f(std::integral_constant<int, 3>{}, c); break;
-            case 2: f(std::integral_constant<int, 2>{}, c); break;
-            case 1: f(std::integral_constant<int, 1>{}, c); break;
-            default: break;
-        }
-    };
-    if (INTERP == 0) {
-        const float dxe = (float)(tp.x0 == INT32_MAX ? tp.x0 : tp.x0 + 1) - tp.fx, dxw = tp.fx - (float)tp.x0;
-        const float dys = (float)(tp.y0 == INT32_MAX ? tp.y0 : tp.y0 + 1) - tp.fy, dyn = tp.fy - (float)tp.y0;
-        const bool ok0 = tp.off[0] >= 0, ok1 = tp.off[1] >= 0, ok2 = tp.off[2] >= 0, ok3 = tp.off[3] >= 0;
-        const int32_t o0 = ok0 ? tp.off[0] : 0, o1 = ok1 ? tp.off[1] : 0, o2 = ok2 ? tp.off[2] : 0,
-                      o3 = ok3 ? tp.off[3] : 0;
-        auto accumulate = [&](float go, float v0, float v1, float v2, float v3) {
-            if (ok0) {
-                gix -= v0 * dys * go;
-                giy -= v0 * dxe * go;
-            }
-            if (ok1) {
-                gix += v1 * dys * go;
-                giy -= v1 * dxw * go;
-            }
-            if (ok2) {
-                gix -= v2 * dyn * go;
-                giy += v2 * dxe * go;
-            }
-            if (ok3) {
-                gix += v3 * dyn * go;
-                giy += v3 * dxw * go;
-            }
-        };
-        if (p.W >= 2) {
-            // The west and east corner of a row are neighbours in memory: one load of two elements (aligned to one
-            // element only) per row instead of two loads halves the addresses the gather puts through the memory
-            // pipeline.  The pair sits at column pb = clamp(x0, 0, W - 2), so it never leaves the row; which half is
-            // which corner follows from pb.  Corners outside the image are skipped by accumulate() as before.
-            using PairBits = typename std::conditional<sizeof(T) == 2, uint32_t, uint64_t>::type;
-            const int32_t x0 = tp.x0, x1 = (tp.x0 == INT32_MAX) ? tp.x0 : tp.x0 + 1;
-            const int32_t y1 = (tp.y0 == INT32_MAX) ? tp.y0 : tp.y0 + 1;
-            const int32_t pb = (x0 < 0) ? 0 : ((x0 > p.W - 2) ? p.W - 2 : x0);
-            const bool lo_w = (x0 == pb), lo_e = (x1 == pb);
-            const int32_t r0 = (tp.y0 >= 0 && tp.y0 < p.H) ? tp.y0 * p.W + pb : 0;
-            const int32_t r1 = (y1 >= 0 && y1 < p.H) ? y1 * p.W + pb : 0;
-            for_groups([&](auto count, int32_t c) {
-                constexpr int U = decltype(count)::value;
-                float go[U];
-                PairBits north[U], south[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const T* xc = x_n + (int64_t)(c + u) * plane_px;
-                    go[u] = ElemIO<T>::load(go_n + (int64_t)(c + u) * points);
-                    __builtin_memcpy(&north[u], xc + r0, sizeof(PairBits));
-                    __builtin_memcpy(&south[u], xc + r1, sizeof(PairBits));
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    T n2[2], s2[2];
-                    __builtin_memcpy(n2, &north[u], sizeof(PairBits));
-                    __builtin_memcpy(s2, &south[u], sizeof(PairBits));
-                    const float nlo = ElemIO<T>::load(&n2[0]), nhi = ElemIO<T>::load(&n2[1]);
-                    const float slo = ElemIO<T>::load(&s2[0]), shi = ElemIO<T>::load(&s2[1]);
-                    accumulate(go[u], lo_w ? nlo : nhi, lo_e ? nlo : nhi, lo_w ? slo : shi, lo_e ? slo : shi);
-                }
-            });
-        } else {
-            for_groups([&](auto count, int32_t c) {
-                constexpr int U = decltype(count)::value;
-                float go[U], v[U][4];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const T* xc = x_n + (int64_t)(c + u) * plane_px;
-                    go[u] = ElemIO<T>::load(go_n + (int64_t)(c + u) * points);
-                    v[u][0] = ElemIO<T>::load(xc + o0);
-                    v[u][1] = ElemIO<T>::load(xc + o1);
-                    v[u][2] = ElemIO<T>::load(xc + o2);
-                    v[u][3] = ElemIO<T>::load(xc + o3);
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    accumulate(go[u], v[u][0], v[u][1], v[u][2], v[u][3]);
-                }
-            });
-        }
-    } else {
-        const float xf = __builtin_floorf(tp.fx), yf = __builtin_floorf(tp.fy);
-        float cx[4], cy[4], cxg[4], cyg[4];
-        cubic_coefficients(cy, tp.fy - yf);
-        cubic_coefficients(cx, tp.fx - xf);
-        cubic_coefficients_grad(cyg, tp.fy - yf);
-        cubic_coefficients_grad(cxg, tp.fx - xf);
-        for (int32_t c = 0; c < p.C; c++) {
-            const T* xc = x_n + (int64_t)c * plane_px;
-            const float go = ElemIO<T>::load(go_n + (int64_t)c * points);
-            T v[16];  // all on their way together; a tap outside the plane counts as 0
-#pragma unroll
-            for (int k = 0; k < 16; k++) {
-                v[k] = xc[tp.off[k] >= 0 ? tp.off[k] : 0];
-            }
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float w = (tp.off[i * 4 + j] >= 0) ? ElemIO<T>::load(&v[i * 4 + j]) : 0.0f;
-                    giy += w * cyg[j] * cx[i] * go;
-                    gix += w * cxg[i] * cy[j] * go;
-                }
-            }
-        }
-    }
-    // products in fp32 first, then the conversion (see contribution())
-    ElemIO<T>::store(dgrid + 2 * idx, as_fp32_value(tp.mx * gix));
-    ElemIO<T>::store(dgrid + 2 * idx + 1, as_fp32_value(tp.my * giy));
+    gs2d_grid_gradient_block<T, INTERP, TILED>(blockIdx.x, gout, x, grid, dgrid, p);
 }
 
 GradGatherArgs gather_args(const GridSamplerGradArgs& a)
@@ -434,6 +251,10 @@ GradGatherArgs gather_args(const GridSamplerGradArgs& a)
     g.grid = a.grid;
     g.dx = a.dx;
     g.scratch = a.scratch;
+    g.x = a.x;
+    g.dgrid = a.dgrid;
+    g.Ho = a.Hout;
+    g.Wo = a.Wout;
     return g;
 }
 
@@ -479,7 +300,9 @@ hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
         }
     }
     if (a.dx != nullptr && !dx_done && a.scratch != nullptr && gs2d_grad_gather_words(a) > 0) {
-        const hipError_t e = run_grad_gather(gather_args(a), stream);
+        GradGatherArgs g = gather_args(a);
+        g.dgrid = dgrid_done ? nullptr : a.dgrid;
+        const hipError_t e = run_grad_gather(g, stream, &dgrid_done);
         if (e != hipSuccess) {
             return e;
         }
@@ -518,26 +341,19 @@ hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
         }
     }
     if (a.dgrid != nullptr && !dgrid_done) {
-        const int64_t total = a.N * a.Hout * a.Wout;
+        const Grid2Launch g = grid2_launch(gather_args(a));
+        if (!g.ok) {
+            return hipErrorInvalidValue;
+        }
         if constexpr (INTERP == 0) {
-            if (const GridTilePlan t = grid_tile_plan(a); t.ok) {
-                p.pieces = (uint32_t)t.tiles;
-                p.by_item = make_fast_div((uint32_t)t.per_item);
-                p.by_tiles_x = make_fast_div((uint32_t)t.tiles_x);
-                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, true>), dim3((unsigned)t.blocks), dim3(kThreads), 0, stream,
-                                   (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, total, p, 0);
+            if (g.tiled) {
+                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, true>), dim3((unsigned)g.blocks), dim3(kGridTileThreads), 0,
+                                   stream, (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, g.p);
                 return hipGetLastError();
             }
         }
-        const int64_t blocks = (total + kThreads - 1) / kThreads;
-        if (blocks > INT32_MAX) {
-            return hipErrorInvalidValue;
-        }
-        const int64_t points = a.Hout * a.Wout;
-        const int32_t blocks_per_item =
-            (points % kThreads == 0 && a.N % 8 == 0 && points / kThreads <= INT32_MAX) ? (int32_t)(points / kThreads) : 0;
-        hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, false>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
-                           (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, total, p, blocks_per_item);
+        hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, false>), dim3((unsigned)g.blocks), dim3(kGridTileThreads), 0, stream,
+                           (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, g.p);
         return hipGetLastError();
     }
     return hipSuccess;

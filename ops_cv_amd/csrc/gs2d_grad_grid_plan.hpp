@@ -4,6 +4,7 @@
 #include <cstdint>
 
 #include "acl_types.hpp"
+#include "gs_grad_gather_plan.hpp"
 #include "launch_limits.hpp"
 
 namespace opscv {
@@ -25,24 +26,34 @@ struct GridTilePlan {
 //
 // Not for bicubic samples, whose sixteen taps share lines within a point already: fp32 8x3x479x637 115 / 138 us, fp16 108 / 153,
 // fp32 2x3x720x1280 106 / 120, 1x4x256x256 -> 512x512 18.0 / 23.5, with border padding 19.6 / 32.3, 4x1x300x400 17.2 / 19.4.
-inline GridTilePlan grid_tile_plan(const GridSamplerGradArgs& a)
+inline GridTilePlan grid_tile_plan(Elem elem, int interp, int64_t N, int64_t H, int64_t W, int64_t Ho, int64_t Wo)
 {
     GridTilePlan p;
-    if (a.interp != 0 || a.N < 1 || a.Hout < 1 || a.Wout < 1 || a.Hout > INT32_MAX / 2 || a.Wout > INT32_MAX / 2 || a.N > INT32_MAX / 2) {
+    if (interp != 0 || N < 1 || Ho < 1 || Wo < 1 || Ho > INT32_MAX / 2 || Wo > INT32_MAX / 2 || N > INT32_MAX / 2) {
         return p;
     }
-    const int64_t tiles_y = (a.Hout + kGridTile - 1) / kGridTile;
-    p.tiles_x = (a.Wout + kGridTile - 1) / kGridTile;
+    const int64_t tiles_y = (Ho + kGridTile - 1) / kGridTile;
+    p.tiles_x = (Wo + kGridTile - 1) / kGridTile;
     p.per_item = p.tiles_x * tiles_y;
-    if (p.per_item > INT32_MAX / 2 / a.N) {
+    if (p.per_item > INT32_MAX / 2 / N) {
         return p;
     }
-    p.tiles = a.N * p.per_item;
+    p.tiles = N * p.per_item;
     p.blocks = (p.tiles + 7) / 8 * 8;
     const int64_t lanes = p.per_item * kGridTileThreads;
-    p.ok = a.Hin * a.Win * elem_size(a.elem) > (64 << 10) && p.tiles >= 512 && lanes - lanes / 5 <= a.Hout * a.Wout &&
+    p.ok = H * W * elem_size(elem) > (64 << 10) && p.tiles >= 512 && lanes - lanes / 5 <= Ho * Wo &&
            fits_launch(p.blocks, kGridTileThreads);
     return p;
+}
+
+inline GridTilePlan grid_tile_plan(const GridSamplerGradArgs& a)
+{
+    return grid_tile_plan(a.elem, a.interp, a.N, a.Hin, a.Win, a.Hout, a.Wout);
+}
+
+inline GridTilePlan grid_tile_plan(const GradGatherArgs& a)
+{
+    return grid_tile_plan(a.elem, a.interp, a.N, a.H, a.W, a.Ho, a.Wo);
 }
 
 }  // namespace opscv

@@ -24,6 +24,7 @@
 #include "gs2d_grad_math.hpp"
 #include "gs3d_grad_math.hpp"
 #include "gs_grad_gather.hpp"
+#include "gs_grad_grid.hpp"
 #include "kernels.hpp"
 #include "options.hpp"
 
@@ -279,31 +280,9 @@ __global__ __launch_bounds__(kThreads) void gs3d_grad_input_kernel(const T* __re
 template <typename T, int INTERP, int U>
 __global__ __launch_bounds__(kThreads) void gs3d_grad_grid_kernel(const T* __restrict__ gout, const T* __restrict__ x,
                                                                    const T* __restrict__ grid, T* __restrict__ dgrid,
-                                                                   int64_t total, Grad3Params p)
+                                                                   Grid3Params p)
 {
-    using Taps = GradTaps3<T, INTERP>;
-    const int64_t idx = (int64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (idx >= total) {
-        return;
-    }
-    (void)gout;
-    (void)x;
-    if (INTERP == 1) {
-        // grid_sampler3_d_grad_simt_det.h:354-356
-        ElemIO<T>::store(dgrid + 3 * idx, 0.0f);
-        ElemIO<T>::store(dgrid + 3 * idx + 1, 0.0f);
-        ElemIO<T>::store(dgrid + 3 * idx + 2, 0.0f);
-        return;
-    }
-    if constexpr (INTERP == 0) {
-        const int32_t points = p.points;
-        const int64_t n = idx / points;
-        const int32_t pt = (int32_t)(idx - n * points);
-        Taps tp;
-        decide_grad_taps3<T, INTERP>(tp, ElemIO<T>::load(grid + 3 * idx), ElemIO<T>::load(grid + 3 * idx + 1),
-                                     ElemIO<T>::load(grid + 3 * idx + 2), p.D, p.H, p.W, p.pad, p.align);
-        gs3d_point_grid_gradient<T, U>(tp, gout, x, dgrid, idx, n, pt, p);
-    }
+    gs3d_grid_gradient_block<T, INTERP, U>(blockIdx.x, gout, x, grid, dgrid, p);
 }
 
 // Voxels per band.  Every workgroup is a chain of dependent LDS round trips, so the chip is filled by workgroups
@@ -340,6 +319,8 @@ GradGatherArgs gather_args(const GridSampler3DGradArgs& a)
     g.grid = a.grid;
     g.dx = a.dx;
     g.scratch = a.gather;
+    g.x = a.x;
+    g.dgrid = a.dgrid;
     return g;
 }
 
@@ -365,7 +346,7 @@ hipError_t launch_interp(const GridSampler3DGradArgs& a, hipStream_t stream)
     }
     bool dgrid_done = false;  // the gather variant's first kernel computes the grid gradient on its way
     if (a.dx != nullptr && a.gather != nullptr && gs3d_grad_gather_words(a) > 0) {
-        const hipError_t e = run_grad_gather(gather_args(a), stream);
+        const hipError_t e = run_grad_gather(gather_args(a), stream, &dgrid_done);
         if (e != hipSuccess) {
             return e;
         }
@@ -435,10 +416,10 @@ hipError_t launch_interp(const GridSampler3DGradArgs& a, hipStream_t stream)
         }
         if (total < kGridGradFewPoints) {
             hipLaunchKernelGGL((gs3d_grad_grid_kernel<T, INTERP, 4>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
-                               (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, total, p);
+                               (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, Grid3Params{p, total});
         } else {
             hipLaunchKernelGGL((gs3d_grad_grid_kernel<T, INTERP, 1>), dim3((unsigned)blocks), dim3(kThreads), 0, stream,
-                               (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, total, p);
+                               (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, Grid3Params{p, total});
         }
         return hipGetLastError();
     }
@@ -503,10 +484,13 @@ int64_t gs3d_grad_gather_words(const GridSampler3DGradArgs& a)
         // 55; 8 x 16x40x40 307 / 72).  Smaller grids seldom have one and cost half as much in slots (19 / 35 us), nor do
         // grids of less than a point per two voxels (13x2x13x41x52 from 9x30x39 28 / 50, 15 of 24 such calls slower sorted;
         // from 0.8 points per voxel on 192 of 243 are faster sorted, on average by 2.7 times).
-        const bool piles = a.pad != 0 && points >= 8192 && 2 * points >= vol;
+        // Batches have such an item more often than single ones: fp16 17x2x24x95x36 from 19x75x28 border (0.49 points per voxel)
+        // 296 us, sorting 93; fp32 23x2 of 7056 voxels and points reflection 152 / 47; but 13x2x27716 voxels at 0.38 border 29 / 47,
+        // 7x9x48620 at 0.23 reflection 38 / 60, 12x3x6840 at 0.52 border 19 / 25.
+        const bool piles = a.pad != 0 && ((points >= 8192 && 2 * points >= vol) || (a.N * points >= 131072 && 20 * points >= 9 * vol));
         // the slots kernels keep an item on one XCD: one or two large items leave most of the chip idle (one item of
-        // 65536 points: 39 / 30 us, with 16 channels 94 / 42; two items 41 / 37; four 39 / 45; one of 36864 27 / 30)
-        const bool few_items = a.N <= 2 && points >= 49152;
+        // 41664 points 34 / 24, of 84600 - / 28; four of 46110 33 / 28; three of 15028 20 / 24)
+        const bool few_items = (a.N <= 2 && points >= 32768) || (a.N <= 4 && points >= 45000);
         if (!piles && !few_items) {
             return 0;
         }

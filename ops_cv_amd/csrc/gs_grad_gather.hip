@@ -732,10 +732,10 @@ int64_t grad_gather_words(const GradGatherArgs& a)
     return pl.ok ? (int64_t)pl.p.lay.item_words * pl.group : 0;
 }
 
-hipError_t run_grad_gather(const GradGatherArgs& a, hipStream_t stream)
+hipError_t run_grad_gather(const GradGatherArgs& a, hipStream_t stream, bool* dgrid_done)
 {
     if (grad_tiles_words(a) > 0) {
-        return run_grad_tiles(a, stream);
+        return run_grad_tiles(a, stream, dgrid_done);
     }
     GatherPlan pl = gather_plan(a);
     if (!pl.ok || a.dx == nullptr || a.gout == nullptr || a.grid == nullptr || a.scratch == nullptr) {

@@ -27,6 +27,10 @@ struct GradGatherArgs {
     const void* grid = nullptr;
     void* dx = nullptr;
     void* scratch = nullptr;  // grad_gather_words() 32-bit words on a 16-byte boundary
+    // the gradient of the grid, for the launches of the input gradient to take along; null: not wanted
+    const void* x = nullptr;
+    void* dgrid = nullptr;
+    int64_t Ho = 0, Wo = 0;   // planes: extents of the grid
 };
 
 constexpr int kGatherThreads = 256;

@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "gs_grad_gather.hpp"
+#include "gs_grad_grid.hpp"
 #include "gs_grad_points.hpp"
 #include "gs_grad_tiles_kernel.hpp"
 #include "gs_grad_tiles_plan.hpp"
@@ -51,10 +52,43 @@ constexpr uint32_t kCountedRun = 32;   // runs of up to as many points are put i
 constexpr uint32_t kSerialMost = 192;  // contributions that a lane merges by itself, and adds by itself where
 constexpr int kFewCrowded = 6;         // more lanes than this of its wavefront have as many as that to do
 
-template <typename T, int DIM, int INTERP>
+// What the bin kernel takes along: nothing, or the gradient of the grid by workgroups behind its own.
+template <int DIM>
+struct GridToo;
+template <>
+struct GridToo<2> {
+    const void* gout;
+    const void* x;
+    void* dgrid;
+    Grid2Params p;
+};
+template <>
+struct GridToo<3> {
+    const void* gout;
+    const void* x;
+    void* dgrid;
+    Grid3Params p;
+};
+
+// GRID: 0: no gradient of the grid; of planes 1 points in rows, 2 in tiles; of volumes 1 a channel's loads at a time, 2 four's
+template <typename T, int DIM, int INTERP, int GRID>
 __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __restrict__ grid, uint32_t* __restrict__ ws,
-                                                                   TilesParams p, uint32_t pieces)
+                                                                   TilesParams p, uint32_t pieces, uint32_t bin_blocks,
+                                                                   GridToo<DIM> too)
 {
+    if constexpr (GRID != 0) {
+        if (blockIdx.x >= bin_blocks) {
+            const uint32_t block = blockIdx.x - bin_blocks;
+            const T* gout = (const T*)too.gout;
+            const T* x = (const T*)too.x;
+            if constexpr (DIM == 2) {
+                gs2d_grid_gradient_block<T, INTERP, GRID == 2>(block, gout, x, grid, (T*)too.dgrid, too.p);
+            } else {
+                gs3d_grid_gradient_block<T, INTERP, GRID == 2 ? 4 : 1>(block, gout, x, grid, (T*)too.dgrid, too.p);
+            }
+            return;
+        }
+    }
     typedef GradTile<DIM> S;
     constexpr int kWaves = kBinThreads / 64;
     constexpr int kSteps = kBinPoints / kBinThreads;
@@ -959,26 +993,61 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
 
 inline uint32_t xcd_blocks(int64_t pieces) { return (uint32_t)((pieces + 7) / 8 * 8); }
 
+template <typename T, int DIM, int INTERP, int GRID>
+hipError_t launch_bin(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t stream, const GridToo<DIM>& too, int64_t grid_blocks)
+{
+    static std::atomic<uint32_t> bin_allowed{0};
+    const hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(gs_tiles_bin_kernel<T, DIM, INTERP, GRID>),
+                                           (int)kTilesMost * (kBinThreads / 64) * 12, bin_allowed);
+    if (e != hipSuccess) {
+        return e;
+    }
+    const uint32_t bins = (uint32_t)a.N * (uint32_t)pl.p.blocks, blocks = xcd_blocks(bins);
+    hipLaunchKernelGGL((gs_tiles_bin_kernel<T, DIM, INTERP, GRID>), dim3(blocks + (uint32_t)grid_blocks), dim3(kBinThreads),
+                       (size_t)pl.bin_lds, stream, (const T*)a.grid, (uint32_t*)a.scratch, pl.p, bins, blocks, too);
+    return hipGetLastError();
+}
+
+// The bin kernel, with the gradient of the whole batch's grid behind its workgroups where that is wanted (a.dgrid).
+template <typename T, int DIM, int INTERP>
+hipError_t run_bin(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t stream)
+{
+    GridToo<DIM> too{};
+    if (a.dgrid == nullptr) {
+        return launch_bin<T, DIM, INTERP, 0>(a, pl, stream, too, 0);
+    }
+    too.gout = a.gout;
+    too.x = a.x;
+    too.dgrid = a.dgrid;
+    if constexpr (DIM == 2) {
+        const Grid2Launch g = grid2_launch(a);
+        too.p = g.p;
+        if constexpr (INTERP == 0) {
+            if (g.tiled) {
+                return launch_bin<T, DIM, INTERP, 2>(a, pl, stream, too, g.blocks);
+            }
+        }
+        return launch_bin<T, DIM, INTERP, 1>(a, pl, stream, too, g.blocks);
+    } else {
+        too.p = grid3_params(a);
+        const int64_t blocks = (too.p.total + kBinThreads - 1) / kBinThreads;
+        return (INTERP == 0 && too.p.total < kGridGradFewPoints) ? launch_bin<T, DIM, INTERP, 2>(a, pl, stream, too, blocks)
+                                                                 : launch_bin<T, DIM, INTERP, 1>(a, pl, stream, too, blocks);
+    }
+}
+
 template <typename T, int DIM, int INTERP, int CB>
 hipError_t launch_tiles(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t stream)
 {
     typedef GradTile<DIM> S;
-    static std::atomic<uint32_t> bin_allowed{0};
-    hipError_t e = allow_dynamic_lds(reinterpret_cast<const void*>(gs_tiles_bin_kernel<T, DIM, INTERP>),
-                                     (int)kTilesMost * (kBinThreads / 64) * 12, bin_allowed);
-    if (e != hipSuccess) {
-        return e;
-    }
+    hipError_t e = hipSuccess;
     static std::atomic<uint32_t> gather_allowed{0};
     e = allow_dynamic_lds(reinterpret_cast<const void*>(gs_tiles_gather_kernel<T, DIM, INTERP, CB>),
                           (int)(kTileBlocksMost + 1) * 8, gather_allowed);
     if (e != hipSuccess) {
         return e;
     }
-    const uint32_t bins = (uint32_t)a.N * (uint32_t)pl.p.blocks;
-    hipLaunchKernelGGL((gs_tiles_bin_kernel<T, DIM, INTERP>), dim3(xcd_blocks(bins)), dim3(kBinThreads), (size_t)pl.bin_lds,
-                       stream, (const T*)a.grid, (uint32_t*)a.scratch, pl.p, bins);
-    e = hipGetLastError();
+    e = run_bin<T, DIM, INTERP>(a, pl, stream);
     if (e != hipSuccess) {
         return e;
     }
@@ -1018,6 +1087,17 @@ hipError_t run_typed(const GradGatherArgs& a, const TilesPlan& pl, hipStream_t s
     }
 }
 
+// Whether the bin kernel takes the gradient of the grid along: its workgroups have the bin's LDS too, which four and more a CU
+// can have.
+bool takes_grid(const GradGatherArgs& a, const TilesPlan& pl)
+{
+    if (a.dgrid == nullptr || a.x == nullptr || pl.group < a.N || pl.bin_lds > 40 * 1024) {
+        return false;
+    }
+    const int64_t blocks = a.dim == 2 ? grid2_launch(a).blocks : (a.N * a.points + kBinThreads - 1) / kBinThreads;
+    return fits_launch(blocks + a.N * (int64_t)pl.p.blocks + 16, kBinThreads);
+}
+
 }  // namespace
 
 int64_t grad_tiles_words(const GradGatherArgs& a)
@@ -1026,16 +1106,19 @@ int64_t grad_tiles_words(const GradGatherArgs& a)
     return pl.ok ? pl.words : 0;
 }
 
-hipError_t run_grad_tiles(const GradGatherArgs& a, hipStream_t stream)
+hipError_t run_grad_tiles(const GradGatherArgs& a, hipStream_t stream, bool* dgrid_done)
 {
     TilesPlan pl = tiles_plan(a);
     if (!pl.ok || a.dx == nullptr || a.gout == nullptr || a.grid == nullptr || a.scratch == nullptr) {
         return hipErrorInvalidValue;
     }
+    // Items in one group: the bin kernel takes the gradient of the grid along.
+    const bool take_grid = takes_grid(a, pl);
     // the items are independent: a group of them after the other, each in all of the scratch
     const int64_t esz = elem_size(a.elem);
     for (int64_t first = 0; first < a.N; first += pl.group) {
         GradGatherArgs g = a;
+        g.dgrid = take_grid ? a.dgrid : nullptr;
         g.N = (a.N - first < pl.group) ? a.N - first : pl.group;
         g.gout = (const char*)a.gout + first * a.C * a.points * esz;
         g.grid = (const char*)a.grid + first * a.points * a.dim * esz;
@@ -1052,6 +1135,7 @@ hipError_t run_grad_tiles(const GradGatherArgs& a, hipStream_t stream)
             return e;
         }
     }
+    *dgrid_done = *dgrid_done || take_grid;
     return hipSuccess;
 }
 

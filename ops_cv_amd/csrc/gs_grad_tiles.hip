@@ -49,8 +49,16 @@ constexpr int kTapBits = 3;
 constexpr uint32_t kNoKey = 0xFFFFFFFFu;
 constexpr uint32_t kNoPlace = 0xFFFFFFFFu;
 constexpr uint32_t kCountedRun = 32;   // runs of up to as many points are put in order by counting, longer ones by ballots
-constexpr uint32_t kSerialMost = 192;  // contributions that a lane merges by itself, and adds by itself where
-constexpr int kFewCrowded = 6;         // more lanes than this of its wavefront have as many as that to do
+// Crowded elements are put in order by a lane each where more than kFewCrowded lanes of a wavefront have one of up to kSerialMost
+// contributions, otherwise one after the other by the wavefront, up to 64 * kRankedRegs contributions by counting.  A lane also
+// adds up to kSerialMost by itself where more lanes than kFewCrowded have as many.  Without the counting and with 192
+// contributions / with it and 192 / 96 / 64 / 48 (and 16 lanes), microseconds of the whole gradient: fp32 reflection
+// 5x4x27x54x51 81 / 66 / 67 / 67 / 66, fp16 3x3x31x45x16 50 / 41 / 41 / 39 / 49, fp32 9x22x25x16x29 86 / 66 / 66 / 67 / 74,
+// planes, fp16 border 29x4x378x312 183 / 162 / 162 / 164 / 163; 22 such gradients together 1.10, 1.10, 1.10 and 1.05 times as
+// fast, and 1.09 with 3 lanes instead of 6.
+constexpr uint32_t kSerialMost = 64;
+constexpr int kFewCrowded = 6;
+constexpr int kRankedRegs = 2;
 
 // What the bin kernel takes along: nothing, or the gradient of the grid by workgroups behind its own.
 template <int DIM>
@@ -577,6 +585,55 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
             done(batch);
         }
     };
+    // The same for up to 64 * kRankedRegs contributions: a key or some a lane, whose place is the number of lesser ones.  (By
+    // itself a lane waits for LDS at every contribution, some 200 clocks; here a contribution costs 10.)
+    auto rank_together = [&](int owner, int lane, uint32_t its_len, auto&& put) {
+        uint32_t first[R], end[R];  // of the runs: where their keys lie in the list, less those of the runs before; sums
+        runs_of_element(first, end);
+        uint32_t sum = 0;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const uint32_t begin = (uint32_t)__builtin_amdgcn_readlane((int)first[r], owner);
+            const uint32_t upto = (uint32_t)__builtin_amdgcn_readlane((int)end[r], owner);
+            first[r] = begin - sum;
+            sum += upto - begin;
+            end[r] = sum;
+        }
+        const uint32_t its_corner = (uint32_t)__builtin_amdgcn_readlane((int)corner, owner);
+        uint32_t own[kRankedRegs], rank[kRankedRegs];
+#pragma unroll
+        for (int m = 0; m < kRankedRegs; m++) {
+            const uint32_t i = (uint32_t)(m * 64 + lane);
+            uint32_t from = first[0];
+#pragma unroll
+            for (int r = 1; r < R; r++) {
+                from = i >= end[r - 1] ? first[r] : from;
+            }
+            own[m] = (i < its_len) ? s_list[from + i] ^ its_corner : kNoKey;
+            rank[m] = 0u;
+        }
+#pragma unroll
+        for (int m = 0; m < kRankedRegs; m++) {
+            const uint32_t n_keys = its_len > (uint32_t)(m * 64) ? its_len - (uint32_t)(m * 64) : 0u;
+            const uint32_t here = n_keys < 64u ? n_keys : 64u;
+            for (uint32_t j = 0; j < here; j += 8u) {
+#pragma unroll
+                for (uint32_t u = 0; u < 8u; u++) {
+                    const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)own[m], (int)(j + u));
+#pragma unroll
+                    for (int q = 0; q < kRankedRegs; q++) {
+                        rank[q] += (other < own[q]) ? 1u : 0u;
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < kRankedRegs; m++) {
+            if ((uint32_t)(m * 64 + lane) < its_len) {
+                put(rank[m], own[m] & kLowBits);
+            }
+        }
+    };
     // The contributions of crowded elements in order to s_sorted, once for all channels: a lane each, or where a single
     // element has hundreds the wavefront together.
     auto merge_crowded = [&]() {
@@ -599,16 +656,23 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
                 sorted = fits ? to : kNoKey;
             }
         }
-        if (fits && len <= kSerialMost) {
+        const bool few = __builtin_popcountll(__builtin_amdgcn_ballot_w64(fits)) <= kFewCrowded;
+        const bool alone = fits && !few && len <= kSerialMost;
+        if (alone) {
             merge_alone([&](uint32_t i, uint32_t k) { s_sorted[sorted + i] = (uint16_t)(k & kLowBits); });
         }
         int lane = t & 63;
         asm volatile("" : "+v"(lane));  // what follows is rare: none of it is worked out ahead
-        uint64_t big = __builtin_amdgcn_ballot_w64(fits && len > kSerialMost);
+        uint64_t big = __builtin_amdgcn_ballot_w64(fits && !alone);
         while (big != 0) {
             const int owner = __builtin_ctzll(big);
             big &= big - 1u;
             uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)sorted, owner);
+            const uint32_t its_len = (uint32_t)__builtin_amdgcn_readlane((int)len, owner);
+            if (its_len <= 64u * kRankedRegs) {
+                rank_together(owner, lane, its_len, [&](uint32_t rank, uint32_t k) { s_sorted[to + rank] = (uint16_t)k; });
+                continue;
+            }
             merge_together(owner, lane, [&](uint32_t rank, uint32_t k) { s_sorted[to + rank] = (uint16_t)k; },
                            [&](uint32_t batch) { to += batch; });
         }

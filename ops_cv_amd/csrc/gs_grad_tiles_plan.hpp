@@ -56,7 +56,9 @@ struct TilesLayout {   // offsets in 32-bit words within an item's scratch
 // nearest 2x4x32x64x64 38 / 33 / 36, 78 / 311 / 194, 119 / 1902 / 633: nearest samples of an eighth of every axis are what the
 // lists remain much faster at.  Nine points of ten on five spots: 1x3x480x640 6156 / 2138 / 1433.
 // Border padding piles points up on few elements, which the gather kernel's wavefronts add together: no limit of contributions
-// (fp16 8x4x256x256 from 360x360 131 / 97 / 100, with the limit 133).
+// (fp16 8x4x256x256 from 360x360 131 / 97 / 100, with the limit 133).  Volumes' borders have elements of 50 to 90 here and
+// there, which the gather kernel's wavefronts put in order by counting: gradients with a limit of 48 / 96 / 192 / none, fp16
+// reflection 11x2x42x18x88 119 / 97 / 97 / 97, bf16 border 3x4x24x61x31 59 / 51 / 52 / 52.
 struct CrowdedTile {
     uint32_t points, contributions;
 };
@@ -67,7 +69,7 @@ inline CrowdedTile crowded_tile(const GradGatherArgs& a)
         return {a.dim == 3 ? 10240u : 12288u, any};
     }
     if (a.dim == 3) {
-        return a.N * a.C <= 48 ? CrowdedTile{1920, 48} : CrowdedTile{6144, 72};
+        return {a.N * a.C <= 48 ? 1920u : 6144u, 96u};
     }
     return {a.C > 8 ? 3072u : 5120u, a.pad == 1 ? any : 48u};
 }

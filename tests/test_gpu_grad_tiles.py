@@ -39,7 +39,7 @@ def _spots(rng, n, count, dim, spread):
 
 # tiles of 32 x 16: one, parts of one, edges on and beside their borders; channels together and in blocks (1 to 4, 8 of a
 # 16-bit type, several blocks); about one point an element, and a round of points more than LDS holds; the third number:
-# points on five spots, so that lanes merge alone (up to 192), the wavefront together, and runs stay single
+# points on five spots, so that lanes merge alone (up to 64), the wavefront together, and runs stay single
 PLANES = [((1, 1, 16, 32), (40, 41), 0.0), ((2, 3, 49, 65), (47, 61), 0.0), ((3, 2, 33, 95), (50, 61), 0.0),
           ((4, 4, 64, 96), (66, 90), 0.0), ((9, 5, 17, 33), (60, 33), 0.0), ((6, 9, 48, 31), (50, 33), 0.0),
           ((6, 21, 50, 64), (52, 66), 0.0), ((6, 7, 20, 40), (40, 39), 0.9), ((16, 2, 18, 34), (65, 60), 0.5)]
@@ -169,6 +169,28 @@ def test_volumes(oracle, device, aclnn, dtype, pad, interp, xs, out, spots):
         z, y, x = np.meshgrid(*axes, indexing="ij")
         grid = np.stack([x, y, z], axis=-1)[None] * rng.uniform(0.9, 1.1, (xs[0], 1, 1, 1, 3)) + rng.normal(0, 0.02, (xs[0],) + out + (3,))
     _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid.reshape((xs[0],) + out + (3,)), rng)
+
+
+# elements with contributions of several cells, as many as a lane, a wavefront by counting and a wavefront by merging put in
+# order: on two elements of a wavefront, and on more than six
+@pytest.mark.parametrize("dtype", ["fp32", "fp16"])
+@pytest.mark.parametrize("elements", [2, 9])
+@pytest.mark.parametrize("xs,out,counts", [((8, 3, 32, 64), (46, 80), (26, 63, 64, 65)), ((10, 1, 32, 64), (40, 90), (127, 128, 129)),
+                                           ((2, 2, 8, 16, 16), (10, 14, 14), (40, 63, 64, 65))])
+def test_crowded_elements(oracle, device, aclnn, dtype, elements, xs, out, counts):
+    rng = np.random.default_rng(4620)
+    points, dim = int(np.prod(out)), len(out)
+    assert host_plans.gradient_tiles(dtype, 0, 1, xs, points) is not None
+    at = rng.uniform(0, 1, (xs[0], points, dim)) * (np.array(xs[:1:-1]) - 1)
+    for n in range(xs[0]):
+        free = iter(rng.permutation(points))
+        for e in range(elements if dim == 2 else min(elements, 5)):  # of volumes on two planes, in rows of 16
+            for row in range(2):
+                around = np.array([3 * e + 2, 9 * row + 4] if dim == 2 else [3 * e + 1, 3 * row + 1, 1])
+                for _ in range(counts[(e + row + n) % len(counts)]):
+                    at[n, next(free)] = around + rng.uniform(-0.9, 0.9, dim)
+    grid = (2 * at + 1) / np.array(xs[:1:-1]) - 1
+    _check(aclnn, oracle, device, dtype, 0, 1, xs, out, grid.reshape((xs[0],) + out + (dim,)), rng)
 
 
 def test_special_grid_values(oracle, device, aclnn):

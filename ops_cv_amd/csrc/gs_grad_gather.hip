@@ -19,6 +19,11 @@
 //           list of their own; meanwhile spare workgroups sort the runs of more than 64 entries.
 //   crowded one wavefront per listed element: merges the element's runs, 64 entries at a time, in the reference's
 //           order; the lanes compute the 64 contributions of a channel at once and one lane adds them up in order.
+//           A chain of waits, so everything that does not depend on the sums is on its way before them: the runs' next
+//           entries, the next channels' gradOutput, the operands of the additions; the places of two runs' entries in
+//           each other are found together, by a fixed number of steps.  Both gradients before / so, border padding: fp32
+//           4x2x600x736 721 / 440 us, 3x1x520x609 -> 605x708 1031 / 674, 4x2x301x505 378 / 268, 3x3x210x328 182 / 132, fp16 2x4x360x552
+//           95 / 82; nearest fp32 3x2x304x576 222 / 144.
 //
 // Input gradient of fp32 8x3x479x637 from as many grid points (rotations of up to 30 degrees): 2568 us with elections;
 // here clear 6, count 43, place 14, fill 13, gather 107, crowded 5 us.  Count is bound by the rate of atomics (55 G/s;
@@ -45,6 +50,7 @@ namespace {
 constexpr int kThreads = kGatherThreads;
 constexpr int kPlaceCells = 8;       // cells per lane of the place kernel
 constexpr int kPlaceThreads = 256;
+constexpr int kFoldPitch = 68;       // of a channel's contributions in LDS: on the 16-byte grid, channels at different banks
 constexpr int kFoldChans = 16;       // channels whose contributions a crowded element's wavefront computes together
 constexpr uint32_t kNoRank = 0xFFFFFFFFu;
 
@@ -513,9 +519,9 @@ __global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __
     typedef Mode<DIM, INTERP> M;
     constexpr int R = M::kRuns;
     constexpr int kWaves = kThreads / 64;
-    __shared__ uint32_t s_window[kWaves][R][64];  // the next 64 entries of every run
+    __shared__ uint32_t s_window[kWaves][R][64];  // short runs, sorted
     __shared__ uint32_t s_key[kWaves][64];        // the next 64 keys in order
-    __shared__ float s_val[kWaves][kFoldChans][65];
+    __shared__ __align__(16) float s_val[kWaves][kFoldChans][kFoldPitch];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t n = blockIdx.y;
     const uint32_t* wsn = ws + (size_t)n * p.lay.item_words;
@@ -525,7 +531,7 @@ __global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __
     const Coords<T, DIM>* coords = reinterpret_cast<const Coords<T, DIM>*>(wsn + p.lay.coords);
     uint32_t(*window)[64] = s_window[wave];
     uint32_t* keys = s_key[wave];
-    float(*val)[65] = s_val[wave];
+    float(*val)[kFoldPitch] = s_val[wave];
     // the wavefronts of a workgroup share nothing: what a wavefront writes to LDS it reads back itself, in order
     auto landed = [] { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); __builtin_amdgcn_wave_barrier(); };
     for (uint32_t job = blockIdx.x * kWaves + wave; job < jobs; job += gridDim.x * kWaves) {
@@ -559,83 +565,100 @@ __global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __
                 }
             }
         }
+        landed();
+        uint32_t ahead[R];  // the next 64 entries of the long runs
+        auto look_ahead = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                ahead[r] = 0xFFFFFFFFu;
+                if (!whole[r] && (uint32_t)lane < left[r]) {
+                    ahead[r] = from[r][lane];
+                }
+            }
+        };
+        look_ahead();
         float acc = 0.0f;  // of channel c_first + lane
         while (total > 0u) {
-            // the next entries of every run
-            uint32_t mine[R], held[R];
+            // the next entries of every run, and behind a run's last one an entry beyond all
+            uint32_t mine[R], held[R], rank[R];
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 held[r] = left[r] < 64u ? left[r] : 64u;
-                if (!whole[r]) {
-                    landed();
-                    if ((uint32_t)lane < held[r]) {
-                        window[r][lane] = from[r][lane];
-                    }
+                mine[r] = ahead[r];
+                if (whole[r] && (uint32_t)lane < held[r]) {
+                    mine[r] = window[r][skip[r] + lane];
                 }
+                rank[r] = (uint32_t)lane;
             }
-            landed();
+            // the rank of every one of them among all: entries of another run come first when their chunk is earlier, or the
+            // same and their corner's number lower
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                mine[r] = ((uint32_t)lane < held[r]) ? window[r][skip[r] + lane] : 0xFFFFFFFFu;
-            }
-            // the rank of every one of them among all: entries of another run come first when their chunk is
-            // earlier, or the same and their corner's number lower
-            const uint32_t batch = total < 64u ? total : 64u;
-            uint32_t taken[R];
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                uint32_t rank = (uint32_t)lane;
+                for (int o = 0; o < r; o++) {
+                    if (held[r] > 0u && held[o] > 0u) {
+                        // how many of run o lie before this lane's entry of run r, and of run r before its entry of run o
+                        const uint32_t in_r = mine[r] >> 8, in_o = mine[o] >> 8;
+                        uint32_t less_o = 0, less_r = 0;
 #pragma unroll
-                for (int o = 0; o < R; o++) {
-                    if (o != r) {
-                        const uint32_t chunk = (mine[r] >> 8) + ((o < r) ? 1u : 0u);
-                        uint32_t lo = 0, hi = held[o];  // the first entry of run o whose chunk is not below `chunk`
-                        while (lo < hi) {
-                            const uint32_t mid = (lo + hi) >> 1;
-                            if ((window[o][skip[o] + mid] >> 8) < chunk) {
-                                lo = mid + 1u;
-                            } else {
-                                hi = mid;
-                            }
+                        for (uint32_t d = 32; d > 0u; d >>= 1) {
+                            const uint32_t chunk_o = (uint32_t)__shfl((int)in_o, (int)(less_o + d - 1u));
+                            const uint32_t chunk_r = (uint32_t)__shfl((int)in_r, (int)(less_r + d - 1u));
+                            less_o += (chunk_o <= in_r) ? d : 0u;
+                            less_r += (chunk_r < in_o) ? d : 0u;
                         }
-                        rank += lo;
+                        // the last of 64
+                        less_o += ((uint32_t)__shfl((int)in_o, (int)less_o) <= in_r) ? 1u : 0u;
+                        less_r += ((uint32_t)__shfl((int)in_r, (int)less_r) < in_o) ? 1u : 0u;
+                        rank[r] += less_o;
+                        rank[o] += less_r;
                     }
                 }
-                const bool take = (uint32_t)lane < held[r] && rank < batch;
-                if (take) {
-                    keys[rank] = M::key(mine[r], r);
-                }
-                taken[r] = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(take));
             }
+            const uint32_t batch = total < 64u ? total : 64u;
 #pragma unroll
             for (int r = 0; r < R; r++) {
-                left[r] -= taken[r];
+                const bool take = (uint32_t)lane < held[r] && rank[r] < batch;
+                if (take) {
+                    keys[rank[r]] = M::key(mine[r], r);
+                }
+                const uint32_t taken = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(take));
+                left[r] -= taken;
                 if (whole[r]) {
-                    skip[r] += taken[r];
+                    skip[r] += taken;
                 } else {
-                    from[r] += taken[r];
+                    from[r] += taken;
                 }
             }
+            look_ahead();
             total -= batch;
             landed();
             const uint32_t key = keys[(uint32_t)lane < batch ? lane : 0];
             const uint32_t pt = M::q_of(key) - phase;
             const float w = weight_of<T, DIM, INTERP>(coords[pt], M::tap_of(key), x, y, z);
+            const T* go = gout + (n * p.C + c_first) * (int64_t)p.points + pt;
+            T got[kFoldChans];  // of the next channels
+            auto fetch = [&](int32_t g) __attribute__((always_inline)) {
+#pragma unroll
+                for (int j = 0; j < kFoldChans; j++) {
+                    if (g + j < nc) {
+                        got[j] = go[(int64_t)(g + j) * p.points];
+                    }
+                }
+            };
+            fetch(0);
             for (int32_t g = 0; g < nc; g += kFoldChans) {
-                const T* go = gout + (n * p.C + c_first + g) * (int64_t)p.points + pt;
                 landed();
 #pragma unroll
                 for (int j = 0; j < kFoldChans; j++) {
                     if (g + j < nc) {
-                        val[j][lane] = value_of<T, INTERP>(ElemIO<T>::load(go + (int64_t)j * p.points), w);
+                        val[j][lane] = ((uint32_t)lane < batch) ? value_of<T, INTERP>(ElemIO<T>::load(&got[j]), w) : 0.0f;
                     }
                 }
+                fetch(g + kFoldChans);
                 landed();
                 if (lane >= g && lane < g + kFoldChans && lane < nc) {
-                    const float* v = val[lane - g];
-                    for (uint32_t i = 0; i < batch; i++) {
-                        acc = rt<T>(acc + v[i]);
-                    }
+                    acc = add_in_order<T>(acc, val[lane - g], batch);
                 }
             }
             landed();

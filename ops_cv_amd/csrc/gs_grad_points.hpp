@@ -92,6 +92,42 @@ __device__ __forceinline__ float value_of(float go, float w)
     return (INTERP == 1) ? rt<T>(go) : rt<T>(as_fp32_value(w * go));
 }
 
+// A crowded element's sum goes on over `count` of 64 contributions in LDS (on the 16-byte grid, zeros behind the last: they change
+// no sum that started at +0), a chain of additions: its operands are loaded 16 ahead, so that it never waits for LDS.
+template <typename T>
+__device__ __forceinline__ float add_in_order(float sum, const float* values, uint32_t count)
+{
+    float4 a[4], b[4];
+    auto load = [&](float4 (&v)[4], int at) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            v[i] = *reinterpret_cast<const float4*>(values + at + 4 * i);
+        }
+    };
+    auto add = [&](const float4 (&v)[4]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            sum = rt<T>(sum + v[i].x);
+            sum = rt<T>(sum + v[i].y);
+            sum = rt<T>(sum + v[i].z);
+            sum = rt<T>(sum + v[i].w);
+        }
+    };
+    load(a, 0);
+    load(b, 16);
+    add(a);
+    if (count > 16u) {
+        load(a, 32);
+        add(b);
+        if (count > 32u) {
+            load(b, 48);
+            add(a);
+            add(b);
+        }
+    }
+    return sum;
+}
+
 // Work of a launch cut into `per_item` pieces per batch item, dealt out so that neighbouring pieces run on one XCD
 // (workgroups go to the eight XCDs in turn): XCD k takes the k-th eighth of all pieces.  Pieces beyond the last: false.
 __device__ __forceinline__ bool piece_of_block(uint32_t block, uint32_t pieces, uint32_t* piece)

@@ -946,13 +946,7 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
                 landed();
                 // zeros change no sum: padding piles points up with weight 0 on the elements next to an edge
                 if (__builtin_amdgcn_ballot_w64(some) != 0 && lane < CB) {
-                    for (uint32_t s = 0; s < batch; s += 4u) {
-                        const float4 v = *reinterpret_cast<const float4*>(&own.value[lane][s]);
-                        sum = rt<T>(sum + v.x);
-                        sum = rt<T>(sum + v.y);
-                        sum = rt<T>(sum + v.z);
-                        sum = rt<T>(sum + v.w);
-                    }
+                    sum = add_in_order<T>(sum, own.value[lane], batch);
                 }
                 landed();
             };
@@ -961,10 +955,15 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
             const uint32_t its_corner = (uint32_t)__builtin_amdgcn_readlane((int)corner, owner);
             const uint32_t its_len = (uint32_t)__builtin_amdgcn_readlane((int)len, owner);
             if ((from & run) != kNoKey) {
+                auto key_of = [&](uint32_t done) {
+                    const uint32_t i = done + (uint32_t)lane < its_len ? done + (uint32_t)lane : 0u;
+                    return run != kNoKey ? s_list[run + i] ^ its_corner : (uint32_t)s_sorted[from + i];
+                };
+                uint32_t k = key_of(0u);
                 for (uint32_t done = 0; done < its_len; done += 64u) {
-                    const uint32_t batch = its_len - done < 64u ? its_len - done : 64u;
-                    const uint32_t i = done + ((uint32_t)lane < batch ? (uint32_t)lane : 0u);
-                    add_batch(run != kNoKey ? s_list[run + i] ^ its_corner : (uint32_t)s_sorted[from + i], batch);
+                    const uint32_t next = key_of(done + 64u);
+                    add_batch(k, its_len - done < 64u ? its_len - done : 64u);
+                    k = next;
                 }
             } else {
                 merge_together(owner, lane, [&](uint32_t rank, uint32_t k) { own.order[rank] = (uint16_t)k; },

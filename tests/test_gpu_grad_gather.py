@@ -107,6 +107,31 @@ def test_volumes(oracle, device, aclnn, dtype, interp, pad):
         assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref)), (xs, out, span)
 
 
+# contributions of several cells: around the wavefront's steps of 64, and of the parts of 16 that it adds; channels of one
+# group of 16 and of two
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("interp", [0, 2])
+@pytest.mark.parametrize("channels,counts", [(1, (33, 47, 48, 49)), (17, (63, 64, 65, 80)), (5, (81, 128, 129, 200))])
+def test_crowded_elements(oracle, device, aclnn, dtype, interp, channels, counts):
+    import torch
+    rng = np.random.default_rng(4090 + interp)
+    xs, out = (2, channels, 32, 48), (45, 43)
+    at = rng.uniform(0, 1, (xs[0], out[0] * out[1], 2)) * (np.array(xs[:1:-1]) - 1)
+    for n in range(xs[0]):
+        free = iter(rng.permutation(out[0] * out[1]))
+        for e in range(12):
+            around = np.array([4 * e + 2, 9 * (e % 3) + 4])
+            for _ in range(counts[(e + n) % len(counts)]):
+                at[n, next(free)] = around + rng.uniform(-0.9, 0.9, 2)
+    g = ((2 * at + 1) / np.array(xs[:1:-1]) - 1).astype(np.float32).reshape((xs[0],) + out + (2,))
+    x, g, go = (I.cast_np(v, dtype) for v in (rng.standard_normal(xs).astype(np.float32), g, rng.standard_normal(xs[:2] + out).astype(np.float32)))
+    assert host_plans.gradient_tiles(dtype, interp, 1, xs, out[0] * out[1]) is None
+    ref, _ = oracle.grid_sampler2d_backward(go, x, g, interp, 1, False, dtype=I.oracle_code(dtype))
+    got, _ = aclnn.grid_sampler2d_backward(*(I.to_torch(v, dtype, device) for v in (go, x, g)), interp, 1, False, (True, False))
+    torch.cuda.synchronize()
+    assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref))
+
+
 def _group(dtype, interp, pad, xs, points, tiles, per_core=1):
     """items that the variant which takes the call runs at a time"""
     by_tiles = host_plans.gradient_tiles(dtype, interp, pad, xs, points, per_core)

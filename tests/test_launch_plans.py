@@ -151,7 +151,12 @@ TILES = [("fp32", 0, 0, (8, 3, 479, 637), 479 * 637, 178, 86), ("fp16", 0, 2, (1
          ("fp32", 0, 2, (1, 3, 704, 1152), 704 * 1152, 60, 62), ("fp32", 0, 0, (4, 3, 640, 1120), 640 * 1120, 125, 129),
          ("fp32", 0, 0, (4, 3, 608, 1024), 608 * 1024, 116, 114), ("fp32", 0, 2, (4, 3, 608, 1024), 608 * 1024, 131, 139),
          ("fp32", 0, 2, (4, 3, 600, 800), 600 * 800, 107, 99), ("fp32", 0, 0, (4, 4, 64, 128, 128), 64 * 128 * 128, 300, 461),
-         ("fp32", 0, 2, (4, 4, 48, 112, 128), 48 * 112 * 128, 272, 242)]
+         ("fp32", 0, 2, (4, 4, 48, 112, 128), 48 * 112 * 128, 272, 242),
+         # border padding, few items and channels
+         ("fp32", 0, 1, (2, 3, 248, 464), 248 * 464, 64, 105), ("fp32", 0, 1, (1, 1, 376, 632), 376 * 632, 67, 97),
+         ("fp32", 0, 1, (2, 6, 61, 54), 61 * 54, 39, 28), ("bf16", 0, 1, (1, 11, 191, 198), 97 * 100, 39, 27),
+         ("fp32", 0, 1, (3, 1, 520, 609), 605 * 708, 674, 380), ("fp32", 0, 1, (5, 2, 405, 480), 405 * 480, 260, 207),
+         ("fp32", 1, 1, (1, 2, 368, 624), 368 * 624, 47, 39), ("fp32", 1, 1, (2, 1, 408, 600), 792 * 1164, 540, 153)]
 
 
 @pytest.mark.parametrize("dtype,interp,pad,shape,points,lists,tiles", TILES)

@@ -48,7 +48,9 @@ constexpr int kPosBits = 11;           // a point's number in LDS, or kRecords: 
 constexpr int kTapBits = 3;
 constexpr uint32_t kNoKey = 0xFFFFFFFFu;
 constexpr uint32_t kNoPlace = 0xFFFFFFFFu;
-constexpr uint32_t kCountedRun = 32;   // runs of up to as many points are put in order by counting, longer ones by ballots
+// Runs of up to as many points are put in order by counting, longer ones by ballots.  32, 64 or 128: nearest, border padding,
+// 1x1x704x912 73 / 70 / 69, 2x6x136x208 20 / 21 / 22 us; 79 and 22 with 32 and one read of LDS after the other.
+constexpr uint32_t kCountedRun = 64;
 // Crowded elements are put in order by a lane each where more than kFewCrowded lanes of a wavefront have one of up to kSerialMost
 // contributions, otherwise one after the other by the wavefront, up to 64 * kRankedRegs contributions by counting.  A lane also
 // adds up to kSerialMost by itself where more lanes than kFewCrowded have as many.  Without the counting and with 192
@@ -811,8 +813,16 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
                     const uint32_t begin = s_start[cell[k]], end = s_start[cell[k] + 1u];
                     if (end - begin <= kCountedRun) {
                         uint32_t less = 0;
-                        for (uint32_t j = begin; j < end; j++) {
-                            less += (s_list[j] < own_key[k]) ? 1u : 0u;  // of one cell: in the order of their numbers
+                        for (uint32_t j = begin; j < end; j += 4u) {  // of one cell: in the order of their numbers
+                            uint32_t other[4];
+#pragma unroll
+                            for (uint32_t u = 0; u < 4u; u++) {
+                                other[u] = s_list[j + u < end ? j + u : begin];
+                            }
+#pragma unroll
+                            for (uint32_t u = 0; u < 4u; u++) {
+                                less += (j + u < end && other[u] < own_key[k]) ? 1u : 0u;
+                            }
                         }
                         place[k] = begin + less;
                     } else if (rank[k] == 0u) {
@@ -830,14 +840,23 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
             for (uint32_t r = (uint32_t)wave; r < s_longs; r += kWaves) {
                 const uint32_t c = s_long[r];
                 uint32_t to_list = s_start[c];
-                for (uint32_t i0 = 0; i0 < number; i0 += 64u) {
-                    const uint32_t i = i0 + (uint32_t)lane;
-                    const bool member = i < number && s_rare.points.cell[i < number ? i : 0u] == c;
-                    const uint64_t mask = __builtin_amdgcn_ballot_w64(member);
-                    if (member) {
-                        s_list[to_list + bits_below(mask)] = s_rare.points.key[i];
+                for (uint32_t i0 = 0; i0 < number; i0 += 256u) {
+                    uint32_t its_cell[4], key[4];
+#pragma unroll
+                    for (uint32_t u = 0; u < 4u; u++) {
+                        const uint32_t i = i0 + u * 64u + (uint32_t)lane;
+                        its_cell[u] = s_rare.points.cell[i < number ? i : 0u];
+                        key[u] = s_rare.points.key[i < number ? i : 0u];
                     }
-                    to_list += (uint32_t)__builtin_popcountll(mask);
+#pragma unroll
+                    for (uint32_t u = 0; u < 4u; u++) {
+                        const bool member = i0 + u * 64u + (uint32_t)lane < number && its_cell[u] == c;
+                        const uint64_t mask = __builtin_amdgcn_ballot_w64(member);
+                        if (member) {
+                            s_list[to_list + bits_below(mask)] = key[u];
+                        }
+                        to_list += (uint32_t)__builtin_popcountll(mask);
+                    }
                 }
             }
             __syncthreads();

@@ -11,7 +11,7 @@
 //           ascending order.  The points are counted by cell in LDS, every lane finds the runs of the cells that its
 //           element is a corner of, keys them (chunk, tap, number in LDS), sorts the keys in registers and folds
 //           weight times gradOutput, both from LDS, with the reference's roundings.  Elements with more contributions
-//           than keys are merged, run by run, a lane each, or where a single element holds hundreds by the whole
+//           than keys are merged, run by run, a lane each, or, where they are few or long, by the whole
 //           wavefront; more points than LDS holds are taken a run of segments after the other, which are whole chunks
 //           in ascending order.  Tiles that many points fall on are left to a third kernel (gs_grad_tiles_crowded.hip).
 //

@@ -226,12 +226,12 @@ __global__ __launch_bounds__(kThreads) void gs2d_grad_input_kernel(const T* __re
     }
 }
 
-template <typename T, int INTERP, bool TILED>
-__global__ __launch_bounds__(kGridTileThreads) void gs2d_grad_grid_kernel(const T* __restrict__ gout, const T* __restrict__ x,
+template <typename T, int INTERP, bool TILED, int THREADS>
+__global__ __launch_bounds__(THREADS) void gs2d_grad_grid_kernel(const T* __restrict__ gout, const T* __restrict__ x,
                                                                           const T* __restrict__ grid, T* __restrict__ dgrid,
                                                                           Grid2Params p)
 {
-    gs2d_grid_gradient_block<T, INTERP, TILED>(blockIdx.x, gout, x, grid, dgrid, p);
+    gs2d_grid_gradient_block<T, INTERP, TILED, THREADS>(blockIdx.x, gout, x, grid, dgrid, p);
 }
 
 GradGatherArgs gather_args(const GridSamplerGradArgs& a)
@@ -341,19 +341,30 @@ hipError_t launch_interp(const GridSamplerGradArgs& a, hipStream_t stream)
         }
     }
     if (a.dgrid != nullptr && !dgrid_done) {
-        const Grid2Launch g = grid2_launch(gather_args(a));
+        const GradGatherArgs ga = gather_args(a);
+        const bool spread = INTERP != 1 && a.N * ga.points <= kGridSpreadPoints;
+        const Grid2Launch g = grid2_launch(ga, spread ? kGridSpreadThreads : kGridTileThreads);
         if (!g.ok) {
             return hipErrorInvalidValue;
         }
+        const T *gout = (const T*)a.gout, *x = (const T*)a.x, *grid = (const T*)a.grid;
+        const dim3 blocks((unsigned)g.blocks), threads(kGridTileThreads);
         if constexpr (INTERP == 0) {
             if (g.tiled) {
-                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, true>), dim3((unsigned)g.blocks), dim3(kGridTileThreads), 0,
-                                   stream, (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, g.p);
+                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, true, kGridTileThreads>), blocks, threads, 0, stream, gout, x,
+                                   grid, (T*)a.dgrid, g.p);
                 return hipGetLastError();
             }
         }
-        hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, false>), dim3((unsigned)g.blocks), dim3(kGridTileThreads), 0, stream,
-                           (const T*)a.gout, (const T*)a.x, (const T*)a.grid, (T*)a.dgrid, g.p);
+        if constexpr (INTERP != 1) {
+            if (spread) {
+                hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, false, kGridSpreadThreads>), blocks, dim3(kGridSpreadThreads), 0, stream, gout, x, grid,
+                                   (T*)a.dgrid, g.p);
+                return hipGetLastError();
+            }
+        }
+        hipLaunchKernelGGL((gs2d_grad_grid_kernel<T, INTERP, false, kGridTileThreads>), blocks, threads, 0, stream, gout, x, grid,
+                           (T*)a.dgrid, g.p);
         return hipGetLastError();
     }
     return hipSuccess;

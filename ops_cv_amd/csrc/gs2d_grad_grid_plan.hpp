@@ -12,6 +12,14 @@ namespace opscv {
 constexpr int kGridTile = 16;  // square: a lane per grid point of 256
 constexpr int kGridTileThreads = kGridTile * kGridTile;
 
+// Few points are bound by the lines that a CU's loads touch, one wavefront's channel after the other: workgroups of a wavefront
+// bring them to four times as many CUs.  256 / 64 threads, grid gradient alone: bicubic fp32 10x54x32x24 -> 62x46 (28520 points)
+// 47.8 / 41.0 us, 13x8x24x42 -> 20x36 16.8 / 14.9, bilinear bf16 8x52x32x32 -> 61x61 9.9 / 8.5, fp16 3x39x61x51 9.1 / 8.2; beyond,
+// with more wavefronts than two a CU, it depends: 27x51x32x48 (41472 points) 9.9 / 10.8, bicubic 21x5x85x85 -> 45x45 (42525) 12.4 /
+// 11.2, 24x49x42x79 (79632) 15.5 / 19.8.  (A wavefront for either sum of 64 points instead: 47.6 / 48.4 on the first.)
+constexpr int64_t kGridSpreadPoints = 32768;
+constexpr int kGridSpreadThreads = 64;
+
 struct GridTilePlan {
     bool ok = false;
     int64_t tiles_x = 0, per_item = 0, tiles = 0;

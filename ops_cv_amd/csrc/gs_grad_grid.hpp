@@ -29,7 +29,7 @@ struct Grid2Launch {
     int64_t blocks = 0;  // of kGridTileThreads
 };
 
-inline Grid2Launch grid2_launch(const GradGatherArgs& a)
+inline Grid2Launch grid2_launch(const GradGatherArgs& a, int threads = kGridTileThreads)
 {
     Grid2Launch g;
     g.p.C = (int32_t)a.C;
@@ -47,9 +47,9 @@ inline Grid2Launch grid2_launch(const GradGatherArgs& a)
         g.p.by_tiles_x = make_fast_div((uint32_t)t.tiles_x);
         g.blocks = t.blocks;
     } else {
-        g.blocks = (g.p.total + kGridTileThreads - 1) / kGridTileThreads;
-        const int64_t per_item = a.points / kGridTileThreads;
-        g.p.blocks_per_item = (a.points % kGridTileThreads == 0 && a.N % 8 == 0 && per_item <= INT32_MAX) ? (int32_t)per_item : 0;
+        g.blocks = (g.p.total + threads - 1) / threads;
+        const int64_t per_item = a.points / threads;
+        g.p.blocks_per_item = (a.points % threads == 0 && a.N % 8 == 0 && per_item <= INT32_MAX) ? (int32_t)per_item : 0;
     }
     g.ok = g.blocks <= INT32_MAX;
     return g;
@@ -65,7 +65,7 @@ inline Grid2Launch grid2_launch(const GradGatherArgs& a)
 // together, in rows (grid_tile_plan): turned grids, one load after the other / together, fp32 8x3x479x637 114 / 115 us, 2x64x128x128
 // 72 / 62, 8x128x32x32 114 / 116, fp16 134 / 108, 156 / 62, 190 / 101; points at random, whose lines are seldom in the cache, fp32
 // 393 / 395, 118 / 125, 108 / 117, fp16 373 / 370, 154 / 107, 188 / 115.
-template <typename T, int INTERP, bool TILED>
+template <typename T, int INTERP, bool TILED, int THREADS = kGridTileThreads>
 __device__ __forceinline__ void gs2d_grid_gradient_block(uint32_t block_index, const T* __restrict__ gout, const T* __restrict__ x,
                                                          const T* __restrict__ grid, T* __restrict__ dgrid, const Grid2Params& p)
 {
@@ -99,7 +99,7 @@ __device__ __forceinline__ void gs2d_grid_gradient_block(uint32_t block_index, c
             const uint32_t xcd = block_index & 7u, i = block_index >> 3;
             block = ((i / (uint32_t)p.blocks_per_item) * 8u + xcd) * (uint32_t)p.blocks_per_item + i % (uint32_t)p.blocks_per_item;
         }
-        idx = (int64_t)block * kGridTileThreads + threadIdx.x;
+        idx = (int64_t)block * THREADS + threadIdx.x;
         if (idx >= p.total) {
             return;
         }

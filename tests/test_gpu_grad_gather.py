@@ -205,3 +205,19 @@ def test_groups_of_items_in_a_graph(device, aclnn, n, plane, tiles):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(dx, want[i][0]) and torch.equal(dg, want[i][1]), i
+
+
+# the grid gradient of few points, by workgroups of one wavefront: a wavefront's points of two items, an item's workgroups on one
+# XCD, the most points of that launch and one row more
+@pytest.mark.parametrize("dtype", ["fp32", "fp16"])
+@pytest.mark.parametrize("interp", [0, 2])
+@pytest.mark.parametrize("xs,out", [((3, 5, 9, 11), (7, 13)), ((8, 3, 12, 10), (16, 8)), ((8, 9, 20, 31), (64, 64)), ((8, 9, 20, 31), (65, 64))])
+def test_grid_gradient_of_few_points(oracle, device, aclnn, dtype, interp, xs, out):
+    import torch
+    rng = np.random.default_rng(4099 + interp)
+    x, go = (I.cast_np(rng.standard_normal(s).astype(np.float32), dtype) for s in (xs, xs[:2] + out))
+    g = I.cast_np(_grid2d(rng, "random", xs[0], *out), dtype)
+    _, ref = oracle.grid_sampler2d_backward(go, x, g, interp, 0, False, dtype=I.oracle_code(dtype))
+    _, got = aclnn.grid_sampler2d_backward(*(I.to_torch(v, dtype, device) for v in (go, x, g)), interp, 0, False, (False, True))
+    torch.cuda.synchronize()
+    assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref))

@@ -17,13 +17,18 @@
 //           registers and folds gradOutput times weight in that order with the reference's roundings, every channel
 //           from the same list.  Elements with more contributions (border padding piles points up on the edges) go to a
 //           list of their own; meanwhile spare workgroups sort the runs of more than 64 entries.
-//   crowded one wavefront per listed element: merges the element's runs, 64 entries at a time, in the reference's
-//           order; the lanes compute the 64 contributions of a channel at once and one lane adds them up in order.
+//   crowded one wavefront per listed element: puts up to 128 contributions in order by counting the lesser keys of each, more
+//           by merging the element's runs, 64 entries at a time; the lanes compute the 64 contributions of a channel at
+//           once and one lane adds them up in the reference's order.
 //           A chain of waits, so everything that does not depend on the sums is on its way before them: the runs' next
 //           entries, the next channels' gradOutput, the operands of the additions; the places of two runs' entries in
-//           each other are found together, by a fixed number of steps.  Both gradients before / so, border padding: fp32
-//           4x2x600x736 721 / 440 us, 3x1x520x609 -> 605x708 1031 / 674, 4x2x301x505 378 / 268, 3x3x210x328 182 / 132, fp16 2x4x360x552
-//           95 / 82; nearest fp32 3x2x304x576 222 / 144.
+//           each other are found together, in as many steps as the longer one takes.  Both gradients, every step waited for in
+//           turn / so, border padding: fp32 4x2x600x736 721 / 440 us, 3x1x520x609 -> 605x708 1031 / 674, 4x2x301x505 378 / 268,
+//           3x3x210x328 182 / 132, fp16 2x4x360x552 95 / 82; nearest fp32 3x2x304x576 222 / 144.
+//           Dense grids have many elements of a few contributions more than a list, where the steps of full runs were most
+//           of the time.  This kernel, every step in turn / always steps for 64 entries and 64 additions / so: fp16 5x3x41x32x44
+//           -> 57x45x62 reflection 134 / 225 / 74, 22x2x10x85x61 -> 14x125x89 1254 / 1801 / 609, fp32 12x3x32x58x57 ->
+//           39x71x69 border 251 / 317 / 107; bicubic (one run) 1x3x231x430 -> 323x602 138 / 217 / 116.
 //
 // Input gradient of fp32 8x3x479x637 from as many grid points (rotations of up to 30 degrees): 2568 us with elections;
 // here clear 6, count 43, place 14, fill 13, gather 107, crowded 5 us.  Count is bound by the rate of atomics (55 G/s;
@@ -52,6 +57,7 @@ constexpr int kPlaceCells = 8;       // cells per lane of the place kernel
 constexpr int kPlaceThreads = 256;
 constexpr int kFoldPitch = 68;       // of a channel's contributions in LDS: on the 16-byte grid, channels at different banks
 constexpr int kFoldChans = 16;       // channels whose contributions a crowded element's wavefront computes together
+constexpr uint32_t kCountedMost = 128;  // contributions of several runs that are put in order by counting, longer ones by merging
 constexpr uint32_t kNoRank = 0xFFFFFFFFu;
 
 // Grid points per lane of the count and fill kernels: the atomics and the scattered stores of several are on their way
@@ -519,8 +525,8 @@ __global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __
     typedef Mode<DIM, INTERP> M;
     constexpr int R = M::kRuns;
     constexpr int kWaves = kThreads / 64;
-    __shared__ uint32_t s_window[kWaves][R][64];  // short runs, sorted
-    __shared__ uint32_t s_key[kWaves][64];        // the next 64 keys in order
+    __shared__ uint32_t s_window[kWaves][R][64];      // short runs, sorted
+    __shared__ uint32_t s_key[kWaves][kCountedMost];  // keys in order: the next 64, or all
     __shared__ __align__(16) float s_val[kWaves][kFoldChans][kFoldPitch];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int64_t n = blockIdx.y;
@@ -548,11 +554,58 @@ __global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __
         uint32_t skip[R];         // entries of a short run already taken
 #pragma unroll
         for (int r = 0; r < R; r++) {
+            start[r] = (uint32_t)__builtin_amdgcn_readfirstlane((int)start[r]);
+            left[r] = (uint32_t)__builtin_amdgcn_readfirstlane((int)left[r]);
             total += left[r];
             whole[r] = left[r] <= kSortedRun;
             skip[r] = 0u;
             from[r] = wsn + (whole[r] ? p.lay.list : p.lay.ranks) + start[r];
-            if (whole[r] && left[r] > 0u) {
+        }
+        const bool counted = R > 1 && total <= kCountedMost;
+        if (counted) {
+            // a key or two a lane, whose place is the number of lesser ones
+            constexpr int kRegs = (int)(kCountedMost / 64u);
+            uint32_t own[kRegs], rank[kRegs];
+#pragma unroll
+            for (int m = 0; m < kRegs; m++) {
+                const uint32_t i = (uint32_t)(m * 64 + lane);
+                uint32_t before = 0, run = 0, at = 0;
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    if (i >= before) {
+                        run = (uint32_t)r;
+                        at = (uint32_t)(from[r] - wsn) + i - before;
+                    }
+                    before += left[r];
+                }
+                own[m] = (i < total) ? M::key(wsn[at], run) : 0xFFFFFFFFu;
+                rank[m] = 0u;
+            }
+#pragma unroll
+            for (int m = 0; m < kRegs; m++) {
+                const uint32_t most = total > (uint32_t)(m * 64) ? total - (uint32_t)(m * 64) : 0u;
+                const uint32_t here = most < 64u ? most : 64u;
+                for (uint32_t j = 0; j < here; j += 8u) {
+#pragma unroll
+                    for (uint32_t u = 0; u < 8u; u++) {
+                        const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)own[m], (int)(j + u));
+#pragma unroll
+                        for (int q = 0; q < kRegs; q++) {
+                            rank[q] += (other < own[q]) ? 1u : 0u;
+                        }
+                    }
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < kRegs; m++) {
+                if ((uint32_t)(m * 64 + lane) < total) {
+                    keys[rank[m]] = own[m];
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            if (!counted && whole[r] && left[r] > 0u) {
                 const bool have = (uint32_t)lane < left[r];
                 const uint32_t v = have ? from[r][lane] : 0xFFFFFFFFu;
                 uint32_t rank = 0;
@@ -571,69 +624,78 @@ __global__ __launch_bounds__(kThreads) void gs_gather_crowded_kernel(const T* __
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 ahead[r] = 0xFFFFFFFFu;
-                if (!whole[r] && (uint32_t)lane < left[r]) {
+                if (!counted && !whole[r] && (uint32_t)lane < left[r]) {
                     ahead[r] = from[r][lane];
                 }
             }
         };
         look_ahead();
-        float acc = 0.0f;  // of channel c_first + lane
+        uint32_t taken_before = 0;  // of the keys
+        float acc = 0.0f;           // of channel c_first + lane
         while (total > 0u) {
-            // the next entries of every run, and behind a run's last one an entry beyond all
-            uint32_t mine[R], held[R], rank[R];
+            const uint32_t batch = total < 64u ? total : 64u;
+            if (!counted) {
+                // the next entries of every run, and behind a run's last one an entry beyond all
+                uint32_t mine[R], held[R], rank[R];
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                held[r] = left[r] < 64u ? left[r] : 64u;
-                mine[r] = ahead[r];
-                if (whole[r] && (uint32_t)lane < held[r]) {
-                    mine[r] = window[r][skip[r] + lane];
+                for (int r = 0; r < R; r++) {
+                    held[r] = left[r] < 64u ? left[r] : 64u;
+                    mine[r] = ahead[r];
+                    if (whole[r] && (uint32_t)lane < held[r]) {
+                        mine[r] = window[r][skip[r] + lane];
+                    }
+                    rank[r] = (uint32_t)lane;
                 }
-                rank[r] = (uint32_t)lane;
-            }
-            // the rank of every one of them among all: entries of another run come first when their chunk is earlier, or the
-            // same and their corner's number lower
+                // the rank of every one of them among all: entries of another run come first when their chunk is earlier, or the
+                // same and their corner's number lower
 #pragma unroll
-            for (int r = 0; r < R; r++) {
+                for (int r = 0; r < R; r++) {
 #pragma unroll
-                for (int o = 0; o < r; o++) {
-                    if (held[r] > 0u && held[o] > 0u) {
-                        // how many of run o lie before this lane's entry of run r, and of run r before its entry of run o
-                        const uint32_t in_r = mine[r] >> 8, in_o = mine[o] >> 8;
-                        uint32_t less_o = 0, less_r = 0;
+                    for (int o = 0; o < r; o++) {
+                        if (held[r] > 0u && held[o] > 0u) {
+                            const uint32_t longest = held[r] > held[o] ? held[r] : held[o];
+                            // how many of run o lie before this lane's entry of run r, and of run r before its entry of run o
+                            const uint32_t in_r = mine[r] >> 8, in_o = mine[o] >> 8;
+                            uint32_t less_o = 0, less_r = 0;
 #pragma unroll
-                        for (uint32_t d = 32; d > 0u; d >>= 1) {
-                            const uint32_t chunk_o = (uint32_t)__shfl((int)in_o, (int)(less_o + d - 1u));
-                            const uint32_t chunk_r = (uint32_t)__shfl((int)in_r, (int)(less_r + d - 1u));
-                            less_o += (chunk_o <= in_r) ? d : 0u;
-                            less_r += (chunk_r < in_o) ? d : 0u;
+                            for (uint32_t d = 32; d > 0u; d >>= 1) {
+                                if (d > longest) {
+                                    continue;
+                                }
+                                const uint32_t chunk_o = (uint32_t)__shfl((int)in_o, (int)(less_o + d - 1u));
+                                const uint32_t chunk_r = (uint32_t)__shfl((int)in_r, (int)(less_r + d - 1u));
+                                less_o += (chunk_o <= in_r) ? d : 0u;
+                                less_r += (chunk_r < in_o) ? d : 0u;
+                            }
+                            if (longest == 64u) {  // the last one
+                                less_o += ((uint32_t)__shfl((int)in_o, (int)less_o) <= in_r) ? 1u : 0u;
+                                less_r += ((uint32_t)__shfl((int)in_r, (int)less_r) < in_o) ? 1u : 0u;
+                            }
+                            rank[r] += less_o;
+                            rank[o] += less_r;
                         }
-                        // the last of 64
-                        less_o += ((uint32_t)__shfl((int)in_o, (int)less_o) <= in_r) ? 1u : 0u;
-                        less_r += ((uint32_t)__shfl((int)in_r, (int)less_r) < in_o) ? 1u : 0u;
-                        rank[r] += less_o;
-                        rank[o] += less_r;
                     }
                 }
-            }
-            const uint32_t batch = total < 64u ? total : 64u;
 #pragma unroll
-            for (int r = 0; r < R; r++) {
-                const bool take = (uint32_t)lane < held[r] && rank[r] < batch;
-                if (take) {
-                    keys[rank[r]] = M::key(mine[r], r);
+                for (int r = 0; r < R; r++) {
+                    const bool take = (uint32_t)lane < held[r] && rank[r] < batch;
+                    if (take) {
+                        keys[rank[r]] = M::key(mine[r], r);
+                    }
+                    const uint32_t taken = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(take));
+                    left[r] -= taken;
+                    if (whole[r]) {
+                        skip[r] += taken;
+                    } else {
+                        from[r] += taken;
+                    }
                 }
-                const uint32_t taken = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(take));
-                left[r] -= taken;
-                if (whole[r]) {
-                    skip[r] += taken;
-                } else {
-                    from[r] += taken;
-                }
+                look_ahead();
             }
-            look_ahead();
             total -= batch;
             landed();
-            const uint32_t key = keys[(uint32_t)lane < batch ? lane : 0];
+            const uint32_t key = keys[taken_before + ((uint32_t)lane < batch ? (uint32_t)lane : 0u)];
+            taken_before += counted ? batch : 0u;
             const uint32_t pt = M::q_of(key) - phase;
             const float w = weight_of<T, DIM, INTERP>(coords[pt], M::tap_of(key), x, y, z);
             const T* go = gout + (n * p.C + c_first) * (int64_t)p.points + pt;

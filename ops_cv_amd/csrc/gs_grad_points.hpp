@@ -122,7 +122,9 @@ __device__ __forceinline__ float add_in_order(float sum, const float* values, ui
         if (count > 32u) {
             load(b, 48);
             add(a);
-            add(b);
+            if (count > 48u) {
+                add(b);
+            }
         }
     }
     return sum;

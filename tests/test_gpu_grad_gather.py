@@ -132,6 +132,32 @@ def test_crowded_elements(oracle, device, aclnn, dtype, interp, channels, counts
     assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref))
 
 
+# the same of the eight runs of a voxel: up to 128 are put in order by counting, more by merging; around every other voxel all
+# points are in one cell, whose run is sorted apart from 65 on.  Many channels, and more points than the tiles take
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("xs,out,counts", [((2, 26, 8, 16, 16), (10, 14, 14), (40, 63, 64, 65)), ((1, 2, 6, 12, 12), (9, 14, 14), (100, 126, 127, 128, 129)),
+                                           ((1, 3, 6, 12, 12), (20, 20, 20), (130, 190, 260, 700))])
+def test_crowded_voxels(oracle, device, aclnn, dtype, xs, out, counts):
+    import torch
+    rng = np.random.default_rng(4095)
+    points, extent = int(np.prod(out)), np.array(xs[:1:-1])
+    assert host_plans.gradient_tiles(dtype, 0, 1, xs, points) is None
+    at = rng.uniform(0, 1, (xs[0], points, 3)) * (extent - 1)
+    for n in range(xs[0]):
+        free = iter(rng.permutation(points))
+        for e in range(9):
+            around = np.array([3 * (e % 3) + 3, 3 * (e // 3) + 3, 3])
+            for _ in range(counts[(e + n) % len(counts)]):
+                at[n, next(free)] = around + (rng.uniform(0.1, 0.9, 3) if e % 2 else rng.uniform(-0.9, 0.9, 3))
+    g = ((2 * at + 1) / extent - 1).astype(np.float32).reshape((xs[0],) + out + (3,))
+    x, g, go = (I.cast_np(v, dtype) for v in (rng.standard_normal(xs).astype(np.float32), g, rng.standard_normal(xs[:2] + out).astype(np.float32)))
+    ref, _ = oracle.grid_sampler3d_backward(go, x, g, 0, 1, False, dtype=I.oracle_code(dtype))
+    with aclnn.option("gs3d_grad_variant", 3):
+        got, _ = aclnn.grid_sampler3d_backward(*(I.to_torch(v, dtype, device) for v in (go, x, g)), 0, 1, False, (True, False))
+    torch.cuda.synchronize()
+    assert np.array_equal(_bits(I.from_torch(got, dtype)), _bits(ref))
+
+
 def _group(dtype, interp, pad, xs, points, tiles, per_core=1):
     """items that the variant which takes the call runs at a time"""
     by_tiles = host_plans.gradient_tiles(dtype, interp, pad, xs, points, per_core)

@@ -1,6 +1,6 @@
 // Backward of the bilinear resize for gfx950, planes (NCHW): incoming rows in registers, several outgoing rows at a time.
 //
-// Same visits, products and order of the sum as resize_grad_kernel (resize_grad.hip): an outgoing element visits up to ten
+// Same visits, products and order of the sum as resize_grad_kernel (resize_grad.hip): an outgoing element visits up to twelve
 // rows and columns of the incoming gradient, in row-major order.  A lane owns a column of a plane -- the columns of all planes
 // side by side, so that no wavefront is cut by a plane's last column -- and keeps the weights of the columns it visits; a
 // wavefront goes down the incoming rows by itself, without barriers.  A row is loaded in aligned units of 16 bytes, three rows
@@ -301,6 +301,8 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_rows_kernel(const TI
     };
     bool done = false;
     if (any(nx > kRowsColumns)) {
+    } else if (any(nx > 10)) {
+        done = width(std::integral_constant<int, kRowsColumns>{});
     } else if (any(nx > 8)) {
         done = width(std::integral_constant<int, 10>{});
     } else if (any(nx > 6)) {
@@ -334,13 +336,13 @@ hipError_t run_typed(const ResizeGradArgs& a, const RowsPlan& p, hipStream_t str
                        a.inv_scale_w, a.half_pixel ? 0.5f : 0.0f)
     if (p.two) {
         if (p.tall) {
-            OPSCV_RGR(true, 10);
+            OPSCV_RGR(true, kRowsColumns);
         } else {
             OPSCV_RGR(true, 8);
         }
     } else {
         if (p.tall) {
-            OPSCV_RGR(false, 10);
+            OPSCV_RGR(false, kRowsColumns);
         } else {
             OPSCV_RGR(false, 8);
         }

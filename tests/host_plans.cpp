@@ -72,6 +72,13 @@ int resize_grad_rows(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t H
     return p.ok ? 1 : 0;
 }
 
+// most rows, and columns, an outgoing element may visit in the rows kernel
+int resize_grad_rows_visits(int64_t* out)
+{
+    out[0] = kRowsColumns;
+    return 1;
+}
+
 // estimates of the input gradient of planes (nanoseconds): elections, sorting; 0 where the elections run
 int sorting_takes_planes(int elem, int64_t interp, int64_t N, int64_t C, int64_t H, int64_t W, int64_t points, int64_t* out)
 {

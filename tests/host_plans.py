@@ -46,6 +46,13 @@ def resize_grad_rows(dtype, planes, small, large, align=False):
     return _call("resize_grad_rows", 3, dtype, planes, *small, *large, int(align))
 
 
+def resize_grad_rows_visits():
+    """Most rows, and columns, of the incoming gradient that an outgoing element may visit in the rows kernel."""
+    out = (ctypes.c_int64 * 1)()
+    assert lib().resize_grad_rows_visits(out) == 1
+    return out[0]
+
+
 def sorting_takes_planes(dtype, interp, shape, points):
     """(elections, sorting): estimated nanoseconds of the input gradient of (N, C, H, W) planes sampled at `points` points
     an item, None where the elections run."""

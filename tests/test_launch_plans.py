@@ -2,6 +2,7 @@
 holds fewer than 2^24 of them."""
 import random
 
+import numpy as np
 import pytest
 
 import host_plans as P
@@ -84,6 +85,27 @@ RESIZES = [(131072, (3, 3), (7, 7), 19.4, 142), (16384, (20, 5), (41, 11), 24.9,
 @pytest.mark.parametrize("planes,small,large,gather,tiles", RESIZES)
 def test_resize_gradient_of_odd_rows_takes_the_faster_of_two_kernels(dtype, planes, small, large, gather, tiles):
     assert (P.resize_grad_planes(dtype, planes, small, large) is not None) == (tiles < gather)
+
+
+@pytest.mark.parametrize("align", [False, True])
+def test_resize_gradient_rows_hold_what_an_element_visits(align):
+    """growth by four and five, where rounding adds a row or column to 2 / scale: the visits of every element, stepped in single
+    precision as the kernels do"""
+    f, most = np.float32, 0
+    assert P.resize_grad_rows("fp32", 4, (100, 100), (496, 496) if align else (500, 500), align) is not None
+    for growth in (4, 5):
+        for n in range(16, 260, 3):
+            large = growth * (n - 1) + 1 if align else growth * n
+            scale = f(n - 1) / f(large - 1) if align else f(n) / f(large)
+            offset = f(0.0 if align else 0.5)
+            i = np.arange(n, dtype=f)
+            start = np.clip(np.ceil((i - f(1) + offset) * (f(1) / scale) - offset), 0, large)
+            at, visits = (start + offset) * scale - offset, np.zeros(n, int)
+            for k in range(16):
+                visits += (at < i + f(1)) & (start + k < large) & (visits == k)
+                at = at + scale
+            most = max(most, visits.max())
+    assert most == 11 and most <= P.resize_grad_rows_visits()
 
 
 # (bytes of a unit, rows, shrunk, align corners, in pairs): microseconds with kept rows / in pairs

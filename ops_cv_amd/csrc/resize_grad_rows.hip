@@ -36,7 +36,7 @@ __device__ __forceinline__ void wave_fence()
     __builtin_amdgcn_wave_barrier();
 }
 
-// TWO: a lane moves up to two 16-byte units of a row, else one.
+// TWO: a lane moves up to two 16-byte units of a row, else one.  VISITS: most rows that an element visits (RowsPlan::visits).
 template <typename TI, typename TO, bool TWO, int VISITS>
 __global__ __launch_bounds__(kGradThreads) void resize_grad_rows_kernel(const TI* __restrict__ g, TO* __restrict__ y,
                                                                          uint32_t columns, FastDiv by_ws, FastDiv by_groups,
@@ -300,9 +300,9 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_rows_kernel(const TI
         return any(nx < decltype(kx)::value) ? sums(kx, std::true_type{}) : sums(kx, std::false_type{});
     };
     bool done = false;
-    if (any(nx > kRowsColumns)) {
-    } else if (any(nx > 10)) {
-        done = width(std::integral_constant<int, kRowsColumns>{});
+    if (any(nx > (VISITS == kRowsColumns ? kRowsColumns : 10))) {
+    } else if (VISITS == kRowsColumns && any(nx > 10)) {
+        done = width(std::integral_constant<int, VISITS == kRowsColumns ? kRowsColumns : 10>{});
     } else if (any(nx > 8)) {
         done = width(std::integral_constant<int, 10>{});
     } else if (any(nx > 6)) {
@@ -335,16 +335,16 @@ hipError_t run_typed(const ResizeGradArgs& a, const RowsPlan& p, hipStream_t str
                        (int32_t)a.Hs, (int32_t)a.Ws, (int32_t)a.Hd, (int32_t)a.Wd, a.scale_h, a.scale_w, a.inv_scale_h,      \
                        a.inv_scale_w, a.half_pixel ? 0.5f : 0.0f)
     if (p.two) {
-        if (p.tall) {
-            OPSCV_RGR(true, kRowsColumns);
-        } else {
-            OPSCV_RGR(true, 8);
+        switch (p.visits) {
+            case kRowsColumns: OPSCV_RGR(true, kRowsColumns); break;
+            case 10: OPSCV_RGR(true, 10); break;
+            default: OPSCV_RGR(true, 8); break;
         }
     } else {
-        if (p.tall) {
-            OPSCV_RGR(false, kRowsColumns);
-        } else {
-            OPSCV_RGR(false, 8);
+        switch (p.visits) {
+            case kRowsColumns: OPSCV_RGR(false, kRowsColumns); break;
+            case 10: OPSCV_RGR(false, 10); break;
+            default: OPSCV_RGR(false, 8); break;
         }
     }
 #undef OPSCV_RGR

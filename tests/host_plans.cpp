@@ -61,14 +61,14 @@ int resize_grad_planes(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t
     return t.rows > 0 ? 1 : 0;
 }
 
-// rows of a wavefront, whether a lane moves two units of a row, whether an element may visit more than eight rows; 0 where the
+// rows of a wavefront, whether a lane moves two units of a row, rows an element may visit; 0 where the
 // rows kernel is not taken
 int resize_grad_rows(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int align, int64_t* out)
 {
     const RowsPlan p = rows_plan(resize_grad_args(elem, planes, Hs, Ws, Hd, Wd, align));
     out[0] = p.rows;
     out[1] = p.two ? 1 : 0;
-    out[2] = p.tall ? 1 : 0;
+    out[2] = p.visits;
     return p.ok ? 1 : 0;
 }
 

@@ -41,8 +41,7 @@ def resize_grad_planes(dtype, planes, small, large, align=False):
 
 
 def resize_grad_rows(dtype, planes, small, large, align=False):
-    """(outgoing rows of a wavefront, whether a lane moves two units of a row, whether an element may visit more than eight
-    rows) of the resize gradient's rows kernel, None where it is not taken."""
+    """(outgoing rows of a wavefront, whether a lane moves two units of a row, rows that an element may visit) of the resize gradient's rows kernel, None where it is not taken."""
     return _call("resize_grad_rows", 3, dtype, planes, *small, *large, int(align))
 
 

@@ -811,56 +811,38 @@ hipError_t run_planes(const ResizeGradArgs& a, const PlaneTile& t, hipStream_t s
 template <typename TI, typename TO>
 hipError_t run(const ResizeGradArgs& a, hipStream_t stream)
 {
-    const RowsPlan rows = rows_plan(a);
-    if (rows.ok) {
-        return run_resize_grad_rows(a, rows, stream);
+    const ResizeGradPlan plan = resize_grad_plan(a);
+    if (plan.kernel == ResizeGradKernel::Rows) {
+        return run_resize_grad_rows(a, plan.rows, stream);
     }
-    const PlaneTile planes_tile = plane_tile(a);
-    if (planes_tile.rows > 0) {
-        return run_planes<TI, TO>(a, planes_tile, stream);
+    if (plan.kernel == ResizeGradKernel::Planes) {
+        return run_planes<TI, TO>(a, plan.planes, stream);
     }
-    constexpr int32_t kCapWords = kGradCapWords;
-    int32_t lds_words = kCapWords;
-    const int32_t tile_rows = lds_tile_rows(a, kCapWords, &lds_words);
-    // the allocation follows the estimate so that more workgroups share a CU (their load and compute phases overlap);
-    // a rectangle that turns out larger than the estimate is read from global memory by the kernel
-    lds_words = (lds_words + 63) / 64 * 64;
-    lds_words = lds_words < kCapWords ? lds_words : kCapWords;
-    if (tile_rows > 0) {
-        const int64_t ci = a.channels_last ? a.C : 1;
+    if (plan.kernel == ResizeGradKernel::Lds) {
+        const LdsTile& t = plan.lds;
+        const int32_t ci = (int32_t)(a.channels_last ? a.C : 1);
         const int64_t planes = a.channels_last ? a.N : a.N * a.C;
-        const int64_t row_elems = a.Ws * ci;
-        // A workgroup walks over several planes with the tile geometry and column weights it computed once; enough
-        // workgroups are launched to keep every CU supplied (kWantBlocks), the rest of the planes are looped over.
-        const int64_t tiles = ((row_elems + kGradTileCols - 1) / kGradTileCols) * ((a.Hs + tile_rows - 1) / tile_rows);
-        int64_t zdim = (kWantBlocks + tiles - 1) / tiles;
-        zdim = zdim < planes ? zdim : planes;
-        zdim = zdim < 65535 ? zdim : 65535;
-        const int64_t tiles_x = (row_elems + kGradTileCols - 1) / kGradTileCols, tiles_y = (a.Hs + tile_rows - 1) / tile_rows;
-        const int64_t blocks = (tiles * zdim + 7) / 8 * 8;  // padded for the XCD mapping of the kernel
-        if (tiles_y <= 65535 && fits_launch(blocks, kGradThreads)) {
-            const dim3 grid((unsigned)blocks);
 #define OPSCV_RGL(HP, IL)                                                                                            \
-    hipLaunchKernelGGL((resize_grad_lds_kernel<TI, TO, HP, IL>), grid, dim3(kGradThreads), lds_words * 4, stream,     \
+    hipLaunchKernelGGL((resize_grad_lds_kernel<TI, TO, HP, IL>), dim3((unsigned)t.blocks), dim3(kGradThreads),           \
+                       t.lds_words * 4, stream,                                                                      \
                        (const TI*)a.x, (TO*)a.y, planes, (int32_t)a.Hs, (int32_t)a.Ws, (int32_t)a.Hd, (int32_t)a.Wd, \
-                       a.scale_h, a.scale_w, a.inv_scale_h, a.inv_scale_w, tile_rows, lds_words, -0.0f,              \
-                       (uint32_t)tiles_x, (uint32_t)tiles_y, (uint32_t)zdim, (int32_t)ci)
-            if (a.half_pixel) {
-                if (a.channels_last) {
-                    OPSCV_RGL(true, true);
-                } else {
-                    OPSCV_RGL(true, false);
-                }
+                       a.scale_h, a.scale_w, a.inv_scale_h, a.inv_scale_w, t.rows, t.lds_words, -0.0f,               \
+                       (uint32_t)t.tiles_x, (uint32_t)t.tiles_y, (uint32_t)t.slots, ci)
+        if (a.half_pixel) {
+            if (a.channels_last) {
+                OPSCV_RGL(true, true);
             } else {
-                if (a.channels_last) {
-                    OPSCV_RGL(false, true);
-                } else {
-                    OPSCV_RGL(false, false);
-                }
+                OPSCV_RGL(true, false);
             }
-#undef OPSCV_RGL
-            return hipGetLastError();
+        } else {
+            if (a.channels_last) {
+                OPSCV_RGL(false, true);
+            } else {
+                OPSCV_RGL(false, false);
+            }
         }
+#undef OPSCV_RGL
+        return hipGetLastError();
     }
     const int64_t total = a.N * a.C * a.Hs * a.Ws;
     int64_t blocks = (total + kGradThreads - 1) / kGradThreads;
@@ -898,15 +880,14 @@ hipError_t run(const ResizeGradArgs& a, hipStream_t stream)
 
 const char* resize_grad_variant(const ResizeGradArgs& a)
 {
-    if (a.user_scales) {
-        return "resize_grad_gather_scales";
+    switch (resize_grad_plan(a).kernel) {
+        case ResizeGradKernel::Scales: return "resize_grad_gather_scales";
+        case ResizeGradKernel::Rows: return "resize_grad_rows";
+        case ResizeGradKernel::Planes:
+        case ResizeGradKernel::Lds: return "resize_grad_lds";
+        case ResizeGradKernel::Gather: break;
     }
-    if (plane_tile(a).rows > 0) {
-        return "resize_grad_lds";
-    }
-    constexpr int32_t kCapWords = kGradCapWords;
-    const int32_t rows = lds_tile_rows(a, kCapWords);
-    return (rows > 0 && (a.Hs + rows - 1) / rows <= 65535) ? "resize_grad_lds" : "resize_grad_gather";
+    return "resize_grad_gather";
 }
 
 hipError_t launch_resize_grad(const ResizeGradArgs& a, hipStream_t stream)

@@ -42,6 +42,39 @@ inline int32_t lds_tile_rows(const ResizeGradArgs& a, int32_t cap_words, int32_t
     return 0;
 }
 
+struct LdsTile {
+    int32_t rows = 0;      // 0: the variant does not apply
+    int32_t lds_words = 0;
+    int64_t tiles_x = 0, tiles_y = 0;
+    int64_t slots = 0;     // workgroups per tile; each takes every slots-th plane
+    int64_t blocks = 0;    // padded for the XCD mapping of the kernel
+};
+
+inline LdsTile lds_tile(const ResizeGradArgs& a)
+{
+    LdsTile t;
+    const int32_t rows = lds_tile_rows(a, kGradCapWords, &t.lds_words);
+    if (rows <= 0) {
+        return t;
+    }
+    // the allocation follows the estimate so that more workgroups share a CU (their load and compute phases overlap);
+    // a rectangle that turns out larger than the estimate is read from global memory by the kernel
+    t.lds_words = (t.lds_words + 63) / 64 * 64;
+    t.lds_words = t.lds_words < kGradCapWords ? t.lds_words : kGradCapWords;
+    const int64_t planes = a.channels_last ? a.N : a.N * a.C, row_elems = a.Ws * (a.channels_last ? a.C : 1);
+    t.tiles_x = (row_elems + kGradTileCols - 1) / kGradTileCols;
+    t.tiles_y = (a.Hs + rows - 1) / rows;
+    // A workgroup walks over several planes with the tile geometry and column weights it computed once; enough
+    // workgroups are launched to keep every CU supplied (kWantBlocks), the rest of the planes are looped over.
+    const int64_t tiles = t.tiles_x * t.tiles_y;
+    t.slots = (kWantBlocks + tiles - 1) / tiles;
+    t.slots = t.slots < planes ? t.slots : planes;
+    t.slots = t.slots < 65535 ? t.slots : 65535;
+    t.blocks = (tiles * t.slots + 7) / 8 * 8;
+    t.rows = (t.tiles_y <= 65535 && fits_launch(t.blocks, kGradThreads)) ? rows : 0;
+    return t;
+}
+
 // ---- resize_grad_planes_kernel ----
 constexpr int kPlaneCols = 64;
 constexpr int kPlaneVisits = 8;                 // most rows, and most columns, an outgoing element may visit
@@ -230,6 +263,31 @@ inline RowsPlan rows_plan(const ResizeGradArgs& a)
     r.blocks = (tiles * groups + 7) / 8 * 8;
     r.ok = fits_launch(r.blocks, kGradThreads);
     return r;
+}
+
+// ---- the kernel of a call ----
+enum class ResizeGradKernel { Scales, Rows, Planes, Lds, Gather };
+
+struct ResizeGradPlan {
+    ResizeGradKernel kernel = ResizeGradKernel::Gather;
+    RowsPlan rows;
+    PlaneTile planes;
+    LdsTile lds;
+};
+
+inline ResizeGradPlan resize_grad_plan(const ResizeGradArgs& a)
+{
+    ResizeGradPlan p;
+    if (a.user_scales) {
+        p.kernel = ResizeGradKernel::Scales;
+    } else if (p.rows = rows_plan(a); p.rows.ok) {
+        p.kernel = ResizeGradKernel::Rows;
+    } else if (p.planes = plane_tile(a); p.planes.rows > 0) {
+        p.kernel = ResizeGradKernel::Planes;
+    } else if (p.lds = lds_tile(a); p.lds.rows > 0) {
+        p.kernel = ResizeGradKernel::Lds;
+    }
+    return p;
 }
 
 }  // namespace opscv

@@ -399,6 +399,28 @@ def test_upsample_backward_status_codes(aclnn, desc):
     assert _ub(aclnn, desc, grad=(1, 1, 3, 3), osize=(3, 3), sh=1.0, sw=1.0)[2] == "copy"
 
 
+def test_upsample_backward_variant_is_the_kernel_that_runs(aclnn, desc):
+    """opscvExecutorVariant names the kernel, by the same rules as the launch: incoming rows in registers, a rectangle in LDS
+    (channels last; planes that the rows kernel leaves), neither.  Traffic measured on one is not reported for another."""
+    f16, f32 = aclnn.ACL_FLOAT16, aclnn.ACL_FLOAT
+
+    def variant(dt, planes, small, large, align=False):
+        st, _, name = _ub(aclnn, desc, grad=(1, planes) + large, out=(1, planes) + small, osize=large, isize=(1, planes) + small,
+                          dt=dt, align=align, sh=0.0, sw=0.0)
+        assert st == 0
+        return name
+
+    assert variant(f16, 64, (1080, 1920), (2160, 3840), True) == "resize_grad_rows"
+    assert variant(f16, 512, (65, 129), (257, 513)) == "resize_grad_rows"
+    assert variant(f32, 64, (100, 100), (450, 450)) == "resize_grad_rows"
+    assert variant(f32, 512, (56, 56), (224, 224)) == "resize_grad_lds"
+    assert variant(f16, 512, (100, 100), (100, 700)) == "resize_grad_lds"
+    assert variant(f16, 64, (100, 100), (601, 601)) == "resize_grad_gather"
+    assert _ub(aclnn, desc, grad=(1, 200, 300, 3), out=(1, 100, 150, 3), osize=(200, 300), isize=(1, 100, 150, 3),
+               fmt=aclnn.ACL_FORMAT_NHWC, sh=0, sw=0)[2] == "resize_grad_lds"
+    assert aclnn.variant_revision("resize_grad_rows") > 0
+
+
 def _gs3(aclnn, desc, inp=(2, 1, 1, 3, 3), grid=(2, 1, 2, 2, 3), out=(2, 1, 1, 2, 2), dt=None, gdt=None, odt=None,
          interp=0, pad=0, align=False, fmt=None, ofmt=None, **kw):
     dt = aclnn.ACL_FLOAT if dt is None else dt

@@ -275,13 +275,26 @@ struct ResizeGradPlan {
     LdsTile lds;
 };
 
+// Few elements that visit few: done before a wavefront of the rows kernel has its weights and its first rows, by a lane an
+// element of the gather.  Rows / gather in graphs of 64 calls, microseconds: bf16 49 planes of 10x20 from 11x23 3.9 / 2.5, 35 of 21x187
+// from 31x281 4.5 / 3.9, fp16 83 of 8x36 from 6x29 3.6 / 2.4, 144 of 9x196 from 11x245 4.7 / 4.0, fp32 7 of 51x51 from 56x57 3.9 / 2.9,
+// 125 of 14x70 by two 4.6 / 4.1, bf16 622 of 45x5 from 91x11 6.1 / 5.0, 4 of 32x18 by 2.5 4.7 / 4.1, fp16 25 of 127x137 by 0.6 4.8 / 4.2;
+// beyond fp16 421 of 9x62 by two 5.0 / 5.0, 960 of 3x173 from 3x191 4.9 / 5.2, bf16 477 of 6x123 from 10x215 5.4 / 6.0, fp32 3171 of
+// 3x32 from 6x65 5.9 / 6.1, 20 of 116x284 by 1.25 6.1 / 7.2, by 2.5 fp16 2 of 145x132 5.0 / 5.0, 55 of 61x69 5.9 / 7.1.
+inline bool gather_takes_few(const ResizeGradArgs& a)
+{
+    const double elements = (double)a.N * (double)a.C * (double)a.Hs * (double)a.Ws;
+    const double visits = 4.0 / ((double)a.scale_h * (double)a.scale_w);  // of an outgoing element
+    return elements <= 450e3 && ((visits <= 18.5 && elements * visits <= 3e6) || (visits <= 26.0 && elements * visits <= 0.95e6));
+}
+
 inline ResizeGradPlan resize_grad_plan(const ResizeGradArgs& a)
 {
     ResizeGradPlan p;
     if (a.user_scales) {
         p.kernel = ResizeGradKernel::Scales;
     } else if (p.rows = rows_plan(a); p.rows.ok) {
-        p.kernel = ResizeGradKernel::Rows;
+        p.kernel = gather_takes_few(a) ? ResizeGradKernel::Gather : ResizeGradKernel::Rows;
     } else if (p.planes = plane_tile(a); p.planes.rows > 0) {
         p.kernel = ResizeGradKernel::Planes;
     } else if (p.lds = lds_tile(a); p.lds.rows > 0) {

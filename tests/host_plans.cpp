@@ -72,6 +72,13 @@ int resize_grad_rows(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t H
     return p.ok ? 1 : 0;
 }
 
+// kernel of a call: 1 rows, 2 planes, 3 LDS tiles, 4 gather
+int resize_grad_kernel(int elem, int64_t planes, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int align, int64_t* out)
+{
+    out[0] = (int64_t)resize_grad_plan(resize_grad_args(elem, planes, Hs, Ws, Hd, Wd, align)).kernel;
+    return 1;
+}
+
 // most rows, and columns, an outgoing element may visit in the rows kernel
 int resize_grad_rows_visits(int64_t* out)
 {

@@ -45,6 +45,11 @@ def resize_grad_rows(dtype, planes, small, large, align=False):
     return _call("resize_grad_rows", 3, dtype, planes, *small, *large, int(align))
 
 
+def resize_grad_kernel(dtype, planes, small, large, align=False):
+    """"rows", "planes", "lds" or "gather": the kernel that the resize gradient of dense planes on a 16-byte boundary runs."""
+    return (None, "rows", "planes", "lds", "gather")[_call("resize_grad_kernel", 1, dtype, planes, *small, *large, int(align))[0]]
+
+
 def resize_grad_rows_visits():
     """Most rows, and columns, of the incoming gradient that an outgoing element may visit in the rows kernel."""
     out = (ctypes.c_int64 * 1)()

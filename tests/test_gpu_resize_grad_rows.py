@@ -11,13 +11,13 @@ pytestmark = pytest.mark.gpu
 # planes, whole and cut; runs of 2, 4, 6, 8 and 10 columns, wider than the plane too; growth by three, whose integer
 # coordinates three outgoing rows may visit; nine and ten rows (corners aligned, growth by four); a lane's two units; shrinking;
 # two to 64 rows a wavefront; growth by 4.7
-CASES = [((2, 3, 129, 259), (43, 65)), ((5, 7, 28, 27), (14, 9)), ((3, 50, 13, 11), (7, 4)), ((9, 40, 9, 5), (4, 5)),
+CASES = [((2, 3, 129, 259), (43, 65)), ((5, 170, 28, 27), (14, 9)), ((3, 700, 13, 11), (7, 4)), ((9, 2000, 9, 5), (4, 5)),
          ((1, 2, 193, 195), (65, 65)), ((2, 2, 20, 80), (5, 20)), ((1, 3, 64, 64), (16, 16)), ((1, 1, 259, 1021), (65, 256)),
-         ((1, 2, 31, 100), (77, 250)), ((1, 1, 5, 6), (40, 37)), ((1, 1, 1, 1), (9, 70)), ((1, 1, 2, 3), (1, 1)),
+         ((1, 24, 31, 100), (77, 250)), ((3, 120, 5, 6), (40, 37)), ((8, 100, 1, 1), (9, 70)), ((1, 1, 2, 3), (1, 1)),
          ((13, 150, 34, 40), (67, 33)), ((1, 400, 90, 130), (45, 128)), ((3, 7, 98, 78), (21, 17))]
 # growth by five, eleven rows, columns or both
-FIVE = [(False, (2, 5, 75, 325), (15, 65)), (True, (1, 3, 66, 321), (14, 65)), (False, (1, 3, 200, 40), (40, 8)), (True, (30, 1, 161, 43), (33, 43)),
-        (True, (1, 2, 17, 326), (33, 66)), (False, (1, 1, 505, 500), (101, 100))]
+FIVE = [(False, (2, 5, 75, 325), (15, 65)), (True, (1, 3, 66, 321), (14, 65)), (False, (1, 3, 200, 40), (40, 8)), (True, (40, 1, 161, 43), (33, 43)),
+        (True, (3, 100, 17, 326), (33, 66)), (False, (1, 1, 505, 500), (101, 100))]
 
 
 def _check(oracle, device, aclnn, dtype, align, gs, small):
@@ -44,15 +44,14 @@ def _check(oracle, device, aclnn, dtype, align, gs, small):
 @pytest.mark.parametrize("align", [False, True])
 @pytest.mark.parametrize("gs,small", CASES)
 def test_rows(oracle, device, aclnn, dtype, align, gs, small):
-    # rows of a wavefront, two units a lane, rows visited; None where another kernel takes it
-    plan = host_plans.resize_grad_rows(dtype, gs[0] * gs[1], small, gs[2:], align)
-    assert plan is not None or small[1] < 4 or align and 1 in small + gs[2:]
+    assert host_plans.resize_grad_kernel(dtype, gs[0] * gs[1], small, gs[2:], align) == "rows" or small[1] < 4 or align and 1 in small + gs[2:]
     _check(oracle, device, aclnn, dtype, align, gs, small)
 
 
 @pytest.mark.parametrize("dtype", I.DTYPES)
 @pytest.mark.parametrize("align,gs,small", FIVE)
 def test_growth_by_five(oracle, device, aclnn, dtype, align, gs, small):
+    assert host_plans.resize_grad_kernel(dtype, gs[0] * gs[1], small, gs[2:], align) == "rows"
     assert host_plans.resize_grad_rows(dtype, gs[0] * gs[1], small, gs[2:], align)[2] == 12
     _check(oracle, device, aclnn, dtype, align, gs, small)
 
@@ -61,5 +60,5 @@ def test_a_row_refused_behind_others(oracle, device, aclnn):
     """growth by a little less than four, eight visits but for row 2060 of 2354, which rounding gives nine: the wavefronts of 16
     rows that hold it have stored twelve when they find out, and have taken the weights of eight more"""
     gs, small = (1, 27, 9412, 64), (2354, 257)
-    assert host_plans.resize_grad_rows("fp16", 27, small, gs[2:]) == (16, 0, 8)
+    assert host_plans.resize_grad_kernel("fp16", 27, small, gs[2:]) == "rows" and host_plans.resize_grad_rows("fp16", 27, small, gs[2:]) == (16, 0, 8)
     _check(oracle, device, aclnn, "fp16", False, gs, small)

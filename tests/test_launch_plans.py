@@ -87,6 +87,20 @@ def test_resize_gradient_of_odd_rows_takes_the_faster_of_two_kernels(dtype, plan
     assert (P.resize_grad_planes(dtype, planes, small, large) is not None) == (tiles < gather)
 
 
+# (type, planes, small, large, microseconds by rows and by the gather): measured in graphs of 64 calls
+FEW = [("bf16", 49, (10, 20), (11, 23), 3.9, 2.5), ("bf16", 35, (21, 187), (31, 281), 4.5, 3.9), ("fp16", 83, (8, 36), (6, 29), 3.6, 2.4),
+       ("fp16", 570, (11, 13), (16, 19), 4.3, 3.2), ("bf16", 807, (14, 5), (21, 7), 4.3, 3.1), ("fp16", 144, (9, 196), (11, 245), 4.7, 4.0),
+       ("fp32", 7, (51, 51), (56, 57), 3.9, 2.9), ("fp16", 125, (14, 70), (28, 140), 4.6, 4.1), ("bf16", 477, (6, 123), (10, 215), 5.4, 6.0),
+       ("bf16", 622, (45, 5), (91, 11), 6.1, 5.0), ("bf16", 4, (32, 18), (80, 45), 4.7, 4.1), ("fp16", 25, (127, 137), (76, 83), 4.8, 4.2),
+       ("fp32", 3171, (3, 32), (6, 65), 5.9, 6.1), ("fp32", 20, (116, 284), (145, 355), 6.1, 7.2), ("fp16", 55, (61, 69), (152, 172), 5.9, 7.1),
+       ("fp32", 1, (45, 190), (180, 760), 6.6, 7.6)]
+
+
+@pytest.mark.parametrize("dtype,planes,small,large,rows,gather", FEW)
+def test_resize_gradient_of_few_elements_takes_the_faster_kernel(dtype, planes, small, large, rows, gather):
+    assert P.resize_grad_kernel(dtype, planes, small, large) == ("gather" if gather < rows else "rows")
+
+
 @pytest.mark.parametrize("align", [False, True])
 def test_resize_gradient_rows_hold_what_an_element_visits(align):
     """growth by four and five, where rounding adds a row or column to 2 / scale: the visits of every element, stepped in single

@@ -13,10 +13,14 @@ constexpr int kGridTile = 16;  // square: a lane per grid point of 256
 constexpr int kGridTileThreads = kGridTile * kGridTile;
 
 // Few points are bound by the lines that a CU's loads touch, one wavefront's channel after the other: workgroups of a wavefront
-// bring them to four times as many CUs.  256 / 64 threads, grid gradient alone: bicubic fp32 10x54x32x24 -> 62x46 (28520 points)
-// 47.8 / 41.0 us, 13x8x24x42 -> 20x36 16.8 / 14.9, bilinear bf16 8x52x32x32 -> 61x61 9.9 / 8.5, fp16 3x39x61x51 9.1 / 8.2; beyond,
-// with more wavefronts than two a CU, it depends: 27x51x32x48 (41472 points) 9.9 / 10.8, bicubic 21x5x85x85 -> 45x45 (42525) 12.4 /
-// 11.2, 24x49x42x79 (79632) 15.5 / 19.8.  (A wavefront for either sum of 64 points instead: 47.6 / 48.4 on the first.)
+// bring them to four times as many CUs, neighbours on one XCD (in turn over all of them every XCD's L2 fetches most of the planes:
+// fp32 1x155x72x88 -> 69x84 17.4 us with 256 threads, 20.7 in turn, 16.8 so, fp16 16x111x27x50 -> 18x33 16.9 / 18.3 / 14.5, fp32
+// 12x68x44x46 12.4 / 12.4 / 9.0).  256 / 64 threads, grid gradient alone: bicubic fp32 10x54x32x24 -> 62x46 (28520 points) 47.8 / 41.0
+// us, 2x256x56x80 -> 101x145 at random 359 / 208, bilinear bf16 8x52x32x32 -> 61x61 9.9 / 8.5, fp32 1x79x133x238 at random 42.3 / 25.4;
+// 130 draws 1.17 and 1.29 times as fast, four of them slower, one large plane after the other in smooth grids: bicubic fp32 1x200x152x184
+// 181 / 193, fp16 1x201x72x88 -> 112x136 102 / 110.  Beyond, with more wavefronts than two a CU, it depends (measured in turn over
+// the XCDs): 27x51x32x48 (41472 points) 9.9 / 10.8, bicubic 21x5x85x85 -> 45x45 (42525) 12.4 / 11.2, 24x49x42x79 (79632) 15.5 / 19.8.
+// (A wavefront for either sum of 64 points instead: 47.6 / 48.4 on the first.)
 constexpr int64_t kGridSpreadPoints = 32768;
 constexpr int kGridSpreadThreads = 64;
 

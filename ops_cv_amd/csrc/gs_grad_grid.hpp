@@ -18,7 +18,7 @@ struct Grid2Params {
     int32_t C, H, W, Ho, Wo;
     int32_t pad, align;
     int32_t blocks_per_item;  // points in rows: see gs2d_grid_gradient_block
-    uint32_t pieces;          // in tiles: how many, and how they are numbered
+    uint32_t pieces;          // in tiles: how many, and how they are numbered; in rows: workgroups dealt out by XCD, 0: in turn
     FastDiv by_item, by_tiles_x;
     int64_t total;            // points of the batch
 };
@@ -26,7 +26,7 @@ struct Grid2Params {
 struct Grid2Launch {
     bool ok = false, tiled = false;
     Grid2Params p{};
-    int64_t blocks = 0;  // of kGridTileThreads
+    int64_t blocks = 0;  // of as many threads as grid2_launch was asked for
 };
 
 inline Grid2Launch grid2_launch(const GradGatherArgs& a, int threads = kGridTileThreads)
@@ -50,6 +50,10 @@ inline Grid2Launch grid2_launch(const GradGatherArgs& a, int threads = kGridTile
         g.blocks = (g.p.total + threads - 1) / threads;
         const int64_t per_item = a.points / threads;
         g.p.blocks_per_item = (a.points % threads == 0 && a.N % 8 == 0 && per_item <= INT32_MAX) ? (int32_t)per_item : 0;
+        if (threads == kGridSpreadThreads && g.p.blocks_per_item == 0 && g.blocks <= INT32_MAX - 8) {
+            g.p.pieces = (uint32_t)g.blocks;
+            g.blocks = (g.blocks + 7) / 8 * 8;
+        }
     }
     g.ok = g.blocks <= INT32_MAX;
     return g;
@@ -98,6 +102,11 @@ __device__ __forceinline__ void gs2d_grid_gradient_block(uint32_t block_index, c
         if (p.blocks_per_item > 0) {
             const uint32_t xcd = block_index & 7u, i = block_index >> 3;
             block = ((i / (uint32_t)p.blocks_per_item) * 8u + xcd) * (uint32_t)p.blocks_per_item + i % (uint32_t)p.blocks_per_item;
+        } else if (p.pieces > 0) {  // XCD k takes the k-th eighth of the workgroups, as in tiles
+            block = (block_index & 7u) * ((p.pieces + 7u) / 8u) + (block_index >> 3);
+            if (block >= p.pieces) {
+                return;
+            }
         }
         idx = (int64_t)block * THREADS + threadIdx.x;
         if (idx >= p.total) {

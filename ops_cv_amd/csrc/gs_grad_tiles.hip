@@ -80,6 +80,9 @@ struct GridToo<3> {
     Grid3Params p;
 };
 
+// the points of a workgroup of the grid's gradient
+static_assert(kBinThreads == kGridTileThreads && kBinThreads == kChunkPoints3, "a lane a point in the bin kernel's workgroups");
+
 // GRID: 0: no gradient of the grid; of planes 1 points in rows, 2 in tiles; of volumes 1 a channel's loads at a time, 2 four's
 template <typename T, int DIM, int INTERP, int GRID>
 __global__ __launch_bounds__(kBinThreads) void gs_tiles_bin_kernel(const T* __restrict__ grid, uint32_t* __restrict__ ws,

@@ -171,6 +171,41 @@ def test_volumes(oracle, device, aclnn, dtype, pad, interp, xs, out, spots):
     _check(aclnn, oracle, device, dtype, interp, pad, xs, out, grid.reshape((xs[0],) + out + (3,)), rng)
 
 
+# Both gradients, that of the grid by workgroups behind the bins of the same launch: points of planes in 16 x 16 tiles, which end
+# beside the grid's edges, and in rows; nearest; of volumes the loads of four channels together and, from 262144 points on, of one
+BOTH = [(0, (3, 3, 300, 290), (256, 257)), (0, (3, 7, 261, 190), (199, 209)), (0, (3, 2, 33, 95), (50, 61)), (0, (5, 1, 37, 43), (60, 33)),
+        (1, (8, 3, 97, 130), (70, 99)), (0, (2, 3, 5, 9, 17), (8, 9, 12)), (0, (2, 9, 8, 16, 16), (10, 15, 16)),
+        (0, (9, 3, 33, 32, 32), (29, 32, 33)), (1, (3, 2, 17, 25, 33), (17, 25, 33))]
+
+
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("pad", [0, 1, 2])
+@pytest.mark.parametrize("interp,xs,out", BOTH)
+def test_both_gradients_in_one_launch(oracle, device, aclnn, dtype, pad, interp, xs, out):
+    import torch
+    rng = np.random.default_rng(4640 + pad)
+    points = int(np.prod(out))
+    group, _, tiles = host_plans.gradient_tiles(dtype, interp, pad, xs, points)[:3]
+    assert group == xs[0] and tiles * 48 <= 40 << 10  # the bins leave room for the grid's workgroups
+    if len(xs) == 4:
+        in_tiles = interp == 0 and xs[2] * xs[3] > 32768
+        assert (host_plans.grid_gradient_tiles(dtype, interp, xs[0], xs[2:], out) is not None) == in_tiles
+        backward, reference = aclnn.grid_sampler2d_backward, oracle.grid_sampler2d_backward
+        grid = I.affine_grid(rng, xs[0], *out)
+    else:
+        backward, reference = aclnn.grid_sampler3d_backward, oracle.grid_sampler3d_backward
+        axes = [(2 * np.arange(k) + 1) / k - 1 for k in out]
+        z, y, x = np.meshgrid(*axes, indexing="ij")
+        grid = np.stack([x, y, z], axis=-1)[None] * rng.uniform(0.9, 1.1, (xs[0], 1, 1, 1, 3)) + rng.normal(0, 0.02, (xs[0],) + out + (3,))
+    x, g, go = (I.cast_np(v.astype(np.float32), dtype) for v in (rng.standard_normal(xs), grid, rng.standard_normal(xs[:2] + out)))
+    ref = reference(go, x, g, interp, pad, False, dtype=I.oracle_code(dtype))
+    with aclnn.option("gs3d_grad_variant", 3 if len(xs) == 5 else 0):
+        got = backward(*(I.to_torch(v, dtype, device) for v in (go, x, g)), interp, pad, False)
+    torch.cuda.synchronize()
+    for a, b in zip(got, ref):
+        assert np.array_equal(np.ascontiguousarray(I.from_torch(a, dtype)).view(np.uint8), np.ascontiguousarray(b).view(np.uint8))
+
+
 # elements with contributions of several cells, as many as a lane, a wavefront by counting and a wavefront by merging put in
 # order: on two elements of a wavefront, and on more than six
 @pytest.mark.parametrize("dtype", ["fp32", "fp16"])

@@ -234,10 +234,11 @@ def test_groups_of_items_in_a_graph(device, aclnn, n, plane, tiles):
 
 
 # the grid gradient of few points, by workgroups of one wavefront: a wavefront's points of two items, an item's workgroups on one
-# XCD, eighths of the workgroups that are not as many on every one, the most points of that launch and one row more
+# XCD, the most points of that launch and one row more, eighths of the workgroups that are not as many on every one
 @pytest.mark.parametrize("dtype", ["fp32", "fp16"])
 @pytest.mark.parametrize("interp", [0, 2])
-@pytest.mark.parametrize("xs,out", [((3, 5, 9, 11), (7, 13)), ((8, 3, 12, 10), (16, 8)), ((3, 11, 20, 31), (37, 43)), ((8, 9, 20, 31), (64, 64)), ((8, 9, 20, 31), (65, 64))])
+@pytest.mark.parametrize("xs,out", [((3, 5, 9, 11), (7, 13)), ((8, 3, 12, 10), (16, 8)), ((8, 9, 20, 31), (64, 64)), ((8, 9, 20, 31), (65, 64)),
+                                    ((3, 11, 20, 31), (37, 43))])
 def test_grid_gradient_of_few_points(oracle, device, aclnn, dtype, interp, xs, out):
     import torch
     rng = np.random.default_rng(4099 + interp)

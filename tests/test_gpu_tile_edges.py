@@ -181,3 +181,36 @@ def test_shrinking_images(oracle, device, aclnn, dtype, align):
         got = aclnn.upsample_bilinear2d(I.to_torch(x, dtype, device), out, align, channels_last=True)
         torch.cuda.synchronize()
         assert _same(I.from_torch(got, dtype), ref), (xs, out)
+
+
+# (type, planes, small, large, kernel): what resize_grad_rows.hip leaves.  Planes kernel: fp32 rows whose units of 16 bytes are
+# estimated at more than two a lane (planes of 42 to 63 columns that grow by three and four), tiles of 8 rows and of 16,
+# walked in turn and not, cut off at the bottom; few elements of 16-bit planes of up to three columns; more than 2^18 rows, with one,
+# two and eight columns past whole tiles.  Tiles in LDS: growth by more than five along a row, rows of 16 and of 32 bits
+LEFT = [("fp32", 2, (13, 56), (52, 224), "planes"), ("fp32", 17, (33, 63), (66, 190), "planes"), ("fp32", 4309, (7, 61), (15, 244), "planes"),
+        ("fp32", 1501, (40, 55), (20, 220), "planes"), ("fp32", 5201, (33, 3), (20, 4), "planes"), ("fp16", 4099, (33, 3), (129, 12), "planes"),
+        ("bf16", 1337, (96, 2), (336, 8), "planes"), ("fp16", 621, (50, 1), (200, 2), "planes"), ("bf16", 5201, (33, 3), (20, 4), "planes"),
+        ("fp16", 1, (2**18 + 3, 66), (2**19 + 9, 131), "planes"), ("bf16", 1, (2**18 + 3, 65), (2**19 + 9, 129), "planes"),
+        ("fp32", 1, (2**18 + 3, 72), (3 * 2**18 + 2, 216), "planes"),
+        ("fp16", 301, (40, 100), (40, 700), "lds"), ("fp32", 40, (55, 60), (55, 301), "lds"), ("bf16", 64, (37, 200), (28, 1240), "lds")]
+
+
+@pytest.mark.parametrize("dtype,planes,small,large,kernel", LEFT)
+def test_resize_gradient_left_by_rows(oracle, device, aclnn, dtype, planes, small, large, kernel):
+    import torch
+    assert host_plans.resize_grad_kernel(dtype, planes, small, large) == kernel
+    rng = np.random.default_rng(5190)
+    g32 = np.resize(rng.standard_normal(1000003).astype(np.float32), (1, planes) + large)
+    g32[0, 0, 0, -1], g32[0, -1, 3, -2 if large[1] > 2 else 0], g32[0, planes // 2, -1, 0] = np.inf, -np.inf, np.nan
+    g = I.cast_np(g32, dtype)
+    ref = oracle.upsample_bilinear2d_backward(g, small, False, dtype=I.oracle_code(dtype))
+    t = I.to_torch(g, dtype, device)
+    for offset in (0, 1) if planes > 1 and kernel == "planes" else (0,):  # a view that starts off the 16-byte grid
+        base = torch.empty(t.numel() + offset, dtype=t.dtype, device=device)
+        view = base[offset:].view(t.shape)
+        view.copy_(t)
+        got = aclnn.upsample_bilinear2d_backward(view, (1, planes) + small, False)
+        torch.cuda.synchronize()
+        got, a, b = I.from_torch(got, dtype), I.as_f32(I.from_torch(got, dtype), dtype), I.as_f32(ref, dtype)
+        numbers = ~np.isnan(b)
+        assert np.array_equal(np.isnan(a), ~numbers) and _same(got[numbers], ref[numbers]), offset

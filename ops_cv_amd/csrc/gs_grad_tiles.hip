@@ -53,13 +53,18 @@ constexpr uint32_t kNoPlace = 0xFFFFFFFFu;
 constexpr uint32_t kCountedRun = 64;
 // Crowded elements are put in order by a lane each where more than kFewCrowded lanes of a wavefront have one of up to kSerialMost
 // contributions, otherwise one after the other by the wavefront, up to 64 * kRankedRegs contributions by counting.  A lane also
-// adds up to kSerialMost by itself where more lanes than kFewCrowded have as many.  Without the counting and with 192
+// adds up to kSerialMost by itself where more lanes than kFewCrowded have as many.  Longer ones are a lane each where the
+// wavefront has kSideBySide times as many contributions as they: border padding piles points up on all elements of a row, and
+// 32 of 88 contributions one after the other take the wavefront longer than a lane each (fp16 3x4x222x157 border, rotated 119 / 63
+// us, 2x8x609x495 -> 649x527 377 / 178, volumes 6x13x17x11x45 -> 17x11x46 314 / 131; with 8 instead of 12 the elements of
+// some hundred on a corner are a lane's too, fp32 5x2x167x179 78 for 53; with 24 3x6x286x208 remains at 131, 77 so).  Without the counting and with 192
 // contributions / with it and 192 / 96 / 64 / 48 (and 16 lanes), microseconds of the whole gradient: fp32 reflection
 // 5x4x27x54x51 81 / 66 / 67 / 67 / 66, fp16 3x3x31x45x16 50 / 41 / 41 / 39 / 49, fp32 9x22x25x16x29 86 / 66 / 66 / 67 / 74,
 // planes, fp16 border 29x4x378x312 183 / 162 / 162 / 164 / 163; 22 such gradients together 1.10, 1.10, 1.10 and 1.05 times as
 // fast, and 1.09 with 3 lanes instead of 6.
 constexpr uint32_t kSerialMost = 64;
 constexpr int kFewCrowded = 6;
+constexpr uint32_t kSideBySide = 12;
 constexpr int kRankedRegs = 2;
 
 // What the bin kernel takes along: nothing, or the gradient of the grid by workgroups behind its own.
@@ -418,6 +423,7 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
     const int32_t tile_y = tile_yz - tile_z * p.tiles_y;
     const int32_t x0 = tile_x * S::kX, y0 = tile_y * S::kY, z0 = tile_z * S::kZ;
     const int32_t phase = (DIM == 3 && p.items_per_core > 1) ? phase_of(n, p) : 0;
+    auto wave_sum = [&](uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)wave_scan(v), 63); };
     auto waves_before = [&](uint32_t* all) { return sums_before<kWaves>(s_scan, wave, lane, all); };
 
     uint32_t* s_before = s_seg;
@@ -662,7 +668,8 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
             }
         }
         const bool few = __builtin_popcountll(__builtin_amdgcn_ballot_w64(fits)) <= kFewCrowded;
-        const bool alone = fits && !few && len <= kSerialMost;
+        const uint32_t all = wave_sum(fits ? len : 0u);
+        const bool alone = fits && ((!few && len <= kSerialMost) || len * kSideBySide <= all);
         if (alone) {
             merge_alone([&](uint32_t i, uint32_t k) { s_sorted[sorted + i] = (uint16_t)(k & kLowBits); });
         }
@@ -924,7 +931,9 @@ __global__ __launch_bounds__(GradTile<DIM>::kThreads, 4) void gs_tiles_gather_ke
         }
         int lane = t & 63;
         asm volatile("" : "+v"(lane));  // what follows is rare: none of it is worked out ahead
-        const bool together = crowded && (len > kSerialMost || ((sorted & only) != kNoKey && __builtin_popcountll(rare) <= kFewCrowded));
+        const uint32_t all = wave_sum(crowded ? len : 0u);
+        const bool together = crowded && ((len > kSerialMost && len * kSideBySide > all) ||
+                                          ((sorted & only) != kNoKey && __builtin_popcountll(rare) <= kFewCrowded));
         if (crowded && !together) {
             if (only != kNoKey) {
                 for (uint32_t i = 0; i < len; i++) {

@@ -228,6 +228,28 @@ def test_crowded_elements(oracle, device, aclnn, dtype, elements, xs, out, count
     _check(aclnn, oracle, device, dtype, 0, 1, xs, out, grid.reshape((xs[0],) + out + (dim,)), rng)
 
 
+# all elements of a row with more contributions than a wavefront takes one after the other, as border padding makes them: a lane
+# each; of one element in it as many again as of a dozen others: by the wavefront
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("xs,out", [((8, 3, 32, 64), (46, 80)), ((3, 9, 48, 64), (50, 64)), ((6, 2, 8, 16, 16), (10, 14, 14))])
+@pytest.mark.parametrize("each,most", [(40, 0), (70, 0), (36, 400)])
+@pytest.mark.parametrize("edge", [False, True])
+def test_crowded_rows(oracle, device, aclnn, dtype, xs, out, each, most, edge):
+    rng = np.random.default_rng(4630)
+    points, dim = int(np.prod(out)), len(out)
+    assert host_plans.gradient_tiles(dtype, 0, 1, xs, points) is not None
+    at = rng.uniform(0, 1, (xs[0], points, dim)) * (np.array(xs[:1:-1]) - 1)
+    for n in range(xs[0]):
+        free = iter(rng.permutation(points))
+        # beyond the edge, where border padding takes them to the row of the edge, or around a row inside
+        around = np.array([0, -3, -2] if edge else [0, 3, 2])[:dim]
+        for x in range(15):
+            for _ in range(each + (most if x == n + 2 else 0)):
+                at[n, next(free)] = around + np.append(x + rng.uniform(0.1, 0.9), rng.uniform(-0.9, 0.9, dim - 1))
+    grid = (2 * at + 1) / np.array(xs[:1:-1]) - 1
+    _check(aclnn, oracle, device, dtype, 0, 1, xs, out, grid.reshape((xs[0],) + out + (dim,)), rng)
+
+
 def test_special_grid_values(oracle, device, aclnn):
     """points that are no numbers, infinite or far outside have no tile; on and beside the edges of tiles and of the plane"""
     rng = np.random.default_rng(4600)

@@ -484,17 +484,13 @@ int64_t gs3d_grad_gather_words(const GridSampler3DGradArgs& a)
         // 55; 8 x 16x40x40 307 / 72).  Smaller grids seldom have one and cost half as much in slots (19 / 35 us), nor do
         // grids of less than a point per two voxels (13x2x13x41x52 from 9x30x39 28 / 50, 15 of 24 such calls slower sorted;
         // from 0.8 points per voxel on 192 of 243 are faster sorted, on average by 2.7 times).
-        // Large batches have such an item from fewer points on, smooth grids of half to one point per two voxels (0.45 to 0.5) where
-        // border padding has 20000 points an item or reflection 32768, and items below 8192 points from 0.7 points per voxel on.
-        // Slots / sorting: border 16x1x53x39x42 from 41x30x32 199 / 69, 20x4x23x76x27 from 18x59x21 194 / 70, but 8x4x10x52x75 from
-        // 8x40x57 28 / 36, 16x4x18x42x29 from 14x33x23 28 / 40, and on the line 8x3 of 28336 points 36 / 38, 20x8 of 27200 94 / 105;
-        // reflection 16x1x34x58x56 from 27x46x44 275 / 109, 12x6 of 35424 points 277 / 109, but 24x1x8x92x67 from 6x73x53 55 / 68, and
-        // on the line 16x6x59x19x75 from 46x15x58 89 / 114; small items 32x2x11x19x36 border 160 / 40, 20x16x9x51x16 reflection 200 / 71,
-        // but 24x12x29x19x22 from 24x16x19 39 / 52, 22x6x25x23x20 from 21x19x17 33 / 64, and on the line 24x6x21x23x22 from 19x20x20
-        // 35 / 59.  (Of grids that leave the faces alone every one is faster in slots: scaled by 0.8 24x8 of 5797 points 34 / 79.)
-        const bool batch = a.N * points >= 131072;
-        const bool piles = a.pad != 0 && ((points >= 8192 && 2 * points >= vol) || (batch && points < 8192 && 10 * points >= 7 * vol) ||
-                                          (batch && points >= (a.pad == 1 ? 20000 : 32768) && 20 * points >= 9 * vol));
+        // Batches have such an item more often than single ones: from 131072 points and 0.45 points per voxel on they are sorted.
+        // Which side is faster is the grid's doing; slots / sorting over 37 such calls of fewer than 8192 points an item or 0.5 per
+        // voxel: affine grids beyond the volume 3.9 times as fast sorted, near the identity 2.8, none slower; points at random 2.1, seven
+        // slower by up to 1.3 times; grids that stay 3 % inside 0.79, all slower, by up to 1.8 times.  fp16 24x6x41x42x39 from 32x33x31
+        // border 620 / 168 near the identity, inside 92 / 129; fp32 48x9x13x17x33 from 10x13x26 171 / 77, inside 42 / 61, at random 62 /
+        // 83; fp32 15x7x9x54x40 from 7x42x31 reflection 153 / 63, inside 35 / 56.  Below the line 13x2x27716 voxels at 0.38 border 29 / 47.
+        const bool piles = a.pad != 0 && ((points >= 8192 && 2 * points >= vol) || (a.N * points >= 131072 && 20 * points >= 9 * vol));
         // the slots kernels keep an item on one XCD: one or two large items leave most of the chip idle (one item of
         // 41664 points 34 / 24, of 84600 - / 28; four of 46110 33 / 28; three of 15028 20 / 24; but grids scaled by 0.8, twice as
         // many points a tile, one item of 41280 points and one channel 31 / 42, four channels 34 / 33, four items of 45486 38 / 50)

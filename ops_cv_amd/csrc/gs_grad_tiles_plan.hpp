@@ -58,7 +58,11 @@ struct TilesLayout {   // offsets in 32-bit words within an item's scratch
 // Border padding piles points up on few elements, which the gather kernel's wavefronts add together: no limit of contributions
 // (fp16 8x4x256x256 from 360x360 131 / 97 / 100, with the limit 133).  Volumes' borders have elements of 50 to 90 here and
 // there, which the gather kernel's wavefronts put in order by counting: gradients with a limit of 48 / 96 / 192 / none, fp16
-// reflection 11x2x42x18x88 119 / 97 / 97 / 97, bf16 border 3x4x24x61x31 59 / 51 / 52 / 52.
+// reflection 11x2x42x18x88 119 / 97 / 97 / 97, bf16 border 3x4x24x61x31 59 / 51 / 52 / 52.  But border padding piles affine grids
+// up on all of a face, whose tiles outlast the launch unless there is other work, and then few elements of points at random:
+// limit of 48 / 96 over 40 borders of up to 48 items times channels, affine 1.36 times as fast with 48, near the identity 1.01, at
+// random 0.89 (fp32 3x4x40x16x17 62 / 174, 1x10x19x48x26 78 / 138, at random fp16 10x3x16x38x38 99 / 64); 72 / 96 over 13 of up to
+// 150 1.13, 0.97 and 1.01 (24x6x22x22x10 102 / 151); reflection, 38 calls, 1.02, 0.97 and 0.89 (fp16 3x6x21x67x39 at random 163 / 104).
 struct CrowdedTile {
     uint32_t points, contributions;
 };
@@ -69,7 +73,8 @@ inline CrowdedTile crowded_tile(const GradGatherArgs& a)
         return {a.dim == 3 ? 10240u : 12288u, any};
     }
     if (a.dim == 3) {
-        return {a.N * a.C <= 48 ? 1920u : 6144u, 96u};
+        const bool few = a.N * a.C <= 48;
+        return {few ? 1920u : 6144u, a.pad != 1 ? 96u : (few ? 48u : 72u)};
     }
     return {a.C > 8 ? 3072u : 5120u, a.pad == 1 ? any : 48u};
 }

@@ -192,6 +192,22 @@ int grid_gradient_tiles(int elem, int64_t interp, int64_t N, int64_t H, int64_t 
     return p.ok ? 1 : 0;
 }
 
+// points and contributions of an element beyond which a tile is the crowded tiles' kernel's
+int crowded_tiles(int elem, int64_t interp, int64_t pad, int64_t N, int64_t C, int64_t dim, int64_t* out)
+{
+    GradGatherArgs a;
+    a.elem = (Elem)elem;
+    a.dim = (int)dim;
+    a.interp = (int)interp;
+    a.pad = (int)pad;
+    a.N = N;
+    a.C = C;
+    const CrowdedTile t = crowded_tile(a);
+    out[0] = t.points;
+    out[1] = t.contributions;
+    return 1;
+}
+
 // nearest resize by runs of rows: rows of a run, pieces of a row, elements of a piece, bytes of LDS; 0 where another kernel
 // takes it.  `in_chunks`: source rows on the 16-byte grid
 int nearest_rows(int elem, int64_t N, int64_t C, int64_t Hs, int64_t Ws, int64_t Hd, int64_t Wd, int64_t last, int64_t in_chunks,

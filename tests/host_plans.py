@@ -88,6 +88,11 @@ def gradient_tiles(dtype, interp, pad, shape, points, per_core=1):
     return _call("gradient_tiles", 5, dtype, interp, pad, *shape, points, per_core)
 
 
+def crowded_tiles(dtype, interp, pad, n, c, dim):
+    """(points, contributions of an element) beyond which a tile of the sorting input gradient is a crowded one."""
+    return _call("crowded_tiles", 2, dtype, interp, pad, n, c, dim)
+
+
 def grid_gradient_tiles(dtype, interp, n, plane, out):
     """(tiles, workgroups) of the 2-D sampler's grid gradient, None where its points are taken in rows."""
     return _call("grid_gradient_tiles", 2, dtype, interp, n, *plane, *out)

@@ -200,6 +200,17 @@ def test_sorting_takes_the_faster_of_lists_and_tiles(dtype, interp, pad, shape, 
     assert (P.gradient_tiles(dtype, interp, pad, shape, points) is not None) == (tiles < lists)
 
 
+# (type, padding, items, channels, limit that is the faster, microseconds with it and with the other): volumes, affine grids under
+# border padding, of 48 and 96, of 72 and 96; points at random under reflection
+CROWDED = [("fp32", 1, 3, 4, 48, 62, 174), ("fp32", 1, 1, 10, 48, 78, 138), ("bf16", 1, 8, 1, 48, 92, 167), ("fp32", 1, 24, 6, 72, 102, 151),
+           ("bf16", 1, 13, 5, 72, 117, 151), ("fp16", 2, 3, 6, 96, 104, 163), ("fp16", 2, 2, 16, 96, 88, 132)]
+
+
+@pytest.mark.parametrize("dtype,pad,n,c,limit,faster,slower", CROWDED)
+def test_crowded_tiles_of_volumes_have_the_faster_limit(dtype, pad, n, c, limit, faster, slower):
+    assert P.crowded_tiles(dtype, 0, pad, n, c, 3)[1] == limit and faster < slower
+
+
 def test_gradient_tiles_fit_lds_and_the_launch():
     """2048 tiles of 32 x 16 (16 x 8 x 4) and 2047 blocks of 1024 points an item; a block more for chunks that start at a shift"""
     assert P.gradient_tiles("fp32", 0, 0, (1, 1, 16 * 2048, 32), 2000)[2] == 2048

@@ -57,7 +57,8 @@ constexpr uint32_t kCountedRun = 64;
 // wavefront has kSideBySide times as many contributions as they: border padding piles points up on all elements of a row, and
 // 32 of 88 contributions one after the other take the wavefront longer than a lane each (fp16 3x4x222x157 border, rotated 119 / 63
 // us, 2x8x609x495 -> 649x527 377 / 178, volumes 6x13x17x11x45 -> 17x11x46 314 / 131; with 8 instead of 12 the elements of
-// some hundred on a corner are a lane's too, fp32 5x2x167x179 78 for 53; with 24 3x6x286x208 remains at 131, 77 so).  Without the counting and with 192
+// some hundred on a corner are a lane's too, fp32 5x2x167x179 78 for 53; with 24 3x6x286x208 remains at 131, 77 so;
+// points at random close together lose, 11x10x246x80 -> 331x107 154 / 165).  Without the counting and with 192
 // contributions / with it and 192 / 96 / 64 / 48 (and 16 lanes), microseconds of the whole gradient: fp32 reflection
 // 5x4x27x54x51 81 / 66 / 67 / 67 / 66, fp16 3x3x31x45x16 50 / 41 / 41 / 39 / 49, fp32 9x22x25x16x29 86 / 66 / 66 / 67 / 74,
 // planes, fp16 border 29x4x378x312 183 / 162 / 162 / 164 / 163; 22 such gradients together 1.10, 1.10, 1.10 and 1.05 times as

@@ -200,12 +200,16 @@ inline TilesPlan tiles_plan_of(const GradGatherArgs& a)
 // 6x12x136x184 -> 115x156 47 / 34).
 // Not where a single tile outlasts the launch: a workgroup adds the points that border padding piles up on a corner (a few in
 // a hundred of an item) a thousand at a time, in lists a wavefront per element does, and with one or two items of many points
-// and few channels nothing else is left to do meanwhile.  Bilinear, both gradients, lists / tiles: 1x3x384x552 -> 461x663 86 /
-// 158, 2x10x152x224 -> 212x312 84 / 130, 2x3x248x464 64 / 105, 1x1x376x632 67 / 97, but points at random 2x4x578x571 263 / 207; up
-// to 16384 points 2x6x61x54 39 / 28, bf16 1x11x191x198 -> 97x100 39 / 27, 1x4x32x56 -> 45x79 42 / 34; from three items on
-// 5x2x405x480 260 / 207, 4x2x301x505 268 / 170, 3x1x520x609 -> 605x708 674 / 380, 3x4x47x86 40 / 22, and at its worst 3x4x265x296
-// 89 / 121, fp16 5x3x232x296 129 / 154.  Nearest, which adds no weights, 1x2x368x624 47 / 39, 2x1x408x600 -> 792x1164 540 / 153,
-// 3x2x304x576 144 / 77, 1x6x32x48 -> 44x66 20 / 20.
+// and few channels nothing else is left to do meanwhile.  Which side is faster is the grid's doing; bilinear, both gradients, lists /
+// tiles for rotations of up to 30 degrees (five grids), points at random, flow fields that stay inside:
+//   1x3x384x552 -> 461x663        75 / 105  142 / 152   61 / 26     3x4x265x296                62 / 67    99 / 75    48 / 25
+//   2x3x248x464                   80 / 83    98 / 80    46 / 22     fp16 5x3x232x296           76 / 76   110 / 78    50 / 28
+//   2x4x578x571                  110 / 124  248 / 199  110 / 49     3x1x520x609 -> 605x708    198 / 180  282 / 213  123 / 66
+//   fp16 1x6x180x170 (30600)      38 / 33    47 / 42    31 / 21     4x2x301x505               108 / 102  159 / 108   77 / 38
+//   2x6x61x54                     34 / 24    36 / 21    29 / 15     5x2x405x480               176 / 137  219 / 150  113 / 57
+// Over 182 calls of three to nine items tiles are 1.06, 1.37 and 1.64 times as fast, rotated ones slower in 64 (fp32 3x1x271x180 44 / 73
+// at worst); over 13 of one and two items beyond 32768 points 0.89, 1.15 and 1.82, over 27 below 1.27, 1.32 and 1.50.  Nearest, which
+// adds no weights, 1x2x368x624 47 / 39, 2x1x408x600 -> 792x1164 540 / 153, 3x2x304x576 144 / 77, 1x6x32x48 -> 44x66 20 / 20.
 // Nor for many channels of volumes (12x31x18x62x20 142 / 159, 3x26x27x18x31 42 / 46; nearest 23x10x28x67x49 114 / 130,
 // 5x28x9x71x45 35 / 39; 7x19x30x20x91 175 / 151, nearest 9x6x52x46x37 67 / 55).
 // Not in planes and volumes of many tiles: every block of points clears, sums and writes a count per tile, and from 1706 tiles
@@ -242,7 +246,7 @@ inline bool tiles_are_faster(const GradGatherArgs& a)
     if (a.interp == 0 && a.elem == Elem::BF16 && (a.H > 64 || a.W > 64) && a.points >= elements) {
         return false;
     }
-    return a.pad != 1 || a.interp == 1 || a.N >= 3 || a.points <= 16384 || a.N * (a.C + 4) >= 48;
+    return a.pad != 1 || a.interp == 1 || a.N >= 3 || a.points <= 32768 || a.N * (a.C + 4) >= 48;
 }
 
 inline TilesPlan tiles_plan(const GradGatherArgs& a)

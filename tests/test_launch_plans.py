@@ -192,7 +192,10 @@ TILES = [("fp32", 0, 0, (8, 3, 479, 637), 479 * 637, 178, 86), ("fp16", 0, 2, (1
          ("fp32", 0, 1, (2, 3, 248, 464), 248 * 464, 64, 105), ("fp32", 0, 1, (1, 1, 376, 632), 376 * 632, 67, 97),
          ("fp32", 0, 1, (2, 6, 61, 54), 61 * 54, 39, 28), ("bf16", 0, 1, (1, 11, 191, 198), 97 * 100, 39, 27),
          ("fp32", 0, 1, (3, 1, 520, 609), 605 * 708, 674, 380), ("fp32", 0, 1, (5, 2, 405, 480), 405 * 480, 260, 207),
-         ("fp32", 1, 1, (1, 2, 368, 624), 368 * 624, 47, 39), ("fp32", 1, 1, (2, 1, 408, 600), 792 * 1164, 540, 153)]
+         ("fp32", 1, 1, (1, 2, 368, 624), 368 * 624, 47, 39), ("fp32", 1, 1, (2, 1, 408, 600), 792 * 1164, 540, 153),
+         # points at random, and rotated
+         ("fp32", 0, 1, (3, 4, 265, 296), 265 * 296, 99, 75), ("fp16", 0, 1, (5, 3, 232, 296), 232 * 296, 110, 78),
+         ("fp16", 0, 1, (1, 6, 180, 170), 180 * 170, 38, 33), ("fp32", 0, 1, (1, 3, 384, 552), 461 * 663, 75, 105)]
 
 
 @pytest.mark.parametrize("dtype,interp,pad,shape,points,lists,tiles", TILES)

@@ -19,8 +19,9 @@
 // tile that a point reaches; all that is scattered happens in LDS.
 //
 // fp32 8x3x479x637 from as many points (rotations of up to 30 degrees), operands from memory: lists through global memory
-// (gs_grad_gather.hip) 188 us in six kernels, here bin 21, gather 73 and 4.6 for a list of crowded tiles that is empty (bin 19
-// and gather 69 before there was one: where a point lies in its tile, and scalar registers that the way out takes).  Bin: 34 us with an LDS atomic a point, which the
+// (gs_grad_gather.hip) 188 us in six kernels, here bin 21, gather 71 and 4.5 for a list of crowded tiles that is empty (bin 19
+// and gather 69 before there was one: where a point lies in its tile, and scalar registers that the way out takes).  With the gradient
+// of the grid in its launch bin takes 53.5, 21 and 33 as two launches: they hardly overlap.  Bin: 34 us with an LDS atomic a point, which the
 // 64 lanes of a wavefront on one tile take in turn, 20 with a run of lanes entered at once.  Gather is bound by its chain of
 // steps, not by a unit: 550 vector, 400 scalar and 49 LDS instructions a wavefront (34 us of issue), and seven waits for memory
 // or the other wavefronts (segments, records, points; counts, starts, lists, keys) at two workgroups per CU.  Without fetching,

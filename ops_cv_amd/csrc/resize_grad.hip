@@ -488,7 +488,8 @@ __global__ __launch_bounds__(kGradThreads) void resize_grad_lds_kernel(const TI*
 }
 
 // Planes whose elements grow by up to four a side (at most eight visited rows and columns) and that resize_grad_rows.hip leaves
-// (planes of 1 GiB, 2^18 rows): the rectangle stays in the element type and comes by asynchronous copies.
+// (rows_plan: mostly fp32 planes of 42 to 63 columns, and of up to three columns): the rectangle stays in the element type and
+// comes by asynchronous copies.
 //
 // A workgroup owns 64 outgoing columns by 16 or 8 outgoing rows, a wavefront every fourth of the rows.  The row segments
 // the tile visits are copied from the 16-byte boundary before their first byte to the one after their last (the bytes

@@ -207,12 +207,16 @@ struct RowsPlan {
     int64_t blocks = 0;    // padded for the XCD mapping of the kernel
 };
 
-// Taken wherever it can: growth by up to five, planes (rows from 2^18 on and planes of 1 GiB are left to the kernels above).
+// Planes that grow by up to five.  Left to the kernels above: more than 2^18 rows; planes of 1 GiB and more, or, of fewer than 64
+// columns, of 2 GiB over the planes that a wavefront may reach (span); up to three columns of fewer than 2^19 elements; and rows whose
+// units of 16 bytes are estimated at more than two a lane.  That estimate counts whole planes where a wavefront has 64 columns
+// of them, some of which it cuts: fp32 planes of 55 to 63 columns that grow by three, 48 to 63 by 3.5, 42 to 63 by four, 28 to 63 by 4.5
+// are left although what they load fits (71 units at most by four).
 // Against them, medians of three runs, device time in microseconds before / with it: bf16 8x64x65x129 from 257x513 58 / 44, fp32 81 / 57,
 // fp16 64x128 from 256x512 53 / 41; growth by two fp32 4x16x270x480 43 / 32, fp16 16x64x56x56 29 / 17, 4x16x1080x1920 437 / 415, bf16
 // 512x32x14x14 43 / 17; growth by 1.1 fp32 2000 planes of 82x424 315 / 164, fp16 182 / 143; shrunk by 0.5 120 / 104 and 30 / 29 (64
-// planes of 400x600), by 0.35 28 / 28.  Growth by four with aligned corners, where an element visits nine rows and columns, had no
-// kernel but the gather: fp16 85 planes of 539x108 206 / 54.8.  Over 260 random shapes (1 to 20000 planes of 2 to 1500 columns, growth by
+// planes of 400x600), by 0.35 28 / 28.  Growth by four with aligned corners, where an element visits nine rows and columns: fp16 85
+// planes of 539x108 206 (tiles of two rows in LDS) / 54.8.  Over 260 random shapes (1 to 20000 planes of 2 to 1500 columns, growth by
 // 0.25 to 4) 1.57 times as fast, none slower by more than a microsecond.
 inline RowsPlan rows_plan(const ResizeGradArgs& a)
 {

@@ -250,6 +250,18 @@ def test_crowded_rows(oracle, device, aclnn, dtype, xs, out, each, most, edge):
     _check(aclnn, oracle, device, dtype, 0, 1, xs, out, grid.reshape((xs[0],) + out + (dim,)), rng)
 
 
+# border padding of one and two items around the most points that are taken by tiles there, rotated so that points pile up
+@pytest.mark.parametrize("dtype", I.DTYPES)
+@pytest.mark.parametrize("xs,out,taken", [((1, 6, 190, 180), (180, 182), True), ((2, 2, 190, 180), (180, 182), True), ((1, 6, 180, 190), (182, 181), False)])
+def test_border_padding_of_few_items(oracle, device, aclnn, dtype, xs, out, taken):
+    rng = np.random.default_rng(4640)
+    assert (host_plans.gradient_tiles(dtype, 0, 1, xs, out[0] * out[1]) is not None) == taken
+    y, x = np.meshgrid(np.linspace(-1, 1, out[0]), np.linspace(-1, 1, out[1]), indexing="ij")
+    turn = np.array([[0.9, -0.5], [0.6, 1.1]])
+    grid = np.broadcast_to(np.stack([x, y], -1) @ turn, (xs[0],) + out + (2,)) + rng.uniform(-0.02, 0.02, (xs[0], 1, 1, 2))
+    _check(aclnn, oracle, device, dtype, 0, 1, xs, out, grid, rng)
+
+
 def test_special_grid_values(oracle, device, aclnn):
     """points that are no numbers, infinite or far outside have no tile; on and beside the edges of tiles and of the plane"""
     rng = np.random.default_rng(4600)
